@@ -339,8 +339,8 @@ int lgx_copy_image(const lgx_image *src, lgx_image *dst, lgx_stream_t stream);
 
 /* Number of gather launch shapes (lgx_gather_params.tile indexes them). */
 int lgx_gather_tiles(void);
-/* A launch shape: info[0..4] = slice pixels per workgroup in x and y, waves
- * per SIMD the registers are held to (1 = the compiler's choice), pipelined
+/* A launch shape: info[0..4] = slice pixels of four waves in x and y (a wave
+ * holds info[0] x info[1] / 4 of them), waves per SIMD the registers are held to (1 = the compiler's choice), pipelined
  * step loop (0/1), swizzled levels (0/1).  A swizzling shape re-lays the
  * pyramid levels whose texel columns the lanes of a wave share modulo
  * F = grid >> level (F >= 2, power-of-two grid) into column-swizzled copies
@@ -370,8 +370,9 @@ int lgx_gather_batch_create(const lgx_gather_params *p, const void *const *works
 int lgx_gather_batch_set_tile(lgx_gather_batch *b, int32_t tile);
 /* Logical blocks (tiles x slices) of all views together. */
 int64_t lgx_gather_batch_blocks(const lgx_gather_batch *b);
-/* workgroups: persistent workgroups (rounded up to a multiple of 8);
- * 0 = one per logical block.  Workgroups take blocks from per-XCD counters
+/* workgroups: persistent workgroups of four waves (the launch has as many
+ * waves, its workgroups rounded up to a multiple of 8); 0 = as many waves as
+ * the chip holds, or fewer if the blocks are fewer.  Workgroups take blocks from per-XCD counters
  * that the launch zeroes first (with a kernel: capturable), so launches of
  * ONE batch must not overlap in time (different batches may). */
 int lgx_gather_batch_launch(const lgx_gather_batch *b, int32_t workgroups, lgx_stream_t stream);
@@ -392,7 +393,7 @@ typedef struct {
 typedef struct {
   int32_t dirs, max_steps, levels, grid, sampler, footprint_dirs;
   int32_t tile;       /* gather launch shape */
-  int32_t workgroups; /* persistent gather workgroups, 0 = one per block */
+  int32_t workgroups; /* persistent gather workgroups, 0 = as many as the chip holds */
   int32_t grid_y;     /* interleave pattern height (lgx_gather_params), <= 0 = grid */
   int32_t chunks;     /* views, in ascending pixel count, are gathered in this many persistent launches
                          (<= 0: 4); each chunk's U-Nets run before the next chunk's gather */

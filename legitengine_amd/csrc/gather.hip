@@ -2,8 +2,10 @@
 // running SSVGI/indirectLighting.frag:114-272 as a gfx950 compute kernel.
 //
 // Design (MI355X):
-//  * Thread mapping per 4x4 interleave slice: every workgroup covers a tile
-//    of ONE slice (all pixels with the same pattern index), so a wavefront's
+//  * Thread mapping per 4x4 interleave slice: every workgroup covers 64
+//    pixels of ONE slice (all with the same pattern index); its waves take
+//    the directions of these pixels in turn (split_waves: how many waves),
+//    and their shares are added through LDS in direction order.  A wavefront's
 //    64 lanes share the Hammersley offsets, i.e. the screen directions and
 //    the geometric step offsets.  Those come from per-slice tables in the
 //    workspace (scalar loads), and all lanes march parallel rays 4 px apart:
@@ -35,6 +37,11 @@ namespace lgx {
 // Buffer resource word 3 of the gfx9 family (raw, untyped 32-bit access).
 static constexpr int kBufferConfig = 0x00020000;
 
+// SPLIT kernels (all but the step-counting ones): the waves of a workgroup
+// share the directions of 64 pixels.  At most kMaxSplit waves; the shares
+// of kRound directions (3 x 64 values each) are in LDS at a time.
+static constexpr int kMaxSplit = 8, kRound = 16, kShare = 3 * 64;
+
 template <class T> struct GatherArgs {
   T inv_vp[16];
   T cam[3];
@@ -65,6 +72,8 @@ template <class T> struct GatherArgs {
   int *step_counts;
   int *hit_counts;  // COUNT only, may be null
   int tile_w, tile_h, tiles_x, n_blocks;
+  int round;  // SPLIT kernels: directions between two ordered sums
+  int split;  // host side: waves sharing a pixel's directions (0: one wave does all of them)
   int occ;   // host side: which register allocation to launch
   int pipe;  // host side: which step loop to launch
   int swz;   // host side: the fine levels are column-swizzled copies
@@ -274,21 +283,37 @@ template <class T> LGX_D size_t point_index(T sx, T sy, int lw, int lh, int pitc
 // T: per-step arithmetic; A: accumulation of the slice contributions and of
 // the direction sum (float/float, double/double, or float/double).
 // One workgroup's share: logical block b (slice k = b % (grid grid_y), tile b / (grid grid_y)).
+// part: LDS for the shares of a.round directions (kShare values each).
+// Bound by VALU issue and by the latency of each step's dependent texel
+// fetch, which only enough waves hide; one wave per pixel block and all its
+// directions left 1024 waves (one per SIMD) for a 256 x 256 image: 153 us
+// there with 16 directions, 57 us with the directions over 8 waves; at 1080p
+// with 32 directions 2.90 -> 2.69 ms (a shorter tail).
 // ARGS: GatherArgs<T> as the kernel's argument, or in constant memory
 // (address space 4, the multi-view kernel's per-view table): either way the
 // compiler reads its fields as scalars.
 template <class T, class A, int SAMPLER, int RFMT, int NFMT, bool COUNT, bool PIPE, bool SWZ, class ARGS>
-LGX_D void gather_block(ARGS &a, const uint32_t b) {
+LGX_D void gather_block(ARGS &a, const uint32_t b, A *part) {
+  constexpr bool SPLIT = !COUNT;
+  // SPLIT: this lane's pixel of the tile, the wave (uniform) and the waves of the workgroup
+  const uint32_t px = SPLIT ? threadIdx.x & 63u : threadIdx.x;
+  const int wave = SPLIT ? (int)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
+  const int waves = SPLIT ? (int)(blockDim.x >> 6) : 1;
   const int g2 = a.grid * a.grid_y;
   const int k = (int)(b % (uint32_t)g2);
   const int t = (int)(b / (uint32_t)g2);
   const int kx = k % a.grid, ky = k / a.grid;
-  const int lx = (t % a.tiles_x) * a.tile_w + (int)(threadIdx.x % (uint32_t)a.tile_w);
-  const int ly = (t / a.tiles_x) * a.tile_h + (int)(threadIdx.x / (uint32_t)a.tile_w);
-  if (lx >= a.lcells_x || ly >= a.lcells_y) return;
+  const int lx = (t % a.tiles_x) * a.tile_w + (int)(px % (uint32_t)a.tile_w);
+  const int ly = (t / a.tiles_x) * a.tile_h + (int)(px / (uint32_t)a.tile_w);
   const int sx = a.sx0 + lx, sy = a.sy0 + ly;
-  const int x = sx * a.grid + kx, y = sy * a.grid_y + ky;
-  if (x < a.rx0 || x >= a.rx1 || y < a.ry0 || y >= a.ry1) return;
+  int x = sx * a.grid + kx, y = sy * a.grid_y + ky;
+  const bool mine = lx < a.lcells_x && ly < a.lcells_y && x >= a.rx0 && x < a.rx1 && y >= a.ry0 && y < a.ry1;
+  if (SPLIT) {  // every lane reaches the barriers: a lane without a pixel reads one in the frame and marches nothing
+    x = mine ? x : a.rx0;
+    y = mine ? y : a.ry0;
+  } else if (!mine) {
+    return;
+  }
 
   const Vec3<T> cam{a.cam[0], a.cam[1], a.cam[2]};
   const T cx = T(x) + T(0.5), cy = T(y) + T(0.5);  // gl_FragCoord (:116)
@@ -313,7 +338,8 @@ LGX_D void gather_block(ARGS &a, const uint32_t b) {
   A sum0 = 0, sum1 = 0, sum2 = 0;
   int step_total = 0, hit_total = 0;
 
-  for (int d = 0; d < a.D; d++) {
+  // the march along direction d: its share of the pixel's sum
+  auto direction = [&](const int d, A &o0, A &o1, A &o2) {
     // the direction and its reciprocals (the host's correctly rounded 1 / d)
     const T dx = dirs[4 * d], dy = dirs[4 * d + 1], idx = dirs[4 * d + 2], idy = dirs[4 * d + 3];
     // :180-183 tangent of the slice through the offset point (the quotient
@@ -609,13 +635,49 @@ LGX_D void gather_block(ARGS &a, const uint32_t b) {
     // :268; for a power-of-two D the quotient is the product with 1 / D
     // (exact), otherwise the IEEE division
     if (a.d_pow2) {
-      sum0 += A(2) * L0 * A(a.inv_d);
-      sum1 += A(2) * L1 * A(a.inv_d);
-      sum2 += A(2) * L2 * A(a.inv_d);
+      o0 = A(2) * L0 * A(a.inv_d);
+      o1 = A(2) * L1 * A(a.inv_d);
+      o2 = A(2) * L2 * A(a.inv_d);
     } else {
-      sum0 += A(2) * L0 / A(a.D);
-      sum1 += A(2) * L1 / A(a.D);
-      sum2 += A(2) * L2 / A(a.D);
+      o0 = A(2) * L0 / A(a.D);
+      o1 = A(2) * L1 / A(a.D);
+      o2 = A(2) * L2 / A(a.D);
+    }
+  };
+
+  if constexpr (SPLIT) {
+    // The waves take the directions of a round in turn and leave each one's
+    // share in LDS; wave 0 adds them in direction order, so the sum is the
+    // one a single wave forms, bit for bit.
+    for (int d0 = 0; d0 < a.D; d0 += a.round) {
+      const int nd = min(a.round, a.D - d0);
+      if (mine)
+        for (int i = wave; i < nd; i += waves) {
+          A o0, o1, o2;
+          direction(d0 + i, o0, o1, o2);
+          A *q = part + i * kShare + px;
+          q[0] = o0;
+          q[64] = o1;
+          q[128] = o2;
+        }
+      __syncthreads();
+      if (wave == 0)
+        for (int i = 0; i < nd; i++) {
+          const A *q = part + i * kShare + px;
+          sum0 += q[0];
+          sum1 += q[64];
+          sum2 += q[128];
+        }
+      __syncthreads();  // before the next round's (or block's) shares overwrite these
+    }
+    if (wave != 0 || !mine) return;
+  } else {
+    for (int d = 0; d < a.D; d++) {
+      A o0, o1, o2;
+      direction(d, o0, o1, o2);
+      sum0 += o0;
+      sum1 += o1;
+      sum2 += o2;
     }
   }
 
@@ -644,8 +706,9 @@ LGX_D void gather_block(ARGS &a, const uint32_t b) {
 // compiler's choice); the launch shapes offer 1 and 8.  PIPE: the step loop
 // that overlaps fetches with arithmetic (Hi-Z sampler).
 template <class T, class A, int SAMPLER, int RFMT, int NFMT, bool COUNT, int OCC, bool PIPE = false, bool SWZ = false>
-__global__ __launch_bounds__(256, OCC) void gather_kernel(const GatherArgs<T> a) {
-  gather_block<T, A, SAMPLER, RFMT, NFMT, COUNT, PIPE, SWZ>(a, xcd_remap(blockIdx.x, (uint32_t)a.n_blocks));
+__global__ __launch_bounds__(COUNT ? 256 : 64 * kMaxSplit, OCC) void gather_kernel(const GatherArgs<T> a) {
+  extern __shared__ __align__(16) unsigned char s_part[];
+  gather_block<T, A, SAMPLER, RFMT, NFMT, COUNT, PIPE, SWZ>(a, xcd_remap(blockIdx.x, (uint32_t)a.n_blocks), (A *)s_part);
 }
 
 // Column-swizzled copies of the fine pyramid levels for the SWZ kernels.
@@ -695,9 +758,10 @@ __global__ __launch_bounds__(256) void swizzle_jobs_kernel(const SwzJob *__restr
 // takes blocks from the other XCDs' chunks in turn (the counters only grow,
 // so every block is taken once), and ends when all eight are exhausted.
 template <class T, class A, int SAMPLER, int RFMT, int NFMT, int OCC, bool PIPE, bool SWZ>
-__global__ __launch_bounds__(256, OCC) void gather_multi_kernel(const GatherArgs<T> *__restrict__ views,
+__global__ __launch_bounds__(64 * kMaxSplit, OCC) void gather_multi_kernel(const GatherArgs<T> *__restrict__ views,
                                                            const uint32_t *__restrict__ first, int n_views,
                                                            uint32_t *next) {
+  extern __shared__ __align__(16) unsigned char s_part[];
   __shared__ uint32_t s_item;
   // the views' arguments are only read: constant memory, so their fields
   // (with a uniform view index) become scalar loads, as a kernel argument's are
@@ -718,7 +782,7 @@ __global__ __launch_bounds__(256, OCC) void gather_multi_kernel(const GatherArgs
       __syncthreads();  // every wave has read s_item before lane 0 overwrites it
       if (it >= c1) break;
       while (v + 1 < n_views && it >= first[v + 1]) v++;  // items of one chunk only grow
-      gather_block<T, A, SAMPLER, RFMT, NFMT, false, PIPE, SWZ>(cviews[v], it - first[v]);
+      gather_block<T, A, SAMPLER, RFMT, NFMT, false, PIPE, SWZ>(cviews[v], it - first[v], (A *)s_part);
     }
   }
 }
@@ -917,30 +981,26 @@ template <class T> static void frame_constants(const lgx_gather_params *p, Gathe
 
 template <class T, class A, int SAMPLER, int RFMT, int NFMT>
 static hipError_t launch_gather(const GatherArgs<T> &a, bool count, hipStream_t s) {
-  dim3 grid((unsigned)a.n_blocks), block(256);
   // the FP32 Hi-Z gather has every variant; the others run the default one
   constexpr bool kAll = sizeof(T) == 4 && sizeof(A) == 4 && SAMPLER == LGX_SAMPLER_HIZ_POINT;
   constexpr int O8 = kAll ? 8 : 1;
-  if (count)
-    hipLaunchKernelGGL((gather_kernel<T, A, SAMPLER, RFMT, NFMT, true, 1>), grid, block, 0, s, a);
-  else if (kAll && a.swz) {  // (make_args sets swz only for this gather)
-    if (a.occ == 8 && a.pipe)
-      hipLaunchKernelGGL((gather_kernel<T, A, SAMPLER, RFMT, NFMT, false, O8, kAll, kAll>), grid, block, 0, s, a);
-    else if (a.occ == 8)
-      hipLaunchKernelGGL((gather_kernel<T, A, SAMPLER, RFMT, NFMT, false, O8, false, kAll>), grid, block, 0, s, a);
-    else if (a.pipe)
-      hipLaunchKernelGGL((gather_kernel<T, A, SAMPLER, RFMT, NFMT, false, 1, kAll, kAll>), grid, block, 0, s, a);
-    else
-      hipLaunchKernelGGL((gather_kernel<T, A, SAMPLER, RFMT, NFMT, false, 1, false, kAll>), grid, block, 0, s, a);
-  } else if (kAll && a.occ == 8 && a.pipe)
-    hipLaunchKernelGGL((gather_kernel<T, A, SAMPLER, RFMT, NFMT, false, O8, kAll>), grid, block, 0, s, a);
-  else if (kAll && a.occ == 8)
-    hipLaunchKernelGGL((gather_kernel<T, A, SAMPLER, RFMT, NFMT, false, O8>), grid, block, 0, s, a);
-  else if (kAll && a.pipe)
-    hipLaunchKernelGGL((gather_kernel<T, A, SAMPLER, RFMT, NFMT, false, 1, kAll>), grid, block, 0, s, a);
-  else
-    hipLaunchKernelGGL((gather_kernel<T, A, SAMPLER, RFMT, NFMT, false, 1>), grid, block, 0, s, a);
-  return hipGetLastError();
+  auto launch = [&](auto kern) {
+    const unsigned threads = a.split ? 64u * (unsigned)a.split : 256u;
+    const size_t lds = a.split ? (size_t)a.round * kShare * sizeof(A) : 0;
+    hipLaunchKernelGGL(kern, dim3((unsigned)a.n_blocks), dim3(threads), lds, s, a);
+    return hipGetLastError();
+  };
+  if (count) return launch(gather_kernel<T, A, SAMPLER, RFMT, NFMT, true, 1>);
+  if (kAll && a.swz) {  // (make_args sets swz only for this gather)
+    if (a.occ == 8 && a.pipe) return launch(gather_kernel<T, A, SAMPLER, RFMT, NFMT, false, O8, kAll, kAll>);
+    if (a.occ == 8) return launch(gather_kernel<T, A, SAMPLER, RFMT, NFMT, false, O8, false, kAll>);
+    if (a.pipe) return launch(gather_kernel<T, A, SAMPLER, RFMT, NFMT, false, 1, kAll, kAll>);
+    return launch(gather_kernel<T, A, SAMPLER, RFMT, NFMT, false, 1, false, kAll>);
+  }
+  if (kAll && a.occ == 8 && a.pipe) return launch(gather_kernel<T, A, SAMPLER, RFMT, NFMT, false, O8, kAll>);
+  if (kAll && a.occ == 8) return launch(gather_kernel<T, A, SAMPLER, RFMT, NFMT, false, O8>);
+  if (kAll && a.pipe) return launch(gather_kernel<T, A, SAMPLER, RFMT, NFMT, false, 1, kAll>);
+  return launch(gather_kernel<T, A, SAMPLER, RFMT, NFMT, false, 1>);
 }
 
 template <class T, class A, int SAMPLER>
@@ -952,8 +1012,8 @@ static hipError_t dispatch_fmt(const GatherArgs<T> &a, int rfmt, int nfmt, bool 
   return hipErrorInvalidValue;
 }
 
-// Launch shapes offered to the autotuner: tile_w x tile_h slice pixels per
-// 256-thread workgroup, the occupancy the registers are allocated for (1: the
+// Launch shapes offered to the autotuner: tile_w x tile_h slice pixels of
+// four waves (a wave holds tile_w x tile_h / 4), the occupancy the registers are allocated for (1: the
 // compiler's choice, 6 waves per SIMD; 8: 64 VGPRs with a few spilled set-up
 // values), the step loop (1: fetches overlapped with arithmetic), and the
 // pyramid layout (1: the fine levels read from column-swizzled copies made in
@@ -1059,11 +1119,47 @@ extern "C" int lgx_gather_tile_info(int32_t tile, int32_t *info) {
   return LGX_OK;
 }
 
+// Pixels a gather launch covers.
+static int64_t launch_pixels(const lgx_gather_params *p) {
+  return p->roi[2] > 0 ? (int64_t)p->roi[2] * p->roi[3] : (int64_t)p->width * p->height;
+}
+
+// Waves that share the directions of 64 pixels.  The chip holds 8192 waves of
+// the gather (8 per SIMD); a launch short of that leaves it idle, and one of a
+// few times that ends in a long tail, since a wave lives as long as its
+// slowest ray times its directions.  More waves per pixel repeat the pixel's
+// set-up and wait for each other at the sums, which weighs most with few
+// directions.  Measured, one / two / four / eight waves (16x16 shapes):
+//   256x256, 16 directions            153 / 88 / 62 / 57 us      (1024 waves of pixels)
+//   512x288, 32 directions            620 / 461 / 335 / 299 us   (2304)
+//   512x288, 4 directions, F = 256    513 / 370 / 293 us
+//   1279x719, 8 directions            214 / 198 / 200 us         (14 K)
+//   1920x1080, 32 directions          2899 / 2769 / 2688 / 2866 us (32 K)
+//   1920x1080, 4 directions, F = 256  2644 / 2450 / 2480 us
+//   256x256 crop, 256 directions      18.2 / 9.4 / 5.8 / 5.8 ms
+//   64x64 crop, 256 directions        19.1 / 8.7 / 4.7 / 2.5 ms
+// The trilinear march has a handful of steps a direction, so a direction is
+// mostly set-up and nothing but an idle chip makes a split worth while
+// (1920x1080, 4 directions: 371 / 374 / 406 us; 480x270: 53 / 45 / 38 us).
+static int split_waves(int64_t pixels, int dirs, int sampler) {
+  const int64_t full = 8192, waves = (pixels + 63) / 64;
+  if (sampler == LGX_SAMPLER_TRILINEAR && dirs < 16) {
+    int k = 1;
+    while (k < 4 && 2 * k <= dirs && waves * k < 2 * full) k *= 2;
+    return k;
+  }
+  if (dirs >= 8 && waves * 4 <= full) return 8;
+  if (dirs >= 16 || (dirs >= 4 && waves * 2 < 2 * full)) return 4;
+  return dirs >= 2 ? 2 : 1;
+}
+
+// split: waves per workgroup, each on its share of the directions (0: the
+// step-counting kernels, whose waves hold all directions of their pixels).
 // jobs: the swizzle copies a swizzling launch needs first, into swz_area
 // (swz_layout's size; null: never swizzle)
 template <class T>
 static int make_args(const lgx_gather_params *p, const void *ws, const lgx_gbuffer *g, const lgx_pyramid *pyr,
-                     lgx_image *out, GatherArgs<T> &a, SwzJobs *jobs = nullptr, void *swz_area = nullptr) {
+                     lgx_image *out, GatherArgs<T> &a, int split, SwzJobs *jobs = nullptr, void *swz_area = nullptr) {
   GatherTableShape s = table_shape(p);
   memset(&a, 0, sizeof(a));
   frame_constants<T>(p, a);
@@ -1149,6 +1245,11 @@ static int make_args(const lgx_gather_params *p, const void *ws, const lgx_gbuff
   a.sy0 = a.ry0 / a.grid_y;
   a.lcells_x = (a.rx1 + a.grid - 1) / a.grid - a.sx0;
   a.lcells_y = (a.ry1 + a.grid_y - 1) / a.grid_y - a.sy0;
+  a.split = split;
+  if (split) {  // the shape's 256 slice pixels are four waves'
+    a.tile_h /= 4;
+    a.round = std::min(a.D, kRound);
+  }
   a.tiles_x = (a.lcells_x + a.tile_w - 1) / a.tile_w;
   int tiles_y = (a.lcells_y + a.tile_h - 1) / a.tile_h;
   a.n_blocks = a.tiles_x * tiles_y * s.g2;
@@ -1160,7 +1261,8 @@ static int gather_impl(const lgx_gather_params *p, void *ws, const lgx_gbuffer *
                        lgx_image *out, hipStream_t stream) {
   GatherArgs<T> a;
   SwzJobs jobs;
-  int rc = make_args<T>(p, ws, g, pyr, out, a, &jobs, (char *)ws + swz_offset(p));
+  int rc = make_args<T>(p, ws, g, pyr, out, a, p->step_counts ? 0 : split_waves(launch_pixels(p), p->dirs, p->sampler), &jobs,
+                        (char *)ws + swz_offset(p));
   if (rc != LGX_OK) return rc;
   hipError_t e;
   if (jobs.n) {
@@ -1240,7 +1342,9 @@ struct lgx_gather_batch {
   std::vector<lgx_pyramid> pyr;
   std::vector<lgx_image> out;
   int sampler = 0, rf = 0, nf = 0, tile = 0;
-  uint32_t total = 0;
+  int split = 1, round = 1;  // waves per workgroup; the largest round of the views
+  uint32_t total = 0;   // blocks the workgroups take
+  int64_t shapes = 0;   // tiles of the launch shape's 256 slice pixels
   void *dev = nullptr;  // GatherArgs<float>[n], uint32 first[n + 1], uint32 next[8] (work counters)
   // swizzling shapes: the views' swizzle jobs, then their copy areas
   // (allocated by the first set_tile to such a shape)
@@ -1288,20 +1392,29 @@ static int gather_batch_upload(lgx_gather_batch *b, int tile) {
     b->swz_bytes = off;
   }
   std::vector<SwzJob> jobs;
-  int rows = 1;
+  int rows = 1, dirs = 1, round = 1;
+  int64_t pixels = 0, shapes = 0;
+  for (const lgx_gather_params &q : b->p) {
+    dirs = std::max(dirs, q.dirs);
+    pixels += launch_pixels(&q);
+  }
+  const int split = split_waves(pixels, dirs, b->sampler);
   for (int i = 0; i < n; i++) {
     lgx_gather_params q = b->p[i];
     q.tile = tile;
     SwzJobs vj;
-    int rc = make_args<float>(&q, b->ws[i], &b->g[i], &b->pyr[i], &b->out[i], args[i], swz ? &vj : nullptr,
+    int rc = make_args<float>(&q, b->ws[i], &b->g[i], &b->pyr[i], &b->out[i], args[i], split, swz ? &vj : nullptr,
                               swz ? (char *)b->swz + area[i] : nullptr);
     if (rc != LGX_OK) return rc;
+    round = std::max(round, args[i].round);
     if (swz)
       for (int k = 0; k < vj.n; k++) {
         jobs.push_back(vj.j[k]);
         rows = std::max(rows, vj.j[k].h);
       }
     first[i + 1] = first[i] + (uint32_t)args[i].n_blocks;
+    const GatherArgs<float> &ga = args[i];
+    shapes += (int64_t)ga.tiles_x * ((ga.lcells_y + ga.tile_h * 4 - 1) / (ga.tile_h * 4)) * ga.grid * ga.grid_y;
   }
   if (!jobs.empty()) {
     rc0 = hip_status(hipMemcpy(b->swz, jobs.data(), jobs.size() * sizeof(SwzJob), hipMemcpyHostToDevice));
@@ -1314,7 +1427,10 @@ static int gather_batch_upload(lgx_gather_batch *b, int tile) {
   int rc = hip_status(hipMemcpy(b->dev, blob.data(), blob.size(), hipMemcpyHostToDevice));
   if (rc != LGX_OK) return rc;
   b->tile = tile;
+  b->split = split;
+  b->round = round;
   b->total = first[n];
+  b->shapes = shapes;
   b->njobs = (int)jobs.size();
   b->job_rows = std::min(rows, 4096);
   return LGX_OK;
@@ -1331,34 +1447,23 @@ static hipError_t launch_multi(const lgx_gather_batch *b, unsigned grid, hipStre
   hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(64), 0, s, next, 8);
   // the Hi-Z sampler has the swizzled variants (make_args sets no jobs otherwise)
   constexpr bool kSwz = SAMPLER == LGX_SAMPLER_HIZ_POINT;
+  auto launch = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(64u * (unsigned)b->split), (size_t)b->round * kShare * sizeof(float), s, args,
+                       first, n, next);
+    return hipGetLastError();
+  };
   if (kSwz && b->njobs) {
     hipLaunchKernelGGL(swizzle_jobs_kernel, dim3((unsigned)b->job_rows, (unsigned)b->njobs), dim3(256), 0, s,
                        (const SwzJob *)b->swz);
-    if (occ8 && pipe)
-      hipLaunchKernelGGL((gather_multi_kernel<float, float, SAMPLER, RFMT, NFMT, 8, true, kSwz>), dim3(grid), dim3(256),
-                         0, s, args, first, n, next);
-    else if (occ8)
-      hipLaunchKernelGGL((gather_multi_kernel<float, float, SAMPLER, RFMT, NFMT, 8, false, kSwz>), dim3(grid),
-                         dim3(256), 0, s, args, first, n, next);
-    else if (pipe)
-      hipLaunchKernelGGL((gather_multi_kernel<float, float, SAMPLER, RFMT, NFMT, 1, true, kSwz>), dim3(grid), dim3(256),
-                         0, s, args, first, n, next);
-    else
-      hipLaunchKernelGGL((gather_multi_kernel<float, float, SAMPLER, RFMT, NFMT, 1, false, kSwz>), dim3(grid),
-                         dim3(256), 0, s, args, first, n, next);
-  } else if (occ8 && pipe)
-    hipLaunchKernelGGL((gather_multi_kernel<float, float, SAMPLER, RFMT, NFMT, 8, true, false>), dim3(grid), dim3(256),
-                       0, s, args, first, n, next);
-  else if (occ8)
-    hipLaunchKernelGGL((gather_multi_kernel<float, float, SAMPLER, RFMT, NFMT, 8, false, false>), dim3(grid),
-                       dim3(256), 0, s, args, first, n, next);
-  else if (pipe)
-    hipLaunchKernelGGL((gather_multi_kernel<float, float, SAMPLER, RFMT, NFMT, 1, true, false>), dim3(grid), dim3(256),
-                       0, s, args, first, n, next);
-  else
-    hipLaunchKernelGGL((gather_multi_kernel<float, float, SAMPLER, RFMT, NFMT, 1, false, false>), dim3(grid),
-                       dim3(256), 0, s, args, first, n, next);
-  return hipGetLastError();
+    if (occ8 && pipe) return launch(gather_multi_kernel<float, float, SAMPLER, RFMT, NFMT, 8, true, kSwz>);
+    if (occ8) return launch(gather_multi_kernel<float, float, SAMPLER, RFMT, NFMT, 8, false, kSwz>);
+    if (pipe) return launch(gather_multi_kernel<float, float, SAMPLER, RFMT, NFMT, 1, true, kSwz>);
+    return launch(gather_multi_kernel<float, float, SAMPLER, RFMT, NFMT, 1, false, kSwz>);
+  }
+  if (occ8 && pipe) return launch(gather_multi_kernel<float, float, SAMPLER, RFMT, NFMT, 8, true, false>);
+  if (occ8) return launch(gather_multi_kernel<float, float, SAMPLER, RFMT, NFMT, 8, false, false>);
+  if (pipe) return launch(gather_multi_kernel<float, float, SAMPLER, RFMT, NFMT, 1, true, false>);
+  return launch(gather_multi_kernel<float, float, SAMPLER, RFMT, NFMT, 1, false, false>);
 }
 
 }  // namespace lgx
@@ -1412,13 +1517,21 @@ extern "C" int lgx_gather_batch_set_tile(lgx_gather_batch *b, int32_t tile) {
   return gather_batch_upload(b, tile);
 }
 
-extern "C" int64_t lgx_gather_batch_blocks(const lgx_gather_batch *b) { return b ? (int64_t)b->total : -1; }
+extern "C" int64_t lgx_gather_batch_blocks(const lgx_gather_batch *b) { return b ? b->shapes : -1; }
 
 extern "C" int lgx_gather_batch_launch(const lgx_gather_batch *b, int32_t workgroups, lgx_stream_t stream) {
   if (!b || workgroups < 0) return LGX_EINVAL;
-  uint32_t grid = workgroups > 0 ? (uint32_t)workgroups : b->total;
+  const int64_t asked = workgroups > 0 ? workgroups : b->shapes;
+  if (asked > (1 << 24)) return LGX_EINVAL;
+  // A workgroup asked for is of four waves: the launch has as many waves.  0
+  // asks for one per block; the chip's 8192 resident waves walk them (each
+  // workgroup ends with an attempt at all eight counters: with one workgroup
+  // per block of 64 pixels those attempts took longer than the gather, 17.5
+  // against 8.5 ms for four views of 7 Mpixel).
+  const uint32_t k = (uint32_t)b->split;
+  uint32_t grid = workgroups > 0 ? std::max(1u, (uint32_t)workgroups * 4u / k) : std::min(b->total, 8192u / k);
   grid = (grid + 7) / 8 * 8;  // the XCD chunking needs a multiple of 8
-  if (grid == 0 || grid > (1u << 24)) return LGX_EINVAL;
+  if (grid == 0) return LGX_EINVAL;
   hipStream_t s = (hipStream_t)stream;
   hipError_t e;
   if (b->sampler == LGX_SAMPLER_HIZ_POINT)
