@@ -10,9 +10,10 @@
 //    the geometric step offsets.  Those come from per-slice tables in the
 //    workspace (scalar loads), and all lanes march parallel rays 4 px apart:
 //    coherent pyramid accesses and near-uniform trip counts.
-//  * Exact early exit: the side fade (:220-228) is zero for every sample
-//    outside the open screen rectangle, the ray leaves that convex region
-//    once and never re-enters, so every later step contributes exactly 0.
+//  * Early exit: the side fade (:220-228) is zero for every sample outside
+//    the open screen rectangle, the ray leaves that convex region once and
+//    never re-enters, so every later step contributes exactly 0.  The march
+//    ends at one offset per direction, the border's or the step count's.
 //  * Per step, the sample's world-space delta is evaluated from per-direction
 //    dot products (the ray through q is affine in the step offset before
 //    normalisation), the horizon test uses a monotone pseudo-angle, and the
@@ -47,6 +48,7 @@ template <class T> struct GatherArgs {
   T cam[3];
   T e0[3], ex[3], ey[3];  // unnormalised ray through screen point s: e0 + s.x*ex + s.y*ey
   T W, H, near_step, log_ratio, ambient;
+  T near_min;  // near_step / the offsets' growth
   int w, h, grid, grid_y, cells_x, cells_y, D, S_tab;  // pattern grid x grid_y
   int d_pow2;      // D is a power of two: x / D == x * inv_d exactly
   double inv_d;    // 1 / D
@@ -85,6 +87,12 @@ template <class T> LGX_D T fast_rsqrt(T v);
 template <> LGX_D float fast_rsqrt<float>(float v) { return __builtin_amdgcn_rsqf(v); }
 template <> LGX_D double fast_rsqrt<double>(double v) { return 1.0 / sqrt(v); }
 
+// A uniform value held in a vector register (float).
+template <class T> LGX_D T vec(T v) {
+  if constexpr (sizeof(T) == 4) asm("" : "+v"(v));
+  return v;
+}
+
 template <class T> LGX_D T fma_(T a, T b, T c) { return fma(a, b, c); }
 
 template <class T> LGX_D T fast_rcp(T v);
@@ -110,12 +118,13 @@ template <class T> LGX_D T div_extent(T q, T b, T rb) {
 // evaluated in float).  The hit branch of the march calls it on every horizon
 // rise, where the library routine's handling of infinities and NaNs (which
 // cannot occur there) costs more than the polynomial.
-template <class T> LGX_D T atan2_finite(T y, T x);
-template <> LGX_D double atan2_finite<double>(double y, double x) { return atan2(y, x); }
-template <> LGX_D float atan2_finite<float>(float y, float x) {
+// NONZERO: the caller's vector is not (0, 0).
+template <bool NONZERO> LGX_D double atan2_finite(double y, double x) { return atan2(y, x); }
+template <bool NONZERO> LGX_D float atan2_finite(float y, float x) {
   const float ax = fabsf(x), ay = fabsf(y);
-  const float mx = fmaxf(ax, ay), mn = fminf(ax, ay);
-  const float t = mx > 0.f ? mn * __builtin_amdgcn_rcpf(mx) : 0.f;
+  const bool steep = ay > ax;
+  const float mx = steep ? ay : ax, mn = steep ? ax : ay;
+  const float t = NONZERO || mx > 0.f ? mn * __builtin_amdgcn_rcpf(mx) : 0.f;
   const float s = t * t;
   float p = -0.004054928198456764f;
   p = fmaf(p, s, 0.021864214912056923f);
@@ -126,41 +135,51 @@ template <> LGX_D float atan2_finite<float>(float y, float x) {
   p = fmaf(p, s, -0.33329862356185913f);
   p = fmaf(p, s, 0.9999993443489075f);
   float r = t * p;
-  r = ay > ax ? 1.5707963705062866f - r : r;
+  r = steep ? 1.5707963705062866f - r : r;
   r = x < 0.f ? 3.1415927410125732f - r : r;
   return copysignf(r, y);
 }
 
-// Radiance texel through a buffer resource (32-bit byte offset against a
-// scalar base): the raw load, and its widening to float, so a fetch can be
+// A pyramid level as a structured buffer: the texel index is the buffer
+// index (the hardware scales it by the stride, one instruction less per fetch
+// than a byte offset), the base, pitch and extent are scalars, and an index
+// past the last row reads 0.
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+LGX_D float struct_load_f32(i32x4 r, int index, int offset, int base, int policy) __asm(
+    "llvm.amdgcn.struct.buffer.load.f32");
+LGX_D f32x2 struct_load_f32x2(i32x4 r, int index, int offset, int base, int policy) __asm(
+    "llvm.amdgcn.struct.buffer.load.v2f32");
+LGX_D f32x4 struct_load_f32x4(i32x4 r, int index, int offset, int base, int policy) __asm(
+    "llvm.amdgcn.struct.buffer.load.v4f32");
+LGX_D i32x4 level_rsrc(const void *base, int stride, int texels) {
+  const uint64_t p = (uint64_t)base;
+  return i32x4{(int)(uint32_t)p, (int)((uint32_t)(p >> 32) & 0xffffu) | (stride << 16), texels, kBufferConfig};
+}
+LGX_D float load_depth(i32x4 r, uint32_t ti) { return struct_load_f32(r, (int)ti, 0, 0, 0); }
+
+// Radiance texel: the raw load, and its widening to float, so a fetch can be
 // issued in one step of the march and consumed in the next.
 template <int FMT> struct RadBuf;
 template <> struct RadBuf<LGX_RGBA16F> {
   static constexpr int kBytes = 8;
-  typedef unsigned int Raw __attribute__((ext_vector_type(2)));
-  static LGX_D Raw raw(__amdgpu_buffer_rsrc_t r, uint32_t ti) {
-    return __builtin_amdgcn_raw_buffer_load_b64(r, (int)(ti * 8u), 0, 0);
-  }
-  static LGX_D float4 load(__amdgpu_buffer_rsrc_t r, uint32_t ti) { return decode(raw(r, ti)); }
-  static LGX_D float4 decode(Raw v) {
+  typedef f32x2 Raw;
+  static LGX_D Raw raw(i32x4 r, uint32_t ti) { return struct_load_f32x2(r, (int)ti, 0, 0, 0); }
+  static LGX_D float4 decode(Raw f) {
+    // the whole vector is reinterpreted at once: a bit cast of one element
+    // of a loaded vector (v[i]) compiles to a read of element 0 here
+    typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+    const u32x2 v = __builtin_bit_cast(u32x2, f);
     return make_float4(h2f((uint16_t)(v[0] & 0xffffu)), h2f((uint16_t)(v[0] >> 16)), h2f((uint16_t)(v[1] & 0xffffu)),
                        h2f((uint16_t)(v[1] >> 16)));
   }
 };
 template <> struct RadBuf<LGX_RGBA32F> {
   static constexpr int kBytes = 16;
-  typedef unsigned int Raw __attribute__((ext_vector_type(4)));
-  static LGX_D Raw raw(__amdgpu_buffer_rsrc_t r, uint32_t ti) {
-    return __builtin_amdgcn_raw_buffer_load_b128(r, (int)(ti * 16u), 0, 0);
-  }
-  static LGX_D float4 load(__amdgpu_buffer_rsrc_t r, uint32_t ti) { return decode(raw(r, ti)); }
-  static LGX_D float4 decode(Raw v) {
-    // the whole vector is reinterpreted at once: a bit cast of one element
-    // of a loaded vector (v[i]) compiles to a read of element 0 here
-    typedef float f32x4 __attribute__((ext_vector_type(4)));
-    const f32x4 f = __builtin_bit_cast(f32x4, v);
-    return make_float4(f.x, f.y, f.z, f.w);
-  }
+  typedef f32x4 Raw;
+  static LGX_D Raw raw(i32x4 r, uint32_t ti) { return struct_load_f32x4(r, (int)ti, 0, 0, 0); }
+  static LGX_D float4 decode(Raw f) { return make_float4(f.x, f.y, f.z, f.w); }
 };
 
 // Texel index iy * pitch + ix with the full-rate 24-bit multiply: rows and
@@ -173,53 +192,87 @@ LGX_D uint32_t texel_index(int iy, int pitch, int ix) {
 // The running horizon maximum of a slice side and the test theta <
 // theta_max of :254, without a division per step.  The pseudo-angle
 // p(y, x) = 1 - x / s for y >= 0 and x / s - 1 for y < 0, s = |x| + |y|, is a
-// monotone stand-in for atan2 on (-pi, pi]; it is copysign(s - x, y) / s, so
-// with s > 0, p(y, x) < P is copysign(s - x, y) < s P: a subtraction, a
-// sign copy, a product and a compare per step, the division only when the
-// maximum P is replaced.  Only the order matters: near-ties decide steps
-// whose contribution h(theta, theta_max) vanishes with the gap.  A zero
-// vector has pseudo-angle 0 (atan2(0, 0) = 0) and is never below.
+// monotone stand-in for atan2 on (-pi, pi].  A sample further along the
+// slice lies on the tangent's side of the centre's eye ray (y = r sin(phi -
+// d/2) + rc sin(d/2) for the angles phi >= d of the sample and of the offset
+// point), so its pseudo-angle is (s - x) / s, and it is below P when s - x <
+// s P: a subtraction, a product and a compare per step, the division only
+// when the maximum is replaced.  Only the order matters: near-ties decide
+// steps whose contribution h(theta, theta_max) vanishes with the gap.
 template <class T> struct HorizonMax {
   T P;
+  // the normal-limited horizon: any vector (a zero vector has angle 0)
   LGX_D void set(T y, T x) {
     const T s = fabs(x) + fabs(y);
     P = s > T(0) ? copysign(s - x, y) * fast_rcp(s) : T(0);
   }
   LGX_D bool below(T y, T x) const {
     const T s = fabs(x) + fabs(y);
-    return copysign(s - x, y) < s * P;
+    return s - x < s * P;
+  }
+  // the maximum replaced by a sample below it (so not a zero vector)
+  LGX_D void lower(T y, T x) {
+    const T s = fabs(x) + fabs(y);
+    P = (s - x) * fast_rcp(s);
   }
 };
 
-// x / b for several x over one b, correctly rounded: r = RN(1/b) once (an
-// IEEE division), then per quotient y = RN(x r) and one fused correction
-// with the exact residual x - y b (Markstein), which rounds to the IEEE
-// quotient when r is the correctly rounded reciprocal (checked against the
-// IEEE division for every significand of b, tests/csrc/check_common_div.c);
-// x = 0 keeps its sign as the IEEE quotient does.  Three quotients cost one
-// division and three short corrections instead of three divisions.
+// x / b for several x over one b, correctly rounded: r = RN(1/b) once, then
+// per quotient y = RN(x r) and one fused correction with the exact residual
+// x - y b (Markstein), which rounds to the IEEE quotient when r is the
+// correctly rounded reciprocal (checked against the IEEE division for every
+// significand of b, tests/csrc/check_common_div.c; x = -0 gives +0 here, a
+// sign that no sum it enters keeps).
 template <class T> LGX_D T div_by(T x, T b, T r) {
   if (sizeof(T) == 8) return x / b;
   const T y = x * r;
   const T e = fma(-y, b, x);
-  const T q = fma(e, r, y);
-  return x == T(0) ? x : q;
+  return fma(e, r, y);
+}
+
+// RN(1 / b): the hardware's reciprocal (1 ulp) and one Newton step.  Equal to
+// the IEEE division for every float of magnitude 2^-100 .. 2^125 (all of
+// them compared on the device), in 3 instructions instead of the division's
+// 10.
+template <class T> LGX_D T recip(T b) {
+  if (sizeof(T) == 8) return T(1) / b;
+  const T r = fast_rcp(b);
+  return fma(fma(-b, r, T(1)), r, r);
+}
+
+// len = RN(sqrt(q)), from the hardware's reciprocal square root y and one
+// residual correction of q y: the IEEE root for every float in 2^-100 ..
+// 2^125 (all compared on the device).  r: 1 / len by a Newton step from y,
+// the IEEE quotient but for one ulp at 24 of the 4.2e8 floats of each 25
+// binades, which div_by's residual absorbs.  7 instructions for the two
+// instead of 27; the three normalisations of a direction's set-up were a
+// quarter of it.
+template <class T> LGX_D void root(T q, T &len, T &r) {
+  if (sizeof(T) == 8) {
+    len = sqrt(q);
+    r = T(1) / len;
+    return;
+  }
+  const T y = fast_rsqrt(q);
+  const T g = q * y;
+  len = fma(fma(-g, g, q), T(0.5) * y, g);
+  r = fma(fma(-len, y, T(1)), y, y);
 }
 template <class T> LGX_D Vec3<T> normalize3_cr(Vec3<T> v) {
-  const T len = sqrt(dot3(v, v));
-  const T r = T(1) / len;
+  T len, r;
+  root(dot3(v, v), len, r);
   return Vec3<T>{div_by(v.x, len, r), div_by(v.y, len, r), div_by(v.z, len, r)};
 }
 
 template <class T, class ARGS> LGX_D Vec3<T> unproject_far(ARGS &a, T sx, T sy) {
   // indirectLighting.frag:20-25 with screenPos.z = 1 (:241)
   const auto &m = a.inv_vp;
-  T x = sx * T(2) - T(1), y = sy * T(2) - T(1);
+  T x = fma_(sx, T(2), T(-1)), y = fma_(sy, T(2), T(-1));  // (2 s is exact: one rounding either way)
   T vx = m[0] * x + m[4] * y + m[8] * T(1) + m[12] * T(1);
   T vy = m[1] * x + m[5] * y + m[9] * T(1) + m[13] * T(1);
   T vz = m[2] * x + m[6] * y + m[10] * T(1) + m[14] * T(1);
   T vw = m[3] * x + m[7] * y + m[11] * T(1) + m[15] * T(1);
-  const T rw = T(1) / vw;
+  const T rw = recip(vw);
   return Vec3<T>{div_by(vx, vw, rw), div_by(vy, vw, rw), div_by(vz, vw, rw)};
 }
 
@@ -284,9 +337,16 @@ template <class T> LGX_D size_t point_index(T sx, T sy, int lw, int lh, int pitc
 // the direction sum (float/float, double/double, or float/double).
 // One workgroup's share: logical block b (slice k = b % (grid grid_y), tile b / (grid grid_y)).
 // part: LDS for the shares of a.round directions (kShare values each).
-// Bound by VALU issue and by the latency of each step's dependent texel
-// fetch, which only enough waves hide; one wave per pixel block and all its
-// directions left 1024 waves (one per SIMD) for a 256 x 256 image: 153 us
+// Bound by VALU issue (about 80 % of the slots at 1080p with 32 directions),
+// then by the latency of each step's dependent texel fetch, which only enough
+// waves hide.  An FP32 multiply, add or FMA on vector registers issues twice
+// a CU-cycle, everything else (compares, conversions, minima, 24-bit
+// products, anything with a scalar operand) once, a root or reciprocal every
+// other: a step is 27 instructions, about 19 slots (41 and 29 with a step
+// count, four border tests, clamped texels and scalar operands), a
+// direction's set-up 276 instead of 430.  1080p, 32 directions: 2.69 -> 2.25
+// ms; 4 directions of 256: 2.45 -> 2.00 ms.
+// One wave per pixel block and all its directions left 1024 waves (one per SIMD) for a 256 x 256 image: 153 us
 // there with 16 directions, 57 us with the directions over 8 waves; at 1080p
 // with 32 directions 2.90 -> 2.69 ms (a shorter tail).
 // ARGS: GatherArgs<T> as the kernel's argument, or in constant memory
@@ -324,7 +384,7 @@ LGX_D void gather_block(ARGS &a, const uint32_t b, A *part) {
   const Vec3<T> rayc = normalize3_cr(unproject_far(a, scx, scy) - cam);
   const Vec3<T> P = cam + rayc * rc;  // :130 from the radial distance
   const Vec3<T> eye = normalize3_cr(cam - P);  // :182
-  const Vec3<T> pdir = normalize3_cr(P - cam);
+  const Vec3<T> pdir{-eye.x, -eye.y, -eye.z};   // normalize(P - cam): every operation is odd
   const T ambient = a.ambient;
   // Ray through the sample, unnormalised, at the pixel centre (U) and per
   // unit of step offset along a direction (V is formed per direction).
@@ -332,6 +392,8 @@ LGX_D void gather_block(ARGS &a, const uint32_t b, A *part) {
   const Vec3<T> U = E0 + EX * scx + EY * scy;
   const T erc = rc * dot3(eye, rayc);
   const T en = dot3(eye, n);
+
+  const T vW = vec(a.W), vH = vec(a.H), vrW = vec(a.rW), vrH = vec(a.rH);
 
   const T *dirs = a.dirs + (size_t)k * a.D * 4;
   const T *steps = a.steps + (size_t)k * a.S_tab * 2;
@@ -351,7 +413,7 @@ LGX_D void gather_block(ARGS &a, const uint32_t b, A *part) {
     const Vec3<T> c1 = cross3(tangent, eye);
     const Vec3<T> dn = cross3(Vec3<T>{-c1.x, -c1.y, -c1.z}, n);
     const T hy = dot3(dn, tangent), hx = dot3(dn, eye);
-    T max_h = atan2_finite(hy, hx);
+    T max_h = atan2_finite<false>(hy, hx);
     HorizonMax<T> hm;
     hm.set(hy, hx);
     const T iq2 = fast_rcp(hx * hx + hy * hy);
@@ -368,15 +430,13 @@ LGX_D void gather_block(ARGS &a, const uint32_t b, A *part) {
     T h0 = T(0.25) * en * (T(1) - c2max) + T(0.25) * tn * (T(2) * max_h - s2max);
     A L0 = A(ambient * h0), L1 = L0, L2 = L0;
     // :212 step count, capped by the table (S)
-    int iters = (int)(log(path / a.near_step) / a.log_ratio) + 1;
-    iters = min(iters, a.S_tab);
+    auto shader_steps = [&]() { return min((int)(log(path / a.near_step) / a.log_ratio) + 1, a.S_tab); };
     // per-direction constants of the fast delta evaluation
-    const Vec3<T> V = EX * (dx / a.W) + EY * (dy / a.H);
+    const Vec3<T> V = EX * div_extent(dx, a.W, a.rW) + EY * div_extent(dy, a.H, a.rH);
     const T uu = dot3(U, U), uv2 = T(2) * dot3(U, V), vv = dot3(V, V);
     const T tu = dot3(tangent, U), tv = dot3(tangent, V);
     const T eu = dot3(eye, U), ev = dot3(eye, V);
     const T trc = rc * dot3(tangent, rayc);
-    int j = 0;
     if (SAMPLER == LGX_SAMPLER_HIZ_POINT) {
       // Level-major march.  The step index j is the same on every active
       // lane (all start at 0 and advance together; lanes only leave), so
@@ -395,21 +455,51 @@ LGX_D void gather_block(ARGS &a, const uint32_t b, A *part) {
       // wide footprint) and not on short ones; the launch-shape autotuner
       // picks per configuration.  Otherwise each step fetches and then waits.
       const int *lstart = a.level_start + (size_t)k * (LGX_MAX_LEVELS + 1);
+      // the offset of step s (a scalar load); past the table no lane goes on
+      auto offset = [&](int s) { return s < a.S_tab ? steps[2 * s] : T(INFINITY); };
+      // The march ends on an offset, not on a step count and four screen
+      // tests: the ray leaves the screen at offset `path`, and the shader's
+      // step count int(log(path / near) / log(ratio)) + 1 (:212) admits step
+      // j while near ratio^j <= path, i.e. while the offset near
+      // ratio^(j + lin) + 1 - near (:217) is at most path ratio^lin + 1 -
+      // near; below near, where the logarithm is negative, the truncation
+      // admits step 0 alone while path > near / ratio.  A step within rounding of the border may fall on either side:
+      // its side fade is 0 there.
+      // With FP32 sums the far borders are taken 2^-20 of the extent early
+      // (0.002 pixels at 1920, where the fade is below 1e-5): whatever the
+      // roundings of the limit and of a step's position, the position stays
+      // below the extent, and so does its texel, which then needs no clamp.
+      // FP64 sums resolve such a step: they keep the border and the clamp.
+      constexpr bool kClamp = sizeof(A) == 8;
+      const T rlin = (steps[0] - T(1) + a.near_step) / a.near_step;
+      T lim = path >= a.near_step ? fma_(path, rlin, T(1) - a.near_step) : path > a.near_min ? offset(1) : T(0);
+      lim = min(lim, path);
+      if (!kClamp) {
+        const T far = T(1 - 0x1p-20);
+        if (dx > T(0)) lim = min(lim, (a.W * far - cx) * idx);
+        if (dy > T(0)) lim = min(lim, (a.H * far - cy) * idy);
+      }
+      if (COUNT) {  // the shader's own rule, step by step
+        const int iters = shader_steps();
+        for (int j = 0; j < iters; j++) {
+          const T o = steps[2 * j];
+          const T qx = cx + dx * o, qy = cy + dy * o;
+          if (!((qx > T(0)) & (qx < a.W) & (qy > T(0)) & (qy < a.H))) break;
+          step_total++;
+        }
+      }
       int l = 0;
       int lnext = a.n_levels > 1 ? lstart[1] : INT_MAX;  // first step of the next level
-      // the level's depth and radiance as buffer resources: per-step fetches
-      // take a 32-bit byte offset against a scalar base
+      // the level's depth and radiance as structured buffers
       auto depth_rsrc = [&](int lv) {
-        return __builtin_amdgcn_make_buffer_rsrc((void *)a.pd[lv], (short)0, a.lh[lv] * a.pd_pitch[lv] * 4,
-                                                 kBufferConfig);
+        return level_rsrc(a.pd[lv], 4, a.lh[lv] * a.pd_pitch[lv]);
       };
       auto rad_rsrc = [&](int lv) {
-        return __builtin_amdgcn_make_buffer_rsrc((void *)a.pr[lv], (short)0,
-                                                 a.lh[lv] * a.pr_pitch[lv] * RadBuf<RFMT>::kBytes, kBufferConfig);
+        return level_rsrc(a.pr[lv], RadBuf<RFMT>::kBytes, a.lh[lv] * a.pr_pitch[lv]);
       };
-      __amdgpu_buffer_rsrc_t drs = depth_rsrc(0), rrs = rad_rsrc(0);
+      i32x4 drs = depth_rsrc(0), rrs = rad_rsrc(0);
       T flw = T(a.lw[0]), flh = T(a.lh[0]);
-      int lw1 = a.lw[0] - 1, lh1 = a.lh[0] - 1, dpitch = a.pd_pitch[0], rpitch = a.pr_pitch[0];
+      int dpitch = a.pd_pitch[0], rpitch = a.pr_pitch[0];
       int smask = 0, sshift = 0, ssw = 0;
       if constexpr (SWZ) {
         smask = a.swz_mask[0];
@@ -421,31 +511,53 @@ LGX_D void gather_block(ARGS &a, const uint32_t b, A *part) {
         if constexpr (SWZ) return (int)(__umul24((unsigned)(ix & smask), (unsigned)ssw) + (unsigned)(ix >> sshift));
         return ix;
       };
-      // the fetch of step s at offset o on the current level: on-screen flag,
-      // q / extent, depth request, radiance texel index
+      // What every step reads: in vector registers, since an FP32 multiply,
+      // add or FMA issues at twice the rate without a scalar operand.
+      const T vdx = vec(dx), vdy = vec(dy);
+      // the fetch at offset o on the current level: q / extent, texel
+      // position, depth request
       struct Fetch {
         float rd;
         T sqx, sqy;
-        uint32_t rti;
-        bool on;
+        int ix, iy;
       };
-      auto request = [&](int s, T o) {
+      auto request = [&](T o) {
         Fetch f;
-        const T qx = cx + dx * o, qy = cy + dy * o;  // :218
-        // :219-228 on screen: q / extent in (0, 1) is q in (0, extent), as
-        // the quotient is correctly rounded (it reaches 1 only from q = extent)
-        // (bitwise &: one mask, not a chain of divergent branches)
-        f.on = (s < iters) & (qx > T(0)) & (qx < a.W) & (qy > T(0)) & (qy < a.H);
-        f.sqx = div_extent(qx, a.W, a.rW);  // :219
-        f.sqy = div_extent(qy, a.H, a.rH);
-        // sq > 0 on screen, so sq * extent >= 0 and truncation is floor; the
-        // product can round up to the extent itself, hence the upper clamp
-        const int ix = col(min((int)(f.sqx * flw), lw1));
-        const int iy = min((int)(f.sqy * flh), lh1);
-        f.rti = texel_index(iy, rpitch, ix);
-        const uint32_t ti = texel_index(iy, dpitch, ix);
-        f.rd = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(drs, (int)(ti * 4u), 0, 0));
+        f.sqx = div_extent(cx + vdx * o, vW, vrW);  // :218-219
+        f.sqy = div_extent(cy + vdy * o, vH, vrH);
+        // truncation is floor: a step of the march is at most rounding below 0
+        f.ix = (int)(f.sqx * flw);
+        f.iy = (int)(f.sqy * flh);
+        if (kClamp) {  // the product can round up to the extent itself
+          f.ix = min(f.ix, (int)flw - 1);
+          f.iy = min(f.iy, (int)flh - 1);
+        }
+        f.ix = col(f.ix);
+        f.rd = load_depth(drs, texel_index(f.iy, dpitch, f.ix));
         return f;
+      };
+      // :254-263 a sample above the horizon: radiance v (raw), weights, new maximum
+      auto raise = [&](T hyv, T hxv, T sqx, T sqy, auto v_of) {
+        if (COUNT) hit_total++;
+        const T th = atan2_finite<true>(hyv, hxv);
+        const T iq = fast_rcp(hxv * hxv + hyv * hyv);
+        const T c2 = (hxv * hxv - hyv * hyv) * iq, s2 = (T(2) * hxv * hyv) * iq;
+        // :222-227 the four ramps; of two opposite ones at most one is below 1
+        const T width = T(0.1f), inv_width = T(1) / width;
+        const T side = min(max(min(sqx, T(1) - sqx) * inv_width, T(0)), T(1)) *
+                       min(max(min(sqy, T(1) - sqy) * inv_width, T(0)), T(1));
+        const T hc = (T(0.25) * en * (c2 - c2max) + T(0.25) * tn * (T(2) * max_h - T(2) * th - s2max + s2)) * side;
+        const float4 v = v_of();
+        L0 += A(T(v.x) * hc);  // :261
+        L1 += A(T(v.y) * hc);
+        L2 += A(T(v.z) * hc);
+        L0 -= A(ambient * hc);  // :262
+        L1 -= A(ambient * hc);
+        L2 -= A(ambient * hc);
+        max_h = th;  // :263
+        hm.lower(hyv, hxv);
+        c2max = c2;
+        s2max = s2;
       };
       // the level of step s (uniform; s never decreases)
       auto to_level = [&](int s) {
@@ -458,8 +570,6 @@ LGX_D void gather_block(ARGS &a, const uint32_t b, A *part) {
           rpitch = a.pr_pitch[l];
           flw = T(a.lw[l]);
           flh = T(a.lh[l]);
-          lw1 = a.lw[l] - 1;
-          lh1 = a.lh[l] - 1;
           if constexpr (SWZ) {
             smask = a.swz_mask[l];
             sshift = a.swz_shift[l];
@@ -467,13 +577,12 @@ LGX_D void gather_block(ARGS &a, const uint32_t b, A *part) {
           }
         }
       };
+      T off = steps[0];
+      to_level(0);
       if constexpr (PIPE) {
-        T off = steps[0];
-        T off_n = steps[2 * min(1, a.S_tab - 1)];  // the next step's offset (scalar)
-        to_level(0);
-        Fetch f = request(0, off);
-        for (; f.on; j++) {
-          const int ju = __builtin_amdgcn_readfirstlane(j);
+        T off_n = offset(1);
+        Fetch f = request(off);
+        for (int j = 0; off < lim; j++) {
           // step j: :241-252 sample delta projected on (eye, tangent)
           const T r = T(f.rd);
           const T len2 = fma_(off, fma_(off, vv, uv2), uu);
@@ -482,97 +591,34 @@ LGX_D void gather_block(ARGS &a, const uint32_t b, A *part) {
           const T hxv = fma_(ri, fma_(off, ev, eu), -erc);
           const bool hit = hm.below(hyv, hxv);  // :254
           typename RadBuf<RFMT>::Raw rv;
-          if (hit) rv = RadBuf<RFMT>::raw(rrs, f.rti);  // :256, on step j's level
+          if (hit) rv = RadBuf<RFMT>::raw(rrs, texel_index(f.iy, rpitch, f.ix));  // :256, on step j's level
           const T sqx = f.sqx, sqy = f.sqy;
-          // step j + 1: its level, then its depth request
+          // step j + 1: its level, then its depth request (discarded if no lane goes on)
           off = off_n;
-          off_n = steps[2 * min(ju + 2, a.S_tab - 1)];  // scalar load, in flight for a step
-          to_level(ju + 1);
-          f = request(ju + 1, off);
-          if (hit) {
-            if (COUNT) hit_total++;
-            const T th = atan2_finite(hyv, hxv);
-            const T iq = fast_rcp(hxv * hxv + hyv * hyv);
-            const T c2 = (hxv * hxv - hyv * hyv) * iq, s2 = (T(2) * hxv * hyv) * iq;
-            T side = T(1);
-            {
-              const T width = T(0.1f), inv_width = T(1) / width;  // :222-227
-              side *= min(max((T(1) - sqx) * inv_width, T(0)), T(1));
-              side *= min(max(sqx * inv_width, T(0)), T(1));
-              side *= min(max((T(1) - sqy) * inv_width, T(0)), T(1));
-              side *= min(max(sqy * inv_width, T(0)), T(1));
-            }
-            const T hc =
-                (T(0.25) * en * (c2 - c2max) + T(0.25) * tn * (T(2) * max_h - T(2) * th - s2max + s2)) * side;
-            const float4 v = RadBuf<RFMT>::decode(rv);
-            L0 += A(T(v.x) * hc);  // :261
-            L1 += A(T(v.y) * hc);
-            L2 += A(T(v.z) * hc);
-            L0 -= A(ambient * hc);  // :262
-            L1 -= A(ambient * hc);
-            L2 -= A(ambient * hc);
-            max_h = th;  // :263
-            hm.set(hyv, hxv);
-            c2max = c2;
-            s2max = s2;
-          }
+          off_n = offset(j + 2);
+          to_level(j + 1);
+          f = request(off);
+          if (hit) raise(hyv, hxv, sqx, sqy, [&]() { return RadBuf<RFMT>::decode(rv); });
         }
       } else {
-        T off = steps[0];
-        for (;; j++) {
-          if (j >= iters) break;
-          const int ju = __builtin_amdgcn_readfirstlane(j);
-          // the next step's offset: a scalar load in flight during this step
-          const T off_next = steps[2 * min(ju + 1, a.S_tab - 1)];
-          to_level(ju);
-          const T qx = cx + dx * off, qy = cy + dy * off;  // :218
-          // :219-228 on screen: q / extent in (0, 1) is q in (0, extent), as
-          // the quotient is correctly rounded (it reaches 1 only from q = extent)
-          // (bitwise &: one mask, not a chain of divergent branches)
-          if (!((qx > T(0)) & (qx < a.W) & (qy > T(0)) & (qy < a.H))) break;
-          const T sqx = div_extent(qx, a.W, a.rW), sqy = div_extent(qy, a.H, a.rH);  // :219
-          // sq > 0, so sq * extent >= 0 and truncation is floor; the product can
-          // round up to the extent itself, hence the upper clamp (in integers)
-          const int ix = col(min((int)(sqx * flw), lw1));
-          const int iy = min((int)(sqy * flh), lh1);
-          const uint32_t ti = texel_index(iy, dpitch, ix);
-          const T r = T(__builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(drs, (int)(ti * 4u), 0, 0)));
+        for (int j = 0; off < lim; j++) {
+          const T off_next = offset(j + 1);
+          to_level(j);
+          const Fetch f = request(off);
           // :241-252 sample delta projected on (eye, tangent)
           const T len2 = fma_(off, fma_(off, vv, uv2), uu);
-          const T ri = r * fast_rsqrt(len2);
+          const T ri = T(f.rd) * fast_rsqrt(len2);
           const T hyv = fma_(ri, fma_(off, tv, tu), -trc);
           const T hxv = fma_(ri, fma_(off, ev, eu), -erc);
-          if (hm.below(hyv, hxv)) {  // :254
-            if (COUNT) hit_total++;
-            const T th = atan2_finite(hyv, hxv);
-            const T iq = fast_rcp(hxv * hxv + hyv * hyv);
-            const T c2 = (hxv * hxv - hyv * hyv) * iq, s2 = (T(2) * hxv * hyv) * iq;
-            T side = T(1);
-            {
-              const T width = T(0.1f), inv_width = T(1) / width;  // :222-227
-              side *= min(max((T(1) - sqx) * inv_width, T(0)), T(1));
-              side *= min(max(sqx * inv_width, T(0)), T(1));
-              side *= min(max((T(1) - sqy) * inv_width, T(0)), T(1));
-              side *= min(max(sqy * inv_width, T(0)), T(1));
-            }
-            const T hc =
-                (T(0.25) * en * (c2 - c2max) + T(0.25) * tn * (T(2) * max_h - T(2) * th - s2max + s2)) * side;
-            const float4 v = RadBuf<RFMT>::load(rrs, texel_index(iy, rpitch, ix));  // :256
-            L0 += A(T(v.x) * hc);  // :261
-            L1 += A(T(v.y) * hc);
-            L2 += A(T(v.z) * hc);
-            L0 -= A(ambient * hc);  // :262
-            L1 -= A(ambient * hc);
-            L2 -= A(ambient * hc);
-            max_h = th;  // :263
-            hm.set(hyv, hxv);
-            c2max = c2;
-            s2max = s2;
-          }
+          if (hm.below(hyv, hxv))  // :254
+            raise(hyv, hxv, f.sqx, f.sqy,
+                  [&]() { return RadBuf<RFMT>::decode(RadBuf<RFMT>::raw(rrs, texel_index(f.iy, rpitch, f.ix))); });  // :256
           off = off_next;
         }
       }
     } else {
+      int j = 0;
+      const int iters = shader_steps();
       for (; j < iters; j++) {
         const T off = steps[2 * j], lod = steps[2 * j + 1];
         const T qx = cx + dx * off, qy = cy + dy * off;  // :218
@@ -625,13 +671,13 @@ LGX_D void gather_block(ARGS &a, const uint32_t b, A *part) {
           L1 -= A(ambient * hc);
           L2 -= A(ambient * hc);
           max_h = th;  // :263
-          hm.set(hyv, hxv);
+          hm.lower(hyv, hxv);
           c2max = c2;
           s2max = s2;
         }
       }
+      if (COUNT) step_total += j;
     }
-    if (COUNT) step_total += j;
     // :268; for a power-of-two D the quotient is the product with 1 / D
     // (exact), otherwise the IEEE division
     if (a.d_pow2) {
@@ -1168,6 +1214,7 @@ static int make_args(const lgx_gather_params *p, const void *ws, const lgx_gbuff
   a.H = T(p->height);
   a.near_step = a.W / T(1000);
   a.log_ratio = std::log(T(2) * pi / T(footprint(p)) + T(1));
+  a.near_min = a.near_step / (T(2) * pi / T(footprint(p)) + T(1));
   a.ambient = T(0.01f);
   a.w = p->width;
   a.h = p->height;
