@@ -3,14 +3,15 @@
 //  * lgx_bilateral: the geometry-aware filter whose weights are written (and
 //    commented out) in denoiser.frag:87-110: w = exp(-|d - dc| * 10.5) *
 //    exp(-|n - nc|^2 * 20) over the taps [-r, r)^2 (y outer, x inner), at
-//    pixel centres with clamp to edge, colour / (sumW + 1e-7).  One 16x16
-//    output tile per workgroup; the tile plus its halo of irradiance, radial
-//    depth and decoded normals is staged in LDS once, so each texel is read
-//    from memory once per pass instead of (2r)^2 times.
+//    pixel centres with clamp to edge, colour / (sumW + 1e-7).  The output
+//    tile of a workgroup plus its halo of irradiance, radial depth and decoded
+//    normals is staged in LDS once, so each texel is read from memory about
+//    once per pass instead of (2r)^2 times.
 //  * lgx_regression_denoise: the live DenoiserPass (denoiser.frag:72-185).
 //  * lgx_composite: finalGatherer.frag:42-58.
 #include <math.h>
 
+#include "device_math.h"
 #include "lgx_internal.h"
 
 namespace lgx {
@@ -28,45 +29,112 @@ struct BilatArgs {
   float ds, ns;
 };
 
-constexpr int kBilatMaxR = 8;
-constexpr int kBilatSpan = 16 + 2 * kBilatMaxR;
+constexpr int kBilatMaxR = 8, kBilatTW = 32;
 
-template <int NFMT> __global__ __launch_bounds__(256) void bilateral_kernel(const BilatArgs a) {
-  __shared__ float4 s_col[kBilatSpan * kBilatSpan];
-  __shared__ float4 s_geo[kBilatSpan * kBilatSpan];  // depth, normal xyz
-  const int r = a.r;
-  const int span = 16 + 2 * r - 1;  // taps reach -r .. r-1
-  const int x0 = blockIdx.x * 16 - r, y0 = blockIdx.y * 16 - r;
-  for (int i = threadIdx.x; i < span * span; i += 256) {
-    const int lx = i % span, ly = i / span;
-    const int gx = min(max(x0 + lx, 0), a.w - 1), gy = min(max(y0 + ly, 0), a.h - 1);
-    s_col[ly * kBilatSpan + lx] = a.in[(size_t)gy * a.in_pitch + gx];
-    const float4 nt = Texel<NFMT>::load(a.normal, (size_t)gy * a.normal_pitch + gx);
-    const Vec3<float> n = oct_decode<float>(nt.x, nt.y);
-    s_geo[ly * kBilatSpan + lx] = make_float4(a.depth[(size_t)gy * a.depth_pitch + gx], n.x, n.y, n.z);
+// One row of taps (n = 2r of them, geometry and colour in LDS) for the
+// outputs LO..HI of a thread's column.
+template <int R, int LO, int HI>
+LGX_D void bilat_row(const float4 *geo, const float4 *col, int n, const float4 (&gc)[R], float4 (&acc)[R]) {
+#pragma unroll 4
+  for (int x = 0; x < n; x++) {
+    const float4 gs = geo[x], c = col[x];
+#pragma unroll
+    for (int k = LO; k <= HI; k++) {
+      // exp(-|dd| ds) exp(-|dn|^2 ns) = exp2(-|dd| kd - |dn|^2 kn), the
+      // depth and normal staged with kd and sqrt(kn): one hardware exp2 (1
+      // ulp) per tap
+      const float dx = gs.y - gc[k].y, dy = gs.z - gc[k].z, dz = gs.w - gc[k].w;
+      const float w = __builtin_amdgcn_exp2f(fmaf(-dz, dz, fmaf(-dy, dy, fmaf(-dx, dx, -fabsf(gs.x - gc[k].x)))));
+      acc[k].x = fmaf(c.x, w, acc[k].x);
+      acc[k].y = fmaf(c.y, w, acc[k].y);
+      acc[k].z = fmaf(c.z, w, acc[k].z);
+      acc[k].w = fmaf(c.w, w, acc[k].w);
+    }
+  }
+}
+// the same for the uniform range lo..hi
+template <int R, int LO = 0, int HI = 0>
+LGX_D void bilat_rows(int lo, int hi, const float4 *geo, const float4 *col, int n, const float4 (&gc)[R],
+                      float4 (&acc)[R]) {
+  if (lo == LO && hi == HI)
+    bilat_row<R, LO, HI>(geo, col, n, gc, acc);
+  else if constexpr (HI + 1 < R)
+    bilat_rows<R, LO, HI + 1>(lo, hi, geo, col, n, gc, acc);
+  else if constexpr (LO + 1 < R)
+    bilat_rows<R, LO + 1, LO + 1>(lo, hi, geo, col, n, gc, acc);
+}
+
+// A workgroup filters 32 x 8R pixels, a thread R pixels of one column, whose
+// windows overlap in all but R - 1 of their rows: a tap read from LDS serves
+// up to R outputs.  Bound by VALU issue (94 % of the slots that this mix of
+// instructions has, by counters): 12 instructions a tap with one exp2 (8
+// FP32, 20 and their scalar operands before), about 190 a pixel for staging
+// and the quotients.  More outputs a thread read less LDS and lose as much
+// to the fewer workgroups that fit it.  2560x1440, r = 4: 121 -> 87 us.
+template <int NFMT, int R> __global__ __launch_bounds__(256) void bilateral_kernel(const BilatArgs a) {
+  extern __shared__ __align__(16) float4 s_bilat[];
+  const int r = a.r, n = 2 * r;
+  constexpr int TW = kBilatTW, TH = 256 / TW * R;
+  const int sw = TW + n - 1, sh = TH + n - 1;  // taps reach -r .. r-1
+  float4 *s_geo = s_bilat, *s_col = s_bilat + sw * sh;  // (depth, normal xyz), colour
+  const int x0 = blockIdx.x * TW - r, y0 = blockIdx.y * TH - r;
+  const float kd = a.ds * 1.44269504f, kn = sqrtf(a.ns * 1.44269504f);
+  // Four texels of the tile a thread at a time, all their loads in flight
+  // together: a load per row waited for its own round trip to memory, which
+  // the few workgroups that fit a CU's LDS do not hide.
+  const int total = sw * sh;
+  const uint32_t inv = ((1u << 20) + sw - 1) / (uint32_t)sw;  // i / sw for i < 4096, sw in 16 .. 79
+  // 32-bit byte offsets from the tile's first image row
+  const int yb = max(y0, 0);
+  const char *b_in = (const char *)(a.in + (size_t)yb * a.in_pitch);
+  const char *b_n = (const char *)a.normal + (size_t)yb * a.normal_pitch * (NFMT == LGX_RG16F ? 4 : 8);
+  const char *b_d = (const char *)(a.depth + (size_t)yb * a.depth_pitch);
+  for (int i0 = threadIdx.x; i0 < total; i0 += 4 * 256) {
+    float4 c[4];
+    float2 nt[4];
+    float d[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      const int i = min(i0 + u * 256, total - 1);
+      const int ly = (int)(((uint32_t)i * inv) >> 20), lx = i - ly * sw;
+      const uint32_t gx = (uint32_t)min(max(x0 + lx, 0), a.w - 1), row = (uint32_t)(min(max(y0 + ly, 0), a.h - 1) - yb);
+      c[u] = *(const float4 *)(b_in + (row * (uint32_t)a.in_pitch + gx) * 16u);
+      const float4 t = Texel<NFMT>::load(b_n + (row * (uint32_t)a.normal_pitch + gx) * (NFMT == LGX_RG16F ? 4u : 8u), 0);
+      nt[u] = make_float2(t.x, t.y);
+      d[u] = *(const float *)(b_d + (row * (uint32_t)a.depth_pitch + gx) * 4u);
+    }
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      const int i = i0 + u * 256;
+      if (i < total) {
+        const Vec3<float> nv = oct_decode_dev<float>(nt[u].x, nt[u].y);
+        s_geo[i] = make_float4(d[u] * kd, nv.x * kn, nv.y * kn, nv.z * kn);
+        s_col[i] = make_float4(c[u].x, c[u].y, c[u].z, 1.0f);
+      }
+    }
   }
   __syncthreads();
-  const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-  const int px = blockIdx.x * 16 + tx, py = blockIdx.y * 16 + ty;
-  if (px >= a.w || py >= a.h) return;
-  const float4 gc = s_geo[(ty + r) * kBilatSpan + tx + r];
-  // exp(-|dd| ds) exp(-|dn|^2 ns) = exp2(-(|dd| ds + |dn|^2 ns) log2(e)): one
-  // hardware exp2 (1 ulp) per tap instead of two library expf
-  const float kd = a.ds * 1.44269504f, kn = a.ns * 1.44269504f;
-  float c0 = 0.f, c1 = 0.f, c2 = 0.f, sw = 0.f;
-  for (int y = -r; y < r; y++)
-    for (int x = -r; x < r; x++) {
-      const int li = (ty + r + y) * kBilatSpan + tx + r + x;
-      const float4 gs = s_geo[li];
-      const float dx = gs.y - gc.y, dy = gs.z - gc.z, dz = gs.w - gc.w;
-      const float wgt = __builtin_amdgcn_exp2f(-(fabsf(gs.x - gc.x) * kd + (dx * dx + dy * dy + dz * dz) * kn));
-      const float4 c = s_col[li];
-      c0 += c.x * wgt;
-      c1 += c.y * wgt;
-      c2 += c.z * wgt;
-      sw += wgt;
-    }
-  a.out[(size_t)py * a.out_pitch + px] = make_float4(c0 / (sw + 1e-7f), c1 / (sw + 1e-7f), c2 / (sw + 1e-7f), 1.0f);
+  const int tx = threadIdx.x % TW, ty = threadIdx.x / TW * R;
+  float4 gc[R], acc[R];
+#pragma unroll
+  for (int k = 0; k < R; k++) {
+    gc[k] = s_geo[(ty + k + r) * sw + tx + r];
+    acc[k] = make_float4(0.f, 0.f, 0.f, 0.f);
+  }
+  // window row j holds the taps of outputs k with 0 <= j - k < 2r
+  for (int j = 0; j < n + R - 1; j++) {
+    const int at = (ty + j) * sw + tx;
+    bilat_rows<R>(max(j - n + 1, 0), min(j, R - 1), s_geo + at, s_col + at, n, gc, acc);
+  }
+  const int px = blockIdx.x * TW + tx, py = blockIdx.y * TH + ty;
+  if (px >= a.w) return;
+#pragma unroll
+  for (int k = 0; k < R; k++) {
+    if (py + k >= a.h) break;
+    const float sum = acc[k].w + 1e-7f, rs = recip(sum);
+    a.out[(size_t)(py + k) * a.out_pitch + px] =
+        make_float4(div_by(acc[k].x, sum, rs), div_by(acc[k].y, sum, rs), div_by(acc[k].z, sum, rs), 1.0f);
+  }
 }
 
 __global__ __launch_bounds__(256) void copy4_kernel(const float4 *in, int ip, float4 *out, int op, int w, int h) {
@@ -155,12 +223,19 @@ extern "C" int lgx_bilateral(const lgx_bilateral_params *p, const lgx_image *in,
   BilatArgs a{(const float4 *)in->ptr, in->pitch, (const float *)g->depth.ptr, g->depth.pitch, g->normal.ptr,
               g->normal.pitch, (float4 *)out->ptr, out->pitch, in->w, in->h, p->radius, p->depth_sharpness,
               p->normal_sharpness};
-  dim3 grid((in->w + 15) / 16, (in->h + 15) / 16);
-  if (g->normal.format == LGX_RG16F)
-    hipLaunchKernelGGL(bilateral_kernel<LGX_RG16F>, grid, dim3(256), 0, s, a);
-  else
-    hipLaunchKernelGGL(bilateral_kernel<LGX_RG32F>, grid, dim3(256), 0, s, a);
-  return hip_status(hipGetLastError());
+  auto launch = [&](auto kern, int R) {
+    const int n = 2 * p->radius, TH = 256 / kBilatTW * R;
+    const size_t lds = (size_t)(kBilatTW + n - 1) * (TH + n - 1) * 2 * sizeof(float4);
+    hipLaunchKernelGGL(kern, dim3((in->w + kBilatTW - 1) / kBilatTW, (in->h + TH - 1) / TH), dim3(256), lds, s, a);
+    return hip_status(hipGetLastError());
+  };
+  const bool h16 = g->normal.format == LGX_RG16F;
+  // Two outputs a thread once their 4096 tiles of 32 x 16 keep every CU's five
+  // workgroups busy for a few rounds (2560x1440, r = 4: 87 against 91 us for
+  // one output; 1279x719, r = 3: 20 against 19 us).
+  if ((int64_t)in->w * in->h >= (int64_t)4096 * 512)
+    return h16 ? launch(bilateral_kernel<LGX_RG16F, 2>, 2) : launch(bilateral_kernel<LGX_RG32F, 2>, 2);
+  return h16 ? launch(bilateral_kernel<LGX_RG16F, 1>, 1) : launch(bilateral_kernel<LGX_RG32F, 1>, 1);
 }
 
 extern "C" int lgx_regression_denoise(const lgx_image *in, const lgx_gbuffer *g, int32_t radius, lgx_image *out,

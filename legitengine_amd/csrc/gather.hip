@@ -31,6 +31,7 @@
 #include <unordered_map>
 #include <vector>
 
+#include "device_math.h"
 #include "lgx_internal.h"
 
 namespace lgx {
@@ -82,22 +83,6 @@ template <class T> struct GatherArgs {
   int sx0, sy0, lcells_x, lcells_y;  // slice cells covered by the launch (region of interest)
   int rx0, ry0, rx1, ry1;            // pixels gathered: [rx0, rx1) x [ry0, ry1)
 };
-
-template <class T> LGX_D T fast_rsqrt(T v);
-template <> LGX_D float fast_rsqrt<float>(float v) { return __builtin_amdgcn_rsqf(v); }
-template <> LGX_D double fast_rsqrt<double>(double v) { return 1.0 / sqrt(v); }
-
-// A uniform value held in a vector register (float).
-template <class T> LGX_D T vec(T v) {
-  if constexpr (sizeof(T) == 4) asm("" : "+v"(v));
-  return v;
-}
-
-template <class T> LGX_D T fma_(T a, T b, T c) { return fma(a, b, c); }
-
-template <class T> LGX_D T fast_rcp(T v);
-template <> LGX_D float fast_rcp<float>(float v) { return __builtin_amdgcn_rcpf(v); }
-template <> LGX_D double fast_rcp<double>(double v) { return 1.0 / v; }
 
 // q / b for the viewport extent b, correctly rounded: y = RN(q * RN(1/b)),
 // one fused correction with the exact residual q - y*b (Markstein).  The
@@ -217,53 +202,6 @@ template <class T> struct HorizonMax {
   }
 };
 
-// x / b for several x over one b, correctly rounded: r = RN(1/b) once, then
-// per quotient y = RN(x r) and one fused correction with the exact residual
-// x - y b (Markstein), which rounds to the IEEE quotient when r is the
-// correctly rounded reciprocal (checked against the IEEE division for every
-// significand of b, tests/csrc/check_common_div.c; x = -0 gives +0 here, a
-// sign that no sum it enters keeps).
-template <class T> LGX_D T div_by(T x, T b, T r) {
-  if (sizeof(T) == 8) return x / b;
-  const T y = x * r;
-  const T e = fma(-y, b, x);
-  return fma(e, r, y);
-}
-
-// RN(1 / b): the hardware's reciprocal (1 ulp) and one Newton step.  Equal to
-// the IEEE division for every float of magnitude 2^-100 .. 2^125 (all of
-// them compared on the device), in 3 instructions instead of the division's
-// 10.
-template <class T> LGX_D T recip(T b) {
-  if (sizeof(T) == 8) return T(1) / b;
-  const T r = fast_rcp(b);
-  return fma(fma(-b, r, T(1)), r, r);
-}
-
-// len = RN(sqrt(q)), from the hardware's reciprocal square root y and one
-// residual correction of q y: the IEEE root for every float in 2^-100 ..
-// 2^125 (all compared on the device).  r: 1 / len by a Newton step from y,
-// the IEEE quotient but for one ulp at 24 of the 4.2e8 floats of each 25
-// binades, which div_by's residual absorbs.  7 instructions for the two
-// instead of 27; the three normalisations of a direction's set-up were a
-// quarter of it.
-template <class T> LGX_D void root(T q, T &len, T &r) {
-  if (sizeof(T) == 8) {
-    len = sqrt(q);
-    r = T(1) / len;
-    return;
-  }
-  const T y = fast_rsqrt(q);
-  const T g = q * y;
-  len = fma(fma(-g, g, q), T(0.5) * y, g);
-  r = fma(fma(-len, y, T(1)), y, y);
-}
-template <class T> LGX_D Vec3<T> normalize3_cr(Vec3<T> v) {
-  T len, r;
-  root(dot3(v, v), len, r);
-  return Vec3<T>{div_by(v.x, len, r), div_by(v.y, len, r), div_by(v.z, len, r)};
-}
-
 template <class T, class ARGS> LGX_D Vec3<T> unproject_far(ARGS &a, T sx, T sy) {
   // indirectLighting.frag:20-25 with screenPos.z = 1 (:241)
   const auto &m = a.inv_vp;
@@ -380,7 +318,7 @@ LGX_D void gather_block(ARGS &a, const uint32_t b, A *part) {
   const T scx = cx / a.W, scy = cy / a.H;           // :118
   const T rc = T(a.depth[(size_t)y * a.depth_pitch + x]);
   const float4 nt = Texel<NFMT>::load(a.normal, (size_t)y * a.normal_pitch + x);
-  const Vec3<T> n = oct_decode<T>(T(nt.x), T(nt.y));  // :133
+  const Vec3<T> n = oct_decode_dev<T>(T(nt.x), T(nt.y));  // :133
   const Vec3<T> rayc = normalize3_cr(unproject_far(a, scx, scy) - cam);
   const Vec3<T> P = cam + rayc * rc;  // :130 from the radial distance
   const Vec3<T> eye = normalize3_cr(cam - P);  // :182
