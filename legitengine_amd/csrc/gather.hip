@@ -40,9 +40,11 @@ namespace lgx {
 static constexpr int kBufferConfig = 0x00020000;
 
 // SPLIT kernels (all but the step-counting ones): the waves of a workgroup
-// share the directions of 64 pixels.  At most kMaxSplit waves; the shares
+// share the directions of 64 pixels.  At most kMaxSplit waves (FP64: half as
+// many, whose registers would spill in a workgroup of 16 waves); the shares
 // of kRound directions (3 x 64 values each) are in LDS at a time.
-static constexpr int kMaxSplit = 8, kRound = 16, kShare = 3 * 64;
+static constexpr int kMaxSplit = 16, kRound = 16, kShare = 3 * 64;
+template <class T> constexpr int max_threads() { return 64 * (sizeof(T) == 8 ? kMaxSplit / 2 : kMaxSplit); }
 
 template <class T> struct GatherArgs {
   T inv_vp[16];
@@ -214,62 +216,83 @@ template <class T, class ARGS> LGX_D Vec3<T> unproject_far(ARGS &a, T sx, T sy) 
   return Vec3<T>{div_by(vx, vw, rw), div_by(vy, vw, rw), div_by(vz, vw, rw)};
 }
 
-template <int FMT> struct RadLoad {
-  static LGX_D float4 at(const void *base, size_t i) { return Texel<FMT>::load(base, i); }
+// Vulkan clamp-to-edge bilinear taps of a point s in one level (u = s W -
+// 1/2, taps floor(u) and the next, weights frac(u)).  At a border, where both
+// taps are the edge texel, the pair is moved inside and the weight saturates,
+// so the two texels of a row are always neighbours and come in one fetch.  A
+// level of one column or row (uniform) has its texel on both sides.
+template <class T> struct TapPos {
+  T al, be;
+  int x, y;
+  LGX_D TapPos(T sx, T sy, int lw, int lh) {
+    const T u = sx * T(lw) - T(0.5), v = sy * T(lh) - T(0.5);
+    const T fu = max(min(floor(u), T(lw - 2)), T(0)), fv = max(min(floor(v), T(lh - 2)), T(0));
+    al = min(max(u - fu, T(0)), T(1));
+    be = min(max(v - fv, T(0)), T(1));
+    x = (int)fu;
+    y = (int)fv;
+  }
+  LGX_D T mix(T p00, T p10, T p01, T p11) const {
+    const T top = fma_(al, p10 - p00, p00), bot = fma_(al, p11 - p01, p01);
+    return fma_(be, bot - top, top);
+  }
 };
-
-// Vulkan clamp-to-edge bilinear in one level (u = s*W - 1/2).
-template <class T, int FMT>
-LGX_D void bilinear(const void *base, int pitch, int lw, int lh, T sx, T sy, T *out, int nch) {
-  T u = sx * T(lw) - T(0.5), v = sy * T(lh) - T(0.5);
-  T fu = floor(u), fv = floor(v);
-  T al = u - fu, be = v - fv;
-  int i0 = (int)fu, j0 = (int)fv;
-  int x0 = min(max(i0, 0), lw - 1), x1 = min(max(i0 + 1, 0), lw - 1);
-  int y0 = min(max(j0, 0), lh - 1), y1 = min(max(j0 + 1, 0), lh - 1);
-  float4 p00 = Texel<FMT>::load(base, (size_t)y0 * pitch + x0);
-  float4 p10 = Texel<FMT>::load(base, (size_t)y0 * pitch + x1);
-  float4 p01 = Texel<FMT>::load(base, (size_t)y1 * pitch + x0);
-  float4 p11 = Texel<FMT>::load(base, (size_t)y1 * pitch + x1);
-  const float *a00 = &p00.x, *a10 = &p10.x, *a01 = &p01.x, *a11 = &p11.x;
-  for (int k = 0; k < nch; k++) {
-    T top = T(a00[k]) * (T(1) - al) + T(a10[k]) * al;
-    T bot = T(a01[k]) * (T(1) - al) + T(a11[k]) * al;
-    out[k] = top * (T(1) - be) + bot * be;
-  }
-}
-
-template <class T, int FMT, class LV, class PI>
-LGX_D void sample_trilinear(const LV &lv, const PI &pitch, const PI &lw, const PI &lh, int nl, T sx, T sy,
-                            T lod, T *out, int nch) {
-  T q = T(nl - 1);
-  T d = lod;
-  if (!(d > T(0))) d = T(0);
-  if (d > q) d = q;
-  int l0 = (int)floor(d);
-  int l1 = min(l0 + 1, nl - 1);
-  T delta = d - T(l0);
-  T a[4], b[4];
-  bilinear<T, FMT>(lv[l0], pitch[l0], lw[l0], lh[l0], sx, sy, a, nch);
-  if (delta > T(0) && l1 != l0) {
-    bilinear<T, FMT>(lv[l1], pitch[l1], lw[l1], lh[l1], sx, sy, b, nch);
-    for (int k = 0; k < nch; k++) out[k] = a[k] * (T(1) - delta) + b[k] * delta;
+template <class T> LGX_D T depth_taps(const float *base, int pitch, int lw, int lh, const TapPos<T> &p) {
+  const i32x4 r = level_rsrc(base, 4, lh * pitch);
+  const uint32_t a = texel_index(p.y, pitch, p.x), b = a + (lh > 1 ? (uint32_t)pitch : 0u);
+  f32x2 t, q;
+  if (lw > 1) {
+    t = struct_load_f32x2(r, (int)a, 0, 0, 0);
+    q = struct_load_f32x2(r, (int)b, 0, 0, 0);
   } else {
-    for (int k = 0; k < nch; k++) out[k] = a[k];
+    t = load_depth(r, a);
+    q = load_depth(r, b);
   }
+  return p.mix(T(t.x), T(t.y), T(q.x), T(q.y));
 }
-
-template <class T> LGX_D int point_level(T lod, int nl) {
-  int l = 0;
-  if (lod > T(0)) l = (int)min(floor(lod), T(nl - 1));
-  return l;
+template <class T, int FMT>
+LGX_D Vec3<T> radiance_taps(const void *base, int pitch, int lw, int lh, const TapPos<T> &p) {
+  typedef RadBuf<FMT> B;
+  const i32x4 r = level_rsrc(base, B::kBytes, lh * pitch);
+  const uint32_t at = texel_index(p.y, pitch, p.x), down = lh > 1 ? (uint32_t)pitch : 0u;
+  float4 t[4];  // (x, y), (x + 1, y), (x, y + 1), (x + 1, y + 1)
+#pragma unroll
+  for (int row = 0; row < 2; row++) {
+    const uint32_t i = at + (row ? down : 0u);
+    typename B::Raw lo, hi;
+    if (FMT == LGX_RGBA16F && lw > 1) {
+      const f32x4 v = struct_load_f32x4(r, (int)i, 0, 0, 0);
+      __builtin_memcpy(&lo, &v, 8);
+      __builtin_memcpy(&hi, (const char *)&v + 8, 8);
+    } else {
+      lo = B::raw(r, i);
+      hi = lw > 1 ? B::raw(r, i + 1) : lo;
+    }
+    t[2 * row] = B::decode(lo);
+    t[2 * row + 1] = B::decode(hi);
+  }
+  return Vec3<T>{p.mix(T(t[0].x), T(t[1].x), T(t[2].x), T(t[3].x)), p.mix(T(t[0].y), T(t[1].y), T(t[2].y), T(t[3].y)),
+                 p.mix(T(t[0].z), T(t[1].z), T(t[2].z), T(t[3].z))};
 }
-template <class T> LGX_D size_t point_index(T sx, T sy, int lw, int lh, int pitch) {
-  T u = floor(sx * T(lw)), v = floor(sy * T(lh));
-  int i = (int)min(max(u, T(0)), T(lw - 1));
-  int j = (int)min(max(v, T(0)), T(lh - 1));
-  return (size_t)j * pitch + i;
-}
+// The trilinear march is bound by VALU issue as well: about 105 instructions a
+// step (130 with 64-bit addresses, IEEE divisions, four clamped single-texel
+// fetches and a select each, 175 at first), 190 a hit.  1080p, 4 directions:
+// 381 -> 270 us.
+// The levels and blend of a step's lod (uniform): clamped to the pyramid, NaN
+// and -inf to level 0.
+template <class T> struct Trilinear {
+  int l0, l1;
+  T f;
+  bool blend;
+  template <class ARGS> LGX_D Trilinear(ARGS &a, T lod) {
+    const T d = lod > T(0) ? min(lod, T(a.n_levels - 1)) : T(0);
+    const T fl = floor(d);
+    l0 = __builtin_amdgcn_readfirstlane((int)fl);
+    l1 = min(l0 + 1, a.n_levels - 1);
+    f = d - fl;  // 0 on the last level
+    blend = __builtin_amdgcn_readfirstlane((int)(f > T(0))) != 0;
+  }
+};
 
 // T: per-step arithmetic; A: accumulation of the slice contributions and of
 // the direction sum (float/float, double/double, or float/double).
@@ -375,6 +398,65 @@ LGX_D void gather_block(ARGS &a, const uint32_t b, A *part) {
     const T tu = dot3(tangent, U), tv = dot3(tangent, V);
     const T eu = dot3(eye, U), ev = dot3(eye, V);
     const T trc = rc * dot3(tangent, rayc);
+    // :254-263 a sample above the horizon: radiance v (raw), weights, new maximum
+    auto raise = [&](T hyv, T hxv, T sqx, T sqy, auto v_of) {
+      if (COUNT) hit_total++;
+      // (FP64 sums of the trilinear mode keep the library's arc tangent and quotients)
+      constexpr bool kLib = sizeof(A) == 8 && SAMPLER == LGX_SAMPLER_TRILINEAR;
+      const T th = kLib ? atan2(hyv, hxv) : atan2_finite<true>(hyv, hxv);
+      const T iq = kLib ? T(1) / (hxv * hxv + hyv * hyv) : fast_rcp(hxv * hxv + hyv * hyv);
+      const T c2 = (hxv * hxv - hyv * hyv) * iq, s2 = (T(2) * hxv * hyv) * iq;
+      // :222-227 the four ramps; of two opposite ones at most one is below 1
+      const T width = T(0.1f), inv_width = T(1) / width;
+      const T side = min(max(min(sqx, T(1) - sqx) * inv_width, T(0)), T(1)) *
+                     min(max(min(sqy, T(1) - sqy) * inv_width, T(0)), T(1));
+      const T hc = (T(0.25) * en * (c2 - c2max) + T(0.25) * tn * (T(2) * max_h - T(2) * th - s2max + s2)) * side;
+      const auto v = v_of();
+      L0 += A(T(v.x) * hc);  // :261
+      L1 += A(T(v.y) * hc);
+      L2 += A(T(v.z) * hc);
+      L0 -= A(ambient * hc);  // :262
+      L1 -= A(ambient * hc);
+      L2 -= A(ambient * hc);
+      max_h = th;  // :263
+      hm.lower(hyv, hxv);
+      c2max = c2;
+      s2max = s2;
+    };
+    // the offset of step s (a scalar load); past the table no lane goes on
+    auto offset = [&](int s) { return s < a.S_tab ? steps[2 * s] : T(INFINITY); };
+    // The march ends on an offset, not on a step count and four screen
+    // tests: the ray leaves the screen at offset `path`, and the shader's
+    // step count int(log(path / near) / log(ratio)) + 1 (:212) admits step
+    // j while near ratio^j <= path, i.e. while the offset near
+    // ratio^(j + lin) + 1 - near (:217) is at most path ratio^lin + 1 -
+    // near; below near, where the logarithm is negative, the truncation
+    // admits step 0 alone while path > near / ratio.  A step within rounding of the border may fall on either side:
+    // its side fade is 0 there.
+    // With FP32 sums the far borders are taken 2^-20 of the extent early
+    // (0.002 pixels at 1920, where the fade is below 1e-5): whatever the
+    // roundings of the limit and of a step's position, the position stays
+    // below the extent, and so does its texel, which then needs no clamp.
+    // FP64 sums resolve such a step: they keep the border and the clamp (as
+    // do the trilinear taps).
+    constexpr bool kClamp = sizeof(A) == 8 || SAMPLER != LGX_SAMPLER_HIZ_POINT;
+    const T rlin = (steps[0] - T(1) + a.near_step) / a.near_step;
+    T lim = path >= a.near_step ? fma_(path, rlin, T(1) - a.near_step) : path > a.near_min ? offset(1) : T(0);
+    lim = min(lim, path);
+    if (!kClamp) {
+      const T far = T(1 - 0x1p-20);
+      if (dx > T(0)) lim = min(lim, (a.W * far - cx) * idx);
+      if (dy > T(0)) lim = min(lim, (a.H * far - cy) * idy);
+    }
+    if (COUNT) {  // the shader's own rule, step by step
+      const int iters = shader_steps();
+      for (int j = 0; j < iters; j++) {
+        const T o = steps[2 * j];
+        const T qx = cx + dx * o, qy = cy + dy * o;
+        if (!((qx > T(0)) & (qx < a.W) & (qy > T(0)) & (qy < a.H))) break;
+        step_total++;
+      }
+    }
     if (SAMPLER == LGX_SAMPLER_HIZ_POINT) {
       // Level-major march.  The step index j is the same on every active
       // lane (all start at 0 and advance together; lanes only leave), so
@@ -393,39 +475,6 @@ LGX_D void gather_block(ARGS &a, const uint32_t b, A *part) {
       // wide footprint) and not on short ones; the launch-shape autotuner
       // picks per configuration.  Otherwise each step fetches and then waits.
       const int *lstart = a.level_start + (size_t)k * (LGX_MAX_LEVELS + 1);
-      // the offset of step s (a scalar load); past the table no lane goes on
-      auto offset = [&](int s) { return s < a.S_tab ? steps[2 * s] : T(INFINITY); };
-      // The march ends on an offset, not on a step count and four screen
-      // tests: the ray leaves the screen at offset `path`, and the shader's
-      // step count int(log(path / near) / log(ratio)) + 1 (:212) admits step
-      // j while near ratio^j <= path, i.e. while the offset near
-      // ratio^(j + lin) + 1 - near (:217) is at most path ratio^lin + 1 -
-      // near; below near, where the logarithm is negative, the truncation
-      // admits step 0 alone while path > near / ratio.  A step within rounding of the border may fall on either side:
-      // its side fade is 0 there.
-      // With FP32 sums the far borders are taken 2^-20 of the extent early
-      // (0.002 pixels at 1920, where the fade is below 1e-5): whatever the
-      // roundings of the limit and of a step's position, the position stays
-      // below the extent, and so does its texel, which then needs no clamp.
-      // FP64 sums resolve such a step: they keep the border and the clamp.
-      constexpr bool kClamp = sizeof(A) == 8;
-      const T rlin = (steps[0] - T(1) + a.near_step) / a.near_step;
-      T lim = path >= a.near_step ? fma_(path, rlin, T(1) - a.near_step) : path > a.near_min ? offset(1) : T(0);
-      lim = min(lim, path);
-      if (!kClamp) {
-        const T far = T(1 - 0x1p-20);
-        if (dx > T(0)) lim = min(lim, (a.W * far - cx) * idx);
-        if (dy > T(0)) lim = min(lim, (a.H * far - cy) * idy);
-      }
-      if (COUNT) {  // the shader's own rule, step by step
-        const int iters = shader_steps();
-        for (int j = 0; j < iters; j++) {
-          const T o = steps[2 * j];
-          const T qx = cx + dx * o, qy = cy + dy * o;
-          if (!((qx > T(0)) & (qx < a.W) & (qy > T(0)) & (qy < a.H))) break;
-          step_total++;
-        }
-      }
       int l = 0;
       int lnext = a.n_levels > 1 ? lstart[1] : INT_MAX;  // first step of the next level
       // the level's depth and radiance as structured buffers
@@ -473,29 +522,6 @@ LGX_D void gather_block(ARGS &a, const uint32_t b, A *part) {
         f.ix = col(f.ix);
         f.rd = load_depth(drs, texel_index(f.iy, dpitch, f.ix));
         return f;
-      };
-      // :254-263 a sample above the horizon: radiance v (raw), weights, new maximum
-      auto raise = [&](T hyv, T hxv, T sqx, T sqy, auto v_of) {
-        if (COUNT) hit_total++;
-        const T th = atan2_finite<true>(hyv, hxv);
-        const T iq = fast_rcp(hxv * hxv + hyv * hyv);
-        const T c2 = (hxv * hxv - hyv * hyv) * iq, s2 = (T(2) * hxv * hyv) * iq;
-        // :222-227 the four ramps; of two opposite ones at most one is below 1
-        const T width = T(0.1f), inv_width = T(1) / width;
-        const T side = min(max(min(sqx, T(1) - sqx) * inv_width, T(0)), T(1)) *
-                       min(max(min(sqy, T(1) - sqy) * inv_width, T(0)), T(1));
-        const T hc = (T(0.25) * en * (c2 - c2max) + T(0.25) * tn * (T(2) * max_h - T(2) * th - s2max + s2)) * side;
-        const float4 v = v_of();
-        L0 += A(T(v.x) * hc);  // :261
-        L1 += A(T(v.y) * hc);
-        L2 += A(T(v.z) * hc);
-        L0 -= A(ambient * hc);  // :262
-        L1 -= A(ambient * hc);
-        L2 -= A(ambient * hc);
-        max_h = th;  // :263
-        hm.lower(hyv, hxv);
-        c2max = c2;
-        s2max = s2;
       };
       // the level of step s (uniform; s never decreases)
       auto to_level = [&](int s) {
@@ -555,66 +581,31 @@ LGX_D void gather_block(ARGS &a, const uint32_t b, A *part) {
         }
       }
     } else {
-      int j = 0;
-      const int iters = shader_steps();
-      for (; j < iters; j++) {
-        const T off = steps[2 * j], lod = steps[2 * j + 1];
-        const T qx = cx + dx * off, qy = cy + dy * off;  // :218
-        const T sqx = qx / a.W, sqy = qy / a.H;          // :219
-        if (!(sqx > T(0) && sqx < T(1) && sqy > T(0) && sqy < T(1))) break;
-        T r;
-        if (SAMPLER == LGX_SAMPLER_HIZ_POINT) {
-          const int l = point_level(lod, a.n_levels);
-          r = T(a.pd[l][point_index(sqx, sqy, a.lw[l], a.lh[l], a.pd_pitch[l])]);
-        } else {
-          T tmp[4];
-          sample_trilinear<T, LGX_R32F>(a.pd, a.pd_pitch, a.lw, a.lh, a.n_levels, sqx, sqy, lod,
-                                        tmp, 1);
-          r = tmp[0];
-        }
+      const T vdx = vec(dx), vdy = vec(dy);
+      for (int j = 0; j < a.S_tab; j++) {
+        const T off = vec(steps[2 * j]), lod = steps[2 * j + 1];
+        if (!(off < lim)) break;
+        const T sqx = div_extent(cx + vdx * off, vW, vrW), sqy = div_extent(cy + vdy * off, vH, vrH);  // :218-219
+        const Trilinear<T> tl(a, lod);
+        const int l0 = tl.l0, l1 = tl.l1;
+        const TapPos<T> p0(sqx, sqy, a.lw[l0], a.lh[l0]), p1(sqx, sqy, a.lw[l1], a.lh[l1]);
+        T r = depth_taps(a.pd[l0], a.pd_pitch[l0], a.lw[l0], a.lh[l0], p0);
+        if (tl.blend) r = fma_(tl.f, depth_taps(a.pd[l1], a.pd_pitch[l1], a.lw[l1], a.lh[l1], p1) - r, r);
         // :241-252 sample delta projected on (eye, tangent)
         const T len2 = fma_(off, fma_(off, vv, uv2), uu);
         const T ri = r * fast_rsqrt(len2);
-        const T hyv = ri * fma_(off, tv, tu) - trc;
-        const T hxv = ri * fma_(off, ev, eu) - erc;
-        if (hm.below(hyv, hxv)) {  // :254
-            if (COUNT) hit_total++;
-          const T th = atan2(hyv, hxv);
-          const T qq = hxv * hxv + hyv * hyv;
-          const T c2 = (hxv * hxv - hyv * hyv) / qq, s2 = (T(2) * hxv * hyv) / qq;
-          T side = T(1);
-          {
-            const T width = T(0.1f), inv_width = T(1) / width;  // :222-227
-            side *= min(max((T(1) - sqx) * inv_width, T(0)), T(1));
-            side *= min(max(sqx * inv_width, T(0)), T(1));
-            side *= min(max((T(1) - sqy) * inv_width, T(0)), T(1));
-            side *= min(max(sqy * inv_width, T(0)), T(1));
-          }
-          const T hc = (T(0.25) * en * (c2 - c2max) + T(0.25) * tn * (T(2) * max_h - T(2) * th - s2max + s2)) * side;
-          T ls[4];
-          if (SAMPLER == LGX_SAMPLER_HIZ_POINT) {
-            const int l = point_level(lod, a.n_levels);
-            float4 v = Texel<RFMT>::load(a.pr[l], point_index(sqx, sqy, a.lw[l], a.lh[l], a.pr_pitch[l]));
-            ls[0] = T(v.x);
-            ls[1] = T(v.y);
-            ls[2] = T(v.z);
-          } else {
-            sample_trilinear<T, RFMT>(a.pr, a.pr_pitch, a.lw, a.lh, a.n_levels, sqx, sqy, lod, ls,
-                                      3);
-          }
-          L0 += A(ls[0] * hc);  // :261
-          L1 += A(ls[1] * hc);
-          L2 += A(ls[2] * hc);
-          L0 -= A(ambient * hc);  // :262
-          L1 -= A(ambient * hc);
-          L2 -= A(ambient * hc);
-          max_h = th;  // :263
-          hm.lower(hyv, hxv);
-          c2max = c2;
-          s2max = s2;
-        }
+        const T hyv = fma_(ri, fma_(off, tv, tu), -trc);
+        const T hxv = fma_(ri, fma_(off, ev, eu), -erc);
+        if (hm.below(hyv, hxv))  // :254
+          raise(hyv, hxv, sqx, sqy, [&]() {  // :256
+            Vec3<T> v = radiance_taps<T, RFMT>(a.pr[l0], a.pr_pitch[l0], a.lw[l0], a.lh[l0], p0);
+            if (tl.blend) {
+              const Vec3<T> w = radiance_taps<T, RFMT>(a.pr[l1], a.pr_pitch[l1], a.lw[l1], a.lh[l1], p1);
+              v = Vec3<T>{fma_(tl.f, w.x - v.x, v.x), fma_(tl.f, w.y - v.y, v.y), fma_(tl.f, w.z - v.z, v.z)};
+            }
+            return v;
+          });
       }
-      if (COUNT) step_total += j;
     }
     // :268; for a power-of-two D the quotient is the product with 1 / D
     // (exact), otherwise the IEEE division
@@ -690,7 +681,7 @@ LGX_D void gather_block(ARGS &a, const uint32_t b, A *part) {
 // compiler's choice); the launch shapes offer 1 and 8.  PIPE: the step loop
 // that overlaps fetches with arithmetic (Hi-Z sampler).
 template <class T, class A, int SAMPLER, int RFMT, int NFMT, bool COUNT, int OCC, bool PIPE = false, bool SWZ = false>
-__global__ __launch_bounds__(COUNT ? 256 : 64 * kMaxSplit, OCC) void gather_kernel(const GatherArgs<T> a) {
+__global__ __launch_bounds__(COUNT ? 256 : max_threads<T>(), OCC) void gather_kernel(const GatherArgs<T> a) {
   extern __shared__ __align__(16) unsigned char s_part[];
   gather_block<T, A, SAMPLER, RFMT, NFMT, COUNT, PIPE, SWZ>(a, xcd_remap(blockIdx.x, (uint32_t)a.n_blocks), (A *)s_part);
 }
@@ -742,7 +733,7 @@ __global__ __launch_bounds__(256) void swizzle_jobs_kernel(const SwzJob *__restr
 // takes blocks from the other XCDs' chunks in turn (the counters only grow,
 // so every block is taken once), and ends when all eight are exhausted.
 template <class T, class A, int SAMPLER, int RFMT, int NFMT, int OCC, bool PIPE, bool SWZ>
-__global__ __launch_bounds__(64 * kMaxSplit, OCC) void gather_multi_kernel(const GatherArgs<T> *__restrict__ views,
+__global__ __launch_bounds__(max_threads<T>(), OCC) void gather_multi_kernel(const GatherArgs<T> *__restrict__ views,
                                                            const uint32_t *__restrict__ first, int n_views,
                                                            uint32_t *next) {
   extern __shared__ __align__(16) unsigned char s_part[];
@@ -965,9 +956,14 @@ template <class T> static void frame_constants(const lgx_gather_params *p, Gathe
 
 template <class T, class A, int SAMPLER, int RFMT, int NFMT>
 static hipError_t launch_gather(const GatherArgs<T> &a, bool count, hipStream_t s) {
-  // the FP32 Hi-Z gather has every variant; the others run the default one
+  // The FP32 Hi-Z gather has every variant; the others run one.  FP32 steps
+  // with FP64 sums: registers for 8 waves per SIMD and the pipelined loop
+  // (256x256 crop, 256 directions: 4.07 ms; 4.13 with the plain loop, 4.86
+  // with the compiler's 99 registers).  Trilinear: 6 waves (1080p, 4
+  // directions: 270 us; 284 at 5, 287 at 8 with spills).
   constexpr bool kAll = sizeof(T) == 4 && sizeof(A) == 4 && SAMPLER == LGX_SAMPLER_HIZ_POINT;
-  constexpr int O8 = kAll ? 8 : 1;
+  constexpr bool kAcc = sizeof(T) == 4 && sizeof(A) == 8 && SAMPLER == LGX_SAMPLER_HIZ_POINT;
+  constexpr int O8 = kAll ? 8 : 1, O1 = kAcc ? 8 : sizeof(T) == 4 && SAMPLER == LGX_SAMPLER_TRILINEAR ? 6 : 1;
   auto launch = [&](auto kern) {
     const unsigned threads = a.split ? 64u * (unsigned)a.split : 256u;
     const size_t lds = a.split ? (size_t)a.round * kShare * sizeof(A) : 0;
@@ -984,7 +980,7 @@ static hipError_t launch_gather(const GatherArgs<T> &a, bool count, hipStream_t 
   if (kAll && a.occ == 8 && a.pipe) return launch(gather_kernel<T, A, SAMPLER, RFMT, NFMT, false, O8, kAll>);
   if (kAll && a.occ == 8) return launch(gather_kernel<T, A, SAMPLER, RFMT, NFMT, false, O8>);
   if (kAll && a.pipe) return launch(gather_kernel<T, A, SAMPLER, RFMT, NFMT, false, 1, kAll>);
-  return launch(gather_kernel<T, A, SAMPLER, RFMT, NFMT, false, 1>);
+  return launch(gather_kernel<T, A, SAMPLER, RFMT, NFMT, false, O1, kAcc>);
 }
 
 template <class T, class A, int SAMPLER>
@@ -1113,25 +1109,28 @@ static int64_t launch_pixels(const lgx_gather_params *p) {
 // few times that ends in a long tail, since a wave lives as long as its
 // slowest ray times its directions.  More waves per pixel repeat the pixel's
 // set-up and wait for each other at the sums, which weighs most with few
-// directions.  Measured, one / two / four / eight waves (16x16 shapes):
-//   256x256, 16 directions            153 / 88 / 62 / 57 us      (1024 waves of pixels)
-//   512x288, 32 directions            620 / 461 / 335 / 299 us   (2304)
-//   512x288, 4 directions, F = 256    513 / 370 / 293 us
-//   1279x719, 8 directions            214 / 198 / 200 us         (14 K)
-//   1920x1080, 32 directions          2899 / 2769 / 2688 / 2866 us (32 K)
-//   1920x1080, 4 directions, F = 256  2644 / 2450 / 2480 us
-//   256x256 crop, 256 directions      18.2 / 9.4 / 5.8 / 5.8 ms
-//   64x64 crop, 256 directions        19.1 / 8.7 / 4.7 / 2.5 ms
+// directions.  Measured, 1 / 2 / 4 / 8 / 16 waves (us, 16x16 shapes):
+//   64x64 crop, 256 directions (64 waves of pixels)  14577 / 7722 / 4068 / 2161 / 1329
+//   128x128 crop, 256 directions (256)               14048 / 7403 / 3849 / 2004 / 1232
+//   256x256 crop, 256 directions (1024)              15892 / 8125 / 4841 / 4860 / 4965
+//   256x256, 16 directions (1024)                    128 / 70 / 45 / 42 / 53
+//   512x288, 32 directions (2304)                    631 / 391 / 286 / 254 / 254
+//   512x288, 4 directions of 256 (2304)              428 / 302 / 228
+//   960x540, 8 directions (8100)                     111 / 96 / 91 / 103
+//   1279x719, 8 directions (14 K)                    158 / 146 / 150 / 175
+//   1920x1080, 32 directions (32 K)                  4085 / 2663 / 2286 / 2453 / 2899
+//   1920x1080, 4 directions of 256 (32 K)            2005 / 1999 / 2077
 // The trilinear march has a handful of steps a direction, so a direction is
-// mostly set-up and nothing but an idle chip makes a split worth while
-// (1920x1080, 4 directions: 371 / 374 / 406 us; 480x270: 53 / 45 / 38 us).
-static int split_waves(int64_t pixels, int dirs, int sampler) {
+// mostly set-up and nothing but an idle chip makes a split worth while:
+//   480x270 / 1280x720 / 1920x1080, 4 directions     47, 32, 28 / 136, 130, 141 / 271, 278, 323
+static int split_waves(int64_t pixels, int dirs, int sampler, int precision) {
   const int64_t full = 8192, waves = (pixels + 63) / 64;
   if (sampler == LGX_SAMPLER_TRILINEAR && dirs < 16) {
     int k = 1;
     while (k < 4 && 2 * k <= dirs && waves * k < 2 * full) k *= 2;
     return k;
   }
+  if (dirs >= 16 && waves * 16 <= full / 2 && precision != LGX_PREC_F64) return 16;
   if (dirs >= 8 && waves * 4 <= full) return 8;
   if (dirs >= 16 || (dirs >= 4 && waves * 2 < 2 * full)) return 4;
   return dirs >= 2 ? 2 : 1;
@@ -1246,8 +1245,8 @@ static int gather_impl(const lgx_gather_params *p, void *ws, const lgx_gbuffer *
                        lgx_image *out, hipStream_t stream) {
   GatherArgs<T> a;
   SwzJobs jobs;
-  int rc = make_args<T>(p, ws, g, pyr, out, a, p->step_counts ? 0 : split_waves(launch_pixels(p), p->dirs, p->sampler), &jobs,
-                        (char *)ws + swz_offset(p));
+  const int split = p->step_counts ? 0 : split_waves(launch_pixels(p), p->dirs, p->sampler, p->precision);
+  int rc = make_args<T>(p, ws, g, pyr, out, a, split, &jobs, (char *)ws + swz_offset(p));
   if (rc != LGX_OK) return rc;
   hipError_t e;
   if (jobs.n) {
@@ -1383,7 +1382,7 @@ static int gather_batch_upload(lgx_gather_batch *b, int tile) {
     dirs = std::max(dirs, q.dirs);
     pixels += launch_pixels(&q);
   }
-  const int split = split_waves(pixels, dirs, b->sampler);
+  const int split = split_waves(pixels, dirs, b->sampler, LGX_PREC_F32);
   for (int i = 0; i < n; i++) {
     lgx_gather_params q = b->p[i];
     q.tile = tile;

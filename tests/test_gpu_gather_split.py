@@ -52,3 +52,23 @@ def test_split_matches_one_wave_and_oracle(extent, roi, grid, dirs, sampler):
             dep, rad = [d.numpy() for d in pyr.dep_b], [r.numpy() for r in pyr.rad_b]
             ref = orc.gather(view, proj, gb["depth"], orc.widen(gb["normal"]), dep, rad, dirs, 64, sampler, grid=grid)
             assert orc.rel_l2(a.numpy()[y:y + rh, x:x + rw], ref[y:y + rh, x:x + rw]) <= 1e-4
+
+
+@pytest.mark.parametrize("kind", ["f32", "mixed"])
+@pytest.mark.parametrize("w,h,levels", [(9, 40, 4), (40, 9, 4), (4, 70, 3), (37, 21, 5)])
+def test_trilinear_narrow_levels(w, h, levels, kind):
+    """Trilinear taps come in pairs of neighbouring texels: levels one texel
+    wide or high, odd extents and every border, against the FP32 oracle (the
+    gather's bar)."""
+    from legitengine_amd import device as dev
+    dev.require_device()
+    sc = lgx.make_scene(6, 8, 2)
+    view, proj = lgx.scene_matrices(sc, w, h)
+    gb = lgx.render_gbuffer_cpu(sc, w, h, kind)
+    g = dev.GBufferDev.from_host(gb)
+    pyr = dev.PyramidDev(g, levels, lgx.SAMPLER_TRILINEAR).build()
+    out = dev.Gather(w, h, 4, 0, lgx.SAMPLER_TRILINEAR)(view, proj, g, pyr)
+    torch.cuda.synchronize()
+    dep, rad = [d.numpy() for d in pyr.dep_b], [orc.widen(r.numpy()) for r in pyr.rad_b]
+    ref = orc.gather(view, proj, gb["depth"], orc.widen(gb["normal"]), dep, rad, 4, 0, lgx.SAMPLER_TRILINEAR)
+    assert orc.rel_l2(out.numpy(), ref) <= 1e-4
