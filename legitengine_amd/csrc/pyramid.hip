@@ -94,6 +94,38 @@ struct BlurArgs {
   int n;
 };
 
+// A texel as fetched, and its channels added to a sum (those the format has).
+template <int FMT> struct BlurTexel;
+template <> struct BlurTexel<LGX_R32F> {
+  typedef float Raw;
+  static LGX_D void add(float4 &s, Raw v) { s.x += v; }
+};
+template <> struct BlurTexel<LGX_RG32F> {
+  typedef float2 Raw;
+  static LGX_D void add(float4 &s, Raw v) {
+    s.x += v.x;
+    s.y += v.y;
+  }
+};
+template <> struct BlurTexel<LGX_RGBA16F> {
+  typedef uint2 Raw;
+  static LGX_D void add(float4 &s, Raw v) {
+    s.x += h2f((uint16_t)(v.x & 0xffffu));
+    s.y += h2f((uint16_t)(v.x >> 16));
+    s.z += h2f((uint16_t)(v.y & 0xffffu));
+    s.w += h2f((uint16_t)(v.y >> 16));
+  }
+};
+template <> struct BlurTexel<LGX_RGBA32F> {
+  typedef float4 Raw;
+  static LGX_D void add(float4 &s, Raw v) {
+    s.x += v.x;
+    s.y += v.y;
+    s.z += v.z;
+    s.w += v.w;
+  }
+};
+
 template <int FMT> __global__ __launch_bounds__(256) void blur_kernel(const BlurArgs a) {
   int jb = 0;
   while (jb + 1 < a.n && (int)blockIdx.x >= a.job[jb + 1].block0) jb++;
@@ -120,6 +152,48 @@ template <int FMT> __global__ __launch_bounds__(256) void blur_kernel(const Blur
     out = make_float4(s.x / tw, s.y / tw, s.z / tw, s.w / tw);
   }
   Store<FMT>::store(J.dst, (size_t)py * J.dp + px, Store<FMT>::round(out));
+}
+
+// The pre-blur of the pyramids, r = 2 (BlurBuilder::ApplyBlur above level 0):
+// a wave takes 64 columns x 4 rows, a thread the 4 rows of its column, whose
+// windows share all but 3 of their 7 rows: 7 loads an output instead of 16,
+// from scalar row bases and one column offset per tap.  Every output keeps
+// the reference's order of additions (x outer, y inner), and 1 / 16 is exact.
+// One output a thread was bound by its 16 loads with 64-bit addresses and
+// four divisions; 2160p levels (44 MB read and written): 38.5 -> 16.6 us.
+template <int FMT> __global__ __launch_bounds__(256) void blur2_kernel(const BlurArgs a) {
+  typedef typename BlurTexel<FMT>::Raw Raw;
+  int jb = 0;
+  while (jb + 1 < a.n && (int)blockIdx.x >= a.job[jb + 1].block0) jb++;
+  const BlurJob &J = a.job[jb];
+  const int t = (int)blockIdx.x - J.block0;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int px = (t % J.tiles_x) * 64 + (int)(threadIdx.x & 63), py = (t / J.tiles_x) * 16 + wave * 4;
+  if (py >= J.h) return;
+  float4 s[4];
+#pragma unroll
+  for (int k = 0; k < 4; k++) s[k] = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+  for (int x = -2; x < 2; x++) {
+    const uint32_t col = (uint32_t)min(max(px + x, 0), J.w - 1) * (uint32_t)sizeof(Raw);
+    Raw v[7];
+#pragma unroll
+    for (int r = 0; r < 7; r++) {
+      const int sy = min(max(py - 2 + r, 0), J.h - 1);  // uniform
+      v[r] = *(const Raw *)((const char *)J.src + (size_t)sy * J.sp * sizeof(Raw) + col);
+    }
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+#pragma unroll
+      for (int y = 0; y < 4; y++) BlurTexel<FMT>::add(s[k], v[k + y]);
+  }
+  if (px >= J.w) return;
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    if (py + k >= J.h) break;
+    const float4 o = make_float4(s[k].x * 0.0625f, s[k].y * 0.0625f, s[k].z * 0.0625f, s[k].w * 0.0625f);
+    Store<FMT>::store(J.dst, (size_t)(py + k) * J.dp + px, Store<FMT>::round(o));
+  }
 }
 
 template <int FMT, int MODE> static hipError_t launch_mips(const MipArgs &a, hipStream_t s) {
@@ -183,6 +257,9 @@ extern "C" int lgx_box_blur(const lgx_image *src, const lgx_image *dst, const in
   memset(&a, 0, sizeof(a));
   a.n = n;
   int blocks = 0;
+  bool r2 = true;  // every radius is the pyramids'
+  for (int i = 0; i < n; i++) r2 = r2 && radius[i] == 2;
+  const int tw = r2 ? 64 : 16;
   for (int i = 0; i < n; i++) {
     if (!image_ok(&src[i]) || !image_ok(&dst[i]) || radius[i] < 0 || radius[i] > 64) return LGX_EINVAL;
     if (src[i].format != fmt || dst[i].format != fmt) return LGX_EFORMAT;
@@ -195,17 +272,23 @@ extern "C" int lgx_box_blur(const lgx_image *src, const lgx_image *dst, const in
     J.sp = src[i].pitch;
     J.dp = dst[i].pitch;
     J.r = radius[i];
-    J.tiles_x = (J.w + 15) / 16;
+    J.tiles_x = (J.w + tw - 1) / tw;
     J.block0 = blocks;
     blocks += J.tiles_x * ((J.h + 15) / 16);
   }
   hipStream_t s = (hipStream_t)stream;
   dim3 grid(blocks), block(256);
+  auto launch = [&](auto kern2, auto kern) {
+    if (r2)
+      hipLaunchKernelGGL(kern2, grid, block, 0, s, a);
+    else
+      hipLaunchKernelGGL(kern, grid, block, 0, s, a);
+  };
   switch (fmt) {
-    case LGX_R32F: hipLaunchKernelGGL(blur_kernel<LGX_R32F>, grid, block, 0, s, a); break;
-    case LGX_RG32F: hipLaunchKernelGGL(blur_kernel<LGX_RG32F>, grid, block, 0, s, a); break;
-    case LGX_RGBA16F: hipLaunchKernelGGL(blur_kernel<LGX_RGBA16F>, grid, block, 0, s, a); break;
-    case LGX_RGBA32F: hipLaunchKernelGGL(blur_kernel<LGX_RGBA32F>, grid, block, 0, s, a); break;
+    case LGX_R32F: launch(blur2_kernel<LGX_R32F>, blur_kernel<LGX_R32F>); break;
+    case LGX_RG32F: launch(blur2_kernel<LGX_RG32F>, blur_kernel<LGX_RG32F>); break;
+    case LGX_RGBA16F: launch(blur2_kernel<LGX_RGBA16F>, blur_kernel<LGX_RGBA16F>); break;
+    case LGX_RGBA32F: launch(blur2_kernel<LGX_RGBA32F>, blur_kernel<LGX_RGBA32F>); break;
     default: return LGX_EFORMAT;
   }
   return hip_status(hipGetLastError());
