@@ -19,7 +19,7 @@ struct ConvArgs {
   int n, h, w;    // output extent
   const bf16 *wt; // packed [9][(ca+cb)/32][cout][32]
   const float *bias;
-  int cout, relu;
+  int cout, relu; // relu: exactly when bias is set (conv3x3 refuses other pairs)
   bf16 *out0;     // channels [0, split)
   int split;
   bf16 *out1;     // channels [split, cout)
@@ -31,12 +31,11 @@ struct ConvArgs {
   const float4 *head_noisy;      // residual, row pitch head_noisy_pitch
   float4 *head_out;              // row pitch head_out_pitch; null = no head
   int head_noisy_pitch, head_out_pitch;
-  // First convolution at inference (cout = 32, an LDS tile, n = 1): the
-  // input records are packed from the noisy image and the G-buffer while
-  // the tile is staged, channels (noisy rgb, depth, normal xy, albedo rgb,
-  // zeros), the values pack_input gives for those records; a and b are
-  // unused.
-  int gin_fmt;  // 0: off; 1: RG16F normal + RGBA8 albedo; 2: RG32F + RGBA32F; 3: records (conv_first_pair)
+  // First convolution (conv_first_pair; conv3x3 refuses it): the input records
+  // are packed from the noisy image and the G-buffer while the tile is
+  // staged, channels (noisy rgb, depth, normal xy, albedo rgb, zeros), the
+  // values pack_input gives for those records; a and b are unused.
+  int gin_fmt;  // 0: off; 1: RG16F normal + RGBA8 albedo; 2: RG32F + RGBA32F; 3: records (gin_x12)
   const float4 *gin_noisy;
   const float *gin_depth;
   const void *gin_normal, *gin_albedo;
@@ -75,8 +74,7 @@ struct WgradArgs {
 };
 
 hipError_t conv3x3(const ConvArgs &a, hipStream_t s);
-// The first convolution from the G-buffer (a0: gin_* set, as for conv3x3,
-// n = 1) or from input records (gin_fmt 3, gin_x12, any n) and the second
+// The first convolution from the G-buffer (a0: gin_* set, n = 1) or from input records (gin_fmt 3, gin_x12, any n) and the second
 // one with its 2x2 pool (a1: out0, pool_out) in one kernel; the first
 // layer's output stays in LDS and also goes to a0.out0 when set (the
 // training forward keeps it for the backward pass).

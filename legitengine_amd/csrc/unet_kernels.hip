@@ -76,45 +76,161 @@ LGX_D bf16x8 load8_clamped(const ConvInput &in, int n, int y, int x, int h, int 
   return *(const bf16x8 *)(in.b + (((size_t)n * h + y) * w + x) * in.cb + (c - in.ca));
 }
 
-// Stores one output row of a wave's register tile: PB blocks of 16 pixels
-// (x0 + pb * 16 + col) x MB blocks of 16 channels (co0 + mb * 16 + kg * 4,
-// 4 per lane): bias (bias_r, this lane's channels), ReLU, the optional
-// mask (four channels in one read), the split into out0 / out1.
-template <int PB, int MB, bool UP = false>
-LGX_D void conv_store_row(const ConvArgs &a, const f32x4 (&acc)[PB][MB], const float (&bias_r)[MB][4], int n, int y,
-                          int x0, int col, int kg, int co0) {
-  typedef bf16 bf16x4 __attribute__((ext_vector_type(4)));
+// The value of the neighbouring lane (lane ^ 1): a DPP quad permutation
+// [1, 0, 3, 2], a modifier of one VALU move (no LDS round trip as a shuffle
+// through ds_bpermute would take).
+LGX_D float lane_xor1(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0xB1, 0xF, 0xF, false));
+}
+
+// One image row of a tensor as a buffer of its own, so a column past the row
+// is past the buffer: reads give 0 and stores are dropped without a branch.
+LGX_D __amdgpu_buffer_rsrc_t row_rsrc(const bf16 *p, size_t row, int w, int stride) {
+  return __builtin_amdgcn_make_buffer_rsrc((void *)(p + row * w * stride), (short)0, w * stride * 2, 0x00020000);
+}
+typedef bf16 bf16x4 __attribute__((ext_vector_type(4)));
+typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+LGX_D void row_store(__amdgpu_buffer_rsrc_t r, int offset, bf16x4 v) {
+  __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), r, offset, 0, 0);
+}
+LGX_D bf16x4 row_load(__amdgpu_buffer_rsrc_t r, int offset) {
+  return __builtin_bit_cast(bf16x4, __builtin_amdgcn_raw_buffer_load_b64(r, offset, 0, 0));
+}
+LGX_D float relu(float v) { return v > 0.f ? v : 0.f; }
+// v with the channels zeroed whose mask is not positive (NaN: zeroed)
+LGX_D bf16x4 masked(bf16x4 v, bf16x4 m) {
 #pragma unroll
-  for (int pb = 0; pb < PB; pb++) {
+  for (int i = 0; i < 4; i++) v[i] = bf2f(m[i]) > 0.f ? v[i] : f2bf(0.f);
+  return v;
+}
+
+// The epilogue of a wave's register tile: WR rows from y0 (uniform) x WP blocks
+// of 16 pixels from x0 (lane: pixel col) x MB blocks of 16 channels from co0
+// (lane: 4 channels of group kg).  Bias and ReLU, rounded to BF16; then
+//  * pool_out: the 2x2 average of the rounded values (rows r, r + 1 are this
+//    lane's, columns x, x + 1 are lanes col, col + 1), summed as
+//    avgpool_kernel sums: (y, x), (y, x+1), (y+1, x), (y+1, x+1);
+//  * UP, channels [0, split): their 2x2 sums in upsample_bwd_kernel's order
+//    (the same), masked at half resolution, instead of the full rows;
+//  * the rows: channels [0, split) to out0, the rest to out1, zeroed where the
+//    mask is not positive.  split is a multiple of 16 (checked on the host),
+//    so a block's half is uniform.
+// Each value is formed once, columns are checked by the row buffers' range, and
+// addresses are a lane offset per pixel block plus constants: with the values
+// formed per use and 64-bit addresses per store, the epilogue of a 64-channel
+// layer with its pool was 1300 of 1560 VALU instructions a tile, as long as the
+// tile's 288 MFMAs.
+template <int WR, int WP, int MB, bool UP>
+LGX_D void conv_epilogue(const ConvArgs &a, const f32x4 (&acc)[WR][WP][MB], const float (&bias_r)[MB][4], int n, int y0,
+                         int x0, int co0, int col, int kg) {
+  y0 = __builtin_amdgcn_readfirstlane(y0);
+  if (y0 >= a.h) return;
+  bf16x4 v[WR][WP][MB];
+  if (a.bias) {  // a forward layer: bias and ReLU (checked on the host); uniform
+#pragma unroll
+    for (int r = 0; r < WR; r++)
+#pragma unroll
+      for (int pb = 0; pb < WP; pb++)
+#pragma unroll
+        for (int mb = 0; mb < MB; mb++) {
+          f32x4 f;
+#pragma unroll
+          for (int i = 0; i < 4; i++) f[i] = relu(acc[r][pb][mb][i] + bias_r[mb][i]);
+          v[r][pb][mb] = __builtin_convertvector(f, bf16x4);
+        }
+  } else {
+#pragma unroll
+    for (int r = 0; r < WR; r++)
+#pragma unroll
+      for (int pb = 0; pb < WP; pb++)
+#pragma unroll
+        for (int mb = 0; mb < MB; mb++) v[r][pb][mb] = __builtin_convertvector(acc[r][pb][mb], bf16x4);
+  }
+  const size_t row0 = (size_t)n * a.h + y0;
+  if constexpr (WR % 2 == 0) {
+    if (a.pool_out || UP) {
+      const int hh = a.h >> 1, ww = a.w >> 1, stride = UP ? a.split : a.cout;
+      bf16 *const dst = UP ? a.up_out : a.pool_out;
+#pragma unroll
+      for (int r = 0; r < WR; r += 2) {
+        if ((y0 + r) >> 1 >= hh) break;  // uniform
+        const size_t hrow = (size_t)n * hh + ((y0 + r) >> 1);
+        const __amdgpu_buffer_rsrc_t rs = row_rsrc(dst, hrow, ww, stride);
+        const __amdgpu_buffer_rsrc_t ms = row_rsrc(UP ? a.up_mask : dst, hrow, ww, stride);
+#pragma unroll
+        for (int pb = 0; pb < WP; pb++) {
+          const int x = x0 + pb * 16 + col;
+          // (odd columns have no pixel here)
+          const int at = col & 1 ? (int)0x80000000u : ((x >> 1) * stride + co0 + kg * 4) * 2;
+#pragma unroll
+          for (int mb = 0; mb < MB; mb++) {
+            if (UP && !(co0 + mb * 16 < a.split)) continue;  // uniform
+            f32x4 f;
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+              const float t = bf2f(v[r][pb][mb][i]), b = bf2f(v[r + 1][pb][mb][i]);
+              const float q = ((t + lane_xor1(t)) + b) + lane_xor1(b);
+              f[i] = UP ? q : q * 0.25f;
+            }
+            bf16x4 o = __builtin_convertvector(f, bf16x4);
+            if (UP) o = masked(o, row_load(ms, at + mb * 32));
+            row_store(rs, at + mb * 32, o);
+          }
+        }
+      }
+    }
+  }
+  // the masks of every row before the stores: for all the compiler knows a
+  // store may alias them, and a read after it would wait for its round trip
+  const bool any_mask = a.mask0 || a.mask1;
+  int at0[WP], at1[WP];  // byte offset of this lane's channels co0.. in a row of out0 / out1
+#pragma unroll
+  for (int pb = 0; pb < WP; pb++) {
     const int x = x0 + pb * 16 + col;
-    if (x >= a.w) continue;
-    const size_t pix = ((size_t)n * a.h + y) * a.w + x;
+    at0[pb] = (x * a.split + co0 + kg * 4) * 2;
+    at1[pb] = (x * (a.cout - a.split) + co0 - a.split + kg * 4) * 2;
+  }
+  if (any_mask) {
+    bf16x4 m[WR][WP][MB];
+#pragma unroll
+    for (int r = 0; r < WR; r++)
+      if (y0 + r < a.h)
+#pragma unroll
+        for (int mb = 0; mb < MB; mb++) {
+          const bool lo = co0 + mb * 16 < a.split;
+          const bf16 *const mask = lo ? a.mask0 : a.mask1;
+          if (!mask || (UP && lo)) continue;
+          const __amdgpu_buffer_rsrc_t rs = row_rsrc(mask, row0 + r, a.w, lo ? a.split : a.cout - a.split);
+#pragma unroll
+          for (int pb = 0; pb < WP; pb++) m[r][pb][mb] = row_load(rs, (lo ? at0[pb] : at1[pb]) + mb * 32);
+        }
+#pragma unroll
+    for (int r = 0; r < WR; r++)
+      if (y0 + r < a.h)
+#pragma unroll
+        for (int mb = 0; mb < MB; mb++) {
+          const bool lo = co0 + mb * 16 < a.split;
+          if (!(lo ? a.mask0 : a.mask1) || (UP && lo)) continue;
+#pragma unroll
+          for (int pb = 0; pb < WP; pb++) v[r][pb][mb] = masked(v[r][pb][mb], m[r][pb][mb]);
+        }
+  }
+#pragma unroll
+  for (int r = 0; r < WR; r++) {
+    if (y0 + r >= a.h) break;  // uniform
+    const __amdgpu_buffer_rsrc_t r0 = row_rsrc(a.out0, row0 + r, a.w, a.split);
+    const __amdgpu_buffer_rsrc_t r1 = row_rsrc(a.out1, row0 + r, a.w, a.cout - a.split);
 #pragma unroll
     for (int mb = 0; mb < MB; mb++) {
-      const int co = co0 + mb * 16 + kg * 4;
-      float v[4];
+      const bool lo = co0 + mb * 16 < a.split;  // uniform
+      if (UP && lo) continue;                   // stored as 2x2 sums at half resolution
 #pragma unroll
-      for (int i = 0; i < 4; i++) {
-        v[i] = acc[pb][mb][i];
-        if (a.bias) v[i] += bias_r[mb][i];
-        if (a.relu) v[i] = v[i] > 0.f ? v[i] : 0.f;
+      for (int pb = 0; pb < WP; pb++) {
+        if (lo)
+          row_store(r0, at0[pb] + mb * 32, v[r][pb][mb]);
+        else
+          row_store(r1, at1[pb] + mb * 32, v[r][pb][mb]);
       }
-      // split is a multiple of 16 (checked on the host), so the half is the
-      // same for the whole 16-channel block: a uniform choice of pointers
-      // (a per-lane choice would become a per-lane read of the arguments)
-      const bool lo = co0 + mb * 16 < a.split;
-      if (UP && lo) continue;  // stored as 2x2 sums at half resolution
-      bf16 *const dst = lo ? a.out0 : a.out1;
-      const bf16 *const mask = lo ? a.mask0 : a.mask1;
-      const int stride = lo ? a.split : a.cout - a.split, cch = lo ? co : co - a.split;
-      if (mask) {
-        const bf16x4 m = *(const bf16x4 *)(mask + pix * stride + cch);
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-          if (!(bf2f(m[i]) > 0.f)) v[i] = 0.f;
-      }
-      bf16x4 o = {f2bf(v[0]), f2bf(v[1]), f2bf(v[2]), f2bf(v[3])};
-      *(bf16x4 *)(dst + pix * stride + cch) = o;
     }
   }
 }
@@ -197,9 +313,6 @@ template <int MB, int PB, int R> __global__ __launch_bounds__(256) void conv3x3_
       }
     }
   }
-  // Epilogue.  Masks are read into registers before the stores they feed:
-  // for all the compiler knows a store may alias them, so a read placed
-  // after a store would wait for that store's memory round trip.
   float bias_r[MB][4];
 #pragma unroll
   for (int mb = 0; mb < MB; mb++) {
@@ -209,12 +322,7 @@ template <int MB, int PB, int R> __global__ __launch_bounds__(256) void conv3x3_
     bias_r[mb][2] = b4.z;
     bias_r[mb][3] = b4.w;
   }
-#pragma unroll
-  for (int r = 0; r < R; r++) {
-    const int y = y0 + r;
-    if (y >= a.h) break;
-    conv_store_row<PB, MB>(a, acc[r], bias_r, n, y, x0, col, kg, 0);
-  }
+  conv_epilogue<R, PB, MB, false>(a, acc, bias_r, n, y0, x0, 0, col, kg);
 }
 
 // The same convolution with the operands staged in LDS.  A workgroup
@@ -232,6 +340,7 @@ template <int MB, int PB, int R> __global__ __launch_bounds__(256) void conv3x3_
 // needs MB = 2, i.e. all 32 channels of a pixel in one workgroup).
 // With one input chunk and no channel split every tile uses the same
 // weights: they stay in LDS from the workgroup's first tile on.
+
 // Raw G-buffer texels of one pixel for the G-buffer-fed first convolution
 // (GIN = 1: RG16F normal, RGBA8 albedo; GIN = 2: RG32F, RGBA32F), kept raw
 // in registers while in flight and converted when staged.
@@ -303,13 +412,6 @@ template <int GIN> LGX_D void gin_pack(const GinRaw<GIN> &r, bf16x8 &v0, bf16x8 
   }
 }
 
-// The value of the neighbouring lane (lane ^ 1): a DPP quad permutation
-// [1, 0, 3, 2], a modifier of one VALU move (no LDS round trip as a shuffle
-// through ds_bpermute would take).
-LGX_D float lane_xor1(float v) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0xB1, 0xF, 0xF, false));
-}
-
 // LDS bytes of conv3x3_lds_kernel<MB, WR, WP> (the layout described in it),
 // and the workgroups per CU that LDS allows, at most 3 (168 VGPRs; 4 would
 // leave 128, fewer than the tiles' accumulators and operands need): the
@@ -323,7 +425,7 @@ constexpr int conv_lds_blocks(int MB, int WR, int WP) {
 
 // UP: the epilogue of an input gradient through an upsample (ConvArgs::up_out),
 // a separate instantiation so the other convolutions keep their registers.
-template <int MB, int WR, int WP, bool HEAD, int GIN = 0, bool UP = false>
+template <int MB, int WR, int WP, bool HEAD, bool UP = false>
 __global__ __launch_bounds__(256, conv_lds_blocks(MB, WR, WP)) void conv3x3_lds_kernel(const ConvArgs a, int tiles_x,
                                                                                       int tiles_y, int splits) {
   constexpr int TH = 4 * WR, TW = 16 * WP, IW = TW + 2, IH = TH + 2;
@@ -376,39 +478,24 @@ __global__ __launch_bounds__(256, conv_lds_blocks(MB, WR, WP)) void conv3x3_lds_
   bf16x8 pin[IN_PER], pw[W_PER];
   uint32_t valid = 0;  // bit i: piece i of pin lies in the image
   const bool w_resident = !HEAD && chunks == 1 && splits == 1;
-  // G-buffer-fed input: one thread per halo pixel, raw texels in flight
-  constexpr int GIN_PER = GIN ? (IH * IW + 255) / 256 : 1;
-  GinRaw<GIN ? GIN : 1> graw[GIN_PER];
   auto fetch = [&](const Tile &tl, int cc, bool with_w) {
-    if constexpr (GIN) {
-      valid = 0;
+    const bool from_a = cc * 32 < a.ca;
+    const bool up = from_a && a.a_up;
+    const int cs = from_a ? a.ca : a.cb;
+    const int sw = up ? (a.w >> 1) : a.w, sh = up ? (a.h >> 1) : a.h;
+    const bf16 *img = (from_a ? a.a : a.b) + (size_t)tl.n * sh * sw * cs + (from_a ? cc * 32 : cc * 32 - a.ca);
+    valid = 0;
 #pragma unroll
-      for (int i = 0; i < GIN_PER; i++) {
-        const int p = min(tid + i * 256, IH * IW - 1);
-        const int y = tl.y0 - 1 + p / IW, x = tl.x0 - 1 + p % IW;
-        const bool ok = y >= 0 && y < a.h && x >= 0 && x < a.w;
-        graw[i] = gin_load<GIN>(a, min(max(y, 0), a.h - 1), min(max(x, 0), a.w - 1));
-        valid |= (uint32_t)ok << i;
-      }
-    } else {
-      const bool from_a = cc * 32 < a.ca;
-      const bool up = from_a && a.a_up;
-      const int cs = from_a ? a.ca : a.cb;
-      const int sw = up ? (a.w >> 1) : a.w, sh = up ? (a.h >> 1) : a.h;
-      const bf16 *img = (from_a ? a.a : a.b) + (size_t)tl.n * sh * sw * cs + (from_a ? cc * 32 : cc * 32 - a.ca);
-      valid = 0;
-#pragma unroll
-      for (int i = 0; i < IN_PER; i++) {
-        int p, part;
-        piece(min(tid + i * 256, IN_PIECES - 1), p, part);
-        p = min(p, NPIX - 1);  // a rounding piece: loaded in bounds, never staged
-        const int y = tl.y0 - 1 + p / IW, x = tl.x0 - 1 + p % IW;
-        const bool ok = y >= 0 && y < a.h && x >= 0 && x < a.w;
-        const int yc = min(max(y, 0), a.h - 1), xc = min(max(x, 0), a.w - 1);
-        const uint32_t off = (uint32_t)((up ? (yc >> 1) : yc) * sw + (up ? (xc >> 1) : xc)) * (uint32_t)cs + part * 8;
-        pin[i] = *(const bf16x8 *)(img + off);
-        valid |= (uint32_t)ok << i;
-      }
+    for (int i = 0; i < IN_PER; i++) {
+      int p, part;
+      piece(min(tid + i * 256, IN_PIECES - 1), p, part);
+      p = min(p, NPIX - 1);  // a rounding piece: loaded in bounds, never staged
+      const int y = tl.y0 - 1 + p / IW, x = tl.x0 - 1 + p % IW;
+      const bool ok = y >= 0 && y < a.h && x >= 0 && x < a.w;
+      const int yc = min(max(y, 0), a.h - 1), xc = min(max(x, 0), a.w - 1);
+      const uint32_t off = (uint32_t)((up ? (yc >> 1) : yc) * sw + (up ? (xc >> 1) : xc)) * (uint32_t)cs + part * 8;
+      pin[i] = *(const bf16x8 *)(img + off);
+      valid |= (uint32_t)ok << i;
     }
     if (!with_w) return;
     const bf16 *wsrc = a.wt + ((size_t)cc * a.cout + tl.co0) * 32;
@@ -425,10 +512,6 @@ __global__ __launch_bounds__(256, conv_lds_blocks(MB, WR, WP)) void conv3x3_lds_
   Tile cur = tile_of(t);
   fetch(cur, 0, true);
   bool stage_w = true;  // false once resident weights are staged
-  if constexpr (GIN) {  // record channels 16-31 are zero on every tile: staged once
-    const bf16x8 z = {};
-    for (int p = tid; p < 2 * IH * IW; p += 256) *(bf16x8 *)(s_in + (2 + p / (IH * IW)) * PLANE_IN + (p % (IH * IW)) * 8) = z;
-  }
   for (;;) {
     f32x4 acc[WR][WP][MB];
 #pragma unroll
@@ -455,26 +538,13 @@ __global__ __launch_bounds__(256, conv_lds_blocks(MB, WR, WP)) void conv3x3_lds_
       }
     }
     for (int cc = 0; cc < chunks; cc++) {
-      if constexpr (GIN) {
 #pragma unroll
-        for (int i = 0; i < GIN_PER; i++) {
-          const int p = tid + i * 256;
-          bf16x8 v0 = {}, v1 = {};
-          if ((valid >> i) & 1u) gin_pack<GIN>(graw[i], v0, v1);
-          if (p < IH * IW) {
-            *(bf16x8 *)(s_in + p * 8) = v0;
-            *(bf16x8 *)(s_in + PLANE_IN + p * 8) = v1;
-          }
-        }
-      } else {
-#pragma unroll
-        for (int i = 0; i < IN_PER; i++) {
-          const int q = tid + i * 256;
-          const bf16x8 z = {};
-          int p, part;
-          piece(q, p, part);
-          if (q < IN_PIECES && p < NPIX) *(bf16x8 *)(s_in + part * PLANE_IN + p * 8) = ((valid >> i) & 1u) ? pin[i] : z;
-        }
+      for (int i = 0; i < IN_PER; i++) {
+        const int q = tid + i * 256;
+        const bf16x8 z = {};
+        int p, part;
+        piece(q, p, part);
+        if (q < IN_PIECES && p < NPIX) *(bf16x8 *)(s_in + part * PLANE_IN + p * 8) = ((valid >> i) & 1u) ? pin[i] : z;
       }
       if (stage_w) {
 #pragma unroll
@@ -563,103 +633,406 @@ __global__ __launch_bounds__(256, conv_lds_blocks(MB, WR, WP)) void conv3x3_lds_
       }
       __syncthreads();  // the next tile's stash overwrites the activations
     } else {
-    if (a.pool_out) {
-      // 2x2 average of the stored (BF16) outputs: rows r, r + 1 are this
-      // lane's, columns x, x + 1 are lanes col, col + 1 (same channel group);
-      // summed in avgpool_kernel's order (y, x), (y, x+1), (y+1, x), (y+1, x+1)
-      const int hh = a.h >> 1, ww = a.w >> 1;
-#pragma unroll
-      for (int r = 0; r + 1 < WR; r += 2) {
-        const int y = cur.y0 + wave * WR + r;  // even
-#pragma unroll
-        for (int pb = 0; pb < WP; pb++) {
-          const int x = cur.x0 + pb * 16 + col;
-#pragma unroll
-          for (int mb = 0; mb < MB; mb++) {
-            const int co = cur.co0 + mb * 16 + kg * 4;
-            float t[4], b[4], tn[4], bn[4];
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-              float v0 = acc[r][pb][mb][i], v1 = acc[r + 1][pb][mb][i];
-              if (a.bias) {
-                v0 += bias_r[mb][i];
-                v1 += bias_r[mb][i];
-              }
-              if (a.relu) {
-                v0 = v0 > 0.f ? v0 : 0.f;
-                v1 = v1 > 0.f ? v1 : 0.f;
-              }
-              t[i] = bf2f(f2bf(v0));
-              b[i] = bf2f(f2bf(v1));
-              tn[i] = lane_xor1(t[i]);
-              bn[i] = lane_xor1(b[i]);
-            }
-            if (!(col & 1) && (y >> 1) < hh && (x >> 1) < ww) {
-              typedef bf16 bf16x4 __attribute__((ext_vector_type(4)));
-              bf16x4 o;
-#pragma unroll
-              for (int i = 0; i < 4; i++) o[i] = f2bf((((t[i] + tn[i]) + b[i]) + bn[i]) * 0.25f);
-              *(bf16x4 *)(a.pool_out + (((size_t)cur.n * hh + (y >> 1)) * ww + (x >> 1)) * a.cout + co) = o;
-            }
-          }
-        }
-      }
-    }
-    if constexpr (UP) {
-      // channels [0, split): 2x2 sums of the stored (BF16) values in
-      // upsample_bwd_kernel's order (y, x), (y, x+1), (y+1, x), (y+1, x+1),
-      // masked at half resolution; rows r, r + 1 are this lane's, columns
-      // x, x + 1 are lanes col, col + 1
-      const int hh = a.h >> 1, ww = a.w >> 1;
-#pragma unroll
-      for (int r = 0; r + 1 < WR; r += 2) {
-        const int y = cur.y0 + wave * WR + r;  // even
-#pragma unroll
-        for (int pb = 0; pb < WP; pb++) {
-          const int x = cur.x0 + pb * 16 + col;
-#pragma unroll
-          for (int mb = 0; mb < MB; mb++) {
-            if (!(cur.co0 + mb * 16 < a.split)) continue;  // uniform
-            const int co = cur.co0 + mb * 16 + kg * 4;
-            float t[4], b[4], tn[4], bn[4];
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-              float v0 = acc[r][pb][mb][i], v1 = acc[r + 1][pb][mb][i];
-              if (a.bias) {
-                v0 += bias_r[mb][i];
-                v1 += bias_r[mb][i];
-              }
-              if (a.relu) {
-                v0 = v0 > 0.f ? v0 : 0.f;
-                v1 = v1 > 0.f ? v1 : 0.f;
-              }
-              t[i] = bf2f(f2bf(v0));
-              b[i] = bf2f(f2bf(v1));
-              tn[i] = lane_xor1(t[i]);
-              bn[i] = lane_xor1(b[i]);
-            }
-            if (!(col & 1) && (y >> 1) < hh && (x >> 1) < ww) {
-              typedef bf16 bf16x4 __attribute__((ext_vector_type(4)));
-              const size_t q = (((size_t)cur.n * hh + (y >> 1)) * ww + (x >> 1)) * a.split + co;
-              const bf16x4 m = *(const bf16x4 *)(a.up_mask + q);
-              bf16x4 o;
-#pragma unroll
-              for (int i = 0; i < 4; i++) o[i] = bf2f(m[i]) > 0.f ? f2bf(((t[i] + tn[i]) + b[i]) + bn[i]) : f2bf(0.f);
-              *(bf16x4 *)(a.up_out + q) = o;
-            }
-          }
-        }
-      }
-    }
-#pragma unroll
-    for (int r = 0; r < WR; r++) {
-      const int y = cur.y0 + wave * WR + r;
-      if (y >= a.h) break;
-      conv_store_row<WP, MB, UP>(a, acc[r], bias_r, cur.n, y, cur.x0, col, kg, cur.co0);
-    }
+    conv_epilogue<WR, WP, MB, UP>(a, acc, bias_r, cur.n, cur.y0 + wave * WR, cur.x0, cur.co0, col, kg);
     }
     t += gridDim.x;
     if (t >= T) break;
+    cur = tile_of(t);
+  }
+}
+
+// conv_epilogue for a tile whose channel blocks are paired: the 16 rows of block
+// mb are channels 32 (mb / 2) + 8 kg + 4 (mb & 1) + i, so a lane holds 8
+// consecutive channels of a pixel in two blocks and a pixel's 32 channels are
+// one 64-byte run of four lanes' 16-byte stores (8-byte stores wrote 32-byte
+// runs, twice as many).  Every store is issued (rows past the image go to an
+// empty buffer): at least kStores, which the caller's wait counts on.
+template <int WR, int WP, int MB, bool UP> constexpr int epilogue_stores() {
+  return WR * WP * MB / 2 / (UP ? 2 : 1);
+}
+// The channel of a row of block mb.  Pairs from 64 channels a workgroup on (128
+// bytes a pixel: 45 us against 58 for the 1080p layer 64 + 64 -> 64); with 32
+// channels the 8-byte stores are the faster ones (67 us against 76 for the
+// full-size 32 -> 32 layer, 125 against 142 for 96 -> 32).
+constexpr bool conv_pairs(int MB) { return MB % 4 == 0; }
+LGX_D int pair_row(bool pairs, int mb, int row) {
+  return pairs ? (mb >> 1) * 32 + (row >> 2) * 8 + (mb & 1) * 4 + (row & 3) : mb * 16 + row;
+}
+typedef float f32x8 __attribute__((ext_vector_type(8)));
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+LGX_D void row_store8(__amdgpu_buffer_rsrc_t r, int offset, bf16x8 v) {
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), r, offset, 0, 0);
+}
+LGX_D bf16x8 row_load8(__amdgpu_buffer_rsrc_t r, int offset) {
+  return __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(r, offset, 0, 0));
+}
+LGX_D bf16x8 masked8(bf16x8 v, bf16x8 m) {
+#pragma unroll
+  for (int i = 0; i < 8; i++) v[i] = bf2f(m[i]) > 0.f ? v[i] : f2bf(0.f);
+  return v;
+}
+template <int WR, int WP, int MB, bool UP>
+LGX_D void conv_epilogue_pairs(const ConvArgs &a, const f32x4 (&acc)[WR][WP][MB], const float (&bias_r)[MB][4], int n,
+                               int y0, int x0, int co0, int col, int kg) {
+  constexpr int MP = MB / 2;
+  y0 = __builtin_amdgcn_readfirstlane(y0);
+  bf16x8 v[WR][WP][MP];
+#pragma unroll
+  for (int r = 0; r < WR; r++)
+#pragma unroll
+    for (int pb = 0; pb < WP; pb++)
+#pragma unroll
+      for (int mp = 0; mp < MP; mp++) {
+        f32x8 f;
+        if (a.bias) {  // a forward layer: bias and ReLU (checked on the host); uniform
+#pragma unroll
+          for (int i = 0; i < 8; i++) f[i] = relu(acc[r][pb][2 * mp + (i >> 2)][i & 3] + bias_r[2 * mp + (i >> 2)][i & 3]);
+        } else {
+#pragma unroll
+          for (int i = 0; i < 8; i++) f[i] = acc[r][pb][2 * mp + (i >> 2)][i & 3];
+        }
+        v[r][pb][mp] = __builtin_convertvector(f, bf16x8);
+      }
+  const size_t row0 = (size_t)n * a.h + y0;
+  if constexpr (WR % 2 == 0) {
+    if (a.pool_out || UP) {
+      const int hh = a.h >> 1, ww = a.w >> 1, stride = UP ? a.split : a.cout;
+      bf16 *const dst = UP ? a.up_out : a.pool_out;
+#pragma unroll
+      for (int r = 0; r < WR; r += 2) {
+        const bool in = (y0 + r) >> 1 < hh;  // uniform
+        const size_t hrow = in ? (size_t)n * hh + ((y0 + r) >> 1) : 0;
+        const __amdgpu_buffer_rsrc_t rs = row_rsrc(dst, hrow, in ? ww : 0, stride);
+        const __amdgpu_buffer_rsrc_t ms = row_rsrc(UP ? a.up_mask : dst, hrow, in ? ww : 0, stride);
+#pragma unroll
+        for (int pb = 0; pb < WP; pb++) {
+          const int x = x0 + pb * 16 + col;
+          // (odd columns have no pixel here)
+          const int at = col & 1 ? (int)0x80000000u : ((x >> 1) * stride + co0 + kg * 8) * 2;
+#pragma unroll
+          for (int mp = 0; mp < MP; mp++) {
+            if (UP && !(co0 + mp * 32 < a.split)) continue;  // uniform
+            f32x8 f;
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+              const float t = bf2f(v[r][pb][mp][i]), b = bf2f(v[r + 1][pb][mp][i]);
+              const float q = ((t + lane_xor1(t)) + b) + lane_xor1(b);
+              f[i] = UP ? q : q * 0.25f;
+            }
+            bf16x8 o = __builtin_convertvector(f, bf16x8);
+            if (UP) o = masked8(o, row_load8(ms, at + mp * 64));
+            row_store8(rs, at + mp * 64, o);
+          }
+        }
+      }
+    }
+  }
+  int at0[WP], at1[WP];  // byte offset of this lane's channels co0.. in a row of out0 / out1
+#pragma unroll
+  for (int pb = 0; pb < WP; pb++) {
+    const int x = x0 + pb * 16 + col;
+    at0[pb] = (x * a.split + co0 + kg * 8) * 2;
+    at1[pb] = (x * (a.cout - a.split) + co0 - a.split + kg * 8) * 2;
+  }
+  if (a.mask0 || a.mask1) {  // all masks before the stores (a read after a store would wait for its round trip)
+    bf16x8 m[WR][WP][MP];
+#pragma unroll
+    for (int r = 0; r < WR; r++)
+#pragma unroll
+      for (int mp = 0; mp < MP; mp++) {
+        const bool lo = co0 + mp * 32 < a.split;
+        const bf16 *const mask = lo ? a.mask0 : a.mask1;
+        if (!mask || (UP && lo)) continue;
+        const bool in = y0 + r < a.h;
+        const __amdgpu_buffer_rsrc_t rs = row_rsrc(mask, in ? row0 + r : 0, in ? a.w : 0, lo ? a.split : a.cout - a.split);
+#pragma unroll
+        for (int pb = 0; pb < WP; pb++) m[r][pb][mp] = row_load8(rs, (lo ? at0[pb] : at1[pb]) + mp * 64);
+      }
+#pragma unroll
+    for (int r = 0; r < WR; r++)
+#pragma unroll
+      for (int mp = 0; mp < MP; mp++) {
+        const bool lo = co0 + mp * 32 < a.split;
+        if (!(lo ? a.mask0 : a.mask1) || (UP && lo)) continue;
+#pragma unroll
+        for (int pb = 0; pb < WP; pb++) v[r][pb][mp] = masked8(v[r][pb][mp], m[r][pb][mp]);
+      }
+  }
+#pragma unroll
+  for (int r = 0; r < WR; r++) {
+    const bool in = y0 + r < a.h;
+    const __amdgpu_buffer_rsrc_t r0 = row_rsrc(a.out0, in ? row0 + r : 0, in ? a.w : 0, a.split);
+    const __amdgpu_buffer_rsrc_t r1 = row_rsrc(a.out1, in ? row0 + r : 0, in ? a.w : 0, a.cout - a.split);
+#pragma unroll
+    for (int mp = 0; mp < MP; mp++) {
+      const bool lo = co0 + mp * 32 < a.split;  // uniform
+      if (UP && lo) continue;                   // stored as 2x2 sums at half resolution
+#pragma unroll
+      for (int pb = 0; pb < WP; pb++) {
+        if (lo)
+          row_store8(r0, at0[pb] + mp * 64, v[r][pb][mp]);
+        else
+          row_store8(r1, at1[pb] + mp * 64, v[r][pb][mp]);
+      }
+    }
+  }
+}
+
+// The same convolution with its operands moved to LDS by direct loads
+// (buffer_load ... lds: no registers and no LDS store instructions).  A
+// workgroup of NW waves computes NW WR rows x 16 WP pixels for MB 16-channel
+// blocks and walks tiles; while the MFMAs read one input buffer the next
+// stage (the tile's next 32-channel chunk, or the next tile's first) lands in
+// the other, with one barrier a stage.  Weights of all chunks stay in LDS
+// when they fit (wres), else they move with their chunk.
+//
+// LDS layout: 64 bytes a pixel (or output channel), the 16-byte channel group g
+// of pixel p in place g ^ (p / 4 % 4).  A wave's direct load fills 1 KB, four
+// lanes to a pixel, so it reads whole 64-byte runs of memory (with a pixel's
+// groups 16 lanes apart, each lane of a quad read another cache line); the
+// exchange of places puts the 16 pixels of an operand read (from any start)
+// on all 64 banks.  Pixels outside the image are offsets outside the buffer,
+// which load as zeros.  Accumulation order is conv3x3_kernel's.
+//
+// What bounds it: the epilogue and the outputs' stores (about 40 % of a layer;
+// without them 64 -> 64 at 960 x 540 takes 33 us instead of 46), then the matrix
+// work; the input loads are hidden.  conv3x3_lds_kernel holds the next stage
+// in registers, which the wide tiles do not have to spare, and issues every
+// element's LDS store: at 960 x 540 its best tile takes 63 us for 64 -> 64
+// against 45 here, 113 against 95 for 192 -> 64 and 57 against 41 for 128 -> 64,
+// at 480 x 270 48 against 37 for 128 -> 128.
+constexpr int dma_in_blocks(int WR, int WP, int NW) { return ((NW * WR + 2) * (16 * WP + 2) + 15) / 16; }
+constexpr int dma_act_bytes(int WR, int WP, int NW, bool head) { return head ? NW * WR * WP * 16 * 80 : 0; }
+// LDS bytes with `slots` weight chunks
+constexpr int dma_lds_bytes(int MB, int WR, int WP, int NW, bool head, int slots) {
+  return (2 * dma_in_blocks(WR, WP, NW) + 9 * MB * slots) * 1024 + dma_act_bytes(WR, WP, NW, head);
+}
+
+template <int MB, int WR, int WP, int NW, int OCC, bool HEAD, bool UP>
+__global__ __launch_bounds__(64 * NW, OCC) void conv3x3_dma_kernel(const ConvArgs a, int tiles_x, int tiles_y, int splits,
+                                                                   int wres) {
+  constexpr int TH = NW * WR, TW = 16 * WP, IW = TW + 2, IH = TH + 2, NPIX = IH * IW;
+  constexpr int NBLK = (NPIX + 15) / 16, NI = (NBLK + NW - 1) / NW, WBLK = 9 * MB, NJ = (WBLK + NW - 1) / NW;
+  constexpr bool PAIRS = conv_pairs(MB);
+  extern __shared__ __align__(16) char s_dma[];
+  char *const s_w = s_dma + 2 * NBLK * 1024;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int col = lane & 15, kg = lane >> 4;
+  const int chunks = (a.ca + a.cb) >> 5;
+  typedef __attribute__((address_space(3))) void LdsVoid;
+  const uint32_t logical = xcd_remap(blockIdx.x, gridDim.x);
+  const int co0 = (int)(logical % (uint32_t)splits) * MB * 16, step = (int)gridDim.x / splits;
+  const int T = tiles_x * tiles_y * a.n;
+  int t = (int)(logical / (uint32_t)splits);
+  if (t >= T) return;  // the whole workgroup, before any barrier
+  struct Tile {
+    int n, y0, x0;
+  };
+  auto tile_of = [&](int u) {
+    Tile r;
+    r.x0 = (u % tiles_x) * TW;
+    u /= tiles_x;
+    r.y0 = (u % tiles_y) * TH;
+    r.n = u / tiles_y;
+    return r;
+  };
+  // this lane's pixel of the wave's i-th input block (row, column of the halo tile) and its channel group
+  const int part = ((lane & 3) ^ (lane >> 4)) * 16;
+  int prow[NI], pcol[NI];
+#pragma unroll
+  for (int i = 0; i < NI; i++) {
+    const int p = (wave + NW * i) * 16 + (lane >> 2);
+    prow[i] = p < NPIX ? p / IW : 1 << 20;  // a pixel past the tile: outside every image
+    pcol[i] = p % IW;
+  }
+  // byte offsets of the wave's pieces in the source of chunk cc (a chunk of the
+  // same tile and source only moves the base), then the loads
+  uint32_t voff[NI];
+  auto dma_in = [&](int buf, const Tile &tl, int cc) {
+    const bool from_a = cc * 32 < a.ca;
+    const int up = from_a && a.a_up ? 1 : 0;
+    const int cs = from_a ? a.ca : a.cb;
+    const int sw = a.w >> up, sh = a.h >> up;
+    const int yb = max(tl.y0 - 1, 0) >> up;  // offsets count from the tile's first row
+    const int ch = from_a ? cc * 32 : cc * 32 - a.ca;
+    const bf16 *base = (from_a ? a.a : a.b) + ((size_t)tl.n * sh + yb) * sw * cs + ch;
+    const size_t left = ((size_t)(sh - yb) * sw * cs - ch) * 2;
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+        (void *)base, (short)0, (int)(left < 0x7fffffffu ? left : 0x7fffffffu), 0x00020000);
+    if (cc == 0 || cc * 32 == a.ca) {
+#pragma unroll
+      for (int i = 0; i < NI; i++) {
+        const int y = tl.y0 - 1 + prow[i], x = tl.x0 - 1 + pcol[i];
+        const bool ok = (uint32_t)y < (uint32_t)a.h && (uint32_t)x < (uint32_t)a.w;
+        const uint32_t off = (uint32_t)(((y >> up) - yb) * sw + (x >> up)) * (uint32_t)(cs * 2) + (uint32_t)part;
+        voff[i] = ok ? off : 0x80000000u;
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < NI; i++)
+      if (wave + NW * i < NBLK)  // uniform
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (LdsVoid *)(s_dma + (buf * NBLK + wave + NW * i) * 1024), 16,
+                                                 (int)voff[i], 0, 0, 0);
+  };
+  const __amdgpu_buffer_rsrc_t wrs =
+      __builtin_amdgcn_make_buffer_rsrc((void *)a.wt, (short)0, 9 * chunks * a.cout * 64, 0x00020000);
+  const int wrow = pair_row(PAIRS, 0, lane >> 2) * 64;  // (block mb: pair_row(PAIRS, mb, 0) rows on)
+  auto dma_w = [&](int slot, int cc) {
+#pragma unroll
+    for (int i = 0; i < NJ; i++) {
+      const int b = wave + NW * i;
+      if (b >= WBLK) continue;  // uniform
+      const int tap = b / MB, mb = b % MB;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(wrs, (LdsVoid *)(s_w + (slot * WBLK + b) * 1024), 16,
+                                               wrow + part, ((tap * chunks + cc) * a.cout + co0 + pair_row(PAIRS, mb, 0)) * 64, 0, 0);
+    }
+  };
+  // LDS offset of the input operand at pixel (wave WR + rr) IW + dx + col, group kg; 16 pixels on is 1 KB on
+  int in_off[WR + 2][3];
+#pragma unroll
+  for (int rr = 0; rr < WR + 2; rr++)
+#pragma unroll
+    for (int dx = 0; dx < 3; dx++) {
+      const int p = (wave * WR + rr) * IW + dx + col;
+      in_off[rr][dx] = p * 64 + (kg ^ ((p >> 2) & 3)) * 16;
+    }
+  Tile cur = tile_of(t);
+  if (wres)
+    for (int cc = 0; cc < chunks; cc++) dma_w(cc, cc);
+  else
+    dma_w(0, 0);
+  float bias_r[MB][4];
+  const float *bsrc = a.bias ? a.bias : (const float *)a.wt;  // (never added without a bias)
+#pragma unroll
+  for (int mb = 0; mb < MB; mb++) {
+    const float4 b4 = *(const float4 *)(bsrc + co0 + pair_row(PAIRS, mb, kg * 4));
+    bias_r[mb][0] = b4.x;
+    bias_r[mb][1] = b4.y;
+    bias_r[mb][2] = b4.z;
+    bias_r[mb][3] = b4.w;
+  }
+  dma_in(0, cur, 0);
+  __syncthreads();  // (waits for the loads)
+  int buf = 0;
+  for (;;) {
+    f32x4 acc[WR][WP][MB];
+#pragma unroll
+    for (int r = 0; r < WR; r++)
+#pragma unroll
+      for (int pb = 0; pb < WP; pb++)
+#pragma unroll
+        for (int mb = 0; mb < MB; mb++) acc[r][pb][mb] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int tn = t + step;
+    for (int cc = 0; cc < chunks; cc++) {
+      // the next stage into the other buffer: every wave is past the barrier that ended its last use
+      const bool more = cc + 1 < chunks || tn < T;
+      if (more) {
+        const int nc = cc + 1 < chunks ? cc + 1 : 0;
+        dma_in(buf ^ 1, cc + 1 < chunks ? cur : tile_of(tn), nc);
+        if (!wres) dma_w(buf ^ 1, nc);
+      }
+      const char *in = s_dma + buf * NBLK * 1024;
+      const char *w = s_w + (wres ? cc : buf) * WBLK * 1024 + col * 64 + (kg ^ (col >> 2)) * 16;
+      // Taps in the order (dx, dy).  The operands of a tap are read while the
+      // previous one's MFMAs run: its weights, and the next column's rows a
+      // third at a time.  (Left to the compiler the reads sit right before
+      // their use, and every tap waits for LDS.)
+      constexpr int ROWS = WR + 2;
+      bf16x8 bx[2][ROWS][WP], aw[2][MB];
+      auto read_row = [&](int dx, int rr) {
+#pragma unroll
+        for (int pb = 0; pb < WP; pb++) bx[dx & 1][rr][pb] = *(const bf16x8 *)(in + in_off[rr][dx] + pb * 1024);
+      };
+      auto read_w = [&](int s) {
+#pragma unroll
+        for (int mb = 0; mb < MB; mb++)
+          aw[s & 1][mb] = *(const bf16x8 *)(w + (((s % 3) * 3 + s / 3) * MB + mb) * 1024);
+      };
+      read_w(0);
+#pragma unroll
+      for (int rr = 0; rr < ROWS; rr++) read_row(0, rr);
+#pragma unroll
+      for (int s = 0; s < 9; s++) {
+        const int dx = s / 3, dy = s % 3;
+        if (s + 1 < 9) read_w(s + 1);
+        if (dx + 1 < 3) {
+#pragma unroll
+          for (int rr = dy * ROWS / 3; rr < (dy + 1) * ROWS / 3; rr++) read_row(dx + 1, rr);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int r = 0; r < WR; r++)
+#pragma unroll
+          for (int pb = 0; pb < WP; pb++)
+#pragma unroll
+            for (int mb = 0; mb < MB; mb++)
+              acc[r][pb][mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(aw[s & 1][mb], bx[dx & 1][r + dy][pb],
+                                                                       acc[r][pb][mb], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if (cc + 1 == chunks) {
+        if constexpr (HEAD) {
+          // the inference head: each wave's activations (BF16, as the unfused
+          // path stores them) through LDS of its own (80 bytes a pixel: reads
+          // of neighbouring pixels on different banks), then a lane per pixel
+          // forms noisy + b + W act in the unfused head's order
+          static_assert(!HEAD || (MB == 2 && WR * WP % 4 == 0), "a lane per pixel");
+          char *act = s_w + (wres ? chunks : 2) * WBLK * 1024 + wave * (WR * TW * 80);
+#pragma unroll
+          for (int r = 0; r < WR; r++)
+#pragma unroll
+            for (int pb = 0; pb < WP; pb++)
+#pragma unroll
+              for (int mb = 0; mb < MB; mb++) {
+                typedef bf16 bf16x4 __attribute__((ext_vector_type(4)));
+                bf16x4 o;
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                  const float v = acc[r][pb][mb][i] + bias_r[mb][i];
+                  o[i] = f2bf(v > 0.f ? v : 0.f);
+                }
+                *(bf16x4 *)(act + (r * TW + pb * 16 + col) * 80 + pair_row(PAIRS, mb, kg * 4) * 2) = o;
+              }
+          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+          for (int p = lane; p < WR * TW; p += 64) {
+            const int y = cur.y0 + wave * WR + p / TW, x = cur.x0 + p % TW;
+            if (y >= a.h || x >= a.w) continue;
+            const float4 c = a.head_noisy[(size_t)y * a.head_noisy_pitch + x];
+            float o[3] = {c.x + a.head_b[0], c.y + a.head_b[1], c.z + a.head_b[2]};
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+              const bf16x8 v = *(const bf16x8 *)(act + p * 80 + q * 16);
+#pragma unroll
+              for (int i = 0; i < 8; i++) {
+                const float f = bf2f(v[i]);
+#pragma unroll
+                for (int k = 0; k < 3; k++) o[k] += a.head_w[k * 32 + q * 8 + i] * f;
+              }
+            }
+            a.head_out[(size_t)y * a.head_out_pitch + x] = make_float4(o[0], o[1], o[2], 1.f);
+          }
+        } else {
+          if constexpr (PAIRS)
+            conv_epilogue_pairs<WR, WP, MB, UP>(a, acc, bias_r, cur.n, cur.y0 + wave * WR, cur.x0, co0, col, kg);
+          else
+            conv_epilogue<WR, WP, MB, UP>(a, acc, bias_r, cur.n, cur.y0 + wave * WR, cur.x0, co0, col, kg);
+        }
+      }
+      if (more) {  // the next stage has landed, and every wave has read this one
+        // A wait for the direct loads alone: the epilogue's stores were issued
+        // after them (memory operations of a wave retire from this counter in
+        // order), and waiting for those too would hold every tile for a
+        // store's round trip.  (conv_epilogue skips rows past the image: no count.)
+        if (!PAIRS || cc + 1 < chunks)
+          asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+        else
+          asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(epilogue_stores<WR, WP, MB, UP>()) : "memory");
+      }
+      buf ^= 1;
+    }
+    if (tn >= T) break;
+    t = tn;
     cur = tile_of(t);
   }
 }
@@ -814,7 +1187,7 @@ __global__ __launch_bounds__(256, 2) void conv_first_pair_kernel(const ConvArgs 
           for (int mb = 0; mb < MB; mb++)
             acc0[j][mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w0[p][mb], bx, acc0[j][mb], 0, 0, 0);
         }
-      // bias, ReLU, BF16 (conv_store_row's rounding), zero outside the image
+      // bias, ReLU, BF16 (conv_epilogue's rounding), zero outside the image
       // (the second layer's padding) -> LDS
 #pragma unroll
       for (int j = 0; j < A_GROUP; j++) {
@@ -831,11 +1204,7 @@ __global__ __launch_bounds__(256, 2) void conv_first_pair_kernel(const ConvArgs 
         for (int mb = 0; mb < MB; mb++) {
           bf16x4 o;
 #pragma unroll
-          for (int i = 0; i < 4; i++) {
-            float v = acc0[j][mb][i] + bias0[mb][i];
-            v = v > 0.f ? v : 0.f;
-            o[i] = f2bf(in ? v : 0.f);
-          }
+          for (int i = 0; i < 4; i++) o[i] = f2bf(in ? relu(acc0[j][mb][i] + bias0[mb][i]) : 0.f);
           *(bf16x4 *)(s_b + (mb * 2 + (kg >> 1)) * PLANE_B + q * 8 + (kg & 1) * 4) = o;
           if (keep) *(bf16x4 *)(a0.out0 + (((size_t)n * a0.h + y) * a0.w + x) * 32 + mb * 16 + kg * 4) = o;
         }
@@ -873,48 +1242,8 @@ __global__ __launch_bounds__(256, 2) void conv_first_pair_kernel(const ConvArgs 
               acc[r][pb][mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(aw[mb], bx[r + dy][pb], acc[r][pb][mb], 0, 0, 0);
       }
     }
-    // 2x2 pool of the stored (BF16) outputs (conv3x3_lds_kernel's pool
-    // epilogue: rows r, r + 1 of this lane, columns x, x + 1 of lanes col,
-    // col + 1, summed in avgpool_kernel's order)
-    {
-      const int hh = a1.h >> 1, ww = a1.w >> 1;
-#pragma unroll
-      for (int r = 0; r + 1 < WR; r += 2) {
-        const int y = y0 + wave * WR + r;
-#pragma unroll
-        for (int pb = 0; pb < WP; pb++) {
-          const int x = x0 + pb * 16 + col;
-#pragma unroll
-          for (int mb = 0; mb < MB; mb++) {
-            const int co = mb * 16 + kg * 4;
-            float tv[4], bv[4], tn[4], bn[4];
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-              float v0 = acc[r][pb][mb][i] + bias1[mb][i], v1 = acc[r + 1][pb][mb][i] + bias1[mb][i];
-              v0 = v0 > 0.f ? v0 : 0.f;
-              v1 = v1 > 0.f ? v1 : 0.f;
-              tv[i] = bf2f(f2bf(v0));
-              bv[i] = bf2f(f2bf(v1));
-              tn[i] = lane_xor1(tv[i]);
-              bn[i] = lane_xor1(bv[i]);
-            }
-            if (!(col & 1) && (y >> 1) < hh && (x >> 1) < ww) {
-              typedef bf16 bf16x4 __attribute__((ext_vector_type(4)));
-              bf16x4 o;
-#pragma unroll
-              for (int i = 0; i < 4; i++) o[i] = f2bf((((tv[i] + tn[i]) + bv[i]) + bn[i]) * 0.25f);
-              *(bf16x4 *)(a1.pool_out + (((size_t)n * hh + (y >> 1)) * ww + (x >> 1)) * 32 + co) = o;
-            }
-          }
-        }
-      }
-    }
-#pragma unroll
-    for (int r = 0; r < WR; r++) {
-      const int y = y0 + wave * WR + r;
-      if (y >= a1.h) break;
-      conv_store_row<WP, MB>(a1, acc[r], bias1, n, y, x0, col, kg, 0);
-    }
+    // with its 2x2 pool
+    conv_epilogue<WR, WP, MB, false>(a1, acc, bias1, n, y0 + wave * WR, x0, 0, col, kg);
     t += gridDim.x;
     if (t >= T) break;
   }
@@ -1455,24 +1784,33 @@ static unsigned grid_for(size_t work, size_t per_block) {
 
 // Register tiles (R rows, PB pixel blocks) offered per output-channel block
 // count MB, accumulators R * PB * MB * 4 VGPRs <= 128; entry 0 is the
-// default, the others are the autotuner's candidates.
+// default, the others are the autotuner's candidates.  Which tile a layer gets
+// is measured at the network's shape (1920 x 1080, us: best register tile /
+// best conv3x3_lds_kernel tile / best conv3x3_dma_kernel tile): 32 -> 32 at full
+// size 84 / 57 / 55; 32 -> 64 at half size 51 / 36 / 27; 128 -> 64 99 / 57 /
+// 41; 64 -> 128 at a quarter 63 / 28 / 22; 192 -> 64 at half size 213 / 113 /
+// 95.  The smallest images go the other way (quarter size of 256 x 256:
+// 12.4 / 13.5 / 19): the direct-load tiles are the largest, and too few of them
+// fill the chip.
 struct ConvTile {
-  int r, pb, lds;  // lds: conv3x3_lds_kernel with WR = r, WP = pb
+  int r, pb, lds;  // lds: 1 conv3x3_lds_kernel, 2 conv3x3_dma_kernel with WR = r, WP = pb
   int mbw;         // lds: output-channel blocks per workgroup (cout / (16 * mbw) splits)
   int per_cu;      // lds: workgroups per CU walking the tiles, 0 = one workgroup per tile
+  int nw;          // dma: waves per workgroup
 };
 static const ConvTile kTiles1[] = {{4, 2, 0, 1, 0}, {2, 4, 0, 1, 0}, {4, 4, 0, 1, 0}, {1, 4, 0, 1, 0}};
-static const ConvTile kTiles2[] = {{4, 2, 0, 2, 0}, {2, 4, 0, 2, 0}, {4, 4, 0, 2, 0}, {1, 4, 0, 2, 0},
-                                   {2, 4, 1, 2, 0}, {2, 2, 1, 2, 0}, {1, 4, 1, 2, 0}, {2, 4, 1, 2, 2},
-                                   {2, 2, 1, 2, 3}, {1, 4, 1, 2, 3}};
-static const ConvTile kTiles4[] = {{2, 2, 0, 4, 0}, {4, 2, 0, 4, 0}, {2, 4, 0, 4, 0}, {1, 4, 0, 4, 0},
-                                   {2, 2, 1, 4, 0}, {1, 4, 1, 4, 0}, {1, 2, 1, 4, 0}, {2, 2, 1, 4, 2},
-                                   {1, 2, 1, 4, 3}, {2, 4, 1, 2, 0}, {2, 2, 1, 2, 3}};
-static const ConvTile kTiles6[] = {{2, 2, 0, 6, 0}, {1, 4, 0, 6, 0}, {1, 2, 0, 6, 0}, {2, 4, 1, 2, 0},
-                                   {2, 2, 1, 2, 3}};
-static const ConvTile kTiles8[] = {{1, 2, 0, 8, 0}, {2, 2, 0, 8, 0}, {1, 4, 0, 8, 0}, {2, 2, 1, 4, 0},
-                                   {1, 2, 1, 4, 3}, {2, 2, 1, 4, 2}};
-static const ConvTile kTiles12[] = {{1, 2, 0, 12, 0}, {2, 1, 0, 12, 0}, {2, 2, 1, 4, 0}, {1, 2, 1, 4, 3}};
+static const ConvTile kTiles2[] = {{4, 2, 0, 2, 0}, {2, 4, 0, 2, 0}, {4, 4, 0, 2, 0},   {1, 4, 0, 2, 0},
+                                   {2, 4, 1, 2, 0}, {2, 2, 1, 2, 0}, {1, 4, 1, 2, 0},   {2, 4, 1, 2, 2},
+                                   {2, 2, 1, 2, 3}, {1, 4, 1, 2, 3}, {2, 2, 2, 2, 2, 4}, {2, 2, 2, 2, 1, 8}};
+static const ConvTile kTiles4[] = {{2, 2, 0, 4, 0}, {4, 2, 0, 4, 0}, {2, 4, 0, 4, 0}, {1, 4, 0, 4, 0},   {2, 2, 1, 4, 0},
+                                   {1, 4, 1, 4, 0}, {1, 2, 1, 4, 0}, {2, 2, 1, 4, 2}, {1, 2, 1, 4, 3},   {2, 4, 1, 2, 0},
+                                   {2, 2, 1, 2, 3}, {2, 2, 2, 4, 1, 4}, {2, 2, 2, 4, 1, 8}};
+static const ConvTile kTiles6[] = {{2, 2, 0, 6, 0}, {1, 4, 0, 6, 0}, {1, 2, 0, 6, 0},
+                                   {2, 4, 1, 2, 0}, {2, 2, 1, 2, 3}, {2, 2, 2, 2, 2, 4}};
+static const ConvTile kTiles8[] = {{1, 2, 0, 8, 0}, {2, 2, 0, 8, 0}, {1, 4, 0, 8, 0},   {2, 2, 1, 4, 0},
+                                   {1, 2, 1, 4, 3}, {2, 2, 1, 4, 2}, {2, 2, 2, 4, 1, 4}, {2, 2, 2, 4, 1, 8}};
+static const ConvTile kTiles12[] = {{1, 2, 0, 12, 0}, {2, 1, 0, 12, 0},   {2, 2, 1, 4, 0},
+                                    {1, 2, 1, 4, 3},  {2, 2, 2, 4, 1, 4}, {2, 2, 2, 4, 1, 8}};
 
 static const ConvTile *conv_tiles(int mb, int *count) {
 #define LGX_TILES(T) \
@@ -1539,26 +1877,41 @@ template <int MBW, int WR, int WP> static void launch_conv_lds(const ConvArgs &a
                          splits);
       return;
     }
-    if (a.gin_fmt == 1) {
-      hipLaunchKernelGGL((conv3x3_lds_kernel<MBW, WR, WP, false, 1>), dim3((unsigned)grid), dim3(256), 0, s, a, tx, ty,
-                         splits);
-      return;
-    }
-    if (a.gin_fmt == 2) {
-      hipLaunchKernelGGL((conv3x3_lds_kernel<MBW, WR, WP, false, 2>), dim3((unsigned)grid), dim3(256), 0, s, a, tx, ty,
-                         splits);
-      return;
-    }
   }
   if constexpr (WR % 2 == 0) {
     if (a.up_out) {
-      hipLaunchKernelGGL((conv3x3_lds_kernel<MBW, WR, WP, false, 0, true>), dim3((unsigned)grid), dim3(256), 0, s, a,
+      hipLaunchKernelGGL((conv3x3_lds_kernel<MBW, WR, WP, false, true>), dim3((unsigned)grid), dim3(256), 0, s, a,
                          tx, ty, splits);
       return;
     }
   }
   hipLaunchKernelGGL((conv3x3_lds_kernel<MBW, WR, WP, false>), dim3((unsigned)grid), dim3(256), 0, s, a, tx, ty,
                      splits);
+}
+
+// Weights resident when two input buffers and all chunks' weights leave room
+// for `per_cu` workgroups' LDS; a tile shape that does not fit either way is
+// an error (none of the network's layers).
+template <int MBW, int WR, int WP, int NW> static hipError_t launch_conv_dma(const ConvArgs &a, int per_cu, hipStream_t s) {
+  const int tx = (a.w + 16 * WP - 1) / (16 * WP), ty = (a.h + NW * WR - 1) / (NW * WR), splits = a.cout / (16 * MBW);
+  const int chunks = (a.ca + a.cb) / 32, cap = 160 * 1024 / per_cu;
+  const bool head = a.head_out != nullptr;
+  const int wres = dma_lds_bytes(MBW, WR, WP, NW, head, chunks) <= cap ? 1 : 0;
+  const int lds = dma_lds_bytes(MBW, WR, WP, NW, head, wres ? chunks : 2);
+  if (lds > 160 * 1024 || (conv_pairs(MBW) && a.split % 32)) return hipErrorInvalidValue;
+  const long tiles = (long)tx * ty * a.n;
+  const long grid = std::min(tiles, std::max(1L, (long)per_cu * cu_count() / splits)) * splits;
+  constexpr int OCC = NW * (NW == 4 && MBW == 2 && WR * WP == 4 ? 2 : 1) / 4;
+  auto launch = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(64 * NW), (size_t)lds, s, a, tx, ty, splits, wres);
+    return hipGetLastError();
+  };
+  if constexpr (MBW == 2) {
+    if (head) return launch(conv3x3_dma_kernel<MBW, WR, WP, NW, OCC, true, false>);
+  }
+  if (head) return hipErrorInvalidValue;
+  if (a.up_out) return launch(conv3x3_dma_kernel<MBW, WR, WP, NW, OCC, false, true>);
+  return launch(conv3x3_dma_kernel<MBW, WR, WP, NW, OCC, false, false>);
 }
 
 template <int MB> static hipError_t conv_mb(const ConvArgs &a, const ConvTile &t, hipStream_t s) {
@@ -1568,7 +1921,7 @@ template <int MB> static hipError_t conv_mb(const ConvArgs &a, const ConvTile &t
     return hipGetLastError(); \
   }
 #define LGX_LDS(MBW, RR, PP) \
-  if (t.lds && t.mbw == MBW && t.r == RR && t.pb == PP) { \
+  if (t.lds == 1 && t.mbw == MBW && t.r == RR && t.pb == PP) { \
     launch_conv_lds<MBW, RR, PP>(a, t.per_cu, s); \
     return hipGetLastError(); \
   }
@@ -1581,23 +1934,27 @@ template <int MB> static hipError_t conv_mb(const ConvArgs &a, const ConvTile &t
   } else {
     LGX_CASE(1, 2) LGX_CASE(2, 1)
   }
+#define LGX_DMA(MBW, RR, PP, NW) \
+  if (t.lds == 2 && t.mbw == MBW && t.r == RR && t.pb == PP && t.nw == NW) \
+    return launch_conv_dma<MBW, RR, PP, NW>(a, t.per_cu, s);
   if constexpr (MB % 2 == 0) {
+    LGX_DMA(2, 2, 2, 4) LGX_DMA(2, 2, 2, 8)
     LGX_LDS(2, 2, 4) LGX_LDS(2, 2, 2) LGX_LDS(2, 1, 4)
   }
   if constexpr (MB % 4 == 0) {
+    LGX_DMA(4, 2, 2, 4) LGX_DMA(4, 2, 2, 8)
     LGX_LDS(4, 2, 2) LGX_LDS(4, 1, 4) LGX_LDS(4, 1, 2)
   }
 #undef LGX_CASE
 #undef LGX_LDS
+#undef LGX_DMA
   return hipErrorInvalidValue;
 }
 
 hipError_t conv3x3(const ConvArgs &a, hipStream_t s) {
-  if (a.cout % 16) return hipErrorInvalidValue;
+  if (a.cout % 16 || (a.bias != nullptr) != (a.relu != 0)) return hipErrorInvalidValue;
   if (a.head_out && (a.cout != 32 || a.n != 1 || !conv3x3_tile_lds(a.cout, a.tile))) return hipErrorInvalidValue;
-  if (a.gin_fmt && (a.gin_fmt > 2 || a.head_out || a.cout != 32 || a.n != 1 || a.ca != 32 || a.cb ||
-                    !conv3x3_tile_lds(a.cout, a.tile)))
-    return hipErrorInvalidValue;
+  if (a.gin_fmt) return hipErrorInvalidValue;  // records packed while staging: conv_first_pair
   if (a.pool_out && (a.head_out || a.mask0 || a.mask1 || !conv3x3_tile_pool(a.cout, a.tile)))
     return hipErrorInvalidValue;
   if (a.up_out && (a.head_out || a.pool_out || a.mask0 || !a.up_mask || a.split < 16 || a.h % 2 || a.w % 2 ||
