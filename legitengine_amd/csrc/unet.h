@@ -41,7 +41,7 @@ struct ConvArgs {
   const void *gin_normal, *gin_albedo;
   int gin_noisy_pitch, gin_depth_pitch, gin_normal_pitch, gin_albedo_pitch;
   const float *gin_x12;  // conv_first_pair with gin_fmt 3: the input records [n][h][w][12]
-  bf16 *rec_out;         // conv_first_pair: optional, the packed 32-channel records of every pixel
+  bf16 *rec_out;         // conv_first_pair with gin_fmt 3: the packed 32-channel records of every pixel
   // Also write the 2x2 average pool of the output (NHWC, h/2 x w/2, cout
   // channels), summed as avgpool_kernel sums it; null = off.  Needs an LDS
   // tile whose waves hold an even number of rows (conv3x3_tile_pool).
@@ -74,10 +74,11 @@ struct WgradArgs {
 };
 
 hipError_t conv3x3(const ConvArgs &a, hipStream_t s);
-// The first convolution from the G-buffer (a0: gin_* set, n = 1) or from input records (gin_fmt 3, gin_x12, any n) and the second
-// one with its 2x2 pool (a1: out0, pool_out) in one kernel; the first
-// layer's output stays in LDS and also goes to a0.out0 when set (the
-// training forward keeps it for the backward pass).
+// The first convolution from the G-buffer (a0: gin_fmt 1 or 2, gin_* set,
+// n = 1) or from input records (gin_fmt 3, gin_x12, any n) and the second one
+// with its 2x2 pool (a1: out0, pool_out) in one kernel.  From the G-buffer the
+// first layer's output stays in LDS; from records it also goes to a0.out0 and
+// the packed records to a0.rec_out, which the backward pass reads.
 hipError_t conv_first_pair(const ConvArgs &a0, const ConvArgs &a1, hipStream_t s);
 int conv3x3_tiles(int cout);  // register tiles offered for this output channel count
 int conv3x3_tile_lds(int cout, int tile);  // 1 if that tile is an LDS tile covering all cout channels

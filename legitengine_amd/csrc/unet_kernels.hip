@@ -18,6 +18,7 @@
 // A is read from the packed weights, B straight from the NHWC activations
 // (16 bytes = 8 channels of one pixel per lane), and each lane's result is 4
 // consecutive output channels of one pixel (one 8-byte store).
+#include <limits.h>
 #include <math.h>
 
 #include <algorithm>
@@ -96,7 +97,7 @@ LGX_D void row_store(__amdgpu_buffer_rsrc_t r, int offset, bf16x4 v) {
 LGX_D bf16x4 row_load(__amdgpu_buffer_rsrc_t r, int offset) {
   return __builtin_bit_cast(bf16x4, __builtin_amdgcn_raw_buffer_load_b64(r, offset, 0, 0));
 }
-LGX_D float relu(float v) { return v > 0.f ? v : 0.f; }
+LGX_D float relu(float v) { return fmaxf(v, 0.f); }  // one instruction; NaN and -0 give +0
 // v with the channels zeroed whose mask is not positive (NaN: zeroed)
 LGX_D bf16x4 masked(bf16x4 v, bf16x4 m) {
 #pragma unroll
@@ -671,6 +672,12 @@ LGX_D bf16x8 masked8(bf16x8 v, bf16x8 m) {
   for (int i = 0; i < 8; i++) v[i] = bf2f(m[i]) > 0.f ? v[i] : f2bf(0.f);
   return v;
 }
+// Element i (a constant) as a float, from the packed words: the compiler turns bf2f(v[i]) of a converted
+// vector into a conversion of that element of its own.
+LGX_D float unpack8(bf16x8 v, int i) {
+  const uint32_t u = __builtin_bit_cast(u32x4, v)[i >> 1];
+  return __builtin_bit_cast(float, i & 1 ? u & 0xffff0000u : u << 16);
+}
 template <int WR, int WP, int MB, bool UP>
 LGX_D void conv_epilogue_pairs(const ConvArgs &a, const f32x4 (&acc)[WR][WP][MB], const float (&bias_r)[MB][4], int n,
                                int y0, int x0, int co0, int col, int kg) {
@@ -1038,214 +1045,291 @@ __global__ __launch_bounds__(64 * NW, OCC) void conv3x3_dma_kernel(const ConvArg
 }
 
 // The first two convolutions in one kernel (inference and the training
-// forward).  A workgroup's tile is 8 x 32 pixels of the second convolution's
-// output.  Its input, the first convolution's output over the tile and a
-// 1-pixel halo (10 x 34), is computed into LDS from the input records of the
-// tile and a 2-pixel halo (12 x 36, packed from the G-buffer or the FP32
-// records while staging, as pack_input_kernel packs them) and goes to HBM
-// only when the backward pass needs it: about half of the two layers' HBM
-// traffic, for 1.33x the first layer's matrix work (the halo).  The first
-// layer's records have 9 channels, padded to 16, so one tap per 32-deep MFMA
-// would leave half of K zero; here taps 2p and 2p + 1 share an MFMA
-// (k = 16 * (tap & 1) + channel; the tenth tap is zero): 5 MFMAs per output
-// block instead of 9.  (conv3x3 on the packed records, one tap per MFMA,
-// rounds the partial sums differently.)  The second convolution is
-// conv3x3_lds_kernel<2, 2, 2> on that LDS tile: the same operand order and
-// the same epilogue, with the 2x2 pool.  Persistent: a workgroup walks the
-// tiles t, t + gridDim.x, ...; the next tile's raw texels are in flight
-// during the current tile's matrix work.
-template <int GIN>
-__global__ __launch_bounds__(256, 2) void conv_first_pair_kernel(const ConvArgs a0, const ConvArgs a1, int tiles_x,
-                                                                 int tiles_y) {
-  constexpr int MB = 2, WR = 2, WP = 2;
-  constexpr int TH = 4 * WR, TW = 16 * WP;  // output tile
-  constexpr int IH = TH + 2, IW = TW + 2;   // first-layer outputs (the second layer's input tile)
-  constexpr int AH = TH + 4, AW = TW + 4;   // input records
-  constexpr int NA = AH * AW, NB = IH * IW;
-  constexpr int PLANE_A = NA * 8, PLANE_B = (NB * 8 + 127) / 128 * 128, PLANE_W = 9 * MB * 16 * 8;
-  constexpr int A_BLOCKS = (NB + 15) / 16;   // 16-pixel blocks of first-layer outputs
-  constexpr int A_PER = (A_BLOCKS + 3) / 4;  // per wave (blocks wave, wave + 4, ...)
-  constexpr int A_GROUP = 3;                 // blocks per pass (shared weight registers)
-  constexpr int GIN_PER = (NA + 255) / 256;
-  constexpr int W_PIECES = 9 * MB * 16 * 4, W_PER = (W_PIECES + 255) / 256;
-  static_assert(A_PER % A_GROUP == 0, "block groups");
-  __shared__ __attribute__((aligned(16))) bf16 s_a[2 * PLANE_A];  // records: channels 0-7, 8-15
-  __shared__ __attribute__((aligned(16))) bf16 s_b[4 * PLANE_B];  // first-layer outputs, 4 x 8 channels
-  __shared__ __attribute__((aligned(16))) bf16 s_w[4 * PLANE_W];  // second-layer weights (resident)
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int col = lane & 15, kg = lane >> 4;
-  const int T = tiles_x * tiles_y * a0.n;  // image-major
-  int t = blockIdx.x;
-  if (t >= T) return;  // the whole workgroup, before any barrier
+// forward): the first one's output goes to HBM only when the backward pass
+// needs it, which is about half of the two layers' traffic.
+//
+// One wave is one workgroup and walks down a strip 30 output columns wide,
+// two rows an iteration: the strip's records (34 columns, packed from the
+// G-buffer or the FP32 records as pack_input_kernel packs them) and the first
+// layer's output (32 columns, two 16-pixel blocks) live in LDS rings of four
+// rows, so each row of either is formed once, and nothing waits at a
+// barrier.  A strip is cut into segments of `len` row pairs so that there are
+// about as many waves as fit the chip; a segment forms two extra rows of the
+// first layer.
+//
+// First layer: its records have 9 channels, padded to 16, so one tap per
+// 32-deep MFMA would leave half of K zero; here taps 2p and 2p + 1 share an
+// MFMA (k = 16 * (tap & 1) + channel; the tenth tap is zero): 5 MFMAs per
+// output block instead of 9.  (conv3x3 on the packed records, one tap per
+// MFMA, rounds the partial sums differently.)  Second layer: conv3x3's order
+// (dx, dy), its weights in registers, with the 2x2 pool.
+//
+// What bounds it: issue.  An iteration has 112 MFMAs (1800 cycles) and 350 other
+// vector instructions, which the two waves of a SIMD overlap in part.  From
+// the G-buffer at 1920 x 1080: 71 us, where 225 MB of traffic take 44 at a
+// copy's rate; with workgroups of four waves that staged an 8 x 32 tile,
+// formed its halo and met at two barriers a tile, 141.  From records with
+// both layers kept (16 x 256 x 256): 60 us for 270 MB, 81 before.
+//
+// LDS: two halves (8 KB apart) of two rows each; iteration k writes half k & 1
+// and reads both.  In a half: records, [plane of 8 channels][row][pixel],
+// then first-layer outputs, the same with four planes; planes are 1280 bytes
+// (a multiple of the banks, as in conv3x3_lds_kernel), rows 640.
+constexpr int kPairCols = 30;           // output columns of a strip
+constexpr int kPairRow = 640, kPairPlane = 2 * kPairRow, kPairOut = 2 * kPairPlane, kPairHalf = 8192;
+// zeros the tenth tap reads (with its zero weights: no 0 * inf), at row and block steps of 640 and 256 bytes
+constexpr int kPairZero = 2 * kPairHalf;
+template <int GIN, bool KEEP>
+__global__ __launch_bounds__(64, 2) void conv_first_pair_kernel(const ConvArgs a0, const ConvArgs a1, int strips,
+                                                                int segs, int len) {
+  __shared__ __attribute__((aligned(256))) char s[2 * kPairHalf + 1024];
+  const int lane = threadIdx.x, col = lane & 15, kg = lane >> 4;
+  const uint32_t id = xcd_remap(blockIdx.x, gridDim.x);
+  const int x0 = (int)(id % (uint32_t)strips) * kPairCols, seg = (int)(id / (uint32_t)strips) % segs,
+            n = (int)(id / (uint32_t)(strips * segs));
+  const int ys = seg * len * 2, pairs = min(len, (a0.h + 1) / 2 - seg * len), h = a0.h, w = a0.w;
   const bf16x8 zero8 = {};
-  // second-layer weights -> LDS (conv3x3_lds_kernel's layout and pieces)
-  {
-    bf16x8 pw[W_PER];
+  // First-layer weights: the A operand of pair p, block mb holds tap 2p + (kg >> 1), channels 8 * (kg & 1)
+  // .. + 7; its rows are ordered (pair_row) so that a lane's outputs are channels 8 kg .. 8 kg + 7.
+  bf16x8 w0[5][2], w1[9][2];
 #pragma unroll
-    for (int i = 0; i < W_PER; i++) {
-      const int q = min(tid + i * 256, W_PIECES - 1);
-      const int row = ((q >> 6) << 4) + (q & 15), part = (q >> 4) & 3;
-      const int tap = row / (MB * 16), co = row % (MB * 16);
-      pw[i] = *(const bf16x8 *)(a1.wt + (size_t)tap * 32 * 32 + (co * 4 + part) * 8);
+  for (int p = 0; p < 5; p++)
+#pragma unroll
+    for (int mb = 0; mb < 2; mb++) {
+      const int tap = 2 * p + (kg >> 1);
+      w0[p][mb] = tap < 9 ? *(const bf16x8 *)(a0.wt + ((size_t)tap * 32 + pair_row(true, mb, col)) * 32 + (kg & 1) * 8)
+                          : zero8;
     }
 #pragma unroll
-    for (int i = 0; i < W_PER; i++) {
-      const int q = tid + i * 256;
-      const int row = ((q >> 6) << 4) + (q & 15), part = (q >> 4) & 3;
-      if (q < W_PIECES) *(bf16x8 *)(s_w + part * PLANE_W + row * 8) = pw[i];
+  for (int tap = 0; tap < 9; tap++)
+#pragma unroll
+    for (int mb = 0; mb < 2; mb++)
+      w1[tap][mb] = *(const bf16x8 *)(a1.wt + ((size_t)tap * 32 + pair_row(true, mb, col)) * 32 + kg * 8);
+  // A first-layer column outside the image has bias -inf: ReLU makes every sum (NaN, too) the zero that the
+  // second layer's padding is.
+  float bias0[2][8], bias1[8];
+#pragma unroll
+  for (int i = 0; i < 8; i++) {
+    const float b = a0.bias[kg * 8 + i];
+#pragma unroll
+    for (int pb = 0; pb < 2; pb++) {
+      const int x = x0 - 1 + pb * 16 + col;
+      bias0[pb][i] = x >= 0 && x < w ? b : -INFINITY;
     }
+    bias1[i] = a1.bias[kg * 8 + i];
   }
-  // first-layer weights in registers: the A operand of pair p, block mb
-  // (output channel mb * 16 + col; k group kg = tap 2p + (kg >> 1),
-  // channels 8 * (kg & 1) .. + 7 of the packed [tap][cout][32] weights)
-  bf16x8 w0[5][MB];
-  int toff[5];  // this lane's tap offset (elements) in the record tile, per pair
+  // this lane's record column (lanes past 33 repeat the last and store nothing)
+  const int rpx = min(lane, 33), rx = x0 - 2 + rpx, rxc = min(max(rx, 0), w - 1);
+  const bool rx_in = rx >= 0 && rx < w;
+  GinRaw<GIN> raw[2];
+  auto fetch = [&](int y) {  // rows y, y + 1 (clamped into the image)
 #pragma unroll
-  for (int p = 0; p < 5; p++) {
-    const int tap = 2 * p + (kg >> 1);
-    toff[p] = tap < 9 ? ((tap / 3) * AW + tap % 3) * 8 : 0;
+    for (int i = 0; i < 2; i++) raw[i] = gin_load<GIN>(a0, min(max(y + i, 0), h - 1), rxc, n);
+  };
+  // rows y, y + 1 into a half: zero outside the image (the first layer's padding); a segment's own pixels
+  // also to rec_out when asked (pack_input_kernel's layout: the training backward reads them)
+  auto stage = [&](int y, int half, bool own) {
 #pragma unroll
-    for (int mb = 0; mb < MB; mb++)
-      w0[p][mb] = tap < 9 ? *(const bf16x8 *)(a0.wt + ((size_t)tap * 32 + mb * 16 + col) * 32 + (kg & 1) * 8) : zero8;
-  }
-  float bias0[MB][4], bias1[MB][4];
-#pragma unroll
-  for (int mb = 0; mb < MB; mb++)
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      bias0[mb][i] = a0.bias[mb * 16 + kg * 4 + i];
-      bias1[mb][i] = a1.bias[mb * 16 + kg * 4 + i];
+    for (int i = 0; i < 2; i++) {
+      const bool in = rx_in && y + i >= 0 && y + i < h;
+      bf16x8 v0, v1;
+      gin_pack<GIN>(raw[i], v0, v1);
+      v0 = in ? v0 : zero8;
+      v1 = in ? v1 : zero8;
+      if (lane < 34) {
+        *(bf16x8 *)(s + half + i * kPairRow + rpx * 16) = v0;
+        *(bf16x8 *)(s + half + kPairPlane + i * kPairRow + rpx * 16) = v1;
+      }
     }
-  GinRaw<GIN> graw[GIN_PER];
-  uint32_t valid = 0;
-  auto fetch = [&](int tt) {
-    const int u = tt % (tiles_x * tiles_y), n = tt / (tiles_x * tiles_y);
-    const int x0 = (u % tiles_x) * TW, y0 = (u / tiles_x) * TH;
-    valid = 0;
+    if constexpr (KEEP) {  // four lanes a pixel, 16 pixels a store, so that a store is one run of memory
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      const int part = lane & 3, px = 2 + (lane >> 2);
+      const char *from = part < 2 ? s + half + part * kPairPlane + px * 16 : s + kPairZero;
 #pragma unroll
-    for (int i = 0; i < GIN_PER; i++) {
-      const int p = min(tid + i * 256, NA - 1);
-      const int y = y0 - 2 + p / AW, x = x0 - 2 + p % AW;
-      const bool ok = y >= 0 && y < a0.h && x >= 0 && x < a0.w;
-      graw[i] = gin_load<GIN>(a0, min(max(y, 0), a0.h - 1), min(max(x, 0), a0.w - 1), n);
-      valid |= (uint32_t)ok << i;
+      for (int i = 0; i < 2; i++) {
+        const bool in = own && y + i < h;
+        const __amdgpu_buffer_rsrc_t rs = row_rsrc(a0.rec_out, in ? (size_t)n * h + y + i : 0, in ? w : 0, 32);
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+          row_store8(rs, px + j * 16 < 2 + kPairCols ? (x0 - 2 + px + j * 16) * 64 + part * 16 : (int)0x80000000u,
+                     *(const bf16x8 *)(from + i * kPairRow + j * 256));
+      }
     }
   };
-  fetch(t);
-  for (;;) {
-    const int u = t % (tiles_x * tiles_y), n = t / (tiles_x * tiles_y);
-    const int x0 = (u % tiles_x) * TW, y0 = (u / tiles_x) * TH;
-    // records -> LDS (zero outside the image: the first layer's padding);
-    // the tile's own pixels also to rec_out when asked (pack_input_kernel's
-    // layout: the training backward reads them)
+  // this lane's kept first-layer columns (1 .. 30, the strip's own) in a row of out0
+  int keep_at[2];
 #pragma unroll
-    for (int i = 0; i < GIN_PER; i++) {
-      const int p = tid + i * 256;
-      bf16x8 v0 = {}, v1 = {};
-      if ((valid >> i) & 1u) gin_pack<GIN>(graw[i], v0, v1);
-      if (p < NA) {
-        *(bf16x8 *)(s_a + p * 8) = v0;
-        *(bf16x8 *)(s_a + PLANE_A + p * 8) = v1;
-        const int ry = p / AW, rx = p % AW;
-        if (a0.rec_out && ((valid >> i) & 1u) && ry >= 2 && ry < 2 + TH && rx >= 2 && rx < 2 + TW) {
-          bf16 *dst = a0.rec_out + (((size_t)n * a0.h + (y0 - 2 + ry)) * a0.w + (x0 - 2 + rx)) * 32;
-          *(bf16x8 *)dst = v0;
-          *(bf16x8 *)(dst + 8) = v1;
-          *(bf16x8 *)(dst + 16) = zero8;
-          *(bf16x8 *)(dst + 24) = zero8;
-        }
+  for (int pb = 0; pb < 2; pb++) {
+    const int c = pb * 16 + col, x = x0 - 1 + c;
+    keep_at[pb] = c >= 1 && c <= kPairCols ? x * 64 + kg * 16 : (int)0x80000000u;
+  }
+  // First layer, rows y (from record rows lo 0, lo 1, hi 0) and y + 1 (lo 1, hi 0, hi 1), to half hi.
+  auto first = [&](int y, int lo, int hi, bool own0, bool own1) {
+    const int lane_off = col * 16 + (kg & 1) * kPairPlane;
+    const int up = kg >> 1;  // the upper tap of a pair
+    const char *const alo = s + lo + lane_off + up * 16, *const ahi = s + hi + lane_off + up * 16;
+    // taps 2 and 3: (row, dx 2) and (row + 1, dx 0)
+    const char *const b0 = s + lo + lane_off + (up ? kPairRow : 32);
+    const char *const b1 = s + lane_off + (up ? hi : lo + kPairRow + 32);
+    const char *const c8 = up ? s + kPairZero : ahi + 32;
+    auto operand = [&](int st, int pb) {
+      const int p = st >> 1, r = st & 1;
+      const char *at;
+      if (p == 0) at = alo + r * kPairRow;                       // taps 0, 1: row r
+      else if (p == 1) at = r ? b1 : b0;                         // taps 2, 3
+      else if (p == 2) at = r ? ahi + 16 : alo + kPairRow + 16;  // taps 4, 5: row r + 1
+      else if (p == 3) at = ahi + r * kPairRow;                  // taps 6, 7: row r + 2
+      else at = c8 + r * kPairRow;                               // tap 8 and, in the upper lanes, zeros
+      return *(const bf16x8 *)(at + pb * 256);
+    };
+    f32x4 acc[2][2][2];
+#pragma unroll
+    for (int r = 0; r < 2; r++)
+#pragma unroll
+      for (int pb = 0; pb < 2; pb++)
+#pragma unroll
+        for (int mb = 0; mb < 2; mb++) acc[r][pb][mb] = f32x4{0.f, 0.f, 0.f, 0.f};
+    constexpr int D = 4;
+    bf16x8 bx[D][2];
+#pragma unroll
+    for (int st = 0; st < D - 1; st++)
+#pragma unroll
+      for (int pb = 0; pb < 2; pb++) bx[st][pb] = operand(st, pb);
+#pragma unroll
+    for (int st = 0; st < 10; st++) {
+      if (st + D - 1 < 10)
+#pragma unroll
+        for (int pb = 0; pb < 2; pb++) bx[(st + D - 1) % D][pb] = operand(st + D - 1, pb);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int pb = 0; pb < 2; pb++) {
+#pragma unroll
+        for (int mb = 0; mb < 2; mb++)
+          acc[st & 1][pb][mb] =
+              __builtin_amdgcn_mfma_f32_16x16x32_bf16(w0[st >> 1][mb], bx[st % D][pb], acc[st & 1][pb][mb], 0, 0, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    // bias, ReLU, BF16 (conv_epilogue's rounding), zero outside the image (the second layer's padding)
+#pragma unroll
+    for (int r = 0; r < 2; r++) {
+      const bool row_in = y + r >= 0 && y + r < h;
+      const bool own = KEEP && (r ? own1 : own0) && row_in;
+      const __amdgpu_buffer_rsrc_t rs = row_rsrc(KEEP ? a0.out0 : nullptr, own ? (size_t)n * h + y + r : 0, own ? w : 0, 32);
+      bf16x8 v[2];
+#pragma unroll
+      for (int pb = 0; pb < 2; pb++) {
+        f32x8 f;
+#pragma unroll
+        for (int i = 0; i < 8; i++) f[i] = relu(acc[r][pb][i >> 2][i & 3] + bias0[pb][i]);
+        v[pb] = __builtin_convertvector(f, bf16x8);
+      }
+      if (!row_in) v[0] = v[1] = zero8;
+#pragma unroll
+      for (int pb = 0; pb < 2; pb++) {
+        *(bf16x8 *)(s + hi + kPairOut + kg * kPairPlane + r * kPairRow + (pb * 16 + col) * 16) = v[pb];
+        if (KEEP) row_store8(rs, keep_at[pb], v[pb]);
       }
     }
-    __syncthreads();
-    if (t + (int)gridDim.x < T) fetch(t + (int)gridDim.x);  // in flight during the matrix work
-    // first layer: this wave's blocks, A_GROUP at a time (not unrolled: one
-    // group's operands live at a time)
-#pragma unroll 1
-    for (int g = 0; g < A_PER; g += A_GROUP) {
-      // this lane's first-layer output pixel in each block of the group
-      // (clamped: the tail block's extra lanes compute a duplicate that is
-      // not stored)
-      int abase[A_GROUP];
+  };
+  // this lane's output columns (30 of 32) in the rows of the output and of the pool
+  int out_at[2], pool_at[2];
 #pragma unroll
-      for (int j = 0; j < A_GROUP; j++) {
-        const int q = min((wave + 4 * (g + j)) * 16 + col, NB - 1);
-        abase[j] = ((q / IW) * AW + q % IW) * 8 + (kg & 1) * PLANE_A;
+  for (int pb = 0; pb < 2; pb++) {
+    const int c = pb * 16 + col, x = x0 + c;
+    out_at[pb] = c < kPairCols ? x * 64 + kg * 16 : (int)0x80000000u;
+    pool_at[pb] = c < kPairCols && !(col & 1) ? (x >> 1) * 64 + kg * 16 : (int)0x80000000u;
+  }
+  // Second layer, output rows y, y + 1 from first-layer rows lo 0, lo 1, hi 0, hi 1, and their pool.
+  auto second = [&](int y, int lo, int hi) {
+    const char *const base = s + kPairOut + kg * kPairPlane + col * 16;
+    auto operand = [&](int st, int pb) {
+      const int dx = st >> 2, rr = st & 3;
+      return *(const bf16x8 *)(base + (rr < 2 ? lo : hi) + (rr & 1) * kPairRow + (pb * 16 + dx) * 16);
+    };
+    f32x4 acc[2][2][2];
+#pragma unroll
+    for (int r = 0; r < 2; r++)
+#pragma unroll
+      for (int pb = 0; pb < 2; pb++)
+#pragma unroll
+        for (int mb = 0; mb < 2; mb++) acc[r][pb][mb] = f32x4{0.f, 0.f, 0.f, 0.f};
+    constexpr int D = 4;
+    bf16x8 bx[D][2];
+#pragma unroll
+    for (int st = 0; st < D - 1; st++)
+#pragma unroll
+      for (int pb = 0; pb < 2; pb++) bx[st][pb] = operand(st, pb);
+#pragma unroll
+    for (int st = 0; st < 12; st++) {
+      const int dx = st >> 2, rr = st & 3;
+      if (st + D - 1 < 12)
+#pragma unroll
+        for (int pb = 0; pb < 2; pb++) bx[(st + D - 1) % D][pb] = operand(st + D - 1, pb);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int r = 0; r < 2; r++) {
+        const int dy = rr - r;
+        if (dy < 0 || dy > 2) continue;
+#pragma unroll
+        for (int pb = 0; pb < 2; pb++)
+#pragma unroll
+          for (int mb = 0; mb < 2; mb++)
+            acc[r][pb][mb] =
+                __builtin_amdgcn_mfma_f32_16x16x32_bf16(w1[dy * 3 + dx][mb], bx[st % D][pb], acc[r][pb][mb], 0, 0, 0);
       }
-      f32x4 acc0[A_GROUP][MB];
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    bf16x8 v[2][2];
 #pragma unroll
-      for (int j = 0; j < A_GROUP; j++)
+    for (int r = 0; r < 2; r++) {
+      const bool in = y + r < h;
+      const __amdgpu_buffer_rsrc_t rs = row_rsrc(a1.out0, in ? (size_t)n * h + y + r : 0, in ? w : 0, 32);
 #pragma unroll
-        for (int mb = 0; mb < MB; mb++) acc0[j][mb] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int pb = 0; pb < 2; pb++) {
+        f32x8 f;
 #pragma unroll
-      for (int p = 0; p < 5; p++)
-#pragma unroll
-        for (int j = 0; j < A_GROUP; j++) {
-          if (wave + 4 * (g + j) >= A_BLOCKS) continue;  // uniform
-          bf16x8 bx = *(const bf16x8 *)(s_a + abase[j] + toff[p]);
-          if (p == 4 && kg >= 2) bx = zero8;  // the tenth tap: zero weights, and no 0 * inf
-#pragma unroll
-          for (int mb = 0; mb < MB; mb++)
-            acc0[j][mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w0[p][mb], bx, acc0[j][mb], 0, 0, 0);
-        }
-      // bias, ReLU, BF16 (conv_epilogue's rounding), zero outside the image
-      // (the second layer's padding) -> LDS
-#pragma unroll
-      for (int j = 0; j < A_GROUP; j++) {
-        const int blk = wave + 4 * (g + j);
-        const int q = blk * 16 + col;
-        if (blk >= A_BLOCKS || q >= NB) continue;
-        const int qy = q / IW, qx = q % IW;
-        const int y = y0 - 1 + qy, x = x0 - 1 + qx;
-        const bool in = y >= 0 && y < a0.h && x >= 0 && x < a0.w;
-        // the tile's own pixels (not the halo) also to HBM, when asked
-        const bool keep = a0.out0 && in && qy >= 1 && qy <= TH && qx >= 1 && qx <= TW;
-        typedef bf16 bf16x4 __attribute__((ext_vector_type(4)));
-#pragma unroll
-        for (int mb = 0; mb < MB; mb++) {
-          bf16x4 o;
-#pragma unroll
-          for (int i = 0; i < 4; i++) o[i] = f2bf(in ? relu(acc0[j][mb][i] + bias0[mb][i]) : 0.f);
-          *(bf16x4 *)(s_b + (mb * 2 + (kg >> 1)) * PLANE_B + q * 8 + (kg & 1) * 4) = o;
-          if (keep) *(bf16x4 *)(a0.out0 + (((size_t)n * a0.h + y) * a0.w + x) * 32 + mb * 16 + kg * 4) = o;
-        }
+        for (int i = 0; i < 8; i++) f[i] = relu(acc[r][pb][i >> 2][i & 3] + bias1[i]);
+        v[r][pb] = __builtin_convertvector(f, bf16x8);
+        row_store8(rs, out_at[pb], v[r][pb]);
       }
     }
-    __syncthreads();
-    // second layer on the LDS tile (conv3x3_lds_kernel's operand order)
-    f32x4 acc[WR][WP][MB];
+    const bool in = (y >> 1) < (h >> 1);
+    const __amdgpu_buffer_rsrc_t ps =
+        row_rsrc(a1.pool_out, in ? (size_t)n * (h >> 1) + (y >> 1) : 0, in ? w >> 1 : 0, 32);
 #pragma unroll
-    for (int r = 0; r < WR; r++)
+    for (int pb = 0; pb < 2; pb++) {
+      f32x8 f;
 #pragma unroll
-      for (int pb = 0; pb < WP; pb++)
-#pragma unroll
-        for (int mb = 0; mb < MB; mb++) acc[r][pb][mb] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int dx = 0; dx < 3; dx++) {
-      bf16x8 bx[WR + 2][WP];
-#pragma unroll
-      for (int rr = 0; rr < WR + 2; rr++)
-#pragma unroll
-        for (int pb = 0; pb < WP; pb++)
-          bx[rr][pb] = *(const bf16x8 *)(s_b + kg * PLANE_B + ((wave * WR + rr) * IW + pb * 16 + col + dx) * 8);
-#pragma unroll
-      for (int dy = 0; dy < 3; dy++) {
-        const int tap = dy * 3 + dx;
-        bf16x8 aw[MB];
-#pragma unroll
-        for (int mb = 0; mb < MB; mb++) aw[mb] = *(const bf16x8 *)(s_w + kg * PLANE_W + ((tap * MB + mb) * 16 + col) * 8);
-#pragma unroll
-        for (int r = 0; r < WR; r++)
-#pragma unroll
-          for (int pb = 0; pb < WP; pb++)
-#pragma unroll
-            for (int mb = 0; mb < MB; mb++)
-              acc[r][pb][mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(aw[mb], bx[r + dy][pb], acc[r][pb][mb], 0, 0, 0);
+      for (int i = 0; i < 8; i++) {
+        const float t = unpack8(v[0][pb], i), b = unpack8(v[1][pb], i);
+        f[i] = (((t + lane_xor1(t)) + b) + lane_xor1(b)) * 0.25f;
       }
+      const bf16x8 o = __builtin_convertvector(f, bf16x8);
+      row_store8(ps, pool_at[pb], o);
     }
-    // with its 2x2 pool
-    conv_epilogue<WR, WP, MB, false>(a1, acc, bias1, n, y0 + wave * WR, x0, 0, col, kg);
-    t += gridDim.x;
-    if (t >= T) break;
+  };
+  // Lanes read what other lanes of the wave wrote: LDS serves a wave in
+  // order, the fence keeps the compiler to that order too.
+  auto fence = [] { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); };
+  *(bf16x8 *)(s + kPairZero + lane * 16) = zero8;
+  fetch(ys - 2);
+  stage(ys - 2, kPairHalf, false);
+  fetch(ys);
+  stage(ys, 0, true);
+  fetch(ys + 2);
+  fence();
+  first(ys - 1, kPairHalf, 0, false, true);
+  fence();
+  for (int k = 1; k <= pairs; k++) {
+    const int hi = (k & 1) * kPairHalf, lo = kPairHalf - hi, y = ys + 2 * k;
+    stage(y, hi, k < pairs);
+    fetch(y + 2);  // (in flight during the matrix work; past the segment: clamped rows nothing reads)
+    fence();
+    first(y - 1, lo, hi, true, k < pairs);
+    fence();
+    second(y - 2, lo, hi);
+    fence();
   }
 }
 
@@ -1980,17 +2064,33 @@ hipError_t conv3x3(const ConvArgs &a, hipStream_t s) {
 hipError_t conv_first_pair(const ConvArgs &a0, const ConvArgs &a1, hipStream_t s) {
   if (a0.gin_fmt < 1 || a0.gin_fmt > 3 || (a0.gin_fmt == 3 ? !a0.gin_x12 : a0.n != 1) || a0.n < 1 ||
       a0.cout != 32 || !a0.wt || !a0.bias || a1.n != a0.n || a1.cout != 32 || a1.split != 32 || !a1.out0 ||
-      !a1.pool_out || !a1.wt || !a1.bias || a1.h != a0.h || a1.w != a0.w || a0.h < 1 || a0.w < 1)
+      !a1.pool_out || !a1.wt || !a1.bias || a1.h != a0.h || a1.w != a0.w || a0.h < 1 || a0.w < 1 ||
+      (a0.out0 != nullptr) != (a0.gin_fmt == 3) || (a0.rec_out != nullptr) != (a0.gin_fmt == 3))
     return hipErrorInvalidValue;
-  const int tx = (a0.w + 31) / 32, ty = (a0.h + 7) / 8;
-  const long tiles = (long)tx * ty * a0.n;
-  const int grid = (int)std::min(tiles, 2L * cu_count());  // two workgroups per CU fit its LDS and registers
+  // Row pairs per segment: of the lengths that fill one to four rounds of the waves that are resident at once
+  // (2 per SIMD) the one that ends first, a segment's first rows counted as 0.4 of an iteration.
+  const int strips = (a0.w + kPairCols - 1) / kPairCols, pairs = (a0.h + 1) / 2;
+  const long waves = 8L * cu_count(), columns = (long)strips * a0.n;
+  int len = pairs, segs = 1;
+  long best = LONG_MAX;
+  for (long r = 1; r <= 4; r++) {
+    const long want = std::min((long)pairs, std::max(1L, r * waves / columns)), l = (pairs + want - 1) / want,
+               k = (pairs + l - 1) / l, cost = (columns * k + waves - 1) / waves * (5 * l + 2);
+    if (cost < best) {
+      best = cost;
+      len = (int)l;
+      segs = (int)k;
+    }
+  }
+  auto launch = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3((unsigned)((long)strips * segs * a0.n)), dim3(64), 0, s, a0, a1, strips, segs, len);
+  };
   if (a0.gin_fmt == 1)
-    hipLaunchKernelGGL(conv_first_pair_kernel<1>, dim3((unsigned)grid), dim3(256), 0, s, a0, a1, tx, ty);
+    launch(conv_first_pair_kernel<1, false>);
   else if (a0.gin_fmt == 2)
-    hipLaunchKernelGGL(conv_first_pair_kernel<2>, dim3((unsigned)grid), dim3(256), 0, s, a0, a1, tx, ty);
+    launch(conv_first_pair_kernel<2, false>);
   else
-    hipLaunchKernelGGL(conv_first_pair_kernel<3>, dim3((unsigned)grid), dim3(256), 0, s, a0, a1, tx, ty);
+    launch(conv_first_pair_kernel<3, true>);
   return hipGetLastError();
 }
 
