@@ -64,7 +64,7 @@ struct WgradArgs {
   const bf16 *dy;  // NHWC cout
   int cout;
   int n, h, w;
-  int rows;        // rows per workgroup (set by conv3x3_wgrad)
+  int rows, cap;   // rows of a strip per wave, and at most per piece of a strip (set by conv3x3_wgrad)
   int cin_log;     // input channels of the master weights (the rest of ca + cb is zero padding)
   float *dw;       // [cout][cin_log][9] (master layout), overwritten
   float *db;       // [cout] bias gradient, overwritten

@@ -37,46 +37,6 @@ LGX_D bf16 f2bf(float v) { return (bf16)v; }
 
 // ------------------------------------------------------------ convolution
 
-// Input addressing shared by forward, input-gradient and weight-gradient
-// kernels: channels [0, ca) come from A (optionally nearest-upsampled from
-// half resolution), [ca, ca+cb) from B.
-struct ConvInput {
-  const bf16 *a;
-  int ca, a_up;
-  const bf16 *b;
-  int cb;
-};
-
-// 16 bytes (8 channels starting at c, c % 8 == 0, within one 32-chunk) of
-// pixel (n, y, x) of the logical input; zero outside the image.
-LGX_D bf16x8 load8(const ConvInput &in, int n, int y, int x, int h, int w, int c) {
-  bf16x8 z = {};
-  if (y < 0 || y >= h || x < 0 || x >= w) return z;
-  if (c < in.ca) {
-    if (in.a_up) {
-      const int hh = h >> 1, ww = w >> 1;
-      return *(const bf16x8 *)(in.a + (((size_t)n * hh + (y >> 1)) * ww + (x >> 1)) * in.ca + c);
-    }
-    return *(const bf16x8 *)(in.a + (((size_t)n * h + y) * w + x) * in.ca + c);
-  }
-  return *(const bf16x8 *)(in.b + (((size_t)n * h + y) * w + x) * in.cb + (c - in.ca));
-}
-
-// The same 16 bytes for a pixel clamped into the image (always a valid
-// read; the caller zeroes what lies outside).
-LGX_D bf16x8 load8_clamped(const ConvInput &in, int n, int y, int x, int h, int w, int c) {
-  y = min(max(y, 0), h - 1);
-  x = min(max(x, 0), w - 1);
-  if (c < in.ca) {
-    if (in.a_up) {
-      const int hh = h >> 1, ww = w >> 1;
-      return *(const bf16x8 *)(in.a + (((size_t)n * hh + (y >> 1)) * ww + (x >> 1)) * in.ca + c);
-    }
-    return *(const bf16x8 *)(in.a + (((size_t)n * h + y) * w + x) * in.ca + c);
-  }
-  return *(const bf16x8 *)(in.b + (((size_t)n * h + y) * w + x) * in.cb + (c - in.ca));
-}
-
 // The value of the neighbouring lane (lane ^ 1): a DPP quad permutation
 // [1, 0, 3, 2], a modifier of one VALU move (no LDS round trip as a shuffle
 // through ds_bpermute would take).
@@ -1335,192 +1295,275 @@ __global__ __launch_bounds__(64, 2) void conv_first_pair_kernel(const ConvArgs a
 
 // Weight and bias gradient of a 3x3 convolution:
 //   dW[tap][ci][co] = sum_p X[p + shift(tap)][ci] * dY[p][co],  db[co] = sum_p dY[p][co]
-// One workgroup: one image, one 32-channel group of the input, a 64-pixel
-// column band and `rows` rows, taken RB rows per round.  Per round the RB + 2
-// input rows and the RB output-gradient rows are staged in LDS transposed
-// (channel-major, written as pixel pairs) so that MFMA operands are 8
-// consecutive pixels of one channel; K runs over pixels.  Three aligned
-// 16-byte reads of an input row give the operands of its three horizontal
-// taps (the shifted ones by an element shift).
-// Wave w owns input half cb = w & 1 and the output blocks mb = (w >> 1) + 2j,
-// all 9 taps: per (row, k chunk) it reads each of its A fragments once for
-// the 9 taps and each tap's B fragment once for its MB / 2 blocks.  Each
-// workgroup stores its partial sums (no atomics) to its own slot of the
-// scratch buffer, part[group][slot][tap][ci % 32][co], and
-// wgrad_reduce_kernel adds the slots in a fixed order.  The workgroups of
-// input group 0 also sum the staged output-gradient rows per channel (the
-// bias gradient) into part_b[slot][co], reduced by bias_reduce_kernel.
-template <int MB, int RB> __global__ __launch_bounds__(256) void conv3x3_wgrad_kernel(const WgradArgs a) {
-  constexpr int XS = 64 + 16;  // staged x range [x0 - 8, x0 + 72): keeps dx = 0 reads 16-byte aligned
-  constexpr int COUT = MB * 16;
-  // LDS layouts.  A 128-bit operand read is served 16 lanes at a time, lanes
-  // col = 0..7 and col = 8..15 of one kg together: with channel rows 44 banks
-  // apart, lanes 0..7 start on 8 banks 4 apart and lanes 8..15 on the other
-  // 8, so the 16 lanes cover the 64 banks once.  A staging store writes one
-  // 32-bit pixel pair per lane, the lanes differing in their 8-channel group
-  // and pixel pair: channel rows 44 banks apart put 8-channel groups 0 or 32
-  // banks apart, and a pad of 512 / COUT banks per 16-channel group (16 for
-  // the 32 input channels) separates the rest.  A staged input row holds 32
-  // channel rows of XS pixels and is 40 banks longer than a multiple of 64,
-  // so a store whose pixel pairs run past the end of a row stays conflict
-  // free.
-  constexpr int CST = 88;                                   // channel-row stride (bf16), XS and 64 pixels used
-  constexpr int XROW = 2896;                                // >= 32 * CST + 2 * 32, 1448 banks = 40 mod 64
-  constexpr int DPAD = 1024 / COUT, DROW = COUT * CST + (COUT / 16) * DPAD;
-  static_assert(XROW >= 32 * CST + 2 * 32 && (XROW / 2) % 64 == 40, "input row layout");
-  __shared__ __align__(16) bf16 xs[(RB + 2) * XROW];
-  __shared__ __align__(16) bf16 ds[RB * DROW];
-  auto xi = [](int rr, int c, int px) { return rr * XROW + c * CST + (c >> 4) * 32 + px; };
-  auto di = [](int rr, int c, int px) { return rr * DROW + c * CST + (c >> 4) * DPAD + px; };
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+// A wave owns 32 output channels x NC blocks of 16 channels of one 32-channel
+// group of the input, all 9 taps (MFMA rows: output channels, columns: input
+// channels, K: 32 pixels of a row), and walks down a 32-pixel strip.  Step r
+// has the input row r (34 pixels) and the gradient row r + 1: the input row's
+// operands of the three horizontal taps serve the gradient rows r - 1, r and
+// r + 1, which are kept in registers, so a step is 18 NC MFMAs on 2 + 3 NC
+// operands.  The rows land in LDS by direct loads, in a ring of four steps of
+// the wave's own: nothing waits at a barrier.  The bias gradient (input
+// group 0) is one more MFMA a block, with a column of ones.
+//
+// LDS is [pixel][32 channels], as in memory; a transposing read
+// (ds_read_b64_tr_b16) gives 16 lanes 4 consecutive pixels of a channel each,
+// so there is no transposition on the way in, and a tap's shift is an address.
+// A lane group's pixels are kg 4 + 0 .. 3 and 16 more on (K in any order, the
+// same for both operands).  The 32-byte halves of pixels 4 to 7 of every 8 are
+// exchanged, which puts the 8 pixels that 32 lanes read on all banks.
+//
+// The pixels (strips x rows) of an image batch are one list, divided evenly
+// over the waves; a wave's share is one or more pieces of strips.  Each
+// workgroup adds its 8 waves' sums and stores them (no atomics) to its own slot
+// of the scratch buffer, part[group][slot][tap][ci % 32][co] and
+// part_b[slot][co]; wgrad_reduce_kernel adds the slots in a fixed order.
+//
+// What bounds it (16 x 256 x 256): 96 -> 32 at full size 56 us, of which 27 are
+// its MFMAs, 9 the direct loads that do not overlap, and 10 a launch's start,
+// first loads and last sums, which are most of the small layers (32 -> 64 at
+// half size 18 us).  Staging pixel pairs through registers into transposed
+// rows and shifting operands by elements, with one workgroup's waves at two
+// barriers a round, it was bound by LDS: 157 and 40 us; 192 -> 64 at half size
+// 114, now 61.
+constexpr int kWgradWaves = 8, kWgradSlot = 34 * 64 + 32 * 64, kWgradRing = 4 * kWgradSlot;
+constexpr int kWgradLds = kWgradWaves * kWgradRing;
+template <int NC> constexpr int wgrad_sums() { return 18 * NC + 2; }  // f32x4 a lane, with the bias
+// The operands of one step: per operand 8 pixels of the lane's channel, kg 4 + 0 .. 3 and 16 (1 KB) on.  In
+// assembly, with its wait: before the builtin of this read the compiler waits for every direct load in
+// flight, the next steps' too (wgrad 96 -> 32 at 256 x 256 x 16: 78 us).
+template <int NC>
+LGX_D void wgrad_operands(int at, const int (&xoff)[3][NC], const int (&doff)[2], bf16x8 (&b)[3][NC], bf16x8 (&d)[2]) {
+  typedef short s16x4 __attribute__((ext_vector_type(4)));
+  s16x4 v[3 * NC + 2][2];
+  int p[3 * NC + 2];
+#pragma unroll
+  for (int k = 0; k < 3 * NC; k++) p[k] = at + xoff[k / NC][k % NC];
+#pragma unroll
+  for (int k = 0; k < 2; k++) p[3 * NC + k] = at + doff[k];
+  if constexpr (NC == 2) {
+    asm volatile(
+        "ds_read_b64_tr_b16 %0, %16\n\tds_read_b64_tr_b16 %1, %16 offset:1024\n\t"
+        "ds_read_b64_tr_b16 %2, %17\n\tds_read_b64_tr_b16 %3, %17 offset:1024\n\t"
+        "ds_read_b64_tr_b16 %4, %18\n\tds_read_b64_tr_b16 %5, %18 offset:1024\n\t"
+        "ds_read_b64_tr_b16 %6, %19\n\tds_read_b64_tr_b16 %7, %19 offset:1024\n\t"
+        "ds_read_b64_tr_b16 %8, %20\n\tds_read_b64_tr_b16 %9, %20 offset:1024\n\t"
+        "ds_read_b64_tr_b16 %10, %21\n\tds_read_b64_tr_b16 %11, %21 offset:1024\n\t"
+        "ds_read_b64_tr_b16 %12, %22\n\tds_read_b64_tr_b16 %13, %22 offset:1024\n\t"
+        "ds_read_b64_tr_b16 %14, %23\n\tds_read_b64_tr_b16 %15, %23 offset:1024\n\t"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(v[0][0]), "=&v"(v[0][1]), "=&v"(v[1][0]), "=&v"(v[1][1]), "=&v"(v[2][0]), "=&v"(v[2][1]),
+          "=&v"(v[3][0]), "=&v"(v[3][1]), "=&v"(v[4][0]), "=&v"(v[4][1]), "=&v"(v[5][0]), "=&v"(v[5][1]),
+          "=&v"(v[3 * NC][0]), "=&v"(v[3 * NC][1]), "=&v"(v[3 * NC + 1][0]), "=&v"(v[3 * NC + 1][1])
+        : "v"(p[0]), "v"(p[1]), "v"(p[2]), "v"(p[3]), "v"(p[4]), "v"(p[5]), "v"(p[3 * NC]), "v"(p[3 * NC + 1])
+        : "memory");
+  } else {
+    asm volatile(
+        "ds_read_b64_tr_b16 %0, %10\n\tds_read_b64_tr_b16 %1, %10 offset:1024\n\t"
+        "ds_read_b64_tr_b16 %2, %11\n\tds_read_b64_tr_b16 %3, %11 offset:1024\n\t"
+        "ds_read_b64_tr_b16 %4, %12\n\tds_read_b64_tr_b16 %5, %12 offset:1024\n\t"
+        "ds_read_b64_tr_b16 %6, %13\n\tds_read_b64_tr_b16 %7, %13 offset:1024\n\t"
+        "ds_read_b64_tr_b16 %8, %14\n\tds_read_b64_tr_b16 %9, %14 offset:1024\n\t"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(v[0][0]), "=&v"(v[0][1]), "=&v"(v[1][0]), "=&v"(v[1][1]), "=&v"(v[2][0]), "=&v"(v[2][1]),
+          "=&v"(v[3][0]), "=&v"(v[3][1]), "=&v"(v[4][0]), "=&v"(v[4][1])
+        : "v"(p[0]), "v"(p[1]), "v"(p[2]), "v"(p[3]), "v"(p[4])
+        : "memory");
+  }
+  auto whole = [&](int k) {
+    return __builtin_bit_cast(bf16x8, __builtin_shufflevector(v[k][0], v[k][1], 0, 1, 2, 3, 4, 5, 6, 7));
+  };
+#pragma unroll
+  for (int k = 0; k < 3 * NC; k++) b[k / NC][k % NC] = whole(k);
+#pragma unroll
+  for (int k = 0; k < 2; k++) d[k] = whole(3 * NC + k);
+}
+template <int NC> __global__ __launch_bounds__(512, 2) void conv3x3_wgrad_kernel(const WgradArgs a) {
+  extern __shared__ __align__(16) char s_wg[];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 15, kg = lane >> 4;
-  const int groups = (a.ca + a.cb) >> 5;
-  // a workgroup computes COUT of the a.cout output channels: channel slice hf
-  const int halves = a.cout / COUT;
-  const int hf = blockIdx.z % halves, zc = blockIdx.z / halves;
-  const int n = zc / groups, g = zc % groups;
-  const int x0 = blockIdx.x * 64, y0 = blockIdx.y * a.rows;
-  const ConvInput in{a.a, a.ca, a.a_up, a.b, a.cb};
-  constexpr int MJ = MB / 2;  // output blocks per wave
-  const int cb = wave & 1, mb0 = wave >> 1;
-  f32x4 acc[9][MJ];
+  const int groups = (a.ca + a.cb) >> 5, units = groups * (a.cout >> 5), slots = (int)gridDim.x / units;
+  // the units of one share of the pixels are neighbours (the same rows, in one XCD's L2)
+  const int id = (int)xcd_remap(blockIdx.x, gridDim.x), slot = id / units, g = id % units % groups,
+            co0 = id % units / groups * 32;
+  const bool from_a = g * 32 < a.ca;
+  const int up = from_a && a.a_up ? 1 : 0;
+  const int cs = from_a ? a.ca : a.cb, ch = from_a ? g * 32 : g * 32 - a.ca;
+  const bf16 *const src = from_a ? a.a : a.b;
+  const int sw = a.w >> up, sh = a.h >> up, bands = (a.w + 31) >> 5;
+  const int items = a.n * bands * a.h;  // (checked on the host)
+  int i0 = (slot * kWgradWaves + wave) * a.rows;
+  const int i1 = min(items, i0 + a.rows);
+  typedef __attribute__((address_space(3))) void LdsVoid;
+  char *const ring = s_wg + wave * kWgradRing;
+  const int ring_at = (int)(uintptr_t)(LdsVoid *)ring;  // in LDS
+  struct Piece {  // dY rows [ys, ye) of a strip; at most cap rows, so that offsets in it stay below 2 GB
+    int n, x0, ys, ye;
+  };
+  auto piece_at = [&](int i) {
+    const int strip = i / a.h, ys = i % a.h;
+    return Piece{strip / bands, strip % bands * 32, ys, min(min(a.h, ys + (i1 - i)), ys + a.cap)};
+  };
+  // Direct loads of one step: input row r (2 KB and the last two pixels, 8 lanes) and gradient row r + 1.
+  // Rows outside the image or the piece, and steps past the end, are past their buffer: zeros.  Five loads,
+  // always: the wait below counts them.  A piece has its buffers (from input row ys - 1, or 0, and gradient
+  // row ys) and lane offsets, a step only its two row offsets: with whole addresses formed per step the
+  // scalar work was as long as the matrix work.
+  const int part = ((lane & 3) ^ (lane >> 4 & 1) * 2) * 16;
+  const int xstep = sw * cs * 2, dstep = a.w * a.cout * 2;
+  int fi = i0, fr = 0, fy = 0, xsize = 0, dsize = 0, xlane[3], dlane[2];
+  Piece fp = {0, 0, 0, 0};
+  __amdgpu_buffer_rsrc_t xr, dr;
+  auto open = [&] {  // the piece at fi
+    fp = piece_at(min(fi, items - 1));
+    fr = fp.ys - 1;
+    fy = max(fr, 0) >> up;
+    xsize = (int)min((long)(sh - fy) * xstep - ch * 2, 0x7fffffffL);
+    dsize = (int)min((long)(a.h - fp.ys) * dstep - co0 * 2, 0x7fffffffL);
+    xr = __builtin_amdgcn_make_buffer_rsrc((void *)(src + ((size_t)fp.n * sh + fy) * sw * cs + ch), (short)0, xsize,
+                                           0x00020000);
+    dr = __builtin_amdgcn_make_buffer_rsrc((void *)(a.dy + ((size_t)fp.n * a.h + fp.ys) * a.w * a.cout + co0), (short)0,
+                                           dsize, 0x00020000);
+#pragma unroll
+    for (int b = 0; b < 3; b++) {
+      const int x = fp.x0 - 1 + b * 16 + (lane >> 2);
+      xlane[b] = (uint32_t)x < (uint32_t)a.w ? (x >> up) * cs * 2 + part : (int)0x80000000u;
+    }
+#pragma unroll
+    for (int b = 0; b < 2; b++) {
+      const int x = fp.x0 + b * 16 + (lane >> 2);
+      dlane[b] = x < a.w ? x * a.cout * 2 + part : (int)0x80000000u;
+    }
+  };
+  char *dst = ring;  // the slot the loads below fill
+  auto load_x = [&](int b0, int b1) {
+    const int row = fi < i1 && (uint32_t)fr < (uint32_t)a.h ? ((fr >> up) - fy) * xstep : xsize;
+#pragma unroll
+    for (int b = b0; b < b1; b++)
+      if (b < 2 || lane < 8)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (LdsVoid *)(dst + b * 1024), 16, xlane[b], row, 0, 0);
+  };
+  auto load_d = [&](int b) {
+    const int row = fi < i1 && fr + 1 < fp.ye ? (fr + 1 - fp.ys) * dstep : dsize;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(dr, (LdsVoid *)(dst + 34 * 64 + b * 1024), 16, dlane[b], row, 0, 0);
+  };
+  auto next = [&] {
+    if (++fr > fp.ye && fi < i1) {
+      fi += fp.ye - fp.ys;
+      if (fi < i1) open();
+    }
+  };
+  open();
+  // lane offsets of the operands: input pixels dx + kg 4 + .., half cb; gradient pixels kg 4 + .., half mb
+  int xoff[3][NC], doff[2];
+#pragma unroll
+  for (int dx = 0; dx < 3; dx++) {
+    const int p = dx + kg * 4 + (col >> 2);
+#pragma unroll
+    for (int cb = 0; cb < NC; cb++) xoff[dx][cb] = p * 64 + (cb ^ (p >> 2 & 1)) * 32 + (col & 3) * 8;
+  }
+#pragma unroll
+  for (int mb = 0; mb < 2; mb++) {
+    const int p = kg * 4 + (col >> 2);
+    doff[mb] = 34 * 64 + p * 64 + (mb ^ (p >> 2 & 1)) * 32 + (col & 3) * 8;
+  }
+  f32x4 acc[9][NC][2], accb[2];
 #pragma unroll
   for (int t = 0; t < 9; t++)
 #pragma unroll
-    for (int j = 0; j < MJ; j++) acc[t][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  // bias partial: thread t sums channel t % COUT over its eighth-, quarter-
-  // or half-row slice of pixels (BP = 256 / COUT slices)
-  constexpr int BP = 256 / COUT, BW = 64 / BP;
-  const int bc = threadIdx.x % COUT, bq = threadIdx.x / COUT;
-  float bsum = 0.f;
-  typedef unsigned short u16;
-  auto pair = [](bf16 lo, bf16 hi) {
-    return (uint32_t)__builtin_bit_cast(u16, lo) | ((uint32_t)__builtin_bit_cast(u16, hi) << 16);
-  };
-  // The next round's rows are loaded into registers while the current
-  // round's matrix work runs (loads unconditional, from clamped in-image
-  // addresses; what lies outside the image or the round is staged as zero).
-  constexpr int XI = ((RB + 2) * (XS / 2) * 4 + 255) / 256;  // input items per thread
-  constexpr int DI = (RB * 32 * (COUT / 8) + 255) / 256;    // output-gradient items per thread
-  bf16x8 px0[XI], px1[XI], pd0[DI], pd1[DI];
-  uint32_t okx = 0, okd = 0;  // bit 2i / 2i+1: item i's first / second pixel lies inside
-  auto fetch = [&](int yr, int nr) {
-    okx = okd = 0;
+    for (int cb = 0; cb < NC; cb++)
 #pragma unroll
-    for (int i = 0; i < XI; i++) {
-      const int e = min((int)threadIdx.x + i * 256, (RB + 2) * (XS / 2) * 4 - 1);
-      const int q = e & 3, pp = (e >> 2) % (XS / 2), rr = (e >> 2) / (XS / 2);
-      const int y = yr + rr - 1, x = x0 - 8 + pp * 2;
-      const bool rowok = rr < nr + 2 && y >= 0 && y < a.h;
-      px0[i] = load8_clamped(in, n, y, x, a.h, a.w, g * 32 + q * 8);
-      px1[i] = load8_clamped(in, n, y, x + 1, a.h, a.w, g * 32 + q * 8);
-      okx |= (uint32_t)(rowok && x >= 0 && x < a.w) << (2 * i);
-      okx |= (uint32_t)(rowok && x + 1 >= 0 && x + 1 < a.w) << (2 * i + 1);
-    }
+      for (int mb = 0; mb < 2; mb++) acc[t][cb][mb] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int i = 0; i < DI; i++) {
-      const int e = min((int)threadIdx.x + i * 256, RB * 32 * (COUT / 8) - 1);
-      const int q = e % (COUT / 8), pp = (e / (COUT / 8)) % 32, rr = e / (COUT / 8) / 32;
-      const int y = min(yr + rr, a.h - 1), x = x0 + pp * 2;
-      const bf16 *row = a.dy + ((size_t)n * a.h + y) * a.w * a.cout + hf * COUT + q * 8;
-      pd0[i] = *(const bf16x8 *)(row + (size_t)min(x, a.w - 1) * a.cout);
-      pd1[i] = *(const bf16x8 *)(row + (size_t)min(x + 1, a.w - 1) * a.cout);
-      okd |= (uint32_t)(rr < nr && x < a.w) << (2 * i);
-      okd |= (uint32_t)(rr < nr && x + 1 < a.w) << (2 * i + 1);
-    }
-  };
-  if (y0 < a.h) fetch(y0, min(RB, min(a.rows, a.h - y0)));
-  for (int r0 = 0; r0 < a.rows; r0 += RB) {
-    const int yr = y0 + r0;
-    if (yr >= a.h) break;  // uniform across the workgroup
-    const int nr = min(RB, min(a.rows - r0, a.h - yr));
-    // input rows yr - 1 .. yr + nr (32 channels of group g), transposed, pixel pairs
+  for (int mb = 0; mb < 2; mb++) accb[mb] = f32x4{0.f, 0.f, 0.f, 0.f};
+  bf16x8 ones, d[3][2];  // d: gradient rows r - 1, r, r + 1
 #pragma unroll
-    for (int i = 0; i < XI; i++) {
-      const int e = (int)threadIdx.x + i * 256;
-      if (e < (RB + 2) * (XS / 2) * 4) {
-        const int q = e & 3, pp = (e >> 2) % (XS / 2), rr = (e >> 2) / (XS / 2);
-        const bf16x8 z = {};
-        const bf16x8 v0 = (okx >> (2 * i)) & 1u ? px0[i] : z, v1 = (okx >> (2 * i + 1)) & 1u ? px1[i] : z;
+  for (int i = 0; i < 8; i++) ones[i] = f2bf(1.f);
 #pragma unroll
-        for (int k = 0; k < 8; k++) *(uint32_t *)&xs[xi(rr, q * 8 + k, pp * 2)] = pair(v0[k], v1[k]);
-      }
-    }
-    // output-gradient rows yr .. yr + nr - 1, transposed, pixel pairs
+  for (int k = 0; k < 3; k++)
 #pragma unroll
-    for (int i = 0; i < DI; i++) {
-      const int e = (int)threadIdx.x + i * 256;
-      if (e < RB * 32 * (COUT / 8)) {
-        const int q = e % (COUT / 8), pp = (e / (COUT / 8)) % 32, rr = e / (COUT / 8) / 32;
-        const bf16x8 z = {};
-        const bf16x8 v0 = (okd >> (2 * i)) & 1u ? pd0[i] : z, v1 = (okd >> (2 * i + 1)) & 1u ? pd1[i] : z;
-#pragma unroll
-        for (int k = 0; k < 8; k++) *(uint32_t *)&ds[di(rr, q * 8 + k, pp * 2)] = pair(v0[k], v1[k]);
-      }
-    }
-    __syncthreads();
-    {  // the next round's rows, in flight during this round's matrix work
-      const int yn = yr + RB;
-      if (r0 + RB < a.rows && yn < a.h) fetch(yn, min(RB, min(a.rows - r0 - RB, a.h - yn)));
-    }
-    if (g == 0) {  // uniform across the workgroup
-      for (int rr = 0; rr < nr; rr++)
-#pragma unroll
-        for (int k = 0; k < BW; k += 8) {
-          const bf16x8 v = *(const bf16x8 *)&ds[di(rr, bc, bq * BW + k)];
-#pragma unroll
-          for (int i = 0; i < 8; i++) bsum += bf2f(v[i]);
-        }
-    }
-    for (int rr = 0; rr < nr; rr++) {
-#pragma unroll
-      for (int kc = 0; kc < 2; kc++) {
-        const int p0 = kc * 32 + kg * 8;
-        bf16x8 av[MJ];  // A: co x pixels
-#pragma unroll
-        for (int j = 0; j < MJ; j++) av[j] = *(const bf16x8 *)&ds[di(rr, (mb0 + 2 * j) * 16 + col, p0)];
-#pragma unroll
-        for (int dy = 0; dy < 3; dy++) {
-          const bf16 *base = &xs[xi(rr + dy, cb * 16 + col, p0 + 8)];  // B: pixels x ci, 16-byte aligned
-          const bf16x8 lo = *(const bf16x8 *)(base - 8), mid = *(const bf16x8 *)base,
-                       hi = *(const bf16x8 *)(base + 8);
-          bf16x8 bm, bp;  // dx = -1: elements base[-1 .. 6]; dx = +1: base[1 .. 8]
-          bm[0] = lo[7];
-#pragma unroll
-          for (int i = 1; i < 8; i++) bm[i] = mid[i - 1];
-#pragma unroll
-          for (int i = 0; i < 7; i++) bp[i] = mid[i + 1];
-          bp[7] = hi[0];
-#pragma unroll
-          for (int j = 0; j < MJ; j++) {
-            acc[dy * 3 + 0][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[j], bm, acc[dy * 3 + 0][j], 0, 0, 0);
-            acc[dy * 3 + 1][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[j], mid, acc[dy * 3 + 1][j], 0, 0, 0);
-            acc[dy * 3 + 2][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[j], bp, acc[dy * 3 + 2][j], 0, 0, 0);
-          }
-        }
-      }
-    }
-    __syncthreads();
+    for (int mb = 0; mb < 2; mb++) d[k][mb] = bf16x8{};
+  for (int k = 0; k < 3; k++) {
+    dst = ring + k * kWgradSlot;
+    load_x(0, 3);
+    load_d(0);
+    load_d(1);
+    next();
   }
-  const size_t slots = (size_t)a.n * gridDim.y * gridDim.x;
-  const size_t slot = ((size_t)n * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x;
-  float *dst = a.part + ((size_t)g * slots + slot) * (9 * 32 * a.cout) + hf * COUT;
+  int at = 0;
+  while (i0 < i1) {
+    const Piece p = piece_at(i0);
+    i0 += p.ye - p.ys;
+    for (int r = p.ys - 1; r <= p.ye; r++) {
+      // this step's five loads have landed (ten later ones are in flight); the slot the next loads go to
+      // was read in the last step
+      asm volatile("s_waitcnt vmcnt(10) lgkmcnt(0)" ::: "memory");
+      dst = ring + (at == 0 ? 3 * kWgradSlot : at - kWgradSlot);
+      const int x = ring_at + at;
+      at = at == 3 * kWgradSlot ? 0 : at + kWgradSlot;
+      bf16x8 b[3][NC];
+      wgrad_operands<NC>(x, xoff, doff, b, d[2]);
+      // vertical tap t: gradient row r + 1 - t, while it is in the piece (uniform)
+      auto taps = [&](int t) {
 #pragma unroll
-  for (int tap = 0; tap < 9; tap++)
+        for (int dx = 0; dx < 3; dx++)
 #pragma unroll
-    for (int j = 0; j < MJ; j++)
-      *(f32x4 *)&dst[(tap * 32 + cb * 16 + col) * a.cout + (mb0 + 2 * j) * 16 + kg * 4] = acc[tap][j];
-  if (g == 0) {
-    // the BP slices of each channel, added in a fixed order (xs is free now)
-    float *red = (float *)&xs[0];
-    red[bq * COUT + bc] = bsum;
-    __syncthreads();
-    if (threadIdx.x < COUT) {
-      float b = 0.f;
+          for (int cb = 0; cb < NC; cb++)
 #pragma unroll
-      for (int k = 0; k < BP; k++) b += red[k * COUT + threadIdx.x];
-      a.part_b[slot * a.cout + hf * COUT + threadIdx.x] = b;
+            for (int mb = 0; mb < 2; mb++)
+              acc[t * 3 + dx][cb][mb] =
+                  __builtin_amdgcn_mfma_f32_16x16x32_bf16(d[2 - t][mb], b[dx][cb], acc[t * 3 + dx][cb][mb], 0, 0, 0);
+      };
+      load_x(0, 2);
+      if (r > p.ys) taps(2);
+      load_x(2, 3);
+      load_d(0);
+      if (r >= p.ys && r < p.ye) taps(1);
+      load_d(1);
+      next();
+      if (r + 1 < p.ye) {
+        taps(0);
+        if (g == 0)
+#pragma unroll
+          for (int mb = 0; mb < 2; mb++)
+            accb[mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(d[2][mb], ones, accb[mb], 0, 0, 0);
+      }
+#pragma unroll
+      for (int mb = 0; mb < 2; mb++) {
+        d[0][mb] = d[1][mb];
+        d[1][mb] = d[2][mb];
+      }
     }
+  }
+  // The waves' sums in a fixed order, through LDS, which holds four waves': waves 4 .. 7 to waves 0 .. 3, then
+  // each wave adds the four of an eighth of the sums and stores it.
+  constexpr int SUMS = wgrad_sums<NC>();
+  f32x4 *const all = (f32x4 *)s_wg + lane;
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+  for (int round = 0; round < 2; round++) {
+    __syncthreads();
+    f32x4 *const mine = all + (size_t)(wave & 3) * SUMS * 64;
+    if ((wave >> 2) != round) {  // round 0: waves 4 .. 7, round 1: waves 0 .. 3
+#pragma unroll
+      for (int k = 0; k < 18 * NC; k++) mine[k * 64] = acc[k / (2 * NC)][k / 2 % NC][k % 2];
+#pragma unroll
+      for (int k = 0; k < 2; k++) mine[(18 * NC + k) * 64] = accb[k];
+    }
+    __syncthreads();
+    if (round == 0 && wave < 4) {
+#pragma unroll
+      for (int k = 0; k < 18 * NC; k++) acc[k / (2 * NC)][k / 2 % NC][k % 2] += mine[k * 64];
+#pragma unroll
+      for (int k = 0; k < 2; k++) accb[k] += mine[(18 * NC + k) * 64];
+    }
+  }
+  float *out = a.part + ((size_t)g * slots + slot) * (9 * 32 * a.cout) + co0 + kg * 4;
+  for (int k = wave; k < SUMS; k += kWgradWaves) {
+    const f32x4 v = ((all[k * 64] + all[(SUMS + k) * 64]) + all[(2 * SUMS + k) * 64]) + all[(3 * SUMS + k) * 64];
+    if (k < 18 * NC)  // tap, input block, output block
+      *(f32x4 *)&out[(k / (2 * NC) * 32 + k / 2 % NC * 16 + col) * a.cout + k % 2 * 16] = v;
+    else if (g == 0 && col == 0)
+      *(f32x4 *)&a.part_b[(size_t)slot * a.cout + co0 + (k - 18 * NC) * 16 + kg * 4] = v;
   }
 }
 
@@ -2094,25 +2137,13 @@ hipError_t conv_first_pair(const ConvArgs &a0, const ConvArgs &a1, hipStream_t s
   return hipGetLastError();
 }
 
-// Weight-gradient workgroups per launch by output-channel count: each stores
-// 9 * 32 * cout FP32 partial sums, about 38 MB per launch at these counts.
-// Workgroups of conv3x3_wgrad_kernel: about the number that are resident at
-// once (2 per CU: the accumulators live in AGPRs, which share the register
-// file with the VGPRs, and LDS), so that the launch is one round of
-// workgroups rather than a round and a fraction with most CUs idle in the
-// fraction.
-static int wgrad_target_blocks(int cout) { return (cout == 128 ? 1 : 2) * cu_count(); }  // x2 slices for 128
-// Output rows staged per round of conv3x3_wgrad_kernel: a round's loads are
-// in flight during the previous round's matrix work, so taller rounds expose
-// that latency fewer times, within two workgroups' LDS per CU (64 channels:
-// 3 rows).
-static constexpr int kWgradRB2 = 4, kWgradRB4 = 3;
-static int wgrad_rb(int cout) { return cout <= 32 ? kWgradRB2 : kWgradRB4; }
+// Workgroups of conv3x3_wgrad_kernel: at most one per CU (its LDS), each with sums of 9 x 32 x 32; rows of
+// a strip per wave at least 8, so that small images have few slots to add.
+static constexpr int kWgradMinRows = 8;
 
 size_t conv3x3_wgrad_scratch_bytes() {
-  size_t m = 0;
-  for (int cout : {32, 64, 128}) m = std::max(m, (size_t)2 * wgrad_target_blocks(cout) * (9 * 32 + 1) * cout * 4);
-  return m;
+  // (the network has at most 16 units of 32 x 32 channels; a bias slot has at most 128)
+  return (size_t)std::max(cu_count(), 16) * (9 * 32 * 32 + 128) * 4;
 }
 
 hipError_t conv3x3_wgrad(WgradArgs a, hipStream_t s) {
@@ -2120,32 +2151,23 @@ hipError_t conv3x3_wgrad(WgradArgs a, hipStream_t s) {
   if ((a.ca + a.cb) % 32 || a.ca % 32 || a.n < 1 || a.h < 1 || a.w < 1 || !a.part || !a.dw || !a.db ||
       a.cin_log < 1 || a.cin_log > a.ca + a.cb)
     return hipErrorInvalidValue;
-  const int groups = (a.ca + a.cb) / 32, bands = (a.w + 63) / 64, target = wgrad_target_blocks(a.cout);
-  const long segs = (long)bands * a.n * groups;  // workgroups per row of rows
-  // rows per workgroup: a multiple of the round height, about `target`
-  // workgroups, at most 2 * target
-  const int rb = wgrad_rb(a.cout);
-  int rows = (int)std::min<long>(a.h, std::max<long>(rb, ((long)a.h * segs + target - 1) / target));
-  rows = (rows + rb - 1) / rb * rb;
-  long blocks = segs * ((a.h + rows - 1) / rows);
-  while (blocks > 2L * target && rows < a.h) {
-    rows += rb;
-    blocks = segs * ((a.h + rows - 1) / rows);
-  }
+  const int groups = (a.ca + a.cb) / 32, units = groups * (a.cout / 32);
+  const long items = (long)a.n * ((a.w + 31) / 32) * a.h;  // rows of strips
+  if (items > INT_MAX / 2) return hipErrorInvalidValue;
+  const long fit = std::max(1, cu_count() / units), per_wg = kWgradWaves * kWgradMinRows;
+  const long wgs = std::min(fit, (items + per_wg - 1) / per_wg);
+  a.rows = (int)((items + wgs * kWgradWaves - 1) / (wgs * kWgradWaves));
+  // a piece's rows (two more are read) within 2 GB of its first
+  a.cap = (int)std::max(1L, std::min((long)a.h, 0x7fffffffL / ((long)a.w * 2 * std::max({a.ca, a.cb, a.cout})) - 3));
+  const int slots = (int)((items + (long)a.rows * kWgradWaves - 1) / ((long)a.rows * kWgradWaves));
   const size_t per = (size_t)9 * 32 * a.cout;
-  const int slots = (int)(blocks / groups);
-  if (((size_t)blocks * per + (size_t)slots * a.cout) * 4 > a.part_bytes) return hipErrorInvalidValue;
-  a.rows = rows;
-  a.part_b = a.part + (size_t)blocks * per;
-  // 128 output channels: the 64-channel kernel on two channel slices (two
-  // workgroups per pixel block; the 128-channel accumulators would leave one
-  // wave per SIMD)
-  const int halves = a.cout == 128 ? 2 : 1;
-  dim3 grid(bands, (a.h + rows - 1) / rows, a.n * groups * halves), block(256);
-  switch (a.cout / 16) {
-    case 2: hipLaunchKernelGGL((conv3x3_wgrad_kernel<2, kWgradRB2>), grid, block, 0, s, a); break;
-    default: hipLaunchKernelGGL((conv3x3_wgrad_kernel<4, kWgradRB4>), grid, block, 0, s, a); break;
-  }
+  if (((size_t)groups * slots * per + (size_t)slots * a.cout) * 4 > a.part_bytes) return hipErrorInvalidValue;
+  a.part_b = a.part + (size_t)groups * slots * per;
+  const bool one = a.cin_log <= 16;  // the other half of the only group's channels is padding
+  const int sums = (one ? wgrad_sums<1>() : wgrad_sums<2>()) * 1024 * kWgradWaves / 2;
+  const size_t lds = std::max(kWgradLds, sums);
+  hipLaunchKernelGGL(one ? conv3x3_wgrad_kernel<1> : conv3x3_wgrad_kernel<2>, dim3((unsigned)(units * slots)),
+                     dim3(64 * kWgradWaves), lds, s, a);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   const int per4 = (int)(per / 4);
