@@ -68,9 +68,18 @@ struct WgradArgs {
   int cin_log;     // input channels of the master weights (the rest of ca + cb is zero padding)
   float *dw;       // [cout][cin_log][9] (master layout), overwritten
   float *db;       // [cout] bias gradient, overwritten
-  float *part;     // scratch for the per-workgroup partial sums
-  float *part_b;   // (set by conv3x3_wgrad) bias partials inside part
-  size_t part_bytes;
+  int slots;              // (set by conv3x3_wgrad, with the next two) partial sums per unit of 32 x 32 channels
+  float *part, *part_b;   // and where they and the bias's are
+};
+// The layers of one backward pass.
+struct WgradTable {
+  WgradArgs l[10];
+  int n;
+  // set by conv3x3_wgrad: layers launched, floats of scratch taken, and the first workgroup of a layer in its launch
+  // (counted over all launches) and in the sums
+  int done;
+  size_t used;
+  int first[11], reduce[11];
 };
 
 hipError_t conv3x3(const ConvArgs &a, hipStream_t s);
@@ -83,7 +92,11 @@ hipError_t conv_first_pair(const ConvArgs &a0, const ConvArgs &a1, hipStream_t s
 int conv3x3_tiles(int cout);  // register tiles offered for this output channel count
 int conv3x3_tile_lds(int cout, int tile);  // 1 if that tile is an LDS tile covering all cout channels
 int conv3x3_tile_pool(int cout, int tile);  // 1 if that tile can write the 2x2 pooled output (pool_out)
-hipError_t conv3x3_wgrad(WgradArgs a, hipStream_t s);
+// The weight gradients of the layers added to the table since the last call, in one launch, as partial sums in
+// part; after at most kWgradLaunches of them conv3x3_wgrad_sums adds those of all layers.
+constexpr int kWgradLaunches = 6;
+hipError_t conv3x3_wgrad(WgradTable &t, float *part, size_t part_bytes, hipStream_t s);
+hipError_t conv3x3_wgrad_sums(const WgradTable &t, hipStream_t s);
 size_t conv3x3_wgrad_scratch_bytes();
 hipError_t pack_input(const float *x12, size_t npix, bf16 *x32, hipStream_t s);
 hipError_t head_fwd_img(const bf16 *d1, const lgx_image &noisy, const float *wh, const float *bh, int out_pitch,

@@ -220,9 +220,10 @@ class Net {
     check(conv3x3(c, s), "conv3x3 input gradient");
   }
 
-  void wgrad(int l, const bf16 *a, int ca, int a_up, const bf16 *b, int cb, const bf16 *dy, int n, int h, int w,
-             hipStream_t s) {
-    WgradArgs g{};
+  // adds layer l's weight gradient to the table of the backward pass
+  void wgrad(WgradTable &t, int l, const bf16 *a, int ca, int a_up, const bf16 *b, int cb, const bf16 *dy, int n, int h,
+             int w) {
+    WgradArgs &g = t.l[t.n++];
     g.a = a;
     g.ca = ca;
     g.a_up = a_up;
@@ -236,9 +237,6 @@ class Net {
     g.cin_log = kLayers[l].cin;
     g.dw = grads + w_off[l];
     g.db = grads + b_off[l];
-    g.part = wpart;
-    g.part_bytes = wpart_bytes;
-    check(conv3x3_wgrad(g, s), "conv3x3_wgrad");
   }
 
   // forward convolution l on the activations of an n x h x w input
@@ -453,33 +451,45 @@ class Net {
     check(head_train(d1, x12, (const float4 *)target, params + head_w_off, params + head_b_off, P, 1.0f / (3.0f * P),
                      loss_kind == LGX_UNET_LOSS_L2, g_d1, grads + head_w_off, grads + head_b_off, loss, s),
           "head_train");
+    // Weight gradients in six launches: the layers of the small resolutions share two (16 x 256 x 256: 137 us; by
+    // themselves, 10 us of each a launch's own, 178), and one sum at the end.  All ten in one launch read their
+    // inputs from HBM once more, when the gradients just written would be in cache: 365 us instead of 284.
+    WgradTable t{};
+    auto launch = [&] { check(conv3x3_wgrad(t, wpart, wpart_bytes, s), "conv3x3_wgrad"); };
     // d1 = relu(conv9(d1a))
-    wgrad(9, d1a, 32, 0, nullptr, 0, g_d1, n, h, w, s);
+    wgrad(t, 9, d1a, 32, 0, nullptr, 0, g_d1, n, h, w);
+    launch();
     dx_layer(9, n, h, w, s);
     // d1a = relu(conv8([up(d2), e1]))
-    wgrad(8, d2, 64, 1, e1, 32, g_d1a, n, h, w, s);
+    wgrad(t, 8, d2, 64, 1, e1, 32, g_d1a, n, h, w);
+    launch();
     dx_layer(8, n, h, w, s);  // and the gradient of d2 through the upsample
     // d2 = relu(conv7(d2a))
-    wgrad(7, d2a, 64, 0, nullptr, 0, g_d2, n, h2, w2, s);
+    wgrad(t, 7, d2a, 64, 0, nullptr, 0, g_d2, n, h2, w2);
     dx_layer(7, n, h, w, s);
     // d2a = relu(conv6([up(b2), e2]))
-    wgrad(6, b2, 128, 1, e2, 64, g_d2a, n, h2, w2, s);
+    wgrad(t, 6, b2, 128, 1, e2, 64, g_d2a, n, h2, w2);
+    launch();
     dx_layer(6, n, h, w, s);  // and the gradient of b2 through the upsample
     // b2 = relu(conv5(b1)), b1 = relu(conv4(p2))
-    wgrad(5, b1, 128, 0, nullptr, 0, g_b2, n, h4, w4, s);
+    wgrad(t, 5, b1, 128, 0, nullptr, 0, g_b2, n, h4, w4);
     dx_layer(5, n, h, w, s);
-    wgrad(4, p2, 64, 0, nullptr, 0, g_b1, n, h4, w4, s);
+    wgrad(t, 4, p2, 64, 0, nullptr, 0, g_b1, n, h4, w4);
     dx_layer(4, n, h, w, s);
     // e2 feeds the pool and the skip
     check(pool_bwd_add(g_e2c, g_p2, e2, n, h2, w2, 64, g_e2, s), "pool_bwd_add");
-    wgrad(3, e2a, 64, 0, nullptr, 0, g_e2, n, h2, w2, s);
+    wgrad(t, 3, e2a, 64, 0, nullptr, 0, g_e2, n, h2, w2);
     dx_layer(3, n, h, w, s);
-    wgrad(2, p1, 32, 0, nullptr, 0, g_e2a, n, h2, w2, s);
+    wgrad(t, 2, p1, 32, 0, nullptr, 0, g_e2a, n, h2, w2);
+    launch();
     dx_layer(2, n, h, w, s);
     check(pool_bwd_add(g_e1c, g_p1, e1, n, h, w, 32, g_e1, s), "pool_bwd_add");
-    wgrad(1, e1a, 32, 0, nullptr, 0, g_e1, n, h, w, s);
+    wgrad(t, 1, e1a, 32, 0, nullptr, 0, g_e1, n, h, w);
+    launch();
     dx_layer(1, n, h, w, s);
-    wgrad(0, x32, 32, 0, nullptr, 0, g_e1a, n, h, w, s);
+    wgrad(t, 0, x32, 32, 0, nullptr, 0, g_e1a, n, h, w);
+    launch();
+    check(conv3x3_wgrad_sums(t, s), "conv3x3_wgrad_sums");
   }
 
   void adam_step(float lr, hipStream_t s) {

@@ -1320,11 +1320,10 @@ __global__ __launch_bounds__(64, 2) void conv_first_pair_kernel(const ConvArgs a
 //
 // What bounds it (16 x 256 x 256): 96 -> 32 at full size 56 us, of which 27 are
 // its MFMAs, 9 the direct loads that do not overlap, and 10 a launch's start,
-// first loads and last sums, which are most of the small layers (32 -> 64 at
-// half size 18 us).  Staging pixel pairs through registers into transposed
-// rows and shifting operands by elements, with one workgroup's waves at two
-// barriers a round, it was bound by LDS: 157 and 40 us; 192 -> 64 at half size
-// 114, now 61.
+// first loads and last sums.  Staging pixel pairs through registers into
+// transposed rows and shifting operands by elements, with one workgroup's
+// waves at two barriers a round, it was bound by LDS: 157 us; the ten layers
+// 570 and 66 for their sums, now 284 and 23.
 constexpr int kWgradWaves = 8, kWgradSlot = 34 * 64 + 32 * 64, kWgradRing = 4 * kWgradSlot;
 constexpr int kWgradLds = kWgradWaves * kWgradRing;
 template <int NC> constexpr int wgrad_sums() { return 18 * NC + 2; }  // f32x4 a lane, with the bias
@@ -1377,14 +1376,13 @@ LGX_D void wgrad_operands(int at, const int (&xoff)[3][NC], const int (&doff)[2]
 #pragma unroll
   for (int k = 0; k < 2; k++) d[k] = whole(3 * NC + k);
 }
-template <int NC> __global__ __launch_bounds__(512, 2) void conv3x3_wgrad_kernel(const WgradArgs a) {
+template <int NC> LGX_D void wgrad_task(const WgradArgs &a, int task) {
   extern __shared__ __align__(16) char s_wg[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 15, kg = lane >> 4;
-  const int groups = (a.ca + a.cb) >> 5, units = groups * (a.cout >> 5), slots = (int)gridDim.x / units;
+  const int groups = (a.ca + a.cb) >> 5, units = groups * (a.cout >> 5), slots = a.slots;
   // the units of one share of the pixels are neighbours (the same rows, in one XCD's L2)
-  const int id = (int)xcd_remap(blockIdx.x, gridDim.x), slot = id / units, g = id % units % groups,
-            co0 = id % units / groups * 32;
+  const int slot = task / units, g = task % units % groups, co0 = task % units / groups * 32;
   const bool from_a = g * 32 < a.ca;
   const int up = from_a && a.a_up ? 1 : 0;
   const int cs = from_a ? a.ca : a.cb, ch = from_a ? g * 32 : g * 32 - a.ca;
@@ -1567,63 +1565,64 @@ template <int NC> __global__ __launch_bounds__(512, 2) void conv3x3_wgrad_kernel
   }
 }
 
-// The fixed-order reductions of conv3x3_wgrad_kernel's per-workgroup partial
-// sums, in one launch.  Blocks [0, nwb): the weight gradient,
-//   dw[co][ci][tap] = sum over slots of part[g][slot][tap][ci % 32][co]
-// written in the master layout for ci < cin_log (g = ci / 32); a workgroup
-// holds 256 / S float4 elements x S slices, slice k sums slots k, k + S, ...
-// and the S slice sums are added in a fixed tree.  Block nwb + co: the bias
-// gradient db[co] = sum over slots of part_b[slot][co], 256 strided partial
-// sums then a fixed tree.  Neither result depends on the order in which
-// workgroups ran.
-template <int S>
-__global__ __launch_bounds__(256) void wgrad_reduce_kernel(const f32x4 *part, int slots, int per4, int groups,
-                                                          int cout, int cin_log, int nwb, const float *part_b,
-                                                          float *dw, float *db) {
-  if ((int)blockIdx.x >= nwb) {  // uniform per workgroup
-    __shared__ float redb[256];
-    const int co = (int)blockIdx.x - nwb;
-    float sb = 0.f;
-    for (int k = threadIdx.x; k < slots; k += 256) sb += part_b[(size_t)k * cout + co];
-    redb[threadIdx.x] = sb;
-    __syncthreads();
-#pragma unroll
-    for (int st = 128; st > 0; st >>= 1) {
-      if ((int)threadIdx.x < st) redb[threadIdx.x] += redb[threadIdx.x + st];
-      __syncthreads();
-    }
-    if (threadIdx.x == 0) db[co] = redb[0];
-    return;
-  }
-  constexpr int E = 256 / S;
-  __shared__ f32x4 red[S][E];
-  const int el = threadIdx.x % E, sl = threadIdx.x / E;
-  const size_t e = (size_t)blockIdx.x * E + el, total = (size_t)groups * per4;
-  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-  if (e < total) {
-    const size_t g = e / per4, f = e % per4;
-    const f32x4 *src = part + g * slots * per4 + f;
-    for (int k = sl; k < slots; k += S) acc += src[(size_t)k * per4];
-  }
-  red[sl][el] = acc;
-  __syncthreads();
-#pragma unroll
-  for (int st = S / 2; st > 0; st >>= 1) {
-    if (sl < st) red[sl][el] += red[sl + st][el];
-    __syncthreads();
-  }
-  if (sl == 0 && e < total) {
-    const int g = (int)(e / per4), f = (int)(e % per4) * 4;
-    const int tap = f / (32 * cout), rem = f % (32 * cout), cl = rem / cout, co = rem % cout;
-    const int ci = g * 32 + cl;
-    if (ci < cin_log) {
-      const f32x4 v = red[0][el];
-#pragma unroll
-      for (int i = 0; i < 4; i++) dw[((size_t)(co + i) * cin_log + ci) * 9 + tap] = v[i];
-    }
-  }
+// The weight gradients of layers l .. t.n - 1: workgroup -> layer -> task (a unit's share).
+__global__ __launch_bounds__(64 * kWgradWaves, 2) void conv3x3_wgrad_kernel(const WgradTable t, int l) {
+  const int id = (int)xcd_remap(blockIdx.x, gridDim.x) + t.first[l];
+  while (id >= t.first[l + 1]) l++;
+  const WgradArgs &a = t.l[l];
+  if (a.cin_log <= 16)  // the other half of the only group's channels is padding
+    wgrad_task<1>(a, id - t.first[l]);
+  else
+    wgrad_task<2>(a, id - t.first[l]);
 }
 
+// The fixed-order sums of the workgroups' partial sums, all layers in one
+// launch.  A workgroup of a layer's weight gradient,
+//   dw[co][ci][tap] = sum over slots of part[g][slot][tap][ci % 32][co]
+// written in the master layout for ci < cin_log (g = ci / 32), has 16 float4
+// elements x 16 slices; slice k sums slots k, k + 16, ... and the slice sums are
+// added in order (256 slots: with 4 slices of 64 loads each, 100 us for the
+// ten layers instead of 23).  A layer's last workgroup: the bias gradient, db[co] =
+// sum over slots of part_b[slot][co], the same way.  Neither result depends on
+// the order in which workgroups ran.
+constexpr int kReduceEl = 16, kReduceSl = 16;
+__global__ __launch_bounds__(256) void wgrad_reduce_kernel(const WgradTable t) {
+  int l = 0;
+  while ((int)blockIdx.x >= t.reduce[l + 1]) l++;
+  const WgradArgs &a = t.l[l];
+  const int blk = (int)blockIdx.x - t.reduce[l], cout = a.cout, slots = a.slots;
+  __shared__ f32x4 red[kReduceSl][kReduceEl];
+  const int el = threadIdx.x % kReduceEl, sl = threadIdx.x / kReduceEl;
+  const bool bias = (int)blockIdx.x + 1 == t.reduce[l + 1];  // uniform per workgroup
+  if (bias) {
+    float *const rb = (float *)red;
+    const int co = (int)threadIdx.x % cout, k0 = (int)threadIdx.x / cout, step = 256 / cout;
+    float sb = 0.f;
+    for (int k = k0; k < slots; k += step) sb += a.part_b[(size_t)k * cout + co];
+    rb[threadIdx.x] = sb;
+    __syncthreads();
+    if (k0) return;
+    for (int k = 1; k < step; k++) sb += rb[k * cout + co];
+    a.db[co] = sb;
+    return;
+  }
+  const int per4 = 9 * 32 * cout / 4;
+  const int e = blk * kReduceEl + el;  // (a workgroup is in one group, and whole)
+  const int g = e / per4, f = e % per4;
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  const f32x4 *src = (const f32x4 *)a.part + (size_t)g * slots * per4 + f;
+  for (int k = sl; k < slots; k += kReduceSl) acc += src[(size_t)k * per4];
+  red[sl][el] = acc;
+  __syncthreads();
+  if (sl) return;
+  f32x4 v = red[0][el];
+#pragma unroll
+  for (int k = 1; k < kReduceSl; k++) v += red[k][el];
+  const int tap = f * 4 / (32 * cout), rem = f * 4 % (32 * cout), ci = g * 32 + rem / cout, co = rem % cout;
+  if (ci < a.cin_log)
+#pragma unroll
+    for (int i = 0; i < 4; i++) a.dw[((size_t)(co + i) * a.cin_log + ci) * 9 + tap] = v[i];
+}
 
 // ------------------------------------------------------------ glue kernels
 
@@ -2137,52 +2136,81 @@ hipError_t conv_first_pair(const ConvArgs &a0, const ConvArgs &a1, hipStream_t s
   return hipGetLastError();
 }
 
-// Workgroups of conv3x3_wgrad_kernel: at most one per CU (its LDS), each with sums of 9 x 32 x 32; rows of
-// a strip per wave at least 8, so that small images have few slots to add.
-static constexpr int kWgradMinRows = 8;
+// Rows of a strip per wave of conv3x3_wgrad_kernel: at least 2.
+static constexpr int kWgradMinRows = 2;
 
 size_t conv3x3_wgrad_scratch_bytes() {
-  // (the network has at most 16 units of 32 x 32 channels; a bias slot has at most 128)
-  return (size_t)std::max(cu_count(), 16) * (9 * 32 * 32 + 128) * 4;
+  // a task has 9 x 32 x 32 sums, and at most 32 channels' bias slots; a launch's tasks are at most the CUs or,
+  // with one each, the units of its layers (52 in the network)
+  return (size_t)kWgradLaunches * (cu_count() + 64) * (9 * 32 * 32 + 32) * 4;
 }
 
-hipError_t conv3x3_wgrad(WgradArgs a, hipStream_t s) {
-  if (a.cout != 32 && a.cout != 64 && a.cout != 128) return hipErrorInvalidValue;
-  if ((a.ca + a.cb) % 32 || a.ca % 32 || a.n < 1 || a.h < 1 || a.w < 1 || !a.part || !a.dw || !a.db ||
-      a.cin_log < 1 || a.cin_log > a.ca + a.cb)
-    return hipErrorInvalidValue;
-  const int groups = (a.ca + a.cb) / 32, units = groups * (a.cout / 32);
-  const long items = (long)a.n * ((a.w + 31) / 32) * a.h;  // rows of strips
-  if (items > INT_MAX / 2) return hipErrorInvalidValue;
-  const long fit = std::max(1, cu_count() / units), per_wg = kWgradWaves * kWgradMinRows;
-  const long wgs = std::min(fit, (items + per_wg - 1) / per_wg);
-  a.rows = (int)((items + wgs * kWgradWaves - 1) / (wgs * kWgradWaves));
-  // a piece's rows (two more are read) within 2 GB of its first
-  a.cap = (int)std::max(1L, std::min((long)a.h, 0x7fffffffL / ((long)a.w * 2 * std::max({a.ca, a.cb, a.cout})) - 3));
-  const int slots = (int)((items + (long)a.rows * kWgradWaves - 1) / ((long)a.rows * kWgradWaves));
-  const size_t per = (size_t)9 * 32 * a.cout;
-  if (((size_t)groups * slots * per + (size_t)slots * a.cout) * 4 > a.part_bytes) return hipErrorInvalidValue;
-  a.part_b = a.part + (size_t)groups * slots * per;
-  const bool one = a.cin_log <= 16;  // the other half of the only group's channels is padding
-  const int sums = (one ? wgrad_sums<1>() : wgrad_sums<2>()) * 1024 * kWgradWaves / 2;
-  const size_t lds = std::max(kWgradLds, sums);
-  hipLaunchKernelGGL(one ? conv3x3_wgrad_kernel<1> : conv3x3_wgrad_kernel<2>, dim3((unsigned)(units * slots)),
-                     dim3(64 * kWgradWaves), lds, s, a);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  const int per4 = (int)(per / 4);
-  const size_t total = (size_t)groups * per4;
-  const f32x4 *part = (const f32x4 *)a.part;
-  auto launch = [&](auto kern, int S) {
-    const int nwb = (int)((total + 256 / S - 1) / (256 / S));
-    hipLaunchKernelGGL(kern, dim3((unsigned)(nwb + a.cout)), dim3(256), 0, s, part, slots, per4, groups, a.cout,
-                       a.cin_log, nwb, (const float *)a.part_b, a.dw, a.db);
+// The units of a launch's layers are divided into tasks of about equal work, as many as there are CUs (a workgroup's
+// LDS takes a CU): the least work T per task for which the sum over layers of units * ceil(work of a unit / T)
+// fits.  A launch has about 10 us of its own (its start, the first loads, the last sums).
+hipError_t conv3x3_wgrad(WgradTable &t, float *part, size_t part_bytes, hipStream_t s) {
+  if (t.done < 0 || t.n <= t.done || t.n > 10 || !part) return hipErrorInvalidValue;
+  const int l0 = t.done;
+  long items[10], units[10], most = 0;
+  for (int l = l0; l < t.n; l++) {
+    const WgradArgs &a = t.l[l];
+    if (a.cout != 32 && a.cout != 64 && a.cout != 128) return hipErrorInvalidValue;
+    if ((a.ca + a.cb) % 32 || a.ca % 32 || a.n < 1 || a.h < 1 || a.w < 1 || !a.dw || !a.db || a.cin_log < 1 ||
+        a.cin_log > a.ca + a.cb || (a.cin_log <= 16 && a.ca + a.cb != 32))
+      return hipErrorInvalidValue;
+    items[l] = (long)a.n * ((a.w + 31) / 32) * a.h;  // rows of strips
+    if (items[l] > INT_MAX / 2) return hipErrorInvalidValue;
+    units[l] = (long)(a.ca + a.cb) / 32 * (a.cout / 32);
+    most = std::max(most, items[l]);
+  }
+  // (a unit with half of the matrix work counts half, though its loads are the same)
+  auto slots_of = [&](int l, long T) {
+    const long per = kWgradWaves * std::max((long)kWgradMinRows, (T * (t.l[l].cin_log <= 16 ? 2 : 1) + kWgradWaves - 1) / kWgradWaves);
+    return (items[l] + per - 1) / per;
   };
-  // about 16 loads per thread
-  if (slots <= 128) launch(wgrad_reduce_kernel<8>, 8);
-  else if (slots <= 256) launch(wgrad_reduce_kernel<16>, 16);
-  else if (slots <= 512) launch(wgrad_reduce_kernel<32>, 32);
-  else launch(wgrad_reduce_kernel<64>, 64);
+  auto tasks_of = [&](long T) {
+    long k = 0;
+    for (int l = l0; l < t.n; l++) k += units[l] * slots_of(l, T);
+    return k;
+  };
+  long lo = 0, hi = most;  // hi fits, or is the fewest tasks there are
+  while (hi - lo > 1) {
+    const long mid = (lo + hi) / 2;
+    (tasks_of(mid) <= cu_count() ? hi : lo) = mid;
+  }
+  size_t used = t.used;
+  int blocks = t.first[l0], sums = t.reduce[l0];
+  const int block0 = blocks;
+  for (int l = l0; l < t.n; l++) {
+    WgradArgs &a = t.l[l];
+    long slots = slots_of(l, hi);
+    a.rows = (int)((items[l] + slots * kWgradWaves - 1) / (slots * kWgradWaves));
+    slots = (items[l] + (long)a.rows * kWgradWaves - 1) / ((long)a.rows * kWgradWaves);
+    a.slots = (int)slots;
+    // a piece's rows (two more are read) within 2 GB of its first
+    a.cap = (int)std::max(1L, std::min((long)a.h, 0x7fffffffL / ((long)a.w * 2 * std::max({a.ca, a.cb, a.cout})) - 3));
+    a.part = part + used;
+    used += (size_t)units[l] * slots * 9 * 32 * 32;
+    a.part_b = part + used;
+    used += (size_t)slots * a.cout;
+    t.first[l] = blocks;
+    t.reduce[l] = sums;
+    blocks += (int)(units[l] * slots);
+    sums += (int)(units[l] * 9 * 32 * 32 / 4 / kReduceEl) + 1;
+  }
+  t.first[t.n] = blocks;
+  t.reduce[t.n] = sums;
+  if (used * 4 > part_bytes) return hipErrorInvalidValue;
+  const size_t lds = std::max(kWgradLds, wgrad_sums<2>() * 1024 * kWgradWaves / 2);
+  t.used = used;
+  t.done = t.n;
+  hipLaunchKernelGGL(conv3x3_wgrad_kernel, dim3((unsigned)(blocks - block0)), dim3(64 * kWgradWaves), lds, s, t, l0);
+  return hipGetLastError();
+}
+
+hipError_t conv3x3_wgrad_sums(const WgradTable &t, hipStream_t s) {
+  if (t.n < 1 || t.done != t.n) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(wgrad_reduce_kernel, dim3((unsigned)t.reduce[t.n]), dim3(256), 0, s, t);
   return hipGetLastError();
 }
 
