@@ -28,9 +28,9 @@ struct ConvArgs {
   // Inference head fused into the epilogue (cout = 32, an LDS tile): instead
   // of storing the activation, out = noisy + head_b + head_w * act per pixel.
   const float *head_w, *head_b;  // [3][32], [3]
-  const float4 *head_noisy;      // residual, row pitch head_noisy_pitch
+  const float *head_in;          // residual: 3 of head_in_floats floats a pixel (16-byte steps), rows of head_in_pitch pixels
   float4 *head_out;              // row pitch head_out_pitch; null = no head
-  int head_noisy_pitch, head_out_pitch;
+  int head_in_floats, head_in_pitch, head_out_pitch;  // (rows over all images)
   // First convolution (conv_first_pair; conv3x3 refuses it): the input records
   // are packed from the noisy image and the G-buffer while the tile is
   // staged, channels (noisy rgb, depth, normal xy, albedo rgb, zeros), the
@@ -99,15 +99,10 @@ hipError_t conv3x3_wgrad(WgradTable &t, float *part, size_t part_bytes, hipStrea
 hipError_t conv3x3_wgrad_sums(const WgradTable &t, hipStream_t s);
 size_t conv3x3_wgrad_scratch_bytes();
 hipError_t pack_input(const float *x12, size_t npix, bf16 *x32, hipStream_t s);
-hipError_t head_fwd_img(const bf16 *d1, const lgx_image &noisy, const float *wh, const float *bh, int out_pitch,
-                        float4 *out, hipStream_t s);
 hipError_t avgpool(const bf16 *x, int n, int h, int w, int c, bf16 *y, hipStream_t s);
 hipError_t pool_bwd_add(const bf16 *dx_in, const bf16 *dpool, const bf16 *act, int n, int h, int w, int c, bf16 *dx,
                         hipStream_t s);
 hipError_t upsample_bwd(const bf16 *dfull, const bf16 *act, int n, int hh, int ww, int c, bf16 *dhalf, hipStream_t s);
-// out row pitch in pixels: rows of w pixels (over all n images) start every out_pitch
-hipError_t head_fwd(const bf16 *d1, const float *x12, const float *wh, const float *bh, size_t npix, int w,
-                    int out_pitch, float4 *out, hipStream_t s);
 // the head's forward, the loss and the head's backward in one pass (training;
 // the head's output is not stored)
 hipError_t head_train(const bf16 *d1, const float *x12, const float4 *target, const float *wh, const float *bh,

@@ -320,21 +320,42 @@ class Net {
     check(conv_first_pair(c0, c1, s), "conv_first_pair");
   }
 
-  // head: also the 1x1 head into out_ (the training step forms the head in
-  // its backward pass instead)
-  void forward(const float *x12, int n, int h, int w, float *out_, hipStream_t s, int out_pitch = 0,
-               bool head = true) {
-    const size_t P = (size_t)n * h * w;
+  // head: the 1x1 head into out_, in the last convolution (the training step
+  // keeps that convolution's output and forms the head in its backward pass)
+  void forward(const float *x12, int n, int h, int w, float *out_, hipStream_t s, bool head = true) {
     ConvArgs c0{};
     c0.gin_fmt = 3;
     c0.gin_x12 = x12;
     c0.rec_out = x32;  // the packed records: the first layer's weight gradient reads them
     first_pair(c0, n, h, w, e1a, s);
-    body(n, h, w, s, 10, 2);
-    if (!head) return;
-    check(head_fwd(d1, x12, params + head_w_off, params + head_b_off, P, w, out_pitch > 0 ? out_pitch : w,
-                   (float4 *)out_, s),
-          "head_fwd");
+    body(n, h, w, s, head ? 9 : 10, 2);
+    if (head) conv_head(n, h, w, x12, 12, w, (float4 *)out_, w, s);
+  }
+
+  // The last convolution with the 1x1 head fused into its epilogue (an LDS
+  // tile over all 32 channels: the autotuned one, else the first offered).
+  void conv_head(int n, int h, int w, const float *in, int in_floats, int in_pitch, float4 *out_, int out_pitch,
+                 hipStream_t s) {
+    ConvArgs c{};
+    c.a = d1a;
+    c.ca = 32;
+    c.n = n;
+    c.h = h;
+    c.w = w;
+    c.wt = wf[9];
+    c.bias = params + b_off[9];
+    c.cout = 32;
+    c.relu = 1;
+    c.split = 32;
+    c.tile = lds_tile32(9);
+    c.head_w = params + head_w_off;
+    c.head_b = params + head_b_off;
+    c.head_in = in;
+    c.head_in_floats = in_floats;
+    c.head_in_pitch = in_pitch;
+    c.head_out = out_;
+    c.head_out_pitch = out_pitch;
+    check(conv3x3(c, s), "conv3x3 with head");
   }
 
   // An LDS tile of a 32-channel convolution: the autotuned one for layer l, else the first offered.
@@ -365,27 +386,7 @@ class Net {
       first_pair(c, 1, h, w, nullptr, s);
     }
     body(1, h, w, s, 9, 2);
-    // the last convolution with the 1x1 head fused into its epilogue (an LDS
-    // tile over all 32 channels: the autotuned one, else the first offered)
-    ConvArgs c{};
-    c.a = d1a;
-    c.ca = 32;
-    c.n = 1;
-    c.h = h;
-    c.w = w;
-    c.wt = wf[9];
-    c.bias = params + b_off[9];
-    c.cout = 32;
-    c.relu = 1;
-    c.split = 32;
-    c.tile = lds_tile32(9);
-    c.head_w = params + head_w_off;
-    c.head_b = params + head_b_off;
-    c.head_noisy = (const float4 *)noisy.ptr;
-    c.head_noisy_pitch = noisy.pitch;
-    c.head_out = (float4 *)out_.ptr;
-    c.head_out_pitch = out_.pitch;
-    check(conv3x3(c, s), "conv3x3 with head");
+    conv_head(1, h, w, (const float *)noisy.ptr, 4, noisy.pitch, (float4 *)out_.ptr, out_.pitch, s);
   }
 
   // Times every register tile of every forward (and, with backward, every
@@ -444,7 +445,7 @@ class Net {
   void backward(const float *x12, const float *target, int n, int h, int w, hipStream_t s) {
     const size_t P = (size_t)n * h * w;
     const int h2 = h / 2, w2 = w / 2, h4 = h / 4, w4 = w / 4;
-    forward(x12, n, h, w, out, s, 0, false);
+    forward(x12, n, h, w, out, s, false);
     // the head's gradient and the loss are accumulated atomically; every
     // convolution gradient is overwritten by its reduction
     check(fill(grads + head_w_off, (size_t)kHeadIn * kHeadOut + kHeadOut + 1, 0.f, s), "fill");  // and the loss

@@ -58,6 +58,10 @@ LGX_D bf16x4 row_load(__amdgpu_buffer_rsrc_t r, int offset) {
   return __builtin_bit_cast(bf16x4, __builtin_amdgcn_raw_buffer_load_b64(r, offset, 0, 0));
 }
 LGX_D float relu(float v) { return fmaxf(v, 0.f); }  // one instruction; NaN and -0 give +0
+// The residual of the inference head at a pixel (the first three of four floats).
+LGX_D float4 head_input(const ConvArgs &a, int n, int y, int x) {
+  return *(const float4 *)(a.head_in + (((size_t)n * a.h + y) * a.head_in_pitch + x) * a.head_in_floats);
+}
 // v with the channels zeroed whose mask is not positive (NaN: zeroed)
 LGX_D bf16x4 masked(bf16x4 v, bf16x4 m) {
 #pragma unroll
@@ -577,7 +581,7 @@ __global__ __launch_bounds__(256, conv_lds_blocks(MB, WR, WP)) void conv3x3_lds_
       for (int p = tid; p < TH * TW; p += 256) {
         const int y = cur.y0 + p / TW, x = cur.x0 + p % TW;
         if (y < a.h && x < a.w) {
-          const float4 c = a.head_noisy[(size_t)y * a.head_noisy_pitch + x];
+          const float4 c = head_input(a, cur.n, y, x);
           float o[3] = {c.x + hw[96], c.y + hw[97], c.z + hw[98]};
 #pragma unroll 1
           for (int q = 0; q < 4; q++) {
@@ -589,7 +593,7 @@ __global__ __launch_bounds__(256, conv_lds_blocks(MB, WR, WP)) void conv3x3_lds_
               for (int k = 0; k < 3; k++) o[k] += hw[k * 32 + q * 8 + i] * f;
             }
           }
-          a.head_out[(size_t)y * a.head_out_pitch + x] = make_float4(o[0], o[1], o[2], 1.f);
+          a.head_out[((size_t)cur.n * a.h + y) * a.head_out_pitch + x] = make_float4(o[0], o[1], o[2], 1.f);
         }
       }
       __syncthreads();  // the next tile's stash overwrites the activations
@@ -965,7 +969,7 @@ __global__ __launch_bounds__(64 * NW, OCC) void conv3x3_dma_kernel(const ConvArg
           for (int p = lane; p < WR * TW; p += 64) {
             const int y = cur.y0 + wave * WR + p / TW, x = cur.x0 + p % TW;
             if (y >= a.h || x >= a.w) continue;
-            const float4 c = a.head_noisy[(size_t)y * a.head_noisy_pitch + x];
+            const float4 c = head_input(a, cur.n, y, x);
             float o[3] = {c.x + a.head_b[0], c.y + a.head_b[1], c.z + a.head_b[2]};
 #pragma unroll
             for (int q = 0; q < 4; q++) {
@@ -977,7 +981,7 @@ __global__ __launch_bounds__(64 * NW, OCC) void conv3x3_dma_kernel(const ConvArg
                 for (int k = 0; k < 3; k++) o[k] += a.head_w[k * 32 + q * 8 + i] * f;
               }
             }
-            a.head_out[(size_t)y * a.head_out_pitch + x] = make_float4(o[0], o[1], o[2], 1.f);
+            a.head_out[((size_t)cur.n * a.h + y) * a.head_out_pitch + x] = make_float4(o[0], o[1], o[2], 1.f);
           }
         } else {
           if constexpr (PAIRS)
@@ -1711,43 +1715,6 @@ __global__ __launch_bounds__(256) void upsample_bwd_kernel(const bf16 *dfull, co
   }
 }
 
-// Output head: out = noisy + W_h * d1 + b_h (1x1, 32 -> 3, FP32 output RGBA).
-__global__ __launch_bounds__(256) void head_fwd_kernel(const bf16 *d1, const float *x12, const float *wh,
-                                                       const float *bh, size_t npix, int w, int out_pitch,
-                                                       float4 *out) {
-  const size_t p = (size_t)blockIdx.x * 256 + threadIdx.x;
-  if (p >= npix) return;
-  float o[3];
-  for (int c = 0; c < 3; c++) o[c] = x12[p * 12 + c] + bh[c];
-  for (int q = 0; q < 4; q++) {
-    const bf16x8 v = *(const bf16x8 *)(d1 + p * 32 + q * 8);
-    for (int i = 0; i < 8; i++) {
-      const float f = bf2f(v[i]);
-      for (int c = 0; c < 3; c++) o[c] += wh[c * 32 + q * 8 + i] * f;
-    }
-  }
-  out[(p / w) * out_pitch + p % w] = make_float4(o[0], o[1], o[2], 1.f);
-}
-
-// The head for inference: the residual comes from the noisy image itself.
-__global__ __launch_bounds__(256) void head_fwd_img_kernel(const bf16 *d1, const float4 *noisy, int np_,
-                                                           const float *wh, const float *bh, int w, int h,
-                                                           int out_pitch, float4 *out) {
-  const size_t p = (size_t)blockIdx.x * 256 + threadIdx.x;
-  if (p >= (size_t)w * h) return;
-  const int x = (int)(p % w), y = (int)(p / w);
-  const float4 c = noisy[(size_t)y * np_ + x];
-  float o[3] = {c.x + bh[0], c.y + bh[1], c.z + bh[2]};
-  for (int q = 0; q < 4; q++) {
-    const bf16x8 v = *(const bf16x8 *)(d1 + p * 32 + q * 8);
-    for (int i = 0; i < 8; i++) {
-      const float f = bf2f(v[i]);
-      for (int k = 0; k < 3; k++) o[k] += wh[k * 32 + q * 8 + i] * f;
-    }
-  }
-  out[(size_t)y * out_pitch + x] = make_float4(o[0], o[1], o[2], 1.f);
-}
-
 // Training: the 1x1 head, the loss and the head's backward in one pass (the
 // head's output is not stored).  One pixel per thread: out = x + b_h + W_h
 // act, summed in head_fwd_kernel's order; mean L1: g = sign(out - target) /
@@ -2079,7 +2046,7 @@ template <int MB> static hipError_t conv_mb(const ConvArgs &a, const ConvTile &t
 
 hipError_t conv3x3(const ConvArgs &a, hipStream_t s) {
   if (a.cout % 16 || (a.bias != nullptr) != (a.relu != 0)) return hipErrorInvalidValue;
-  if (a.head_out && (a.cout != 32 || a.n != 1 || !conv3x3_tile_lds(a.cout, a.tile))) return hipErrorInvalidValue;
+  if (a.head_out && (a.cout != 32 || !a.head_in || !conv3x3_tile_lds(a.cout, a.tile))) return hipErrorInvalidValue;
   if (a.gin_fmt) return hipErrorInvalidValue;  // records packed while staging: conv_first_pair
   if (a.pool_out && (a.head_out || a.mask0 || a.mask1 || !conv3x3_tile_pool(a.cout, a.tile)))
     return hipErrorInvalidValue;
@@ -2218,13 +2185,6 @@ hipError_t pack_input(const float *x12, size_t npix, bf16 *x32, hipStream_t s) {
   hipLaunchKernelGGL(pack_input_kernel, dim3((unsigned)((npix + 63) / 64)), dim3(256), 0, s, x12, npix, x32);
   return hipGetLastError();
 }
-hipError_t head_fwd_img(const bf16 *d1, const lgx_image &noisy, const float *wh, const float *bh, int out_pitch,
-                        float4 *out, hipStream_t s) {
-  const size_t npix = (size_t)noisy.w * noisy.h;
-  hipLaunchKernelGGL(head_fwd_img_kernel, dim3((unsigned)((npix + 255) / 256)), dim3(256), 0, s, d1,
-                     (const float4 *)noisy.ptr, noisy.pitch, wh, bh, noisy.w, noisy.h, out_pitch, out);
-  return hipGetLastError();
-}
 hipError_t avgpool(const bf16 *x, int n, int h, int w, int c, bf16 *y, hipStream_t s) {
   hipLaunchKernelGGL(avgpool_kernel, dim3(grid_for((size_t)n * (h / 2) * (w / 2) * (c / 8), 256)), dim3(256), 0, s, x,
                      n, h, w, c, y);
@@ -2241,12 +2201,6 @@ hipError_t pool_bwd_add(const bf16 *dx_in, const bf16 *dpool, const bf16 *act, i
 hipError_t upsample_bwd(const bf16 *dfull, const bf16 *act, int n, int hh, int ww, int c, bf16 *dhalf, hipStream_t s) {
   hipLaunchKernelGGL(upsample_bwd_kernel, dim3(grid_for((size_t)n * hh * ww * (c / 8), 256)), dim3(256), 0, s, dfull,
                      act, n, hh, ww, c, dhalf);
-  return hipGetLastError();
-}
-hipError_t head_fwd(const bf16 *d1, const float *x12, const float *wh, const float *bh, size_t npix, int w,
-                    int out_pitch, float4 *out, hipStream_t s) {
-  hipLaunchKernelGGL(head_fwd_kernel, dim3((unsigned)((npix + 255) / 256)), dim3(256), 0, s, d1, x12, wh, bh, npix, w,
-                     out_pitch, out);
   return hipGetLastError();
 }
 hipError_t head_train(const bf16 *d1, const float *x12, const float4 *target, const float *wh, const float *bh,
