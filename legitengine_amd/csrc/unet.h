@@ -25,7 +25,7 @@ struct ConvArgs {
   bf16 *out1;     // channels [split, cout)
   const bf16 *mask0, *mask1;
   int tile;       // register tile: an index below conv3x3_tiles(cout), 0 = default
-  // Inference head fused into the epilogue (cout = 32, an LDS tile): instead
+  // Inference head fused into the epilogue (cout = 32, conv3x3_head_tile): instead
   // of storing the activation, out = noisy + head_b + head_w * act per pixel.
   const float *head_w, *head_b;  // [3][32], [3]
   const float *head_in;          // residual: 3 of head_in_floats floats a pixel (16-byte steps), rows of head_in_pitch pixels
@@ -90,7 +90,9 @@ hipError_t conv3x3(const ConvArgs &a, hipStream_t s);
 // the packed records to a0.rec_out, which the backward pass reads.
 hipError_t conv_first_pair(const ConvArgs &a0, const ConvArgs &a1, hipStream_t s);
 int conv3x3_tiles(int cout);  // register tiles offered for this output channel count
-int conv3x3_tile_lds(int cout, int tile);  // 1 if that tile is an LDS tile covering all cout channels
+// The tile of a convolution with head_out: the direct-load tile of four waves (the whole denoise / forward, us:
+// 1920 x 1080 523, the other tiles 523 to 579; 16 x 256 x 256 319, 322 to 335; 256 x 256 84, 85 to 88).
+int conv3x3_head_tile();
 int conv3x3_tile_pool(int cout, int tile);  // 1 if that tile can write the 2x2 pooled output (pool_out)
 // The weight gradients of the layers added to the table since the last call, in one launch, as partial sums in
 // part; after at most kWgradLaunches of them conv3x3_wgrad_sums adds those of all layers.

@@ -332,8 +332,7 @@ class Net {
     if (head) conv_head(n, h, w, x12, 12, w, (float4 *)out_, w, s);
   }
 
-  // The last convolution with the 1x1 head fused into its epilogue (an LDS
-  // tile over all 32 channels: the autotuned one, else the first offered).
+  // The last convolution with the 1x1 head fused into its epilogue.
   void conv_head(int n, int h, int w, const float *in, int in_floats, int in_pitch, float4 *out_, int out_pitch,
                  hipStream_t s) {
     ConvArgs c{};
@@ -347,7 +346,7 @@ class Net {
     c.cout = 32;
     c.relu = 1;
     c.split = 32;
-    c.tile = lds_tile32(9);
+    c.tile = conv3x3_head_tile();
     c.head_w = params + head_w_off;
     c.head_b = params + head_b_off;
     c.head_in = in;
@@ -356,14 +355,6 @@ class Net {
     c.head_out = out_;
     c.head_out_pitch = out_pitch;
     check(conv3x3(c, s), "conv3x3 with head");
-  }
-
-  // An LDS tile of a 32-channel convolution: the autotuned one for layer l, else the first offered.
-  int lds_tile32(int l) const {
-    if (conv3x3_tile_lds(32, fwd_tile[l])) return fwd_tile[l];
-    for (int t = 0; t < conv3x3_tiles(32); t++)
-      if (conv3x3_tile_lds(32, t)) return t;
-    return 0;
   }
 
   // Inference straight from a G-buffer and the noisy image (the values of

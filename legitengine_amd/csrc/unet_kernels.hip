@@ -301,8 +301,6 @@ template <int MB, int PB, int R> __global__ __launch_bounds__(256) void conv3x3_
 // tiles blockIdx.x, blockIdx.x + gridDim.x, ...  Every output is
 // accumulated in the same order as conv3x3_kernel (chunk, dx, dy), so the
 // two kernels give bit-identical results.
-// HEAD: the inference head fused into the epilogue (its own instantiation;
-// needs MB = 2, i.e. all 32 channels of a pixel in one workgroup).
 // With one input chunk and no channel split every tile uses the same
 // weights: they stay in LDS from the workgroup's first tile on.
 
@@ -390,7 +388,7 @@ constexpr int conv_lds_blocks(int MB, int WR, int WP) {
 
 // UP: the epilogue of an input gradient through an upsample (ConvArgs::up_out),
 // a separate instantiation so the other convolutions keep their registers.
-template <int MB, int WR, int WP, bool HEAD, bool UP = false>
+template <int MB, int WR, int WP, bool UP = false>
 __global__ __launch_bounds__(256, conv_lds_blocks(MB, WR, WP)) void conv3x3_lds_kernel(const ConvArgs a, int tiles_x,
                                                                                       int tiles_y, int splits) {
   constexpr int TH = 4 * WR, TW = 16 * WP, IW = TW + 2, IH = TH + 2;
@@ -442,7 +440,7 @@ __global__ __launch_bounds__(256, conv_lds_blocks(MB, WR, WP)) void conv3x3_lds_
   // serialising the prefetch with the matrix work.
   bf16x8 pin[IN_PER], pw[W_PER];
   uint32_t valid = 0;  // bit i: piece i of pin lies in the image
-  const bool w_resident = !HEAD && chunks == 1 && splits == 1;
+  const bool w_resident = chunks == 1 && splits == 1;
   auto fetch = [&](const Tile &tl, int cc, bool with_w) {
     const bool from_a = cc * 32 < a.ca;
     const bool up = from_a && a.a_up;
@@ -491,16 +489,14 @@ __global__ __launch_bounds__(256, conv_lds_blocks(MB, WR, WP)) void conv3x3_lds_
     // unconditional like the tile loads (a layer without bias reads its
     // weights instead and never adds the values).
     float bias_r[MB][4];
-    if constexpr (!HEAD) {  // (the head's epilogue stores to LDS: it reads the bias there)
-      const float *bsrc = a.bias ? a.bias : (const float *)a.wt;
+    const float *bsrc = a.bias ? a.bias : (const float *)a.wt;
 #pragma unroll
-      for (int mb = 0; mb < MB; mb++) {
-        const float4 b4 = *(const float4 *)(bsrc + cur.co0 + mb * 16 + kg * 4);
-        bias_r[mb][0] = b4.x;
-        bias_r[mb][1] = b4.y;
-        bias_r[mb][2] = b4.z;
-        bias_r[mb][3] = b4.w;
-      }
+    for (int mb = 0; mb < MB; mb++) {
+      const float4 b4 = *(const float4 *)(bsrc + cur.co0 + mb * 16 + kg * 4);
+      bias_r[mb][0] = b4.x;
+      bias_r[mb][1] = b4.y;
+      bias_r[mb][2] = b4.z;
+      bias_r[mb][3] = b4.w;
     }
     for (int cc = 0; cc < chunks; cc++) {
 #pragma unroll
@@ -525,7 +521,7 @@ __global__ __launch_bounds__(256, conv_lds_blocks(MB, WR, WP)) void conv3x3_lds_
       // in flight during the matrix work below: the next chunk, or the next tile's first
       if (cc + 1 < chunks)
         fetch(cur, cc + 1, true);
-      else if (!HEAD && t + (int)gridDim.x < T)  // a head launch has one tile per workgroup
+      else if (t + (int)gridDim.x < T)
         fetch(tile_of(t + (int)gridDim.x), 0, !w_resident);
 #pragma unroll
       for (int dx = 0; dx < 3; dx++) {
@@ -554,52 +550,7 @@ __global__ __launch_bounds__(256, conv_lds_blocks(MB, WR, WP)) void conv3x3_lds_
       }
       __syncthreads();  // the next stash overwrites the tiles
     }
-    if constexpr (HEAD) {
-      // fused inference head: the tile's activations (BF16, as the unfused
-      // path stores them) go to LDS, then one thread per pixel forms
-      // noisy + b + W * act in the unfused head's order (bit-identical)
-      bf16 *act = s_in;  // [TH][TW][32]; the input tile is no longer read
-      float *hw = (float *)s_w;  // head weights [3][32] and bias [3]; the chunk weights are no longer read
-      if (tid < 99) hw[tid] = tid < 96 ? a.head_w[tid] : a.head_b[tid - 96];
-#pragma unroll
-      for (int r = 0; r < WR; r++)
-#pragma unroll
-        for (int pb = 0; pb < WP; pb++)
-#pragma unroll
-          for (int mb = 0; mb < MB; mb++) {
-            const int co = mb * 16 + kg * 4;
-            typedef bf16 bf16x4 __attribute__((ext_vector_type(4)));
-            bf16x4 o;
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-              float v = acc[r][pb][mb][i] + a.bias[co + i];
-              o[i] = f2bf(v > 0.f ? v : 0.f);
-            }
-            *(bf16x4 *)(act + ((wave * WR + r) * TW + pb * 16 + col) * 32 + co) = o;
-          }
-      __syncthreads();
-      for (int p = tid; p < TH * TW; p += 256) {
-        const int y = cur.y0 + p / TW, x = cur.x0 + p % TW;
-        if (y < a.h && x < a.w) {
-          const float4 c = head_input(a, cur.n, y, x);
-          float o[3] = {c.x + hw[96], c.y + hw[97], c.z + hw[98]};
-#pragma unroll 1
-          for (int q = 0; q < 4; q++) {
-            const bf16x8 v = *(const bf16x8 *)(act + p * 32 + q * 8);
-#pragma unroll
-            for (int i = 0; i < 8; i++) {
-              const float f = bf2f(v[i]);
-#pragma unroll
-              for (int k = 0; k < 3; k++) o[k] += hw[k * 32 + q * 8 + i] * f;
-            }
-          }
-          a.head_out[((size_t)cur.n * a.h + y) * a.head_out_pitch + x] = make_float4(o[0], o[1], o[2], 1.f);
-        }
-      }
-      __syncthreads();  // the next tile's stash overwrites the activations
-    } else {
     conv_epilogue<WR, WP, MB, UP>(a, acc, bias_r, cur.n, cur.y0 + wave * WR, cur.x0, cur.co0, col, kg);
-    }
     t += gridDim.x;
     if (t >= T) break;
     cur = tile_of(t);
@@ -773,7 +724,7 @@ LGX_D void conv_epilogue_pairs(const ConvArgs &a, const f32x4 (&acc)[WR][WP][MB]
 // against 45 here, 113 against 95 for 192 -> 64 and 57 against 41 for 128 -> 64,
 // at 480 x 270 48 against 37 for 128 -> 128.
 constexpr int dma_in_blocks(int WR, int WP, int NW) { return ((NW * WR + 2) * (16 * WP + 2) + 15) / 16; }
-constexpr int dma_act_bytes(int WR, int WP, int NW, bool head) { return head ? NW * WR * WP * 16 * 80 : 0; }
+constexpr int dma_act_bytes(int WR, int WP, int NW, bool head) { return head ? NW * WR * WP * 16 * 64 + 512 : 0; }
 // LDS bytes with `slots` weight chunks
 constexpr int dma_lds_bytes(int MB, int WR, int WP, int NW, bool head, int slots) {
   return (2 * dma_in_blocks(WR, WP, NW) + 9 * MB * slots) * 1024 + dma_act_bytes(WR, WP, NW, head);
@@ -868,6 +819,10 @@ __global__ __launch_bounds__(64 * NW, OCC) void conv3x3_dma_kernel(const ConvArg
       in_off[rr][dx] = p * 64 + (kg ^ ((p >> 2) & 3)) * 16;
     }
   Tile cur = tile_of(t);
+  char *const s_act = s_w + (wres ? chunks : 2) * WBLK * 1024;
+  // the head's weights and bias, in LDS: read from memory they would wait behind the next stage's loads
+  float *const s_head = (float *)(s_act + NW * WR * TW * 64);
+  if (HEAD && threadIdx.x < 99) s_head[threadIdx.x] = threadIdx.x < 96 ? a.head_w[threadIdx.x] : a.head_b[threadIdx.x - 96];
   if (wres)
     for (int cc = 0; cc < chunks; cc++) dma_w(cc, cc);
   else
@@ -894,6 +849,15 @@ __global__ __launch_bounds__(64 * NW, OCC) void conv3x3_dma_kernel(const ConvArg
 #pragma unroll
         for (int mb = 0; mb < MB; mb++) acc[r][pb][mb] = f32x4{0.f, 0.f, 0.f, 0.f};
     const int tn = t + step;
+    // HEAD: this lane's pixels (lane, lane + 64, .. of the wave's), their residuals ahead of the next stage's loads
+    constexpr int NP = HEAD ? WR * TW / 64 : 1;
+    float4 head_c[NP];
+    if constexpr (HEAD)
+#pragma unroll
+      for (int k = 0; k < NP; k++) {
+        const int p = lane + k * 64, y = min(cur.y0 + wave * WR + p / TW, a.h - 1), x = min(cur.x0 + p % TW, a.w - 1);
+        head_c[k] = head_input(a, cur.n, y, x);
+      }
     for (int cc = 0; cc < chunks; cc++) {
       // the next stage into the other buffer: every wave is past the barrier that ended its last use
       const bool more = cc + 1 < chunks || tn < T;
@@ -944,11 +908,13 @@ __global__ __launch_bounds__(64 * NW, OCC) void conv3x3_dma_kernel(const ConvArg
       if (cc + 1 == chunks) {
         if constexpr (HEAD) {
           // the inference head: each wave's activations (BF16, as the unfused
-          // path stores them) through LDS of its own (80 bytes a pixel: reads
-          // of neighbouring pixels on different banks), then a lane per pixel
-          // forms noisy + b + W act in the unfused head's order
+          // path stores them) through LDS of its own, then a lane per pixel
+          // forms in + b + W act, channel by channel.  1920 x 1080: 75 us, 55
+          // without the head; with 80 bytes a pixel in LDS only one
+          // workgroup fits a CU (108), and with the head's weights read
+          // from memory per tile, behind the next stage's loads, 118.
           static_assert(!HEAD || (MB == 2 && WR * WP % 4 == 0), "a lane per pixel");
-          char *act = s_w + (wres ? chunks : 2) * WBLK * 1024 + wave * (WR * TW * 80);
+          char *act = s_act + wave * (WR * TW * 64);
 #pragma unroll
           for (int r = 0; r < WR; r++)
 #pragma unroll
@@ -962,26 +928,39 @@ __global__ __launch_bounds__(64 * NW, OCC) void conv3x3_dma_kernel(const ConvArg
                   const float v = acc[r][pb][mb][i] + bias_r[mb][i];
                   o[i] = f2bf(v > 0.f ? v : 0.f);
                 }
-                *(bf16x4 *)(act + (r * TW + pb * 16 + col) * 80 + pair_row(PAIRS, mb, kg * 4) * 2) = o;
+                // (the 16-byte place of channels 8 c .. 8 c + 7 of pixel p is c ^ (p / 4 % 4))
+                *(bf16x4 *)(act + (r * TW + pb * 16 + col) * 64 + ((mb * 2 + (kg >> 1)) ^ (col >> 2)) * 16 + (kg & 1) * 8) = o;
               }
           __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+          // (a buffer from the wave's first row: one store a pixel whatever lies outside, which the wait counts on)
+          const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+              (void *)(a.head_out + ((size_t)cur.n * a.h + cur.y0 + wave * WR) * a.head_out_pitch), (short)0, 0x7fffffff,
+              0x00020000);
 #pragma unroll
-          for (int p = lane; p < WR * TW; p += 64) {
-            const int y = cur.y0 + wave * WR + p / TW, x = cur.x0 + p % TW;
-            if (y >= a.h || x >= a.w) continue;
-            const float4 c = head_input(a, cur.n, y, x);
-            float o[3] = {c.x + a.head_b[0], c.y + a.head_b[1], c.z + a.head_b[2]};
+          for (int k = 0; k < NP; k++) {
+            const int p = lane + k * 64, r = p / TW, x = cur.x0 + p % TW;
+            const float4 c = head_c[k];
+            const f32x4 hb = *(const f32x4 *)(s_head + 96);
+            float o[3] = {c.x + hb[0], c.y + hb[1], c.z + hb[2]};
 #pragma unroll
             for (int q = 0; q < 4; q++) {
-              const bf16x8 v = *(const bf16x8 *)(act + p * 80 + q * 16);
+              const bf16x8 v = *(const bf16x8 *)(act + p * 64 + (q ^ (p >> 2 & 3)) * 16);
+              f32x4 hw[3][2];
+#pragma unroll
+              for (int k3 = 0; k3 < 3; k3++)
+#pragma unroll
+                for (int i = 0; i < 2; i++) hw[k3][i] = *(const f32x4 *)(s_head + k3 * 32 + q * 8 + i * 4);
 #pragma unroll
               for (int i = 0; i < 8; i++) {
                 const float f = bf2f(v[i]);
 #pragma unroll
-                for (int k = 0; k < 3; k++) o[k] += a.head_w[k * 32 + q * 8 + i] * f;
+                for (int k3 = 0; k3 < 3; k3++) o[k3] += hw[k3][i >> 2][i & 3] * f;
               }
             }
-            a.head_out[((size_t)cur.n * a.h + y) * a.head_out_pitch + x] = make_float4(o[0], o[1], o[2], 1.f);
+            const f32x4 out = {o[0], o[1], o[2], 1.f};
+            const bool in = cur.y0 + wave * WR + r < a.h && x < a.w;
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, out), rs,
+                                                   in ? (r * a.head_out_pitch + x) * 16 : (int)0x80000000u, 0, 0);
           }
         } else {
           if constexpr (PAIRS)
@@ -995,8 +974,10 @@ __global__ __launch_bounds__(64 * NW, OCC) void conv3x3_dma_kernel(const ConvArg
         // after them (memory operations of a wave retire from this counter in
         // order), and waiting for those too would hold every tile for a
         // store's round trip.  (conv_epilogue skips rows past the image: no count.)
-        if (!PAIRS || cc + 1 < chunks)
+        if (cc + 1 < chunks || (!PAIRS && !HEAD))
           asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+        else if constexpr (HEAD)
+          asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(NP) : "memory");
         else
           asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(epilogue_stores<WR, WP, MB, UP>()) : "memory");
       }
@@ -1921,11 +1902,11 @@ static const ConvTile *conv_tiles(int mb, int *count) {
 #undef LGX_TILES
 }
 
-int conv3x3_tile_lds(int cout, int tile) {
-  int n = 0;
-  if (cout % 16) return 0;
-  const ConvTile *t = conv_tiles(cout / 16, &n);
-  return t && tile >= 0 && tile < n && t[tile].lds && t[tile].mbw * 16 == cout;
+int conv3x3_head_tile() {
+  const int n = (int)(sizeof(kTiles2) / sizeof(kTiles2[0]));
+  int t = 0;
+  while (t + 1 < n && kTiles2[t].lds != 2) t++;
+  return t;
 }
 
 int conv3x3_tile_pool(int cout, int tile) {
@@ -1964,21 +1945,14 @@ template <int MBW, int WR, int WP> static void launch_conv_lds(const ConvArgs &a
   const int tx = (a.w + 16 * WP - 1) / (16 * WP), ty = (a.h + 4 * WR - 1) / (4 * WR), splits = a.cout / (16 * MBW);
   const long tiles = (long)tx * ty * a.n * splits;
   long grid = per_cu > 0 ? std::min(tiles, (long)per_cu * cu_count()) : tiles;
-  if constexpr (MBW == 2) {
-    if (a.head_out) {  // one tile per workgroup: nothing is prefetched across the head's epilogue
-      hipLaunchKernelGGL((conv3x3_lds_kernel<MBW, WR, WP, true>), dim3((unsigned)tiles), dim3(256), 0, s, a, tx, ty,
-                         splits);
-      return;
-    }
-  }
   if constexpr (WR % 2 == 0) {
     if (a.up_out) {
-      hipLaunchKernelGGL((conv3x3_lds_kernel<MBW, WR, WP, false, true>), dim3((unsigned)grid), dim3(256), 0, s, a,
+      hipLaunchKernelGGL((conv3x3_lds_kernel<MBW, WR, WP, true>), dim3((unsigned)grid), dim3(256), 0, s, a,
                          tx, ty, splits);
       return;
     }
   }
-  hipLaunchKernelGGL((conv3x3_lds_kernel<MBW, WR, WP, false>), dim3((unsigned)grid), dim3(256), 0, s, a, tx, ty,
+  hipLaunchKernelGGL((conv3x3_lds_kernel<MBW, WR, WP>), dim3((unsigned)grid), dim3(256), 0, s, a, tx, ty,
                      splits);
 }
 
@@ -1999,7 +1973,7 @@ template <int MBW, int WR, int WP, int NW> static hipError_t launch_conv_dma(con
     hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(64 * NW), (size_t)lds, s, a, tx, ty, splits, wres);
     return hipGetLastError();
   };
-  if constexpr (MBW == 2) {
+  if constexpr (MBW == 2 && NW == 4) {
     if (head) return launch(conv3x3_dma_kernel<MBW, WR, WP, NW, OCC, true, false>);
   }
   if (head) return hipErrorInvalidValue;
@@ -2046,7 +2020,7 @@ template <int MB> static hipError_t conv_mb(const ConvArgs &a, const ConvTile &t
 
 hipError_t conv3x3(const ConvArgs &a, hipStream_t s) {
   if (a.cout % 16 || (a.bias != nullptr) != (a.relu != 0)) return hipErrorInvalidValue;
-  if (a.head_out && (a.cout != 32 || !a.head_in || !conv3x3_tile_lds(a.cout, a.tile))) return hipErrorInvalidValue;
+  if (a.head_out && (a.cout != 32 || !a.head_in || a.tile != conv3x3_head_tile())) return hipErrorInvalidValue;
   if (a.gin_fmt) return hipErrorInvalidValue;  // records packed while staging: conv_first_pair
   if (a.pool_out && (a.head_out || a.mask0 || a.mask1 || !conv3x3_tile_pool(a.cout, a.tile)))
     return hipErrorInvalidValue;
