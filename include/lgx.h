@@ -349,12 +349,12 @@ int lgx_gather_tiles(void);
  * identical results. */
 int lgx_gather_tile_info(int32_t tile, int32_t *info);
 
-/* ---- several views of uneven resolution in one persistent launch ----
+/* ---- several views of uneven resolution in one launch ----
  * No counterpart in the reference (its frame loop, main.cpp:269-312, renders
  * one view per frame); built for serving many views per submission.
  *
- * lgx_gather_batch: the IndirectLightPass of n views as ONE launch of a
- * persistent kernel whose workgroups walk the views' tiles.  Each item is
+ * lgx_gather_batch: the IndirectLightPass of n views as ONE launch, with a
+ * workgroup per block or persistent workgroups that walk the views' tiles.  Each item is
  * what lgx_gather takes, checked the same way; all share LGX_PREC_F32, the
  * sampler, the tile and the radiance / normal formats (RGBA16F + RG16F or
  * RGBA32F + RG32F); step_counts must be NULL; at most 2978 views (the
@@ -371,16 +371,16 @@ int lgx_gather_batch_set_tile(lgx_gather_batch *b, int32_t tile);
 /* Logical blocks (tiles x slices) of all views together. */
 int64_t lgx_gather_batch_blocks(const lgx_gather_batch *b);
 /* workgroups: persistent workgroups of four waves (the launch has as many
- * waves, its workgroups rounded up to a multiple of 8); 0 = as many waves as
- * the chip holds, or fewer if the blocks are fewer.  Workgroups take blocks from per-XCD counters
- * that the launch zeroes first (with a kernel: capturable), so launches of
- * ONE batch must not overlap in time (different batches may). */
+ * waves, its workgroups rounded up to a multiple of 8), which take blocks
+ * from per-XCD counters that the launch zeroes first (with a kernel:
+ * capturable); 0 = a workgroup per block.  Launches of ONE batch must not
+ * overlap in time (different batches may). */
 int lgx_gather_batch_launch(const lgx_gather_batch *b, int32_t workgroups, lgx_stream_t stream);
 void lgx_gather_batch_destroy(lgx_gather_batch *b);
 
 /* lgx_batch: the denoised path for n views (own G-buffers and cameras).
  * The views, in ascending pixel count, form `chunks` chunks; per chunk the
- * mips, Hi-Z and pre-blur of its views and ONE persistent lgx_gather_batch
+ * mips, Hi-Z and pre-blur of its views and ONE lgx_gather_batch
  * launch over them, then the U-Net of each of its views, smallest first,
  * and a device timestamp as each view completes, all on the caller's stream.  The whole batch can be
  * captured into ONE hipGraph and replayed. */
@@ -393,9 +393,9 @@ typedef struct {
 typedef struct {
   int32_t dirs, max_steps, levels, grid, sampler, footprint_dirs;
   int32_t tile;       /* gather launch shape */
-  int32_t workgroups; /* persistent gather workgroups, 0 = as many as the chip holds */
+  int32_t workgroups; /* persistent gather workgroups, 0 = a workgroup per block */
   int32_t grid_y;     /* interleave pattern height (lgx_gather_params), <= 0 = grid */
-  int32_t chunks;     /* views, in ascending pixel count, are gathered in this many persistent launches
+  int32_t chunks;     /* views, in ascending pixel count, are gathered in this many launches
                          (<= 0: 4); each chunk's U-Nets run before the next chunk's gather */
 } lgx_batch_config;
 /* net: created with max n >= 1 and max h x w covering every view; NULL =

@@ -3,7 +3,7 @@
 //
 // The views, in ascending pixel count, form a few chunks.  Per chunk the
 // stream builds the views' mips / Hi-Z / pre-blur (small launches), gathers
-// all of the chunk's views in one persistent launch (lgx_gather_batch) and
+// all of the chunk's views in one launch (lgx_gather_batch) and
 // then runs the U-Net of each of the chunk's views, smallest first.  Small
 // views therefore complete after a fraction of the batch.  (U-Nets on a
 // second stream, overlapping the next chunk's gather, waited for the
@@ -58,7 +58,7 @@ struct lgx_batch {
   std::vector<std::vector<int>> chunks;   // consecutive runs of `order`
   std::vector<void *> blocks;
   std::map<std::pair<int, int>, void *> ws;  // gather tables per extent
-  std::vector<lgx_gather_batch *> gbs;    // one persistent gather per chunk
+  std::vector<lgx_gather_batch *> gbs;    // one gather per chunk
   lgx_unet *net = nullptr;
   unsigned long long *ts = nullptr;  // device [n + 1]
   hipGraph_t graph = nullptr;

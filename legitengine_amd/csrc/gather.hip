@@ -762,6 +762,29 @@ __global__ __launch_bounds__(max_threads<T>(), OCC) void gather_multi_kernel(con
   }
 }
 
+// The same views with a workgroup per block, in the views' order, dispatched
+// by the hardware: blocks of a view go to the XCDs in contiguous bands, as
+// gather_kernel's.  For launches that say no number of workgroups: a persistent
+// launch of the chip's 8192 waves takes 7.18 ms for a batch of 512x512,
+// 1280x720, 1920x1080 and 2560x1440 (4 directions of 256, a launch per view),
+// this one 6.71: the hardware replaces each workgroup as it ends.
+template <class T, class A, int SAMPLER, int RFMT, int NFMT, int OCC, bool PIPE, bool SWZ>
+__global__ __launch_bounds__(max_threads<T>(), OCC) void gather_views_kernel(const GatherArgs<T> *__restrict__ views,
+                                                           const uint32_t *__restrict__ first, int n_views) {
+  extern __shared__ __align__(16) unsigned char s_part[];
+  typedef const GatherArgs<T> __attribute__((address_space(4))) CArgs;  // (as in gather_multi_kernel)
+  CArgs *cviews = (CArgs *)views;
+  int v = 0;
+  for (int hi = n_views - 1; v < hi;) {  // the last view that starts at or before this block
+    const int mid = (v + hi + 1) / 2;
+    if (first[mid] <= blockIdx.x) v = mid;
+    else hi = mid - 1;
+  }
+  const uint32_t f = first[v];
+  gather_block<T, A, SAMPLER, RFMT, NFMT, false, PIPE, SWZ>(cviews[v], xcd_remap(blockIdx.x - f, first[v + 1] - f),
+                                                            (A *)s_part);
+}
+
 __global__ void zero_u32_kernel(uint32_t *p, int n) {
   if ((int)threadIdx.x < n) p[threadIdx.x] = 0u;
 }
@@ -1317,7 +1340,7 @@ extern "C" int lgx_gather(const lgx_gather_params *p, void *workspace, const lgx
   return gather_impl<float, float>(p, workspace, g, pyr, out, (hipStream_t)stream);
 }
 
-// ---------------------------------------------------------------- several views, one persistent launch
+// ---------------------------------------------------------------- several views, one launch
 
 struct lgx_gather_batch {
   std::vector<lgx_gather_params> p;
@@ -1420,6 +1443,7 @@ static int gather_batch_upload(lgx_gather_batch *b, int tile) {
   return LGX_OK;
 }
 
+// grid 0: a workgroup per block; else persistent workgroups
 template <int SAMPLER, int RFMT, int NFMT>
 static hipError_t launch_multi(const lgx_gather_batch *b, unsigned grid, hipStream_t s) {
   const bool occ8 = kTiles[b->tile][2] == 8, pipe = kTiles[b->tile][3] == 1;
@@ -1427,27 +1451,33 @@ static hipError_t launch_multi(const lgx_gather_batch *b, unsigned grid, hipStre
   const GatherArgs<float> *args = (const GatherArgs<float> *)b->dev;
   const uint32_t *first = (const uint32_t *)((const unsigned char *)b->dev + (size_t)n * sizeof(GatherArgs<float>));
   uint32_t *next = (uint32_t *)(first + n + 1);
-  // a kernel, not a memset, so the launch can be captured into a graph
-  hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(64), 0, s, next, 8);
   // the Hi-Z sampler has the swizzled variants (make_args sets no jobs otherwise)
   constexpr bool kSwz = SAMPLER == LGX_SAMPLER_HIZ_POINT;
-  auto launch = [&](auto kern) {
-    hipLaunchKernelGGL(kern, dim3(grid), dim3(64u * (unsigned)b->split), (size_t)b->round * kShare * sizeof(float), s, args,
-                       first, n, next);
-    return hipGetLastError();
-  };
-  if (kSwz && b->njobs) {
+  const bool swz = kSwz && b->njobs;
+  if (swz)
     hipLaunchKernelGGL(swizzle_jobs_kernel, dim3((unsigned)b->job_rows, (unsigned)b->njobs), dim3(256), 0, s,
                        (const SwzJob *)b->swz);
-    if (occ8 && pipe) return launch(gather_multi_kernel<float, float, SAMPLER, RFMT, NFMT, 8, true, kSwz>);
-    if (occ8) return launch(gather_multi_kernel<float, float, SAMPLER, RFMT, NFMT, 8, false, kSwz>);
-    if (pipe) return launch(gather_multi_kernel<float, float, SAMPLER, RFMT, NFMT, 1, true, kSwz>);
-    return launch(gather_multi_kernel<float, float, SAMPLER, RFMT, NFMT, 1, false, kSwz>);
+  // a kernel, not a memset, so the launch can be captured into a graph
+  if (grid) hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(64), 0, s, next, 8);
+  const dim3 block(64u * (unsigned)b->split);
+  const size_t lds = (size_t)b->round * kShare * sizeof(float);
+  auto launch = [&](auto multi, auto views) {
+    if (grid)
+      hipLaunchKernelGGL(multi, dim3(grid), block, lds, s, args, first, n, next);
+    else
+      hipLaunchKernelGGL(views, dim3(b->total), block, lds, s, args, first, n);
+    return hipGetLastError();
+  };
+#define LGX_MULTI(OCC, PIPE, SWZ) \
+  launch(gather_multi_kernel<float, float, SAMPLER, RFMT, NFMT, OCC, PIPE, SWZ>, \
+         gather_views_kernel<float, float, SAMPLER, RFMT, NFMT, OCC, PIPE, SWZ>)
+  if (swz) {
+    if (occ8) return pipe ? LGX_MULTI(8, true, kSwz) : LGX_MULTI(8, false, kSwz);
+    return pipe ? LGX_MULTI(1, true, kSwz) : LGX_MULTI(1, false, kSwz);
   }
-  if (occ8 && pipe) return launch(gather_multi_kernel<float, float, SAMPLER, RFMT, NFMT, 8, true, false>);
-  if (occ8) return launch(gather_multi_kernel<float, float, SAMPLER, RFMT, NFMT, 8, false, false>);
-  if (pipe) return launch(gather_multi_kernel<float, float, SAMPLER, RFMT, NFMT, 1, true, false>);
-  return launch(gather_multi_kernel<float, float, SAMPLER, RFMT, NFMT, 1, false, false>);
+  if (occ8) return pipe ? LGX_MULTI(8, true, false) : LGX_MULTI(8, false, false);
+  return pipe ? LGX_MULTI(1, true, false) : LGX_MULTI(1, false, false);
+#undef LGX_MULTI
 }
 
 }  // namespace lgx
@@ -1507,15 +1537,18 @@ extern "C" int lgx_gather_batch_launch(const lgx_gather_batch *b, int32_t workgr
   if (!b || workgroups < 0) return LGX_EINVAL;
   const int64_t asked = workgroups > 0 ? workgroups : b->shapes;
   if (asked > (1 << 24)) return LGX_EINVAL;
-  // A workgroup asked for is of four waves: the launch has as many waves.  0
-  // asks for one per block; the chip's 8192 resident waves walk them (each
-  // workgroup ends with an attempt at all eight counters: with one workgroup
-  // per block of 64 pixels those attempts took longer than the gather, 17.5
-  // against 8.5 ms for four views of 7 Mpixel).
+  // A workgroup asked for is of four waves: the launch has as many waves, its
+  // workgroups a multiple of 8 for the XCD chunking.  0 asks for a workgroup
+  // per block: no counters (with them, each workgroup ends with an attempt at
+  // all eight: 17.5 ms for four views of 7 Mpixel), unless the launch would
+  // pass the grid's 2^32 threads; then the chip's 8192 resident waves.
   const uint32_t k = (uint32_t)b->split;
-  uint32_t grid = workgroups > 0 ? std::max(1u, (uint32_t)workgroups * 4u / k) : std::min(b->total, 8192u / k);
-  grid = (grid + 7) / 8 * 8;  // the XCD chunking needs a multiple of 8
-  if (grid == 0) return LGX_EINVAL;
+  uint32_t grid = 0;
+  if (workgroups > 0 || (uint64_t)b->total * 64 * k > 0xffffffffu) {
+    grid = workgroups > 0 ? std::max(1u, (uint32_t)workgroups * 4u / k) : std::min(b->total, 8192u / k);
+    grid = (grid + 7) / 8 * 8;
+  }
+  if (!grid && !b->total) return LGX_EINVAL;
   hipStream_t s = (hipStream_t)stream;
   hipError_t e;
   if (b->sampler == LGX_SAMPLER_HIZ_POINT)

@@ -383,7 +383,7 @@ class UNet:
 
 
 class GatherBatch:
-    """Several views' gathers in one persistent launch (lgx_gather_batch_*).
+    """Several views' gathers in one launch (lgx_gather_batch_*).
     items: (Gather, GBufferDev, PyramidDev, out DImage, view, proj) tuples."""
 
     def __init__(self, items):
