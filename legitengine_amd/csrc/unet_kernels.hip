@@ -709,11 +709,13 @@ LGX_D void conv_epilogue_pairs(const ConvArgs &a, const f32x4 (&acc)[WR][WP][MB]
 // when they fit (wres), else they move with their chunk.
 //
 // LDS layout: 64 bytes a pixel (or output channel), the 16-byte channel group g
-// of pixel p in place g ^ (p / 4 % 4).  A wave's direct load fills 1 KB, four
+// of pixel p in place g ^ 2 (p / 4 % 2).  A wave's direct load fills 1 KB, four
 // lanes to a pixel, so it reads whole 64-byte runs of memory (with a pixel's
 // groups 16 lanes apart, each lane of a quad read another cache line); the
-// exchange of places puts the 16 pixels of an operand read (from any start)
-// on all 64 banks.  Pixels outside the image are offsets outside the buffer,
+// exchange of places puts the lanes of an operand read that are served
+// together (8 of one group and the 8 others of the next one) on all 64 banks
+// from any first pixel; g ^ (p / 4 % 4) does so only from every fourth, and
+// half of the LDS cycles were conflicts (96 -> 32 at 1080p 131 us, now 126).  Pixels outside the image are offsets outside the buffer,
 // which load as zeros.  Accumulation order is conv3x3_kernel's.
 //
 // What bounds it: the epilogue and the outputs' stores (about 40 % of a layer;
@@ -759,7 +761,7 @@ __global__ __launch_bounds__(64 * NW, OCC) void conv3x3_dma_kernel(const ConvArg
     return r;
   };
   // this lane's pixel of the wave's i-th input block (row, column of the halo tile) and its channel group
-  const int part = ((lane & 3) ^ (lane >> 4)) * 16;
+  const int part = ((lane & 3) ^ (lane >> 4 & 1) * 2) * 16;
   int prow[NI], pcol[NI];
 #pragma unroll
   for (int i = 0; i < NI; i++) {
@@ -816,7 +818,7 @@ __global__ __launch_bounds__(64 * NW, OCC) void conv3x3_dma_kernel(const ConvArg
 #pragma unroll
     for (int dx = 0; dx < 3; dx++) {
       const int p = (wave * WR + rr) * IW + dx + col;
-      in_off[rr][dx] = p * 64 + (kg ^ ((p >> 2) & 3)) * 16;
+      in_off[rr][dx] = p * 64 + (kg ^ (p >> 2 & 1) * 2) * 16;
     }
   Tile cur = tile_of(t);
   char *const s_act = s_w + (wres ? chunks : 2) * WBLK * 1024;
@@ -867,7 +869,7 @@ __global__ __launch_bounds__(64 * NW, OCC) void conv3x3_dma_kernel(const ConvArg
         if (!wres) dma_w(buf ^ 1, nc);
       }
       const char *in = s_dma + buf * NBLK * 1024;
-      const char *w = s_w + (wres ? cc : buf) * WBLK * 1024 + col * 64 + (kg ^ (col >> 2)) * 16;
+      const char *w = s_w + (wres ? cc : buf) * WBLK * 1024 + col * 64 + (kg ^ (col >> 2 & 1) * 2) * 16;
       // Taps in the order (dx, dy).  The operands of a tap are read while the
       // previous one's MFMAs run: its weights, and the next column's rows a
       // third at a time.  (Left to the compiler the reads sit right before
