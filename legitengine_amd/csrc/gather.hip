@@ -767,7 +767,8 @@ __global__ __launch_bounds__(max_threads<T>(), OCC) void gather_multi_kernel(con
 // gather_kernel's.  For launches that say no number of workgroups: a persistent
 // launch of the chip's 8192 waves takes 7.18 ms for a batch of 512x512,
 // 1280x720, 1920x1080 and 2560x1440 (4 directions of 256, a launch per view),
-// this one 6.71: the hardware replaces each workgroup as it ends.
+// this one 6.71, and 32 views of 63 Mpixel with their U-Nets 86.4 against 71.9:
+// the hardware replaces each workgroup as it ends.
 template <class T, class A, int SAMPLER, int RFMT, int NFMT, int OCC, bool PIPE, bool SWZ>
 __global__ __launch_bounds__(max_threads<T>(), OCC) void gather_views_kernel(const GatherArgs<T> *__restrict__ views,
                                                            const uint32_t *__restrict__ first, int n_views) {

@@ -715,16 +715,16 @@ LGX_D void conv_epilogue_pairs(const ConvArgs &a, const f32x4 (&acc)[WR][WP][MB]
 // exchange of places puts the lanes of an operand read that are served
 // together (8 of one group and the 8 others of the next one) on all 64 banks
 // from any first pixel; g ^ (p / 4 % 4) does so only from every fourth, and
-// half of the LDS cycles were conflicts (96 -> 32 at 1080p 131 us, now 126).  Pixels outside the image are offsets outside the buffer,
-// which load as zeros.  Accumulation order is conv3x3_kernel's.
+// half of the LDS cycles were conflicts (96 -> 32 at 1080p 131 us, now 126).
+// Pixels outside the image are offsets outside the buffer, which load as zeros.  Accumulation order is conv3x3_kernel's.
 //
 // What bounds it: the epilogue and the outputs' stores (about 40 % of a layer;
 // without them 64 -> 64 at 960 x 540 takes 33 us instead of 46), then the matrix
 // work; the input loads are hidden.  conv3x3_lds_kernel holds the next stage
 // in registers, which the wide tiles do not have to spare, and issues every
 // element's LDS store: at 960 x 540 its best tile takes 63 us for 64 -> 64
-// against 45 here, 113 against 95 for 192 -> 64 and 57 against 41 for 128 -> 64,
-// at 480 x 270 48 against 37 for 128 -> 128.
+// against 45 here, 113 against 91 for 192 -> 64 and 57 against 40 for 128 -> 64,
+// at 480 x 270 47 against 36 for 128 -> 128.
 constexpr int dma_in_blocks(int WR, int WP, int NW) { return ((NW * WR + 2) * (16 * WP + 2) + 15) / 16; }
 constexpr int dma_act_bytes(int WR, int WP, int NW, bool head) { return head ? NW * WR * WP * 16 * 64 + 512 : 0; }
 // LDS bytes with `slots` weight chunks
@@ -1863,9 +1863,9 @@ static unsigned grid_for(size_t work, size_t per_block) {
 // default, the others are the autotuner's candidates.  Which tile a layer gets
 // is measured at the network's shape (1920 x 1080, us: best register tile /
 // best conv3x3_lds_kernel tile / best conv3x3_dma_kernel tile): 32 -> 32 at full
-// size 84 / 57 / 55; 32 -> 64 at half size 51 / 36 / 27; 128 -> 64 99 / 57 /
-// 41; 64 -> 128 at a quarter 63 / 28 / 22; 192 -> 64 at half size 213 / 113 /
-// 95.  The smallest images go the other way (quarter size of 256 x 256:
+// size 84 / 57 / 55; 32 -> 64 at half size 51 / 36 / 26; 128 -> 64 99 / 57 /
+// 40; 64 -> 128 at a quarter 63 / 27 / 23; 192 -> 64 at half size 213 / 113 /
+// 91.  The smallest images go the other way (quarter size of 256 x 256:
 // 12.4 / 13.5 / 19): the direct-load tiles are the largest, and too few of them
 // fill the chip.
 struct ConvTile {
