@@ -93,6 +93,7 @@ int conv3x3_tiles(int cout);  // register tiles offered for this output channel 
 // The tile of a convolution with head_out: the direct-load tile of four waves (the whole denoise / forward, us:
 // 1920 x 1080 523, the other tiles 523 to 579; 16 x 256 x 256 319, 322 to 335; 256 x 256 84, 85 to 88).
 int conv3x3_head_tile();
+int conv3x3_default_tile(int cout, long pixels);  // of a network that was not autotuned
 int conv3x3_tile_pool(int cout, int tile);  // 1 if that tile can write the 2x2 pooled output (pool_out)
 // The weight gradients of the layers added to the table since the last call, in one launch, as partial sums in
 // part; after at most kWgradLaunches of them conv3x3_wgrad_sums adds those of all layers.

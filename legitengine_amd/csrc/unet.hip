@@ -72,7 +72,7 @@ class Net {
       *g_e1a;
   int adam_t = 0;
   // register tile of each layer's forward and input-gradient convolution
-  // (an index below conv3x3_tiles(cout)); set by autotune()
+  // (an index below conv3x3_tiles(cout)): by the largest extents at first, then as autotune() measures
   int fwd_tile[10] = {}, dx_tile[10] = {};
 
   void *alloc(size_t bytes) {
@@ -114,6 +114,11 @@ class Net {
       wt[l] = l == 0 ? nullptr : (bf16 *)alloc((size_t)9 * L.cin_pad * L.cout * 2);
     }
     const size_t P = (size_t)n * h * w, P2 = P / 4, P4 = P / 16;
+    for (int l = 0; l < 10; l++) {
+      const long pixels = (long)(l == 4 || l == 5 ? P4 : l == 2 || l == 3 || l == 6 || l == 7 ? P2 : P);
+      fwd_tile[l] = conv3x3_default_tile(kLayers[l].cout, pixels);
+      dx_tile[l] = conv3x3_default_tile(kLayers[l].cin_pad, pixels);
+    }
     auto A = [&](size_t pix, int c) { return (bf16 *)alloc(pix * c * 2); };
     x32 = A(P, 32);
     e1a = A(P, 32);

@@ -68,3 +68,17 @@ def test_denoise_equals_register_tiles(dev, h, w):
     for k in range(2):
         net.set_tiles(picks(COUTS, k), [0] * 10)
         assert net.denoise(g, noisy).numpy().tobytes() == ref.tobytes(), k
+
+
+@pytest.mark.parametrize("n,h,w", [(1, 4, 4), (1, 400, 400), (1, 448, 896), (1, 800, 1024)])
+def test_default_tiles(dev, n, h, w):
+    """A new network's tiles, below and above the rule's pixel counts (40000
+    and 200000 at a layer's resolution), are offered ones and change no bit."""
+    x, _ = inputs(n, h, w)
+    net = dev.UNet(n, h, w, seed=3)
+    f, d = net.tiles()
+    for t, c in zip(f + d, COUTS + CINS):
+        assert 0 <= t < lgx.lib().lgx_unet_conv_tiles(c)
+    out = net.forward(x).cpu().numpy()
+    net.set_tiles([0] * 10, [0] * 10)
+    assert net.forward(x).cpu().numpy().tobytes() == out.tobytes()
