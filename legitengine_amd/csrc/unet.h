@@ -34,7 +34,7 @@ struct ConvArgs {
   // First convolution (conv_first_pair; conv3x3 refuses it): the input records
   // are packed from the noisy image and the G-buffer while the tile is
   // staged, channels (noisy rgb, depth, normal xy, albedo rgb, zeros), the
-  // values pack_input gives for those records; a and b are unused.
+  // records' values; a and b are unused.
   int gin_fmt;  // 0: off; 1: RG16F normal + RGBA8 albedo; 2: RG32F + RGBA32F; 3: records (gin_x12)
   const float4 *gin_noisy;
   const float *gin_depth;
@@ -101,7 +101,6 @@ constexpr int kWgradLaunches = 6;
 hipError_t conv3x3_wgrad(WgradTable &t, float *part, size_t part_bytes, hipStream_t s);
 hipError_t conv3x3_wgrad_sums(const WgradTable &t, hipStream_t s);
 size_t conv3x3_wgrad_scratch_bytes();
-hipError_t pack_input(const float *x12, size_t npix, bf16 *x32, hipStream_t s);
 hipError_t avgpool(const bf16 *x, int n, int h, int w, int c, bf16 *y, hipStream_t s);
 hipError_t pool_bwd_add(const bf16 *dx_in, const bf16 *dpool, const bf16 *act, int n, int h, int w, int c, bf16 *dx,
                         hipStream_t s);

@@ -345,8 +345,8 @@ template <int GIN> LGX_D GinRaw<GIN> gin_load(const ConvArgs &a, int y, int x, i
   return r;
   }
 }
-// The first 16 channels of the pixel's input record (pack_input_kernel's
-// values for the record the G-buffer and the noisy image give).
+// The first 16 channels of the pixel's input: noisy irradiance rgb, depth, oct
+// normal xy, albedo rgb and zeros (a record has 12 floats, the last 3 unused).
 template <int GIN> LGX_D void gin_pack(const GinRaw<GIN> &r, bf16x8 &v0, bf16x8 &v1) {
   if constexpr (GIN == 3) {
     v0 = bf16x8{f2bf(r.a.x), f2bf(r.a.y), f2bf(r.a.z), f2bf(r.a.w), f2bf(r.b.x), f2bf(r.b.y), f2bf(r.b.z), f2bf(r.b.w)};
@@ -997,7 +997,7 @@ __global__ __launch_bounds__(64 * NW, OCC) void conv3x3_dma_kernel(const ConvArg
 //
 // One wave is one workgroup and walks down a strip 30 output columns wide,
 // two rows an iteration: the strip's records (34 columns, packed from the
-// G-buffer or the FP32 records as pack_input_kernel packs them) and the first
+// G-buffer or the FP32 records by gin_pack) and the first
 // layer's output (32 columns, two 16-pixel blocks) live in LDS rings of four
 // rows, so each row of either is formed once, and nothing waits at a
 // barrier.  A strip is cut into segments of `len` row pairs so that there are
@@ -1074,7 +1074,7 @@ __global__ __launch_bounds__(64, 2) void conv_first_pair_kernel(const ConvArgs a
     for (int i = 0; i < 2; i++) raw[i] = gin_load<GIN>(a0, min(max(y + i, 0), h - 1), rxc, n);
   };
   // rows y, y + 1 into a half: zero outside the image (the first layer's padding); a segment's own pixels
-  // also to rec_out when asked (pack_input_kernel's layout: the training backward reads them)
+  // also to rec_out when asked (32 channels, the upper 16 zero: the training backward reads them)
   auto stage = [&](int y, int half, bool own) {
 #pragma unroll
     for (int i = 0; i < 2; i++) {
@@ -1613,21 +1613,6 @@ __global__ __launch_bounds__(256) void wgrad_reduce_kernel(const WgradTable t) {
 
 // ------------------------------------------------------------ glue kernels
 
-// Network input: [noisy irradiance rgb, depth, oct normal xy, albedo rgb, 0...]
-// from a compact FP32 record of 12 floats per pixel (the last 3 unused).
-__global__ __launch_bounds__(256) void pack_input_kernel(const float *x12, size_t npix, bf16 *x32) {
-  const size_t p = (size_t)blockIdx.x * 64 + (threadIdx.x >> 2);
-  const int q = threadIdx.x & 3;  // 8-channel quarter
-  if (p >= npix) return;
-  bf16x8 v = {};
-  if (q == 0) {
-    for (int i = 0; i < 8; i++) v[i] = f2bf(x12[p * 12 + i]);
-  } else if (q == 1) {
-    v[0] = f2bf(x12[p * 12 + 8]);
-  }
-  *(bf16x8 *)(x32 + p * 32 + q * 8) = v;
-}
-
 __global__ __launch_bounds__(256) void avgpool_kernel(const bf16 *x, int n, int h, int w, int c, bf16 *y) {
   // y[n][h/2][w/2][c] = mean of the 2x2 children
   const int hh = h >> 1, ww = w >> 1;
@@ -1700,7 +1685,7 @@ __global__ __launch_bounds__(256) void upsample_bwd_kernel(const bf16 *dfull, co
 
 // Training: the 1x1 head, the loss and the head's backward in one pass (the
 // head's output is not stored).  One pixel per thread: out = x + b_h + W_h
-// act, summed in head_fwd_kernel's order; mean L1: g = sign(out - target) /
+// act, summed channel by channel; mean L1: g = sign(out - target) /
 // count per channel, mean squared error (l2): g = 2 (out - target) / count;
 // dd1 = mask(d1 > 0) W_h^T g (per channel, the three products in channel
 // order).  A thread keeps 3 x 32 head-weight partial sums; they are reduced
@@ -2172,10 +2157,6 @@ hipError_t conv3x3_wgrad_sums(const WgradTable &t, hipStream_t s) {
   return hipGetLastError();
 }
 
-hipError_t pack_input(const float *x12, size_t npix, bf16 *x32, hipStream_t s) {
-  hipLaunchKernelGGL(pack_input_kernel, dim3((unsigned)((npix + 63) / 64)), dim3(256), 0, s, x12, npix, x32);
-  return hipGetLastError();
-}
 hipError_t avgpool(const bf16 *x, int n, int h, int w, int c, bf16 *y, hipStream_t s) {
   hipLaunchKernelGGL(avgpool_kernel, dim3(grid_for((size_t)n * (h / 2) * (w / 2) * (c / 8), 256)), dim3(256), 0, s, x,
                      n, h, w, c, y);
