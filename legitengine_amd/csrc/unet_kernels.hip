@@ -1850,8 +1850,11 @@ static unsigned grid_for(size_t work, size_t per_block) {
 // best conv3x3_lds_kernel tile / best conv3x3_dma_kernel tile): 32 -> 32 at full
 // size 84 / 57 / 55; 32 -> 64 at half size 51 / 36 / 26; 128 -> 64 99 / 57 /
 // 40; 64 -> 128 at a quarter 63 / 27 / 23; 192 -> 64 at half size 213 / 113 /
-// 91.  The smallest images go the other way (quarter size of 256 x 256:
-// 12.4 / 13.5 / 19): the direct-load tiles are the largest, and too few of them
+// 91.  The input gradient 32 -> 96 (16 x 256 x 256: 151 / 90 / 82) is fastest
+// with 16 columns a tile, whose registers let four waves share a SIMD; others
+// are not (32 -> 32 at full size 59 with it).  The smallest images go the other
+// way (quarter size of 256 x 256: 12.4 / 13.5 / 19): the direct-load tiles are
+// the largest, and too few of them
 // fill the chip.
 struct ConvTile {
   int r, pb, lds;  // lds: 1 conv3x3_lds_kernel, 2 conv3x3_dma_kernel with WR = r, WP = pb
@@ -1867,7 +1870,7 @@ static const ConvTile kTiles4[] = {{2, 2, 0, 4, 0}, {4, 2, 0, 4, 0}, {2, 4, 0, 4
                                    {1, 4, 1, 4, 0}, {1, 2, 1, 4, 0}, {2, 2, 1, 4, 2}, {1, 2, 1, 4, 3},   {2, 4, 1, 2, 0},
                                    {2, 2, 1, 2, 3}, {2, 2, 2, 4, 1, 4}, {2, 2, 2, 4, 1, 8}};
 static const ConvTile kTiles6[] = {{2, 2, 0, 6, 0}, {1, 4, 0, 6, 0}, {1, 2, 0, 6, 0},
-                                   {2, 4, 1, 2, 0}, {2, 2, 1, 2, 3}, {2, 2, 2, 2, 2, 4}};
+                                   {2, 4, 1, 2, 0}, {2, 2, 1, 2, 3}, {2, 2, 2, 2, 2, 4}, {2, 1, 2, 2, 2, 8}};
 static const ConvTile kTiles8[] = {{1, 2, 0, 8, 0}, {2, 2, 0, 8, 0}, {1, 4, 0, 8, 0},   {2, 2, 1, 4, 0},
                                    {1, 2, 1, 4, 3}, {2, 2, 1, 4, 2}, {2, 2, 2, 4, 1, 4}, {2, 2, 2, 4, 1, 8}};
 static const ConvTile kTiles12[] = {{1, 2, 0, 12, 0}, {2, 1, 0, 12, 0},   {2, 2, 1, 4, 0},
@@ -1897,7 +1900,7 @@ int conv3x3_default_tile(int cout, long pixels) {
   switch (cout) {
     case 32: return 10;
     case 64: return pixels >= 200000 ? 12 : pixels >= 40000 ? 11 : 8;
-    case 96: return pixels >= 200000 ? 5 : 4;
+    case 96: return pixels >= 200000 ? 6 : 4;
     case 128: return pixels >= 40000 ? 7 : 4;
     case 192: return pixels >= 40000 ? 5 : 4;
     default: return 0;
@@ -1970,7 +1973,7 @@ template <int MBW, int WR, int WP, int NW> static hipError_t launch_conv_dma(con
   if (lds > 160 * 1024 || (conv_pairs(MBW) && a.split % 32)) return hipErrorInvalidValue;
   const long tiles = (long)tx * ty * a.n;
   const long grid = std::min(tiles, std::max(1L, (long)per_cu * cu_count() / splits)) * splits;
-  constexpr int OCC = NW * (NW == 4 && MBW == 2 && WR * WP == 4 ? 2 : 1) / 4;
+  constexpr int OCC = NW * ((NW == 4 && MBW == 2 && WR * WP == 4) || WR * WP == 2 ? 2 : 1) / 4;
   auto launch = [&](auto kern) {
     hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(64 * NW), (size_t)lds, s, a, tx, ty, splits, wres);
     return hipGetLastError();
@@ -2006,6 +2009,9 @@ template <int MB> static hipError_t conv_mb(const ConvArgs &a, const ConvTile &t
 #define LGX_DMA(MBW, RR, PP, NW) \
   if (t.lds == 2 && t.mbw == MBW && t.r == RR && t.pb == PP && t.nw == NW) \
     return launch_conv_dma<MBW, RR, PP, NW>(a, t.per_cu, s);
+  if constexpr (MB == 6) {
+    LGX_DMA(2, 2, 1, 8)
+  }
   if constexpr (MB % 2 == 0) {
     LGX_DMA(2, 2, 2, 4) LGX_DMA(2, 2, 2, 8)
     LGX_LDS(2, 2, 4) LGX_LDS(2, 2, 2) LGX_LDS(2, 1, 4)
