@@ -34,18 +34,19 @@ constexpr int kBilatMaxR = 8, kBilatTW = 32;
 // One row of taps (n = 2r of them, geometry and colour in LDS) for the
 // outputs LO..HI of a thread's column.
 template <int R, int LO, int HI>
-LGX_D void bilat_row(const float4 *geo, const float4 *col, int n, float kd, const float4 (&gc)[R], float4 (&acc)[R]) {
+LGX_D void bilat_row(const float4 *geo, const float4 *col, int n, float kd, float kn, const float4 (&gc)[R], float4 (&acc)[R]) {
 #pragma unroll 4
   for (int x = 0; x < n; x++) {
     const float4 gs = geo[x], c = col[x];
 #pragma unroll
     for (int k = LO; k <= HI; k++) {
-      // exp(-|dd| ds) exp(-|dn|^2 ns) = exp2(-|dd| kd - |dn|^2 kn), the
-      // normal staged with sqrt(kn): one hardware exp2 (1 ulp) per tap.  kd
-      // multiplies the difference, which is exact for neighbouring depths:
-      // of depths scaled first every product would round at its own size
+      // exp(-|dd| ds) exp(-|dn|^2 ns) = exp2(-|dd| kd - |dn|^2 kn): one
+      // hardware exp2 (1 ulp) per tap.  kd and kn (of any sign) multiply the
+      // differences, which are exact for neighbours: of values scaled first
+      // every product would round at its own size
       const float dx = gs.y - gc[k].y, dy = gs.z - gc[k].z, dz = gs.w - gc[k].w;
-      const float w = __builtin_amdgcn_exp2f(fmaf(-dz, dz, fmaf(-dy, dy, fmaf(-dx, dx, -fabsf(gs.x - gc[k].x) * kd))));
+      const float dn2 = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
+      const float w = __builtin_amdgcn_exp2f(fmaf(-dn2, kn, -fabsf(gs.x - gc[k].x) * kd));
       acc[k].x = fmaf(c.x, w, acc[k].x);
       acc[k].y = fmaf(c.y, w, acc[k].y);
       acc[k].z = fmaf(c.z, w, acc[k].z);
@@ -55,20 +56,20 @@ LGX_D void bilat_row(const float4 *geo, const float4 *col, int n, float kd, cons
 }
 // the same for the uniform range lo..hi
 template <int R, int LO = 0, int HI = 0>
-LGX_D void bilat_rows(int lo, int hi, const float4 *geo, const float4 *col, int n, float kd, const float4 (&gc)[R],
+LGX_D void bilat_rows(int lo, int hi, const float4 *geo, const float4 *col, int n, float kd, float kn, const float4 (&gc)[R],
                       float4 (&acc)[R]) {
   if (lo == LO && hi == HI)
-    bilat_row<R, LO, HI>(geo, col, n, kd, gc, acc);
+    bilat_row<R, LO, HI>(geo, col, n, kd, kn, gc, acc);
   else if constexpr (HI + 1 < R)
-    bilat_rows<R, LO, HI + 1>(lo, hi, geo, col, n, kd, gc, acc);
+    bilat_rows<R, LO, HI + 1>(lo, hi, geo, col, n, kd, kn, gc, acc);
   else if constexpr (LO + 1 < R)
-    bilat_rows<R, LO + 1, LO + 1>(lo, hi, geo, col, n, kd, gc, acc);
+    bilat_rows<R, LO + 1, LO + 1>(lo, hi, geo, col, n, kd, kn, gc, acc);
 }
 
 // A workgroup filters 32 x 8R pixels, a thread R pixels of one column, whose
 // windows overlap in all but R - 1 of their rows: a tap read from LDS serves
 // up to R outputs.  Bound by VALU issue (94 % of the slots that this mix of
-// instructions has, by counters): 13 instructions a tap with one exp2 (20 and
+// instructions has, by counters): 14 instructions a tap with one exp2 (20 and
 // their scalar operands before), about 190 a pixel for staging and the
 // quotients.  More outputs a thread read less LDS and lose as much
 // to the fewer workgroups that fit it.  2560x1440, r = 4: 133 -> 94 us a call.
@@ -79,7 +80,7 @@ template <int NFMT, int R> __global__ __launch_bounds__(256) void bilateral_kern
   const int sw = TW + n - 1, sh = TH + n - 1;  // taps reach -r .. r-1
   float4 *s_geo = s_bilat, *s_col = s_bilat + sw * sh;  // (depth, normal xyz), colour
   const int x0 = blockIdx.x * TW - r, y0 = blockIdx.y * TH - r;
-  const float kd = vec(a.ds * 1.44269504f), kn = sqrtf(a.ns * 1.44269504f);
+  const float kd = vec(a.ds * 1.44269504f), kn = vec(a.ns * 1.44269504f);
   // Four texels of the tile a thread at a time, all their loads in flight
   // together: a load per row waited for its own round trip to memory, which
   // the few workgroups that fit a CU's LDS do not hide.
@@ -109,7 +110,7 @@ template <int NFMT, int R> __global__ __launch_bounds__(256) void bilateral_kern
       const int i = i0 + u * 256;
       if (i < total) {
         const Vec3<float> nv = oct_decode_dev<float>(nt[u].x, nt[u].y);
-        s_geo[i] = make_float4(d[u], nv.x * kn, nv.y * kn, nv.z * kn);
+        s_geo[i] = make_float4(d[u], nv.x, nv.y, nv.z);
         s_col[i] = make_float4(c[u].x, c[u].y, c[u].z, 1.0f);
       }
     }
@@ -125,7 +126,7 @@ template <int NFMT, int R> __global__ __launch_bounds__(256) void bilateral_kern
   // window row j holds the taps of outputs k with 0 <= j - k < 2r
   for (int j = 0; j < n + R - 1; j++) {
     const int at = (ty + j) * sw + tx;
-    bilat_rows<R>(max(j - n + 1, 0), min(j, R - 1), s_geo + at, s_col + at, n, kd, gc, acc);
+    bilat_rows<R>(max(j - n + 1, 0), min(j, R - 1), s_geo + at, s_col + at, n, kd, kn, gc, acc);
   }
   const int px = blockIdx.x * TW + tx, py = blockIdx.y * TH + ty;
   if (px >= a.w) return;

@@ -54,3 +54,11 @@ def test_background_at_the_largest_float(w, h, radius):
 def test_negative_depth_sharpness(w, h, radius):
     out, ref = run(w, h, radius, ds=-1.5)
     assert orc.rel_l2(out, ref) <= 1e-5
+
+
+@pytest.mark.parametrize("w,h,radius", SIZES)
+@pytest.mark.parametrize("ns", [-0.5, 0.0, 1e4, 1e6])
+def test_normal_sharpness(w, h, radius, ns):
+    out, ref = run(w, h, radius, ns=ns)
+    assert np.isfinite(out).all()
+    assert orc.rel_l2(out, ref) <= 1e-5
