@@ -62,3 +62,22 @@ def test_normal_sharpness(w, h, radius, ns):
     out, ref = run(w, h, radius, ns=ns)
     assert np.isfinite(out).all()
     assert orc.rel_l2(out, ref) <= 1e-5
+
+
+@pytest.mark.parametrize("w,h,radius", SIZES)
+def test_infinite_irradiance(w, h, radius):
+    """Taps of +inf and -inf: sums of one sign stay infinite, mixed ones are
+    NaN, as the oracle's."""
+    def spots(a):
+        a[5:h // 4, 3, 0] = np.inf
+        a[7, 9:w // 3, 1] = -np.inf
+        a[h // 2, w // 2, 2] = np.inf
+        a[h // 2 + 1, w // 2 + 1, 2] = -np.inf
+        return a
+    out, ref = run(w, h, radius, ns=5.0, irradiance=spots)  # (no weight so small that it may be flushed to 0)
+    assert np.isinf(ref).any() and np.isnan(ref).any()
+    assert np.array_equal(np.isnan(out), np.isnan(ref))
+    assert np.array_equal(out[np.isinf(ref)], ref[np.isinf(ref)])
+    f = np.isfinite(ref)
+    assert np.isfinite(out[f]).all()
+    assert np.linalg.norm((out[f] - ref[f]).astype(np.float64)) <= 1e-5 * np.linalg.norm(ref[f].astype(np.float64))
