@@ -16,6 +16,13 @@ template <class T> LGX_D T vec(T v) {
   return v;
 }
 
+// A value that the compiler takes for a new one (what is formed from it is not
+// merged with what was formed before).
+template <class T> LGX_D T opaque(T v) {
+  asm("" : "+v"(v));
+  return v;
+}
+
 template <class T> LGX_D T fma_(T a, T b, T c) { return fma(a, b, c); }
 
 template <class T> LGX_D T fast_rcp(T v);

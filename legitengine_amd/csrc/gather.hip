@@ -32,6 +32,7 @@
 #include <vector>
 
 #include "device_math.h"
+#include "gather_taps.h"
 #include "lgx_internal.h"
 
 namespace lgx {
@@ -216,28 +217,9 @@ template <class T, class ARGS> LGX_D Vec3<T> unproject_far(ARGS &a, T sx, T sy) 
   return Vec3<T>{div_by(vx, vw, rw), div_by(vy, vw, rw), div_by(vz, vw, rw)};
 }
 
-// Vulkan clamp-to-edge bilinear taps of a point s in one level (u = s W -
-// 1/2, taps floor(u) and the next, weights frac(u)).  At a border, where both
-// taps are the edge texel, the pair is moved inside and the weight saturates,
-// so the two texels of a row are always neighbours and come in one fetch.  A
-// level of one column or row (uniform) has its texel on both sides.
-template <class T> struct TapPos {
-  T al, be;
-  int x, y;
-  LGX_D TapPos(T sx, T sy, int lw, int lh) {
-    const T u = sx * T(lw) - T(0.5), v = sy * T(lh) - T(0.5);
-    const T fu = max(min(floor(u), T(lw - 2)), T(0)), fv = max(min(floor(v), T(lh - 2)), T(0));
-    al = min(max(u - fu, T(0)), T(1));
-    be = min(max(v - fv, T(0)), T(1));
-    x = (int)fu;
-    y = (int)fv;
-  }
-  LGX_D T mix(T p00, T p10, T p01, T p11) const {
-    const T top = fma_(al, p10 - p00, p00), bot = fma_(al, p11 - p01, p01);
-    return fma_(be, bot - top, top);
-  }
-};
-template <class T> LGX_D T depth_taps(const float *base, int pitch, int lw, int lh, const TapPos<T> &p) {
+// The texels of a tap position: one fetch per row where the level has a pair
+// of columns (uniform).
+template <class T> LGX_D Quad<T> depth_quad(const float *base, int pitch, int lw, int lh, const TapPos<T> &p) {
   const i32x4 r = level_rsrc(base, 4, lh * pitch);
   const uint32_t a = texel_index(p.y, pitch, p.x), b = a + (lh > 1 ? (uint32_t)pitch : 0u);
   f32x2 t, q;
@@ -248,10 +230,10 @@ template <class T> LGX_D T depth_taps(const float *base, int pitch, int lw, int 
     t = load_depth(r, a);
     q = load_depth(r, b);
   }
-  return p.mix(T(t.x), T(t.y), T(q.x), T(q.y));
+  return Quad<T>{T(t.x), T(t.y), T(q.x), T(q.y)};
 }
 template <class T, int FMT>
-LGX_D Vec3<T> radiance_taps(const void *base, int pitch, int lw, int lh, const TapPos<T> &p) {
+LGX_D Vec3<Quad<T>> radiance_quad(const void *base, int pitch, int lw, int lh, const TapPos<T> &p) {
   typedef RadBuf<FMT> B;
   const i32x4 r = level_rsrc(base, B::kBytes, lh * pitch);
   const uint32_t at = texel_index(p.y, pitch, p.x), down = lh > 1 ? (uint32_t)pitch : 0u;
@@ -271,8 +253,9 @@ LGX_D Vec3<T> radiance_taps(const void *base, int pitch, int lw, int lh, const T
     t[2 * row] = B::decode(lo);
     t[2 * row + 1] = B::decode(hi);
   }
-  return Vec3<T>{p.mix(T(t[0].x), T(t[1].x), T(t[2].x), T(t[3].x)), p.mix(T(t[0].y), T(t[1].y), T(t[2].y), T(t[3].y)),
-                 p.mix(T(t[0].z), T(t[1].z), T(t[2].z), T(t[3].z))};
+  return Vec3<Quad<T>>{{T(t[0].x), T(t[1].x), T(t[2].x), T(t[3].x)},
+                       {T(t[0].y), T(t[1].y), T(t[2].y), T(t[3].y)},
+                       {T(t[0].z), T(t[1].z), T(t[2].z), T(t[3].z)}};
 }
 // The trilinear march is bound by VALU issue as well: about 105 instructions a
 // step (130 with 64-bit addresses, IEEE divisions, four clamped single-texel
@@ -589,8 +572,30 @@ LGX_D void gather_block(ARGS &a, const uint32_t b, A *part) {
         const Trilinear<T> tl(a, lod);
         const int l0 = tl.l0, l1 = tl.l1;
         const TapPos<T> p0(sqx, sqy, a.lw[l0], a.lh[l0]), p1(sqx, sqy, a.lw[l1], a.lh[l1]);
-        T r = depth_taps(a.pd[l0], a.pd_pitch[l0], a.lw[l0], a.lh[l0], p0);
-        if (tl.blend) r = fma_(tl.f, depth_taps(a.pd[l1], a.pd_pitch[l1], a.lw[l1], a.lh[l1], p1) - r, r);
+        auto depth_at = [&](int l, const TapPos<T> &p) { return depth_quad(a.pd[l], a.pd_pitch[l], a.lw[l], a.lh[l], p); };
+        auto radiance_at = [&](int l, const TapPos<T> &p) {
+          return radiance_quad<T, RFMT>(a.pr[l], a.pr_pitch[l], a.lw[l], a.lh[l], p);
+        };
+        // A sample that is not finite has an infinite texel among its taps: fetched again, for nothing is kept for
+        // it (24 more spilled registers otherwise), and blended tap by tap.
+        auto depth_again = [&](int l) {
+          const T ux = opaque(sqx), uy = opaque(sqy);
+          const int lw = a.lw[l], lh = a.lh[l];
+          return clamped_taps(ux, uy, lw, lh, depth_at(l, TapPos<T>(ux, uy, lw, lh)));
+        };
+        auto radiance_again = [&](int l) {
+          const T ux = opaque(sqx), uy = opaque(sqy);
+          const int lw = a.lw[l], lh = a.lh[l];
+          const Vec3<Quad<T>> q = radiance_at(l, TapPos<T>(ux, uy, lw, lh));
+          return Vec3<T>{clamped_taps(ux, uy, lw, lh, q.x), clamped_taps(ux, uy, lw, lh, q.y),
+                         clamped_taps(ux, uy, lw, lh, q.z)};
+        };
+        T r = p0.mix(depth_at(l0, p0));
+        if (tl.blend) r = TapPos<T>::lerp(tl.f, r, p1.mix(depth_at(l1, p1)));
+        if (!finite_tap(r)) {
+          r = depth_again(l0);
+          if (tl.blend) r = r * (T(1) - tl.f) + depth_again(l1) * tl.f;
+        }
         // :241-252 sample delta projected on (eye, tangent)
         const T len2 = fma_(off, fma_(off, vv, uv2), uu);
         const T ri = r * fast_rsqrt(len2);
@@ -598,10 +603,16 @@ LGX_D void gather_block(ARGS &a, const uint32_t b, A *part) {
         const T hxv = fma_(ri, fma_(off, ev, eu), -erc);
         if (hm.below(hyv, hxv))  // :254
           raise(hyv, hxv, sqx, sqy, [&]() {  // :256
-            Vec3<T> v = radiance_taps<T, RFMT>(a.pr[l0], a.pr_pitch[l0], a.lw[l0], a.lh[l0], p0);
+            const Vec3<Quad<T>> q0 = radiance_at(l0, p0);
+            Vec3<T> v{p0.mix(q0.x), p0.mix(q0.y), p0.mix(q0.z)};
             if (tl.blend) {
-              const Vec3<T> w = radiance_taps<T, RFMT>(a.pr[l1], a.pr_pitch[l1], a.lw[l1], a.lh[l1], p1);
-              v = Vec3<T>{fma_(tl.f, w.x - v.x, v.x), fma_(tl.f, w.y - v.y, v.y), fma_(tl.f, w.z - v.z, v.z)};
+              const Vec3<Quad<T>> q1 = radiance_at(l1, p1);
+              v = Vec3<T>{TapPos<T>::lerp(tl.f, v.x, p1.mix(q1.x)), TapPos<T>::lerp(tl.f, v.y, p1.mix(q1.y)),
+                          TapPos<T>::lerp(tl.f, v.z, p1.mix(q1.z))};
+            }
+            if (!finite_tap(v.x + v.y + v.z)) {
+              v = radiance_again(l0);
+              if (tl.blend) v = v * (T(1) - tl.f) + radiance_again(l1) * tl.f;
             }
             return v;
           });

@@ -1,0 +1,21 @@
+"""The gather's host-and-device arithmetic, called on the CPU in the kernels'
+precision (the programs in tests/csrc say what they compare and why their
+bounds are what they are)."""
+import os
+import subprocess
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+def program(tmp_path, name):
+    exe = str(tmp_path / name)
+    subprocess.run(["g++", "-O2", "-std=c++17", "-ffp-contract=off", "-I", os.path.join(ROOT, "legitengine_amd", "csrc"),
+                    "-o", exe, os.path.join(ROOT, "tests", "csrc", name + ".cpp")], check=True)
+    return exe
+
+
+def test_trilinear_taps(tmp_path):
+    r = subprocess.run([program(tmp_path, "check_taps")], capture_output=True, text=True, timeout=300)
+    assert r.stdout.startswith("ok "), r.stdout
+    samples, at_infinite, missed = (int(v) for v in r.stdout.split()[1:])
+    assert samples == 4000000 and at_infinite > 10000 and missed > 100000
