@@ -90,7 +90,26 @@ def build_integration_example(verbose=False):
     return EXAMPLE_BIN
 
 
+DEVICE_MATH_SRC = os.path.join(ROOT, "tests", "csrc", "check_device_math.hip")
+DEVICE_MATH_BIN = os.path.join(ROOT, "tests", "csrc", "check_device_math")
+
+
+def build_device_math_check(verbose=False):
+    """Compiles the check of the device kernels' short arithmetic, with the
+    library's own flags; the GPU tests run it."""
+    tmp = DEVICE_MATH_BIN + ".tmp"
+    cmd = [HIPCC, f"--offload-arch={ARCH}", *HIP_FLAGS, DEVICE_MATH_SRC, "-o", tmp]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"compile failed: {' '.join(cmd)}\n{r.stdout}\n{r.stderr}")
+    os.replace(tmp, DEVICE_MATH_BIN)
+    if verbose:
+        print(f"built {DEVICE_MATH_BIN}")
+    return DEVICE_MATH_BIN
+
+
 if __name__ == "__main__":
     build(verbose=True)
     build_integration_example(verbose=True)
+    build_device_math_check(verbose=True)
     sys.exit(0)

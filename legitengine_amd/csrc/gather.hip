@@ -99,35 +99,6 @@ template <class T> LGX_D T div_extent(T q, T b, T rb) {
   return fma(e, rb, y);
 }
 
-// atan2(y, x) for finite arguments (atan2(0, 0) = 0), float: octant
-// reduction to t = min(|x|, |y|) / max(|x|, |y|) in [0, 1] and
-// atan(t) = t P(t^2) with a degree-7 polynomial fitted to atan(t) / t on
-// [0, 1] by iteratively reweighted least squares (max error 4e-8; 1.2e-7
-// evaluated in float).  The hit branch of the march calls it on every horizon
-// rise, where the library routine's handling of infinities and NaNs (which
-// cannot occur there) costs more than the polynomial.
-// NONZERO: the caller's vector is not (0, 0).
-template <bool NONZERO> LGX_D double atan2_finite(double y, double x) { return atan2(y, x); }
-template <bool NONZERO> LGX_D float atan2_finite(float y, float x) {
-  const float ax = fabsf(x), ay = fabsf(y);
-  const bool steep = ay > ax;
-  const float mx = steep ? ay : ax, mn = steep ? ax : ay;
-  const float t = NONZERO || mx > 0.f ? mn * __builtin_amdgcn_rcpf(mx) : 0.f;
-  const float s = t * t;
-  float p = -0.004054928198456764f;
-  p = fmaf(p, s, 0.021864214912056923f);
-  p = fmaf(p, s, -0.05591406673192978f);
-  p = fmaf(p, s, 0.0964231863617897f);
-  p = fmaf(p, s, -0.1390867531299591f);
-  p = fmaf(p, s, 0.19946573674678802f);
-  p = fmaf(p, s, -0.33329862356185913f);
-  p = fmaf(p, s, 0.9999993443489075f);
-  float r = t * p;
-  r = steep ? 1.5707963705062866f - r : r;
-  r = x < 0.f ? 3.1415927410125732f - r : r;
-  return copysignf(r, y);
-}
-
 // A pyramid level as a structured buffer: the texel index is the buffer
 // index (the hardware scales it by the stride, one instruction less per fetch
 // than a byte offset), the base, pitch and extent are scalars, and an index
@@ -384,11 +355,9 @@ LGX_D void gather_block(ARGS &a, const uint32_t b, A *part) {
     // :254-263 a sample above the horizon: radiance v (raw), weights, new maximum
     auto raise = [&](T hyv, T hxv, T sqx, T sqy, auto v_of) {
       if (COUNT) hit_total++;
-      // (FP64 sums of the trilinear mode keep the library's arc tangent and quotients)
-      constexpr bool kLib = sizeof(A) == 8 && SAMPLER == LGX_SAMPLER_TRILINEAR;
-      const T th = kLib ? atan2(hyv, hxv) : atan2_finite<true>(hyv, hxv);
-      const T iq = kLib ? T(1) / (hxv * hxv + hyv * hyv) : fast_rcp(hxv * hxv + hyv * hyv);
-      const T c2 = (hxv * hxv - hyv * hyv) * iq, s2 = (T(2) * hxv * hyv) * iq;
+      // (the trilinear mode: the library's arc tangent and IEEE quotients, 1080p with 4 directions 397 -> 415 us a frame)
+      T th, c2, s2;
+      slice_angle<SAMPLER == LGX_SAMPLER_TRILINEAR>(hyv, hxv, th, c2, s2);
       // :222-227 the four ramps; of two opposite ones at most one is below 1
       const T width = T(0.1f), inv_width = T(1) / width;
       const T side = min(max(min(sqx, T(1) - sqx) * inv_width, T(0)), T(1)) *
