@@ -42,23 +42,24 @@ template <class T> LGX_D T div_by(T x, T b, T r) {
   return fma(e, r, y);
 }
 
-// RN(1 / b): the hardware's reciprocal (1 ulp) and one Newton step.  Equal to
-// the IEEE division for every float of magnitude 2^-100 .. 2^125 (all of
-// them compared on the device), in 3 instructions instead of the division's
-// 10.
+// RN(1 / b) for 2^-126 <= |b| < 2^126: the hardware's reciprocal (1 ulp) and
+// one Newton step, 3 instructions instead of the division's 10
+// (tests/csrc/check_device_math.hip compares all significands on the device,
+// here and below).
 template <class T> LGX_D T recip(T b) {
   if (sizeof(T) == 8) return T(1) / b;
   const T r = fast_rcp(b);
   return fma(fma(-b, r, T(1)), r, r);
 }
 
-// len = RN(sqrt(q)), from the hardware's reciprocal square root y and one
-// residual correction of q y: the IEEE root for every float in 2^-100 ..
-// 2^125 (all compared on the device).  r: 1 / len by a Newton step from y,
-// the IEEE quotient but for one ulp at 24 of the 4.2e8 floats of each 25
-// binades, which div_by's residual absorbs.  7 instructions for the two
+// len = RN(sqrt(q)) for finite q >= 2^-100, from the hardware's reciprocal
+// square root y and one residual correction of q y.  r: 1 / len by a Newton
+// step from y, the IEEE quotient but for the lengths (2 - 2^-23) 2^k, where
+// it is an ulp below; a quotient by one of those is an ulp off for x a power
+// of two and the IEEE one for every other x.  7 instructions for the two
 // instead of 27; the three normalisations of a direction's set-up were a
-// quarter of it.
+// quarter of it.  (A branch to IEEE operations for other q costs the gather's
+// set-up registers; its callers see to the range.)
 template <class T> LGX_D void root(T q, T &len, T &r) {
   if (sizeof(T) == 8) {
     len = sqrt(q);

@@ -109,7 +109,9 @@ template <int NFMT, int R> __global__ __launch_bounds__(256) void bilateral_kern
     for (int u = 0; u < 4; u++) {
       const int i = i0 + u * 256;
       if (i < total) {
-        const Vec3<float> nv = oct_decode_dev<float>(nt[u].x, nt[u].y);
+        Vec3<float> nv = oct_decode_dev<float>(nt[u].x, nt[u].y);
+        // (a length whose square overflows: uniform, no wave of unit normals goes there)
+        if (__builtin_amdgcn_ballot_w64(fabsf(nt[u].x) + fabsf(nt[u].y) > 1e18f)) nv = oct_decode<float>(nt[u].x, nt[u].y);
         s_geo[i] = make_float4(d[u], nv.x, nv.y, nv.z);
         s_col[i] = make_float4(c[u].x, c[u].y, c[u].z, 1.0f);
       }

@@ -49,7 +49,8 @@ template <class T> constexpr int max_threads() { return 64 * (sizeof(T) == 8 ? k
 
 template <class T> struct GatherArgs {
   T inv_vp[16];
-  T cam[3];
+  T cam[3];  // in units of 1 / unit, as inv_vp's points are
+  T unit;
   T e0[3], ex[3], ey[3];  // unnormalised ray through screen point s: e0 + s.x*ex + s.y*ey
   T W, H, near_step, log_ratio, ambient;
   T near_min;  // near_step / the offsets' growth
@@ -297,7 +298,15 @@ LGX_D void gather_block(ARGS &a, const uint32_t b, A *part) {
   const float4 nt = Texel<NFMT>::load(a.normal, (size_t)y * a.normal_pitch + x);
   const Vec3<T> n = oct_decode_dev<T>(T(nt.x), T(nt.y));  // :133
   const Vec3<T> rayc = normalize3_cr(unproject_far(a, scx, scy) - cam);
-  const Vec3<T> P = cam + rayc * rc;  // :130 from the radial distance
+  // The radial distance in the units of cam.  Only the direction of what it
+  // scales is used, so one whose square is below the roots' range is made
+  // longer.  (Formed again per direction: kept, it costs the pipelined loop
+  // a wave per SIMD.)
+  auto radial = [&]() {
+    const T v = opaque(rc) * a.unit;
+    return v < T(0x1p-49) ? v * T(0x1p100) : v;
+  };
+  const Vec3<T> P = cam + rayc * radial();  // :130 from the radial distance
   const Vec3<T> eye = normalize3_cr(cam - P);  // :182
   const Vec3<T> pdir{-eye.x, -eye.y, -eye.z};   // normalize(P - cam): every operation is odd
   const T ambient = a.ambient;
@@ -322,7 +331,7 @@ LGX_D void gather_block(ARGS &a, const uint32_t b, A *part) {
     // :180-183 tangent of the slice through the offset point (the quotient
     // by the extent is the IEEE one, as for the step positions)
     const T ox = div_extent(cx + dx * T(10e-1), a.W, a.rW), oy = div_extent(cy + dy * T(10e-1), a.H, a.rH);
-    const Vec3<T> offp = cam + normalize3_cr(unproject_far(a, ox, oy) - cam) * rc;
+    const Vec3<T> offp = cam + normalize3_cr(unproject_far(a, ox, oy) - cam) * radial();
     const Vec3<T> tangent = normalize3_cr(normalize3_cr(offp - cam) - pdir);
     // :193-198 normal-limited initial horizon
     const Vec3<T> c1 = cross3(tangent, eye);
@@ -939,8 +948,6 @@ template <class T> static void frame_constants(const lgx_gather_params *p, Gathe
     for (int i = 0; i < 16; i++) invvp[i] = inv.m[i];
     for (int i = 0; i < 3; i++) cam[i] = iv.m[12 + i];
   }
-  for (int i = 0; i < 16; i++) a.inv_vp[i] = T(invvp[i]);
-  for (int i = 0; i < 3; i++) a.cam[i] = T(cam[i]);
   // v(s) = invVP * (2s-1, 1, 1) = c0*(2sx-1) + c1*(2sy-1) + c2 + c3;
   // ray(s) ~ sign(v.w) * (v.xyz - cam * v.w), affine in s.
   double base[4], c0[4], c1[4];
@@ -956,6 +963,23 @@ template <class T> static void frame_constants(const lgx_gather_params *p, Gathe
     a.ex[i] = T(sg * (c0[i] - cam[i] * c0[3]));
     a.ey[i] = T(sg * (c1[i] - cam[i] * c1[3]));
   }
+  // The kernel's reciprocals and roots cover 2^-126 .. 2^126 and squares from
+  // 2^-100 on.  The homogeneous scale of the matrix and the unit of length do
+  // not matter to it (only directions are formed): where the far plane's w or
+  // its distance is outside 2^-40 .. 2^60, a power of two brings it near 1.
+  auto near_one = [](double v) {
+    return v == 0 || !std::isfinite(v) || (std::fabs(v) >= 0x1p-40 && std::fabs(v) <= 0x1p60) ? 1.0
+                                                                                               : std::ldexp(1.0, -std::ilogb(v));
+  };
+  double far = 0;
+  for (int i = 0; i < 3; i++) {
+    const double d = (base[i] + 0.5 * c0[i] + 0.5 * c1[i]) / wc - cam[i];
+    far += d * d;
+  }
+  const double ws = near_one(wc), unit = near_one(std::sqrt(far));
+  for (int i = 0; i < 16; i++) a.inv_vp[i] = T(invvp[i] * ws * (i % 4 < 3 ? unit : 1.0));
+  for (int i = 0; i < 3; i++) a.cam[i] = T(cam[i] * unit);
+  a.unit = T(unit);
 }
 
 template <class T, class A, int SAMPLER, int RFMT, int NFMT>

@@ -81,3 +81,20 @@ def test_infinite_irradiance(w, h, radius):
     f = np.isfinite(ref)
     assert np.isfinite(out[f]).all()
     assert np.linalg.norm((out[f] - ref[f]).astype(np.float64)) <= 1e-5 * np.linalg.norm(ref[f].astype(np.float64))
+
+
+@pytest.mark.parametrize("w,h,radius", SIZES)
+def test_normals_of_any_length(w, h, radius):
+    """Encoded normals far outside the square: a length whose square overflows
+    divides to zero, as in the oracle."""
+    from legitengine_amd import device as dev
+    dev.require_device()
+    gb = lgx.render_gbuffer_cpu(lgx.make_scene(9, 8, 2), w, h, "f32")
+    gb["normal"][3:h // 3, ::5] *= np.float32(1e21)
+    gb["normal"][h // 2:, ::7] *= np.float32(1e6)
+    inp = np.random.default_rng(w).random((h, w, 4), dtype=np.float32)
+    out = dev.bilateral(dev.DImage.from_numpy(inp, lgx.RGBA32F), dev.GBufferDev.from_host(gb), radius=radius)
+    torch.cuda.synchronize()
+    ref = orc.bilateral(inp, gb["depth"], orc.widen(gb["normal"]), radius)
+    assert np.isfinite(ref).all()
+    assert orc.rel_l2(out.numpy(), ref) <= 1e-5
