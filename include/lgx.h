@@ -109,7 +109,9 @@ typedef struct {
   int32_t sampler;   /* LGX_SAMPLER_* */
   int32_t precision; /* LGX_PREC_*: F64 computes and accumulates in double (output RGBA64F) */
   int32_t out_layout;/* LGX_OUT_*: SLICES writes the output deinterleaved (grid x grid slices) */
-  int32_t *step_counts; /* optional device int32[W*H]: on-screen steps per pixel (sum over dirs), NULL = off */
+  int32_t *step_counts; /* optional device int32[W*H]: steps taken per pixel (sum over dirs), NULL = off; in the
+                           outermost 2^-19 of the extent, where the side fade (:220-228) is below 2e-5, the
+                           shader's on-screen steps, which the march may end just before */
   int32_t tile;      /* launch shape: an index below lgx_gather_tiles() (0 = default) */
   int32_t roi[4];    /* x0, y0, w, h: gather only these pixels (w = 0: the whole frame); output stays full-frame */
   int32_t footprint_dirs; /* direction count in the step growth and lod (indirectLighting.frag:212,217,234);

@@ -32,6 +32,7 @@
 #include <vector>
 
 #include "device_math.h"
+#include "gather_march.h"
 #include "gather_taps.h"
 #include "lgx_internal.h"
 
@@ -344,17 +345,10 @@ LGX_D void gather_block(ARGS &a, const uint32_t b, A *part) {
     T c2max = (hx * hx - hy * hy) * iq2, s2max = (T(2) * hx * hy) * iq2;
     const T tn = dot3(tangent, n);
     // :202-204 path to the screen border
-    T path;
-    {
-      const T ix = idx, iy = idy;
-      T t1 = (T(0) - cx) * ix, t2 = (a.W - cx) * ix, t3 = (T(0) - cy) * iy, t4 = (a.H - cy) * iy;
-      path = fabs(min(max(t1, t2), max(t3, t4)));
-    }
+    const T path = border_path(cx, cy, a.W, a.H, idx, idy);
     // :209 ambient term: h(0, max_h)
     T h0 = T(0.25) * en * (T(1) - c2max) + T(0.25) * tn * (T(2) * max_h - s2max);
     A L0 = A(ambient * h0), L1 = L0, L2 = L0;
-    // :212 step count, capped by the table (S)
-    auto shader_steps = [&]() { return min((int)(log(path / a.near_step) / a.log_ratio) + 1, a.S_tab); };
     // per-direction constants of the fast delta evaluation
     const Vec3<T> V = EX * div_extent(dx, a.W, a.rW) + EY * div_extent(dy, a.H, a.rH);
     const T uu = dot3(U, U), uv2 = T(2) * dot3(U, V), vv = dot3(V, V);
@@ -386,38 +380,13 @@ LGX_D void gather_block(ARGS &a, const uint32_t b, A *part) {
     };
     // the offset of step s (a scalar load); past the table no lane goes on
     auto offset = [&](int s) { return s < a.S_tab ? steps[2 * s] : T(INFINITY); };
-    // The march ends on an offset, not on a step count and four screen
-    // tests: the ray leaves the screen at offset `path`, and the shader's
-    // step count int(log(path / near) / log(ratio)) + 1 (:212) admits step
-    // j while near ratio^j <= path, i.e. while the offset near
-    // ratio^(j + lin) + 1 - near (:217) is at most path ratio^lin + 1 -
-    // near; below near, where the logarithm is negative, the truncation
-    // admits step 0 alone while path > near / ratio.  A step within rounding of the border may fall on either side:
-    // its side fade is 0 there.
-    // With FP32 sums the far borders are taken 2^-20 of the extent early
-    // (0.002 pixels at 1920, where the fade is below 1e-5): whatever the
-    // roundings of the limit and of a step's position, the position stays
-    // below the extent, and so does its texel, which then needs no clamp.
-    // FP64 sums resolve such a step: they keep the border and the clamp (as
-    // do the trilinear taps).
+    // The steps below an offset limit (march_limit).  FP64 sums resolve a step
+    // at the far border: they keep the border and the texel's clamp, as do the
+    // trilinear taps.
     constexpr bool kClamp = sizeof(A) == 8 || SAMPLER != LGX_SAMPLER_HIZ_POINT;
-    const T rlin = (steps[0] - T(1) + a.near_step) / a.near_step;
-    T lim = path >= a.near_step ? fma_(path, rlin, T(1) - a.near_step) : path > a.near_min ? offset(1) : T(0);
-    lim = min(lim, path);
-    if (!kClamp) {
-      const T far = T(1 - 0x1p-20);
-      if (dx > T(0)) lim = min(lim, (a.W * far - cx) * idx);
-      if (dy > T(0)) lim = min(lim, (a.H * far - cy) * idy);
-    }
-    if (COUNT) {  // the shader's own rule, step by step
-      const int iters = shader_steps();
-      for (int j = 0; j < iters; j++) {
-        const T o = steps[2 * j];
-        const T qx = cx + dx * o, qy = cy + dy * o;
-        if (!((qx > T(0)) & (qx < a.W) & (qy > T(0)) & (qy < a.H))) break;
-        step_total++;
-      }
-    }
+    T lim = march_limit(path, a.near_step, a.near_min, steps[0], offset(1));
+    if (!kClamp) lim = inside_far(lim, cx, cy, a.W, a.H, dx, dy, idx, idy);
+    int marched = 0;  // COUNT: steps taken
     if (SAMPLER == LGX_SAMPLER_HIZ_POINT) {
       // Level-major march.  The step index j is the same on every active
       // lane (all start at 0 and advance together; lanes only leave), so
@@ -530,6 +499,7 @@ LGX_D void gather_block(ARGS &a, const uint32_t b, A *part) {
           const T off_next = offset(j + 1);
           to_level(j);
           const Fetch f = request(off);
+          if (COUNT) marched++;
           // :241-252 sample delta projected on (eye, tangent)
           const T len2 = fma_(off, fma_(off, vv, uv2), uu);
           const T ri = T(f.rd) * fast_rsqrt(len2);
@@ -546,6 +516,7 @@ LGX_D void gather_block(ARGS &a, const uint32_t b, A *part) {
       for (int j = 0; j < a.S_tab; j++) {
         const T off = vec(steps[2 * j]), lod = steps[2 * j + 1];
         if (!(off < lim)) break;
+        if (COUNT) marched++;
         const T sqx = div_extent(cx + vdx * off, vW, vrW), sqy = div_extent(cy + vdy * off, vH, vrH);  // :218-219
         const Trilinear<T> tl(a, lod);
         const int l0 = tl.l0, l1 = tl.l1;
@@ -595,6 +566,25 @@ LGX_D void gather_block(ARGS &a, const uint32_t b, A *part) {
             return v;
           });
       }
+    }
+    if (COUNT) {
+      // The steps taken, but those in the border's fringe (2^-19 of the extent, a fade below 2e-5) or within
+      // rounding of the step count's end as the shader's own rule has them: it may admit them and the limit
+      // not, or the other way round.
+      const int iters = min((int)(log(path / a.near_step) / a.log_ratio) + 1, a.S_tab);
+      int rule = 0;
+      for (; rule < iters; rule++) {
+        const T qx = cx + dx * steps[2 * rule], qy = cy + dy * steps[2 * rule];
+        if (!((qx > T(0)) & (qx < a.W) & (qy > T(0)) & (qy < a.H))) break;
+      }
+      auto fringe = [&](int j) {
+        const T o = steps[2 * j], px = (cx + dx * o) / a.W, py = (cy + dy * o) / a.H;
+        return min(min(px, T(1) - px), min(py, T(1) - py)) <= T(0x1p-19) ||
+               fabs(o - growth_limit(path, a.near_step, steps[0])) <= o * T(0x1p-19);
+      };
+      while (marched < rule && fringe(marched)) marched++;
+      while (marched > rule && fringe(marched - 1)) marched--;
+      step_total += marched;
     }
     // :268; for a power-of-two D the quotient is the product with 1 / D
     // (exact), otherwise the IEEE division

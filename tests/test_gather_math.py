@@ -19,3 +19,13 @@ def test_trilinear_taps(tmp_path):
     assert r.stdout.startswith("ok "), r.stdout
     samples, at_infinite, missed = (int(v) for v in r.stdout.split()[1:])
     assert samples == 4000000 and at_infinite > 10000 and missed > 100000
+
+
+def test_march_limit(tmp_path):
+    exe = program(tmp_path, "check_gather_limit")
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=300)
+    assert r.stdout.startswith("ok "), r.stdout
+    assert int(r.stdout.split()[1]) > 10 ** 6
+    for mistake in (1, 2, 3, 4):
+        r = subprocess.run([exe, str(mistake)], capture_output=True, text=True, timeout=300)
+        assert r.returncode == 1 and "footprint" in r.stdout, (mistake, r.stdout)
