@@ -981,7 +981,6 @@ static hipError_t launch_gather(const GatherArgs<T> &a, bool count, hipStream_t 
   // directions: 270 us; 284 at 5, 287 at 8 with spills).
   constexpr bool kAll = sizeof(T) == 4 && sizeof(A) == 4 && SAMPLER == LGX_SAMPLER_HIZ_POINT;
   constexpr bool kAcc = sizeof(T) == 4 && sizeof(A) == 8 && SAMPLER == LGX_SAMPLER_HIZ_POINT;
-  constexpr int O8 = kAll ? 8 : 1, O1 = kAcc ? 8 : sizeof(T) == 4 && SAMPLER == LGX_SAMPLER_TRILINEAR ? 6 : 1;
   auto launch = [&](auto kern) {
     const unsigned threads = a.split ? 64u * (unsigned)a.split : 256u;
     const size_t lds = a.split ? (size_t)a.round * kShare * sizeof(A) : 0;
@@ -989,16 +988,21 @@ static hipError_t launch_gather(const GatherArgs<T> &a, bool count, hipStream_t 
     return hipGetLastError();
   };
   if (count) return launch(gather_kernel<T, A, SAMPLER, RFMT, NFMT, true, 1>);
-  if (kAll && a.swz) {  // (make_args sets swz only for this gather)
-    if (a.occ == 8 && a.pipe) return launch(gather_kernel<T, A, SAMPLER, RFMT, NFMT, false, O8, kAll, kAll>);
-    if (a.occ == 8) return launch(gather_kernel<T, A, SAMPLER, RFMT, NFMT, false, O8, false, kAll>);
-    if (a.pipe) return launch(gather_kernel<T, A, SAMPLER, RFMT, NFMT, false, 1, kAll, kAll>);
-    return launch(gather_kernel<T, A, SAMPLER, RFMT, NFMT, false, 1, false, kAll>);
+  if constexpr (kAll) {
+    if (a.swz) {
+      if (a.occ == 8 && a.pipe) return launch(gather_kernel<T, A, SAMPLER, RFMT, NFMT, false, 8, true, true>);
+      if (a.occ == 8) return launch(gather_kernel<T, A, SAMPLER, RFMT, NFMT, false, 8, false, true>);
+      if (a.pipe) return launch(gather_kernel<T, A, SAMPLER, RFMT, NFMT, false, 1, true, true>);
+      return launch(gather_kernel<T, A, SAMPLER, RFMT, NFMT, false, 1, false, true>);
+    }
+    if (a.occ == 8 && a.pipe) return launch(gather_kernel<T, A, SAMPLER, RFMT, NFMT, false, 8, true>);
+    if (a.occ == 8) return launch(gather_kernel<T, A, SAMPLER, RFMT, NFMT, false, 8>);
+    if (a.pipe) return launch(gather_kernel<T, A, SAMPLER, RFMT, NFMT, false, 1, true>);
+    return launch(gather_kernel<T, A, SAMPLER, RFMT, NFMT, false, 1>);
+  } else {
+    constexpr int OCC = kAcc ? 8 : sizeof(T) == 4 && SAMPLER == LGX_SAMPLER_TRILINEAR ? 6 : 1;
+    return launch(gather_kernel<T, A, SAMPLER, RFMT, NFMT, false, OCC, kAcc>);
   }
-  if (kAll && a.occ == 8 && a.pipe) return launch(gather_kernel<T, A, SAMPLER, RFMT, NFMT, false, O8, kAll>);
-  if (kAll && a.occ == 8) return launch(gather_kernel<T, A, SAMPLER, RFMT, NFMT, false, O8>);
-  if (kAll && a.pipe) return launch(gather_kernel<T, A, SAMPLER, RFMT, NFMT, false, 1, kAll>);
-  return launch(gather_kernel<T, A, SAMPLER, RFMT, NFMT, false, O1, kAcc>);
 }
 
 template <class T, class A, int SAMPLER>
