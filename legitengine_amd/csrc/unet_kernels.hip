@@ -1862,18 +1862,18 @@ struct ConvTile {
   int per_cu;      // lds: workgroups per CU walking the tiles, 0 = one workgroup per tile
   int nw;          // dma: waves per workgroup
 };
-static const ConvTile kTiles1[] = {{4, 2, 0, 1, 0}, {2, 4, 0, 1, 0}, {4, 4, 0, 1, 0}, {1, 4, 0, 1, 0}};
-static const ConvTile kTiles2[] = {{4, 2, 0, 2, 0}, {2, 4, 0, 2, 0}, {4, 4, 0, 2, 0},   {1, 4, 0, 2, 0},
+static constexpr ConvTile kTiles1[] = {{4, 2, 0, 1, 0}, {2, 4, 0, 1, 0}, {4, 4, 0, 1, 0}, {1, 4, 0, 1, 0}};
+static constexpr ConvTile kTiles2[] = {{4, 2, 0, 2, 0}, {2, 4, 0, 2, 0}, {4, 4, 0, 2, 0},   {1, 4, 0, 2, 0},
                                    {2, 4, 1, 2, 0}, {2, 2, 1, 2, 0}, {1, 4, 1, 2, 0},   {2, 4, 1, 2, 2},
                                    {2, 2, 1, 2, 3}, {1, 4, 1, 2, 3}, {2, 2, 2, 2, 2, 4}, {2, 2, 2, 2, 1, 8}};
-static const ConvTile kTiles4[] = {{2, 2, 0, 4, 0}, {4, 2, 0, 4, 0}, {2, 4, 0, 4, 0}, {1, 4, 0, 4, 0},   {2, 2, 1, 4, 0},
+static constexpr ConvTile kTiles4[] = {{2, 2, 0, 4, 0}, {4, 2, 0, 4, 0}, {2, 4, 0, 4, 0}, {1, 4, 0, 4, 0},   {2, 2, 1, 4, 0},
                                    {1, 4, 1, 4, 0}, {1, 2, 1, 4, 0}, {2, 2, 1, 4, 2}, {1, 2, 1, 4, 3},   {2, 4, 1, 2, 0},
                                    {2, 2, 1, 2, 3}, {2, 2, 2, 4, 1, 4}, {2, 2, 2, 4, 1, 8}};
-static const ConvTile kTiles6[] = {{2, 2, 0, 6, 0}, {1, 4, 0, 6, 0}, {1, 2, 0, 6, 0},
+static constexpr ConvTile kTiles6[] = {{2, 2, 0, 6, 0}, {1, 4, 0, 6, 0}, {1, 2, 0, 6, 0},
                                    {2, 4, 1, 2, 0}, {2, 2, 1, 2, 3}, {2, 2, 2, 2, 2, 4}, {2, 1, 2, 2, 2, 8}};
-static const ConvTile kTiles8[] = {{1, 2, 0, 8, 0}, {2, 2, 0, 8, 0}, {1, 4, 0, 8, 0},   {2, 2, 1, 4, 0},
+static constexpr ConvTile kTiles8[] = {{1, 2, 0, 8, 0}, {2, 2, 0, 8, 0}, {1, 4, 0, 8, 0},   {2, 2, 1, 4, 0},
                                    {1, 2, 1, 4, 3}, {2, 2, 1, 4, 2}, {2, 2, 2, 4, 1, 4}, {2, 2, 2, 4, 1, 8}};
-static const ConvTile kTiles12[] = {{1, 2, 0, 12, 0}, {2, 1, 0, 12, 0},   {2, 2, 1, 4, 0},
+static constexpr ConvTile kTiles12[] = {{1, 2, 0, 12, 0}, {2, 1, 0, 12, 0},   {2, 2, 1, 4, 0},
                                     {1, 2, 1, 4, 3},  {2, 2, 2, 4, 1, 4}, {2, 2, 2, 4, 1, 8}};
 
 static const ConvTile *conv_tiles(int mb, int *count) {
@@ -1896,21 +1896,37 @@ static const ConvTile *conv_tiles(int mb, int *count) {
 // where they fill the chip, below that the LDS tiles with the most workgroups: a pass with
 // them takes 1.00 to 1.02 times the autotuned one from 16 x 16 to 2560 x 1440 (1.10 at 2 x 512 x 512); with the
 // tables' first entries 1280 x 720 took 523 us instead of 274 and 2560 x 1440 1746 instead of 941.
+// (Named by their shapes, which must be in the tables: an index would follow another tile's insertion.)
+template <size_t N> constexpr int tile_index(const ConvTile (&tiles)[N], const ConvTile &t) {
+  for (size_t i = 0; i < N; i++)
+    if (tiles[i].r == t.r && tiles[i].pb == t.pb && tiles[i].lds == t.lds && tiles[i].mbw == t.mbw &&
+        tiles[i].per_cu == t.per_cu && tiles[i].nw == t.nw)
+      return (int)i;
+  return -1;
+}
 int conv3x3_default_tile(int cout, long pixels) {
+  constexpr int dma2 = tile_index(kTiles2, {2, 2, 2, 2, 2, 4});
+  constexpr int lds4 = tile_index(kTiles4, {1, 2, 1, 4, 3}), dma4 = tile_index(kTiles4, {2, 2, 2, 4, 1, 4}),
+                wide4 = tile_index(kTiles4, {2, 2, 2, 4, 1, 8});
+  constexpr int lds6 = tile_index(kTiles6, {2, 2, 1, 2, 3}), dma6 = tile_index(kTiles6, {2, 1, 2, 2, 2, 8});
+  constexpr int lds8 = tile_index(kTiles8, {1, 2, 1, 4, 3}), wide8 = tile_index(kTiles8, {2, 2, 2, 4, 1, 8});
+  constexpr int dma12 = tile_index(kTiles12, {2, 2, 2, 4, 1, 4}), wide12 = tile_index(kTiles12, {2, 2, 2, 4, 1, 8});
+  static_assert(dma2 >= 0 && lds4 >= 0 && dma4 >= 0 && wide4 >= 0 && lds6 >= 0 && dma6 >= 0 && lds8 >= 0 &&
+                    wide8 >= 0 && dma12 >= 0 && wide12 >= 0,
+                "not in its table");
   switch (cout) {
-    case 32: return 10;
-    case 64: return pixels >= 200000 ? 12 : pixels >= 40000 ? 11 : 8;
-    case 96: return pixels >= 200000 ? 6 : 4;
-    case 128: return pixels >= 40000 ? 7 : 4;
-    case 192: return pixels >= 40000 ? 5 : 4;
+    case 32: return dma2;
+    case 64: return pixels >= 200000 ? wide4 : pixels >= 40000 ? dma4 : lds4;
+    case 96: return pixels >= 200000 ? dma6 : lds6;
+    case 128: return pixels >= 40000 ? wide8 : lds8;
+    case 192: return pixels >= 40000 ? wide12 : dma12;
     default: return 0;
   }
 }
 
 int conv3x3_head_tile() {
-  const int n = (int)(sizeof(kTiles2) / sizeof(kTiles2[0]));
-  int t = 0;
-  while (t + 1 < n && kTiles2[t].lds != 2) t++;
+  constexpr int t = tile_index(kTiles2, {2, 2, 2, 2, 2, 4});
+  static_assert(t >= 0, "not in its table");
   return t;
 }
 
