@@ -68,11 +68,12 @@ LGX_D void bilat_rows(int lo, int hi, const float4 *geo, const float4 *col, int 
 
 // A workgroup filters 32 x 8R pixels, a thread R pixels of one column, whose
 // windows overlap in all but R - 1 of their rows: a tap read from LDS serves
-// up to R outputs.  Bound by VALU issue (94 % of the slots that this mix of
-// instructions has, by counters): 14 instructions a tap with one exp2 (20 and
-// their scalar operands before), about 190 a pixel for staging and the
-// quotients.  More outputs a thread read less LDS and lose as much
-// to the fewer workgroups that fit it.  2560x1440, r = 4: 133 -> 95 us a call.
+// up to R outputs.  Bound by VALU issue (1.19 instructions a CU-cycle by
+// counters; the taps' mix alone can reach 1.37): 14 instructions a tap with
+// one exp2 (20 and their scalar operands before), about 330 a pixel for
+// staging and the quotients.  More outputs a thread read less LDS and lose as
+// much to the fewer workgroups that fit it.  2560x1440, r = 4: 133 -> 94 us a
+// call.
 template <int NFMT, int R> __global__ __launch_bounds__(256) void bilateral_kernel(const BilatArgs a) {
   extern __shared__ __align__(16) float4 s_bilat[];
   const int r = a.r, n = 2 * r;
@@ -105,17 +106,26 @@ template <int NFMT, int R> __global__ __launch_bounds__(256) void bilateral_kern
       nt[u] = make_float2(t.x, t.y);
       d[u] = *(const float *)(b_d + (row * (uint32_t)a.depth_pitch + gx) * 4u);
     }
+    // (a normal whose squared length overflows: uniform, no wave of unit normals goes there)
+    float longest = 0.f;
 #pragma unroll
-    for (int u = 0; u < 4; u++) {
-      const int i = i0 + u * 256;
-      if (i < total) {
-        Vec3<float> nv = oct_decode_dev<float>(nt[u].x, nt[u].y);
-        // (a length whose square overflows: uniform, no wave of unit normals goes there)
-        if (__builtin_amdgcn_ballot_w64(fabsf(nt[u].x) + fabsf(nt[u].y) > 1e18f)) nv = oct_decode<float>(nt[u].x, nt[u].y);
-        s_geo[i] = make_float4(d[u], nv.x, nv.y, nv.z);
-        s_col[i] = make_float4(c[u].x, c[u].y, c[u].z, 1.0f);
+    for (int u = 0; u < 4; u++) longest = fmaxf(longest, fabsf(nt[u].x) + fabsf(nt[u].y));
+    const bool ieee = __builtin_amdgcn_ballot_w64(longest > 1e18f) != 0;
+    auto stage = [&](auto decode) {
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        const int i = i0 + u * 256;
+        if (i < total) {
+          const Vec3<float> nv = decode(nt[u].x, nt[u].y);
+          s_geo[i] = make_float4(d[u], nv.x, nv.y, nv.z);
+          s_col[i] = make_float4(c[u].x, c[u].y, c[u].z, 1.0f);
+        }
       }
-    }
+    };
+    if (ieee)
+      stage([](float x, float y) { return oct_decode<float>(x, y); });
+    else
+      stage([](float x, float y) { return oct_decode_dev<float>(x, y); });
   }
   __syncthreads();
   const int tx = threadIdx.x % TW, ty = threadIdx.x / TW * R;
@@ -135,8 +145,8 @@ template <int NFMT, int R> __global__ __launch_bounds__(256) void bilateral_kern
 #pragma unroll
   for (int k = 0; k < R; k++) {
     if (py + k >= a.h) break;
-    // IEEE quotients: an infinite sum stays infinite (2560x1440, r = 4: 95.1 us a call,
-    // 93.7 with one reciprocal and its corrections, which are NaN there)
+    // IEEE quotients: an infinite sum stays infinite (1.4 us of the 94 at 2560x1440, r = 4, over one reciprocal and
+    // its corrections, which give NaN there)
     const float sum = acc[k].w + 1e-7f;
     a.out[(size_t)(py + k) * a.out_pitch + px] = make_float4(acc[k].x / sum, acc[k].y / sum, acc[k].z / sum, 1.0f);
   }
@@ -236,8 +246,8 @@ extern "C" int lgx_bilateral(const lgx_bilateral_params *p, const lgx_image *in,
   };
   const bool h16 = g->normal.format == LGX_RG16F;
   // Two outputs a thread once their 4096 tiles of 32 x 16 keep every CU's five
-  // workgroups busy for a few rounds (2560x1440, r = 4: 87 against 91 us for
-  // one output; 1279x719, r = 3: 20 against 19 us).
+  // workgroups busy for a few rounds (2560x1440, r = 4: 96 against 101 us a
+  // call for one output; 1279x719, r = 3: 23.5 against 20.8 us).
   if ((int64_t)in->w * in->h >= (int64_t)4096 * 512)
     return h16 ? launch(bilateral_kernel<LGX_RG16F, 2>, 2) : launch(bilateral_kernel<LGX_RG32F, 2>, 2);
   return h16 ? launch(bilateral_kernel<LGX_RG16F, 1>, 1) : launch(bilateral_kernel<LGX_RG32F, 1>, 1);
