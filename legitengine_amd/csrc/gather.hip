@@ -230,10 +230,10 @@ LGX_D Vec3<Quad<T>> radiance_quad(const void *base, int pitch, int lw, int lh, c
                        {T(t[0].y), T(t[1].y), T(t[2].y), T(t[3].y)},
                        {T(t[0].z), T(t[1].z), T(t[2].z), T(t[3].z)}};
 }
-// The trilinear march is bound by VALU issue as well: about 105 instructions a
-// step (130 with 64-bit addresses, IEEE divisions, four clamped single-texel
-// fetches and a select each, 175 at first), 190 a hit.  1080p, 4 directions:
-// 381 -> 270 us.
+// The trilinear march is bound by VALU issue as well: about 107 instructions a
+// step (130 with 64-bit addresses, four clamped single-texel fetches and a
+// select each, 175 at first), the library's arc tangent and two divisions a
+// hit.  1080p, 4 directions, under the profiler: 387 -> 312 us.
 // The levels and blend of a step's lod (uniform): clamped to the pyramid, NaN
 // and -inf to level 0.
 template <class T> struct Trilinear {
@@ -261,8 +261,8 @@ template <class T> struct Trilinear {
 // products, anything with a scalar operand) once, a root or reciprocal every
 // other: a step is 27 instructions, about 19 slots (41 and 29 with a step
 // count, four border tests, clamped texels and scalar operands), a
-// direction's set-up 276 instead of 430.  1080p, 32 directions: 2.69 -> 2.25
-// ms; 4 directions of 256: 2.45 -> 2.00 ms.
+// direction's set-up about 280 instead of 430.  1080p, 32 directions: 2.69 ->
+// 2.25 ms; 4 directions of 256: 2.45 -> 2.00 ms.
 // One wave per pixel block and all its directions left 1024 waves (one per SIMD) for a 256 x 256 image: 153 us
 // there with 16 directions, 57 us with the directions over 8 waves; at 1080p
 // with 32 directions 2.90 -> 2.69 ms (a shorter tail).
@@ -380,12 +380,26 @@ LGX_D void gather_block(ARGS &a, const uint32_t b, A *part) {
     };
     // the offset of step s (a scalar load); past the table no lane goes on
     auto offset = [&](int s) { return s < a.S_tab ? steps[2 * s] : T(INFINITY); };
-    // The steps below an offset limit (march_limit).  FP64 sums resolve a step
-    // at the far border: they keep the border and the texel's clamp, as do the
-    // trilinear taps.
-    constexpr bool kClamp = sizeof(A) == 8 || SAMPLER != LGX_SAMPLER_HIZ_POINT;
-    T lim = march_limit(path, a.near_step, a.near_min, steps[0], offset(1));
+    // FP32 sums take the steps below an offset limit (march_limit), which may
+    // have another step within rounding of the border or of the step count's
+    // end than the shader's rule; FP64 sums resolve such a step (4e-8 of a
+    // 256-direction crop with a row of pixels at such a place) and keep the
+    // rule itself, four compares and a count a step: 256 x 256, 256
+    // directions 4.95 -> 5.33 ms.
+    constexpr bool kRule = sizeof(A) == 8;
+    constexpr bool kClamp = kRule || SAMPLER != LGX_SAMPLER_HIZ_POINT;
+    T lim = T(0);
+    if (!kRule) lim = march_limit(path, a.near_step, a.near_min, steps[0], offset(1));
     if (!kClamp) lim = inside_far(lim, cx, cy, a.W, a.H, dx, dy, idx, idy);
+    const int iters = kRule || COUNT ? min((int)(log(path / a.near_step) / a.log_ratio) + 1, a.S_tab) : 0;  // :212
+    // What every step reads: in vector registers, since an FP32 multiply,
+    // add or FMA issues at twice the rate without a scalar operand.
+    const T vdx = vec(dx), vdy = vec(dy);
+    // whether step j at offset o, position q, is taken (bitwise: one mask, not a chain of branches)
+    auto taken = [&](int j, T o, T qx, T qy) {
+      if constexpr (kRule) return (j < iters) & (qx > T(0)) & (qx < vW) & (qy > T(0)) & (qy < vH);
+      else return o < lim;
+    };
     int marched = 0;  // COUNT: steps taken
     if (SAMPLER == LGX_SAMPLER_HIZ_POINT) {
       // Level-major march.  The step index j is the same on every active
@@ -428,20 +442,20 @@ LGX_D void gather_block(ARGS &a, const uint32_t b, A *part) {
         if constexpr (SWZ) return (int)(__umul24((unsigned)(ix & smask), (unsigned)ssw) + (unsigned)(ix >> sshift));
         return ix;
       };
-      // What every step reads: in vector registers, since an FP32 multiply,
-      // add or FMA issues at twice the rate without a scalar operand.
-      const T vdx = vec(dx), vdy = vec(dy);
       // the fetch at offset o on the current level: q / extent, texel
       // position, depth request
       struct Fetch {
         float rd;
         T sqx, sqy;
         int ix, iy;
+        bool on;  // the step is taken
       };
-      auto request = [&](T o) {
+      auto request = [&](int j, T o) {
         Fetch f;
-        f.sqx = div_extent(cx + vdx * o, vW, vrW);  // :218-219
-        f.sqy = div_extent(cy + vdy * o, vH, vrH);
+        const T qx = cx + vdx * o, qy = cy + vdy * o;  // :218-219
+        f.on = taken(j, o, qx, qy);
+        f.sqx = div_extent(qx, vW, vrW);
+        f.sqy = div_extent(qy, vH, vrH);
         // truncation is floor: a step of the march is at most rounding below 0
         f.ix = (int)(f.sqx * flw);
         f.iy = (int)(f.sqy * flh);
@@ -475,8 +489,8 @@ LGX_D void gather_block(ARGS &a, const uint32_t b, A *part) {
       to_level(0);
       if constexpr (PIPE) {
         T off_n = offset(1);
-        Fetch f = request(off);
-        for (int j = 0; off < lim; j++) {
+        Fetch f = request(0, off);
+        for (int j = 0; f.on; j++) {
           // step j: :241-252 sample delta projected on (eye, tangent)
           const T r = T(f.rd);
           const T len2 = fma_(off, fma_(off, vv, uv2), uu);
@@ -491,14 +505,16 @@ LGX_D void gather_block(ARGS &a, const uint32_t b, A *part) {
           off = off_n;
           off_n = offset(j + 2);
           to_level(j + 1);
-          f = request(off);
+          f = request(j + 1, off);
           if (hit) raise(hyv, hxv, sqx, sqy, [&]() { return RadBuf<RFMT>::decode(rv); });
         }
       } else {
-        for (int j = 0; off < lim; j++) {
+        for (int j = 0;; j++) {
+          if (!kRule && !(off < lim)) break;
           const T off_next = offset(j + 1);
           to_level(j);
-          const Fetch f = request(off);
+          const Fetch f = request(j, off);
+          if (kRule && !f.on) break;
           if (COUNT) marched++;
           // :241-252 sample delta projected on (eye, tangent)
           const T len2 = fma_(off, fma_(off, vv, uv2), uu);
@@ -512,12 +528,12 @@ LGX_D void gather_block(ARGS &a, const uint32_t b, A *part) {
         }
       }
     } else {
-      const T vdx = vec(dx), vdy = vec(dy);
       for (int j = 0; j < a.S_tab; j++) {
         const T off = vec(steps[2 * j]), lod = steps[2 * j + 1];
-        if (!(off < lim)) break;
+        const T qx = cx + vdx * off, qy = cy + vdy * off;  // :218-219
+        if (!taken(j, off, qx, qy)) break;
         if (COUNT) marched++;
-        const T sqx = div_extent(cx + vdx * off, vW, vrW), sqy = div_extent(cy + vdy * off, vH, vrH);  // :218-219
+        const T sqx = div_extent(qx, vW, vrW), sqy = div_extent(qy, vH, vrH);
         const Trilinear<T> tl(a, lod);
         const int l0 = tl.l0, l1 = tl.l1;
         const TapPos<T> p0(sqx, sqy, a.lw[l0], a.lh[l0]), p1(sqx, sqy, a.lw[l1], a.lh[l1]);
@@ -571,7 +587,6 @@ LGX_D void gather_block(ARGS &a, const uint32_t b, A *part) {
       // The steps taken, but those in the border's fringe (2^-19 of the extent, a fade below 2e-5) or within
       // rounding of the step count's end as the shader's own rule has them: it may admit them and the limit
       // not, or the other way round.
-      const int iters = min((int)(log(path / a.near_step) / a.log_ratio) + 1, a.S_tab);
       int rule = 0;
       for (; rule < iters; rule++) {
         const T qx = cx + dx * steps[2 * rule], qy = cy + dy * steps[2 * rule];
@@ -976,9 +991,9 @@ template <class T, class A, int SAMPLER, int RFMT, int NFMT>
 static hipError_t launch_gather(const GatherArgs<T> &a, bool count, hipStream_t s) {
   // The FP32 Hi-Z gather has every variant; the others run one.  FP32 steps
   // with FP64 sums: registers for 8 waves per SIMD and the pipelined loop
-  // (256x256 crop, 256 directions: 4.07 ms; 4.13 with the plain loop, 4.86
-  // with the compiler's 99 registers).  Trilinear: 6 waves (1080p, 4
-  // directions: 270 us; 284 at 5, 287 at 8 with spills).
+  // (256x256 crop, 256 directions, with the offset limit: 4.07 ms; 4.13 with the
+  // plain loop, 4.86 with the compiler's 99 registers).  Trilinear: 6 waves (1080p, 4
+  // directions, under the profiler: 312 us; 356 at 4, 334 at 5, 324 at 7).
   constexpr bool kAll = sizeof(T) == 4 && sizeof(A) == 4 && SAMPLER == LGX_SAMPLER_HIZ_POINT;
   constexpr bool kAcc = sizeof(T) == 4 && sizeof(A) == 8 && SAMPLER == LGX_SAMPLER_HIZ_POINT;
   auto launch = [&](auto kern) {
