@@ -193,50 +193,26 @@ template <class T, class ARGS> LGX_D Vec3<T> unproject_far(ARGS &a, T sx, T sy) 
   return Vec3<T>{div_by(vx, vw, rw), div_by(vy, vw, rw), div_by(vz, vw, rw)};
 }
 
-// The texels of a tap position: one fetch per row where the level has a pair
-// of columns (uniform).
-template <class T> LGX_D Quad<T> depth_quad(const float *base, int pitch, int lw, int lh, const TapPos<T> &p) {
+template <class T> LGX_D T depth_taps(const float *base, int pitch, int lh, const TapPos<T> &p) {
   const i32x4 r = level_rsrc(base, 4, lh * pitch);
-  const uint32_t a = texel_index(p.y, pitch, p.x), b = a + (lh > 1 ? (uint32_t)pitch : 0u);
-  f32x2 t, q;
-  if (lw > 1) {
-    t = struct_load_f32x2(r, (int)a, 0, 0, 0);
-    q = struct_load_f32x2(r, (int)b, 0, 0, 0);
-  } else {
-    t = load_depth(r, a);
-    q = load_depth(r, b);
-  }
-  return Quad<T>{T(t.x), T(t.y), T(q.x), T(q.y)};
+  const float t00 = load_depth(r, texel_index(p.y0, pitch, p.x0)), t10 = load_depth(r, texel_index(p.y0, pitch, p.x1));
+  const float t01 = load_depth(r, texel_index(p.y1, pitch, p.x0)), t11 = load_depth(r, texel_index(p.y1, pitch, p.x1));
+  return p.mix(T(t00), T(t10), T(t01), T(t11));
 }
-template <class T, int FMT>
-LGX_D Vec3<Quad<T>> radiance_quad(const void *base, int pitch, int lw, int lh, const TapPos<T> &p) {
+template <class T, int FMT> LGX_D Vec3<T> radiance_taps(const void *base, int pitch, int lh, const TapPos<T> &p) {
   typedef RadBuf<FMT> B;
   const i32x4 r = level_rsrc(base, B::kBytes, lh * pitch);
-  const uint32_t at = texel_index(p.y, pitch, p.x), down = lh > 1 ? (uint32_t)pitch : 0u;
-  float4 t[4];  // (x, y), (x + 1, y), (x, y + 1), (x + 1, y + 1)
-#pragma unroll
-  for (int row = 0; row < 2; row++) {
-    const uint32_t i = at + (row ? down : 0u);
-    typename B::Raw lo, hi;
-    if (FMT == LGX_RGBA16F && lw > 1) {
-      const f32x4 v = struct_load_f32x4(r, (int)i, 0, 0, 0);
-      __builtin_memcpy(&lo, &v, 8);
-      __builtin_memcpy(&hi, (const char *)&v + 8, 8);
-    } else {
-      lo = B::raw(r, i);
-      hi = lw > 1 ? B::raw(r, i + 1) : lo;
-    }
-    t[2 * row] = B::decode(lo);
-    t[2 * row + 1] = B::decode(hi);
-  }
-  return Vec3<Quad<T>>{{T(t[0].x), T(t[1].x), T(t[2].x), T(t[3].x)},
-                       {T(t[0].y), T(t[1].y), T(t[2].y), T(t[3].y)},
-                       {T(t[0].z), T(t[1].z), T(t[2].z), T(t[3].z)}};
+  const typename B::Raw r00 = B::raw(r, texel_index(p.y0, pitch, p.x0)), r10 = B::raw(r, texel_index(p.y0, pitch, p.x1)),
+                        r01 = B::raw(r, texel_index(p.y1, pitch, p.x0)), r11 = B::raw(r, texel_index(p.y1, pitch, p.x1));
+  const float4 a = B::decode(r00), b = B::decode(r10), c = B::decode(r01), d = B::decode(r11);
+  return Vec3<T>{p.mix(T(a.x), T(b.x), T(c.x), T(d.x)), p.mix(T(a.y), T(b.y), T(c.y), T(d.y)),
+                 p.mix(T(a.z), T(b.z), T(c.z), T(d.z))};
 }
-// The trilinear march is bound by VALU issue as well: about 107 instructions a
-// step (130 with 64-bit addresses, four clamped single-texel fetches and a
-// select each, 175 at first), the library's arc tangent and two divisions a
-// hit.  1080p, 4 directions, under the profiler: 387 -> 312 us.
+// The trilinear march is bound by VALU issue as well: eight fetches, seven
+// blends of four instructions and the taps' positions a step, the library's
+// arc tangent and two divisions a hit.  Structured fetches (no 64-bit
+// addresses), the step's invariants in vector registers and registers for 6
+// waves per SIMD: 1080p frame with 4 directions 510 -> 426 us.
 // The levels and blend of a step's lod (uniform): clamped to the pyramid, NaN
 // and -inf to level 0.
 template <class T> struct Trilinear {
@@ -361,7 +337,7 @@ LGX_D void gather_block(ARGS &a, const uint32_t b, A *part) {
     // :254-263 a sample above the horizon: radiance v (raw), weights, new maximum
     auto raise = [&](T hyv, T hxv, T sqx, T sqy, auto v_of) {
       if (COUNT) hit_total++;
-      // (the trilinear mode: the library's arc tangent and IEEE quotients, 1080p with 4 directions 397 -> 415 us a frame)
+      // (the trilinear mode: the library's arc tangent and IEEE quotients, 18 us of a 1080p frame with 4 directions)
       T th, c2, s2;
       slice_angle<SAMPLER == LGX_SAMPLER_TRILINEAR>(hyv, hxv, th, c2, s2);
       // :222-227 the four ramps; of two opposite ones at most one is below 1
@@ -383,14 +359,15 @@ LGX_D void gather_block(ARGS &a, const uint32_t b, A *part) {
     };
     // the offset of step s (a scalar load); past the table no lane goes on
     auto offset = [&](int s) { return s < a.S_tab ? steps[2 * s] : T(INFINITY); };
-    // FP32 sums take the steps below an offset limit (march_limit), which may
-    // have another step within rounding of the border or of the step count's
-    // end than the shader's rule; FP64 sums resolve such a step (4e-8 of a
-    // 256-direction crop with a row of pixels at such a place) and keep the
+    // FP32 sums of the Hi-Z sampler take the steps below an offset limit
+    // (march_limit), which may have another step within rounding of the border
+    // or of the step count's end than the shader's rule; FP64 sums resolve
+    // such a step (4e-8 of a 256-direction crop with a row of pixels at such a
+    // place), the trilinear sampler's hit counts show it, and both keep the
     // rule itself, four compares and a count a step: 256 x 256, 256
-    // directions 4.95 -> 5.33 ms.
-    constexpr bool kRule = sizeof(A) == 8;
-    constexpr bool kClamp = kRule || SAMPLER != LGX_SAMPLER_HIZ_POINT;
+    // directions, FP64 sums 4.95 -> 5.33 ms.
+    constexpr bool kRule = sizeof(A) == 8 || SAMPLER == LGX_SAMPLER_TRILINEAR;
+    constexpr bool kClamp = kRule;
     T lim = T(0);
     if (!kRule) lim = march_limit(path, a.near_step, a.near_min, steps[0], offset(1));
     if (!kClamp) lim = inside_far(lim, cx, cy, a.W, a.H, dx, dy, idx, idy);
@@ -540,47 +517,19 @@ LGX_D void gather_block(ARGS &a, const uint32_t b, A *part) {
         const Trilinear<T> tl(a, lod);
         const int l0 = tl.l0, l1 = tl.l1;
         const TapPos<T> p0(sqx, sqy, a.lw[l0], a.lh[l0]), p1(sqx, sqy, a.lw[l1], a.lh[l1]);
-        auto depth_at = [&](int l, const TapPos<T> &p) { return depth_quad(a.pd[l], a.pd_pitch[l], a.lw[l], a.lh[l], p); };
-        auto radiance_at = [&](int l, const TapPos<T> &p) {
-          return radiance_quad<T, RFMT>(a.pr[l], a.pr_pitch[l], a.lw[l], a.lh[l], p);
-        };
-        // A sample that is not finite has an infinite texel among its taps: fetched again, for nothing is kept for
-        // it (24 more spilled registers otherwise), and blended tap by tap.
-        auto depth_again = [&](int l) {
-          const T ux = opaque(sqx), uy = opaque(sqy);
-          const int lw = a.lw[l], lh = a.lh[l];
-          return clamped_taps(ux, uy, lw, lh, depth_at(l, TapPos<T>(ux, uy, lw, lh)));
-        };
-        auto radiance_again = [&](int l) {
-          const T ux = opaque(sqx), uy = opaque(sqy);
-          const int lw = a.lw[l], lh = a.lh[l];
-          const Vec3<Quad<T>> q = radiance_at(l, TapPos<T>(ux, uy, lw, lh));
-          return Vec3<T>{clamped_taps(ux, uy, lw, lh, q.x), clamped_taps(ux, uy, lw, lh, q.y),
-                         clamped_taps(ux, uy, lw, lh, q.z)};
-        };
-        T r = p0.mix(depth_at(l0, p0));
-        if (tl.blend) r = TapPos<T>::lerp(tl.f, r, p1.mix(depth_at(l1, p1)));
-        if (!finite_tap(r)) {
-          r = depth_again(l0);
-          if (tl.blend) r = r * (T(1) - tl.f) + depth_again(l1) * tl.f;
-        }
+        T r = depth_taps(a.pd[l0], a.pd_pitch[l0], a.lh[l0], p0);
+        if (tl.blend) r = TapPos<T>::lerp(tl.f, r, depth_taps(a.pd[l1], a.pd_pitch[l1], a.lh[l1], p1));
         // :241-252 sample delta projected on (eye, tangent)
         const T len2 = fma_(off, fma_(off, vv, uv2), uu);
         const T ri = r * fast_rsqrt(len2);
-        const T hyv = fma_(ri, fma_(off, tv, tu), -trc);
-        const T hxv = fma_(ri, fma_(off, ev, eu), -erc);
+        const T hyv = ri * fma_(off, tv, tu) - trc;
+        const T hxv = ri * fma_(off, ev, eu) - erc;
         if (hm.below(hyv, hxv))  // :254
           raise(hyv, hxv, sqx, sqy, [&]() {  // :256
-            const Vec3<Quad<T>> q0 = radiance_at(l0, p0);
-            Vec3<T> v{p0.mix(q0.x), p0.mix(q0.y), p0.mix(q0.z)};
+            Vec3<T> v = radiance_taps<T, RFMT>(a.pr[l0], a.pr_pitch[l0], a.lh[l0], p0);
             if (tl.blend) {
-              const Vec3<Quad<T>> q1 = radiance_at(l1, p1);
-              v = Vec3<T>{TapPos<T>::lerp(tl.f, v.x, p1.mix(q1.x)), TapPos<T>::lerp(tl.f, v.y, p1.mix(q1.y)),
-                          TapPos<T>::lerp(tl.f, v.z, p1.mix(q1.z))};
-            }
-            if (!finite_tap(v.x + v.y + v.z)) {
-              v = radiance_again(l0);
-              if (tl.blend) v = v * (T(1) - tl.f) + radiance_again(l1) * tl.f;
+              const Vec3<T> w = radiance_taps<T, RFMT>(a.pr[l1], a.pr_pitch[l1], a.lh[l1], p1);
+              v = Vec3<T>{TapPos<T>::lerp(tl.f, v.x, w.x), TapPos<T>::lerp(tl.f, v.y, w.y), TapPos<T>::lerp(tl.f, v.z, w.z)};
             }
             return v;
           });
@@ -996,7 +945,7 @@ static hipError_t launch_gather(const GatherArgs<T> &a, bool count, hipStream_t 
   // with FP64 sums: registers for 8 waves per SIMD and the pipelined loop
   // (256x256 crop, 256 directions, with the offset limit: 4.07 ms; 4.13 with the
   // plain loop, 4.86 with the compiler's 99 registers).  Trilinear: 6 waves (1080p, 4
-  // directions, under the profiler: 312 us; 356 at 4, 334 at 5, 324 at 7).
+  // directions, under the profiler: 330 to 334 us at 4 to 7, 357 at 8).
   constexpr bool kAll = sizeof(T) == 4 && sizeof(A) == 4 && SAMPLER == LGX_SAMPLER_HIZ_POINT;
   constexpr bool kAcc = sizeof(T) == 4 && sizeof(A) == 8 && SAMPLER == LGX_SAMPLER_HIZ_POINT;
   auto launch = [&](auto kern) {
