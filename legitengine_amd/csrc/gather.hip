@@ -336,7 +336,6 @@ LGX_D void gather_block(ARGS &a, const uint32_t b, A *part) {
     const T trc = rc * dot3(tangent, rayc);
     // :254-263 a sample above the horizon: radiance v (raw), weights, new maximum
     auto raise = [&](T hyv, T hxv, T sqx, T sqy, auto v_of) {
-      if (COUNT) hit_total++;
       // (the trilinear mode: the library's arc tangent and IEEE quotients, 18 us of a 1080p frame with 4 directions)
       T th, c2, s2;
       slice_angle<SAMPLER == LGX_SAMPLER_TRILINEAR>(hyv, hxv, th, c2, s2);
@@ -367,17 +366,20 @@ LGX_D void gather_block(ARGS &a, const uint32_t b, A *part) {
     // rule itself, four compares and a count a step: 256 x 256, 256
     // directions, FP64 sums 4.95 -> 5.33 ms.
     constexpr bool kRule = sizeof(A) == 8 || SAMPLER == LGX_SAMPLER_TRILINEAR;
-    constexpr bool kClamp = kRule;
+    constexpr bool kClamp = kRule || COUNT;
     T lim = T(0);
     if (!kRule) lim = march_limit(path, a.near_step, a.near_min, steps[0], offset(1));
-    if (!kClamp) lim = inside_far(lim, cx, cy, a.W, a.H, dx, dy, idx, idy);
+    if (!kRule) lim = inside_far(lim, cx, cy, a.W, a.H, dx, dy, idx, idy);
     const int iters = kRule || COUNT ? min((int)(log(path / a.near_step) / a.log_ratio) + 1, a.S_tab) : 0;  // :212
     // What every step reads: in vector registers, since an FP32 multiply,
     // add or FMA issues at twice the rate without a scalar operand.
     const T vdx = vec(dx), vdy = vec(dy);
-    // whether step j at offset o, position q, is taken (bitwise: one mask, not a chain of branches)
+    // whether the rule has step j, at position q (bitwise: one mask, not a chain of branches), and whether it is taken
+    auto ruled = [&](int j, T qx, T qy) {
+      return (j < iters) & (qx > T(0)) & (qx < vW) & (qy > T(0)) & (qy < vH);
+    };
     auto taken = [&](int j, T o, T qx, T qy) {
-      if constexpr (kRule) return (j < iters) & (qx > T(0)) & (qx < vW) & (qy > T(0)) & (qy < vH);
+      if constexpr (kRule) return ruled(j, qx, qy);
       else return o < lim;
     };
     int marched = 0;  // COUNT: steps taken
@@ -490,20 +492,29 @@ LGX_D void gather_block(ARGS &a, const uint32_t b, A *part) {
         }
       } else {
         for (int j = 0;; j++) {
-          if (!kRule && !(off < lim)) break;
+          if (!kRule && !COUNT && !(off < lim)) break;
           const T off_next = offset(j + 1);
           to_level(j);
           const Fetch f = request(j, off);
           if (kRule && !f.on) break;
-          if (COUNT) marched++;
+          // COUNT: also the steps that only the rule has, for its count of hits
+          bool rule = true;
+          if (COUNT) {
+            rule = ruled(j, cx + vdx * off, cy + vdy * off);
+            if (!(rule | f.on)) break;
+            marched += f.on;
+          }
           // :241-252 sample delta projected on (eye, tangent)
           const T len2 = fma_(off, fma_(off, vv, uv2), uu);
           const T ri = T(f.rd) * fast_rsqrt(len2);
           const T hyv = fma_(ri, fma_(off, tv, tu), -trc);
           const T hxv = fma_(ri, fma_(off, ev, eu), -erc);
-          if (hm.below(hyv, hxv))  // :254
-            raise(hyv, hxv, f.sqx, f.sqy,
-                  [&]() { return RadBuf<RFMT>::decode(RadBuf<RFMT>::raw(rrs, texel_index(f.iy, rpitch, f.ix))); });  // :256
+          if (hm.below(hyv, hxv)) {  // :254
+            if (COUNT) hit_total += rule;
+            if (!COUNT || f.on)
+              raise(hyv, hxv, f.sqx, f.sqy,
+                    [&]() { return RadBuf<RFMT>::decode(RadBuf<RFMT>::raw(rrs, texel_index(f.iy, rpitch, f.ix))); });  // :256
+          }
           off = off_next;
         }
       }
@@ -524,7 +535,8 @@ LGX_D void gather_block(ARGS &a, const uint32_t b, A *part) {
         const T ri = r * fast_rsqrt(len2);
         const T hyv = ri * fma_(off, tv, tu) - trc;
         const T hxv = ri * fma_(off, ev, eu) - erc;
-        if (hm.below(hyv, hxv))  // :254
+        if (hm.below(hyv, hxv)) {  // :254
+          if (COUNT) hit_total++;
           raise(hyv, hxv, sqx, sqy, [&]() {  // :256
             Vec3<T> v = radiance_taps<T, RFMT>(a.pr[l0], a.pr_pitch[l0], a.lh[l0], p0);
             if (tl.blend) {
@@ -533,6 +545,7 @@ LGX_D void gather_block(ARGS &a, const uint32_t b, A *part) {
             }
             return v;
           });
+        }
       }
     }
     if (COUNT) {
@@ -1111,7 +1124,7 @@ static int64_t launch_pixels(const lgx_gather_params *p) {
 //   1920x1080, 4 directions of 256 (32 K)            2005 / 1999 / 2077
 // The trilinear march has a handful of steps a direction, so a direction is
 // mostly set-up and nothing but an idle chip makes a split worth while:
-//   480x270 / 1280x720 / 1920x1080, 4 directions     47, 32, 28 / 136, 130, 141 / 271, 278, 323
+//   480x270 / 1280x720 / 1920x1080, 4 directions     52, 39, 34 / 152, 147, 153 / 287, 296, 321
 static int split_waves(int64_t pixels, int dirs, int sampler, int precision) {
   const int64_t full = 8192, waves = (pixels + 63) / 64;
   if (sampler == LGX_SAMPLER_TRILINEAR && dirs < 16) {
