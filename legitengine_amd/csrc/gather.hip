@@ -238,10 +238,10 @@ template <class T> struct Trilinear {
 // waves hide.  An FP32 multiply, add or FMA on vector registers issues twice
 // a CU-cycle, everything else (compares, conversions, minima, 24-bit
 // products, anything with a scalar operand) once, a root or reciprocal every
-// other: a step is 27 instructions, about 19 slots (41 and 29 with a step
+// other: a step is 28 instructions, about 20 slots (41 and 29 with a step
 // count, four border tests, clamped texels and scalar operands), a
 // direction's set-up about 280 instead of 430.  1080p, 32 directions: 2.69 ->
-// 2.25 ms; 4 directions of 256: 2.45 -> 2.00 ms.
+// 2.28 ms; 4 directions of 256: 2.45 -> 2.04 ms.
 // One wave per pixel block and all its directions left 1024 waves (one per SIMD) for a 256 x 256 image: 153 us
 // there with 16 directions, 57 us with the directions over 8 waves; at 1080p
 // with 32 directions 2.90 -> 2.69 ms (a shorter tail).

@@ -911,8 +911,9 @@ __global__ __launch_bounds__(64 * NW, OCC) void conv3x3_dma_kernel(const ConvArg
         if constexpr (HEAD) {
           // the inference head: each wave's activations (BF16, as the unfused
           // path stores them) through LDS of its own, then a lane per pixel
-          // forms in + b + W act, channel by channel.  1920 x 1080: 75 us, 55
-          // without the head; with 80 bytes a pixel in LDS only one
+          // forms in + b + W act, channel by channel.  1920 x 1080: 65 us, 55
+          // without the head (the residual's read is waited for before the
+          // tile's first MFMA); with 80 bytes a pixel in LDS only one
           // workgroup fits a CU (108), and with the head's weights read
           // from memory per tile, behind the next stage's loads, 118.
           static_assert(!HEAD || (MB == 2 && WR * WP % 4 == 0), "a lane per pixel");
