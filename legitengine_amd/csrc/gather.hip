@@ -284,7 +284,7 @@ LGX_D void gather_block(ARGS &a, const uint32_t b, A *part) {
   // a wave per SIMD.)
   auto radial = [&]() {
     const T v = opaque(rc) * a.unit;
-    return v < T(0x1p-49) ? v * T(0x1p100) : v;
+    return fabs(v) < T(0x1p-49) ? v * T(0x1p100) : v;
   };
   const Vec3<T> P = cam + rayc * radial();  // :130 from the radial distance
   const Vec3<T> eye = normalize3_cr(cam - P);  // :182

@@ -52,7 +52,7 @@ def test_unit_of_length(sampler, exponent):
     assert orc.rel_l2(out, ref) <= 1e-6
 
 
-@pytest.mark.parametrize("sampler,marker", [(HIZ, 1e-15), (TRI, 1e-15), (TRI, 1e-20)])
+@pytest.mark.parametrize("sampler,marker", [(HIZ, 1e-15), (TRI, 1e-15), (TRI, 1e-20), (HIZ, -1.0), (TRI, -1.0)])
 def test_distances_of_next_to_nothing(sampler, marker):
     dev, view, proj, gb = setup()
     for i in (12, 13, 14):
